@@ -13,20 +13,32 @@
 //   tokens exceeds u * (kept mass), u in [0, 1) supplied by the caller (the
 //   inverse of the distribution torch.multinomial draws from).
 //
-// No sort: the k-th largest z and the top-p boundary are found by radix
-// selection over an order-preserving 32-bit key of z, 8 bits per pass, from
-// histograms of token counts (top-k) or of the mass exp(z - max) (top-p), in
-// 2^-40 fixed point, so that every sum is exact and independent of the order
+// No sort.  Both cuts (the k-th largest z, the top-p boundary) are found in
+// two levels.  The row's tokens are counted (top-k) and their masses
+// exp(z - max), in 2^-40 fixed point, added (top-p) in kSampBins equal bins
+// of max - z; a token more than 28 below the maximum has mass 0, so the bins
+// span at most that.  Every sum is an exact integer, independent of the order
 // the atomics land in; top_p is applied to the kept mass as top_p * sum,
-// which is the normalized condition.  Each workgroup builds its histogram in
-// LDS and adds it into the pass's row histogram with device-scope atomics
-// (the first launch zeroes those; top-k's first pass, in that launch, keeps
-// one histogram per workgroup instead).  Every launch reads the row again
-// from L2 (608 KB at V = 151936); a workgroup that needs the outcome of the
-// previous pass re-derives it from that pass's histogram (identical in every
-// workgroup), so no workgroup waits for another.  The first pass of each
-// selection rides on the launch before it (the max pass, the softmax-sum
-// pass).  Rows are independent (grid.y).  Differences from
+// which is the normalized condition.  The bins of the two cuts (or, while the
+// kept mass still depends on the k-th token, the few bins its bounds allow)
+// hold the only undecided tokens: a few hundred of 151936.  They are listed
+// per slice, and one workgroup per row finds the exact keys among them
+// (order-preserving 32-bit keys of z, 256 ranges per step), adds up the
+// slices and draws.  Four launches for any cut: maximum, bins, lists, draw
+// (three without a cut).
+//
+// What bounds it: the launches and the latency of each one's serial chain;
+// the logits (608 KB at V = 151936) are read from L2 three times.  Measured
+// in a HIP graph at V = 151936, against one launch per 8 key bits of each cut
+// over the whole row (7 launches with top-p, 10 with top-k as well): one row,
+// top-p 32.5 -> 18.4 us, top-k and top-p 49.5 -> 23.1, top-k 30.3 -> 16.8, no
+// cut 12.6 -> 10.7; eight rows, both cuts 63.6 -> 27.1.  Per launch at one
+// row: 3.0 (maximum), 4.5, 5.0, 6.6 us.  512 bins: 256 and 1024 ran within
+// 2% at one row; 1024 was 25% slower at 16 rows (more atomics per slice).
+//
+// No workgroup waits for another: what a launch needs from the one before it
+// (maximum, bins) every workgroup derives for itself.  Rows are independent
+// (grid.y).  Differences from
 // the reference's sort-based form: the top-p rule walks the tokens in the
 // order of z, where the sort walks the fp32 probabilities, so of two tokens
 // whose probabilities round to the same fp32 value the larger z comes first
@@ -42,42 +54,43 @@
 namespace sbq {
 
 constexpr int kSampThreads = 1024;
-constexpr int kSampMaxBlocks = 64;   // workgroups per row (one wave's lanes sum their per-workgroup values)
-constexpr int kSampCopies = 16;      // LDS copies of each histogram bin (atomics of one wave spread over them)
-constexpr double kSampFix = 1099511627776.0;  // 2^40: exp(z - max) in (0, 1] -> fixed point
+constexpr int kSampWaves = kSampThreads / 64;
+constexpr int kSampMaxBlocks = 64;   // workgroups (slices) per row: one wave's lanes hold a value of each
+constexpr int kSampBins = 512;       // bins of max - z
+constexpr int kSampCopies = 8;       // LDS copies of each bin (atomics of one wave spread over them)
+constexpr int kSampUnroll = 4;       // tokens in flight per thread
+constexpr int kSampList = 512;       // undecided tokens listed per slice (a slice with more is read again)
+constexpr uint32_t kSampTied = 1u << 31;  // a slice's undecided tokens are more than that and share one key
+constexpr float kSampRange = 28.0f;  // exp(-28) < 2^-40: a mass of 0 from here down
 
 // Per-row scratch, from the row's first byte (each part 256-byte aligned).
 struct SampRow {
-  static constexpr int64_t kHead = 0;                       // SampHead
-  static constexpr int64_t kMax = 256;                      // float [G]
-  static constexpr int64_t kNan = kMax + 512;               // int [G]
-  static constexpr int64_t kEsum = kNan + 512;              // uint64 [G]: mass of the tokens top-k keeps
-  static constexpr int64_t kBsum = kEsum + 512;             // uint64 [G]: mass of the tokens both keep (boundary ties aside)
-  static constexpr int64_t kTie = kBsum + 512;              // int [G]: tokens of the top-p boundary key
-  static constexpr int64_t kState = kTie + 256;             // SampState [2]
-  static constexpr int64_t kHist = kState + 256;            // uint64 [G][256]: top-k pass 0, per workgroup
-  static constexpr int64_t kGh = kHist + kSampMaxBlocks * 256 * 8;  // uint64 [7][256]: the later passes' sums
-  static constexpr int64_t kBytes = kGh + 7 * 256 * 8;
+  static constexpr int64_t kHead = 0;                      // SampHead
+  static constexpr int64_t kMax = 256;                     // float [G]
+  static constexpr int64_t kMin = kMax + 256;              // float [G]
+  static constexpr int64_t kNan = kMin + 256;              // int [G]
+  static constexpr int64_t kSum = kNan + 256;              // uint64 [G]: mass above every undecided bin
+  static constexpr int64_t kNum = kSum + 512;              // uint32 [G]: undecided tokens of the slice (| kSampTied)
+  static constexpr int64_t kMass = kNum + 256;             // uint64 [kSampBins]
+  static constexpr int64_t kCount = kMass + kSampBins * 8; // uint32 [kSampBins]
+  static constexpr int64_t kList = kCount + kSampBins * 4; // uint32 [G][kSampList]: keys of the undecided tokens
+  static constexpr int64_t kBytes = kList + kSampMaxBlocks * kSampList * 4;
 };
 static_assert(kSampMaxBlocks * 8 <= 512 && kSampMaxBlocks * 4 <= 256 && kSampMaxBlocks <= 64,
-              "per-block arrays fit their slots and one wave");
+              "per-slice arrays fit their slots and one wave");
+static_assert(kSampMaxBlocks % kSampWaves == 0, "the draw's waves own whole sets of slices");
 
+// The undecided bins of a row, recorded by the list launch for the draw.
 struct SampHead {
-  uint32_t kth;    // key of the k-th largest z (0: no top-k)
-  uint32_t tkey;   // key of the top-p boundary (0: no top-p)
-  float m;         // max z
-  int valid;       // 0: a NaN or an infinite max (the reference raises)
-  int tie_n;       // top-p keeps the first tie_n tokens of key tkey (vocabulary order) ...
+  int valid;      // 0: a NaN or an infinite max (the reference raises)
+  float m, inv;   // max z; bins per unit of max - z
+  int kbin;       // the bin of the k-th largest z (-1: top-k masks nothing of mass)
+  int krest;      // its rank within that bin, from the top
+  int lo, hi;     // the top-p boundary lies in bins lo .. hi (lo > hi: no top-p)
   int pad;
-  uint64_t tie_f;  // ... each of mass tie_f (0: no such tokens)
-};
-
-// Radix descent state before a pass: the key bits found so far and the
-// remaining rank (top-k) or the mass above the region (top-p).
-struct SampState {
-  uint32_t prefix;
-  uint32_t pad;
-  uint64_t rest;
+  uint64_t kabove;  // mass of the bins above kbin
+  uint64_t labove;  // mass of the bins above lo
+  uint64_t total;   // mass of the row
 };
 
 struct SampArgs {
@@ -88,7 +101,6 @@ struct SampArgs {
   int k;                 // min(top_k, V), or 0
   double top_p;          // 0 without top-p
   uint8_t* ws;
-  int64_t ws_row;        // bytes per row (SampRow::kBytes)
   const float* u;        // [M] uniforms in [0, 1)
   int64_t* tokens;       // [M]
 };
@@ -106,493 +118,668 @@ __device__ __forceinline__ float samp_unkey(uint32_t k) {
 
 __device__ __forceinline__ float samp_z(const SampArgs& a, const float* row, int i) { return row[i] / a.T; }
 
-// fixed-point mass exp(z - m) of a token top-k keeps (0 for masked ones)
-__device__ __forceinline__ uint64_t samp_efix(float z, uint32_t kth, float m) {
-  if (samp_key(z) < kth) return 0;
-  return (uint64_t)((double)expf(z - m) * kSampFix);  // exp(z - m) <= 1: exact in double after the scaling
+// fixed-point mass exp(z - m) * 2^40, truncated: the 24-bit significand of
+// the float exp(z - m) <= 1, shifted (its exponent field is at most 127)
+__device__ __forceinline__ uint64_t samp_efix(float z, float m) {
+  const uint32_t b = __float_as_uint(expf(z - m));
+  const int sh = (int)(b >> 23) - (150 - 40);
+  const uint64_t s = (b & 0x7fffffu) | 0x800000u;
+  return sh >= 0 ? s << sh : s >> min(-sh, 63);
+}
+
+// Bin of z: equal steps of m - z, 0 at the maximum.  Rounding and truncation
+// are monotone, so a larger z never has a larger bin, and equal z share one.
+__device__ __forceinline__ int samp_bin(float z, float m, float inv) {
+  return (int)fminf((m - z) * inv, (float)(kSampBins - 1));
 }
 
 // The top-p bound on the mass above a token: mass_above < top_p * S (S: the
 // mass top-k keeps) <=> mass_above < thr, for integer masses.
 __device__ __forceinline__ uint64_t samp_thr(double top_p, uint64_t S) { return (uint64_t)ceil(top_p * (double)S); }
 
-__device__ __forceinline__ uint8_t* samp_row_ws(const SampArgs& a) { return a.ws + (int64_t)blockIdx.y * a.ws_row; }
+__device__ __forceinline__ uint8_t* samp_row_ws(const SampArgs& a) { return a.ws + (int64_t)blockIdx.y * SampRow::kBytes; }
 
-// LDS histogram of 256 bins x kSampCopies (lane l adds to copy l % copies,
-// so a wave whose keys share a bin hits kSampCopies addresses, not one).
-__device__ __forceinline__ void hist_clear(uint64_t* H) {
-  for (int b = threadIdx.x; b < 256 * kSampCopies; b += blockDim.x) H[b] = 0;
-}
-__device__ __forceinline__ void hist_add(uint64_t* H, uint32_t bin, uint64_t v) {
-  atomicAdd((unsigned long long*)&H[bin * kSampCopies + (threadIdx.x & (kSampCopies - 1))], (unsigned long long)v);
-}
-__device__ __forceinline__ void hist_store(const uint64_t* H, uint64_t* out) {
-  for (int b = threadIdx.x; b < 256; b += blockDim.x) {
-    uint64_t s = 0;
-#pragma unroll
-    for (int c = 0; c < kSampCopies; ++c) s += H[b * kSampCopies + c];
-    out[b] = s;
+// The tokens [i0, i1) of the row as `n` consecutive threads, of which this is
+// number `t`, take them: kSampUnroll loads in flight, indexes clamped to the
+// range, surplus ones skipped.  The first round is loaded on construction
+// (ahead of what the caller still has to find out: an L2 latency less per
+// launch).
+struct SampTokens {
+  const float* row;
+  int i0, i1, t, n;
+  float x[kSampUnroll];
+
+  __device__ __forceinline__ SampTokens(const float* row_, int i0_, int i1_, int t_, int n_)
+      : row(row_), i0(i0_), i1(i1_), t(t_), n(n_) {
+    load(i0 + t);
   }
-}
-// add the workgroup's histogram into the row's (zeroed by the first launch)
-__device__ __forceinline__ void hist_accumulate(const uint64_t* H, uint64_t* gh) {
-  for (int b = threadIdx.x; b < 256; b += blockDim.x) {
-    uint64_t s = 0;
+  __device__ __forceinline__ void load(int b) {
 #pragma unroll
-    for (int c = 0; c < kSampCopies; ++c) s += H[b * kSampCopies + c];
-    if (s) __hip_atomic_fetch_add((unsigned long long*)&gh[b], (unsigned long long)s, __ATOMIC_RELAXED,
-                                  __HIP_MEMORY_SCOPE_AGENT);
+    for (int u = 0; u < kSampUnroll; ++u) x[u] = row[max(min(b + u * n, i1 - 1), 0)];
   }
+  // f(i, z) for each token
+  template <typename F>
+  __device__ __forceinline__ void each(float T, F f) {
+    for (int b = i0 + t; b < i1; b += kSampUnroll * n) {
+      if (b != i0 + t) load(b);
+#pragma unroll
+      for (int u = 0; u < kSampUnroll; ++u)
+        if (b + u * n < i1) f(b + u * n, x[u] / T);
+    }
+  }
+};
+
+// v of the lane that the DPP control names, 0 where it names none
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t samp_dpp0(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint64_t samp_dpp0(uint64_t v) {
+  return (uint64_t)samp_dpp0<CTRL, ROWS>((uint32_t)v) | (uint64_t)samp_dpp0<CTRL, ROWS>((uint32_t)(v >> 32)) << 32;
 }
 
+// Inclusive prefix sum over the lanes of one wave: within the rows of 16
+// lanes, then across them (lane moves, no LDS round trips).
+template <typename T>
+__device__ __forceinline__ T wave_prefix(T v) {
+  v += samp_dpp0<0x111, 0xf>(v);  // row_shr 1, 2, 4, 8
+  v += samp_dpp0<0x112, 0xf>(v);
+  v += samp_dpp0<0x114, 0xf>(v);
+  v += samp_dpp0<0x118, 0xf>(v);
+  v += samp_dpp0<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+  v += samp_dpp0<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+  return v;
+}
+// The last lane's value.
+__device__ __forceinline__ uint32_t wave_last(uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane((int)v, 63); }
+__device__ __forceinline__ uint64_t wave_last(uint64_t v) {
+  return (uint64_t)wave_last((uint32_t)v) | (uint64_t)wave_last((uint32_t)(v >> 32)) << 32;
+}
+template <typename T>
+__device__ __forceinline__ T wave_total(T v) { return wave_last(wave_prefix(v)); }
+
+// Block sum, every thread the result.  red: kSampWaves words, reused after
+// the caller's next barrier.
 __device__ __forceinline__ uint64_t samp_block_sum_u64(uint64_t v, uint64_t* red) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  const int w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  if ((threadIdx.x & 63) == 0) red[w] = v;
+  const int lane = threadIdx.x & 63;
+  v = wave_total(v);
+  if (lane == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
-  uint64_t s = 0;
-  for (int i = 0; i < nw; ++i) s += red[i];
-  __syncthreads();
+  return wave_total(lane < kSampWaves ? red[lane] : (uint64_t)0);
+}
+
+// The row's maximum, bins and validity from the first launch's per-slice
+// values (identical in every wave and workgroup).
+struct SampScale {
+  float m, inv;
+  bool valid, clamped;  // clamped: the last bin holds only tokens of mass 0
+};
+__device__ __forceinline__ SampScale samp_scale(const SampArgs& a, const uint8_t* w) {
+  const int lane = threadIdx.x & 63, g = min(lane, a.G - 1);
+  const float mxl = ((const float*)(w + SampRow::kMax))[g], mnl = ((const float*)(w + SampRow::kMin))[g];
+  const int nl = ((const int*)(w + SampRow::kNan))[g];
+  SampScale s;
+  s.m = wave_max(mxl);
+  const float mn = wave_min(mnl);
+  s.valid = __ballot(nl != 0) == 0 && s.m < INFINITY && s.m > -INFINITY;
+  const float range = s.m - mn;
+  s.clamped = !(range < kSampRange);
+  s.inv = (float)(kSampBins - 1) / (s.clamped ? kSampRange : fmaxf(range, 1e-30f));
   return s;
 }
 
-// Two block sums at once (one pair of barriers); red: 32 words.
-__device__ __forceinline__ void samp_block_sum2_u64(uint64_t& v0, uint64_t& v1, uint64_t* red) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    v0 += __shfl_xor(v0, o);
-    v1 += __shfl_xor(v1, o);
-  }
-  const int w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  if ((threadIdx.x & 63) == 0) {
-    red[w] = v0;
-    red[16 + w] = v1;
-  }
-  __syncthreads();
-  uint64_t s0 = 0, s1 = 0;
-  for (int i = 0; i < nw; ++i) {
-    s0 += red[i];
-    s1 += red[16 + i];
-  }
-  __syncthreads();
-  v0 = s0;
-  v1 = s1;
-}
-
-// Sum of v over the G <= 64 lanes of one wave (exact), every lane the result.
-__device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
-}
-
-// sum over g < G of a per-workgroup array, by the lanes of each wave (one
-// load per lane, all in flight; identical in every wave and workgroup)
-__device__ __forceinline__ uint64_t samp_sum_g(const uint64_t* p, int G) {
-  const int lane = threadIdx.x & 63;
-  return wave_sum_u64(lane < G ? p[lane] : 0);
-}
-
-// One radix step from the previous pass's histograms (every workgroup of the
-// row computes the same result): top-k (MASS false) takes the digit whose
-// bin holds the remaining rank counted from the top; top-p (MASS true) the
-// lowest digit whose bins above leave the mass above the region below thr.
-// The G histograms are summed by all threads (four partial sums per bin,
-// added in a fixed order); wave 0 then finds the digit, four bins per lane,
-// with suffix sums across the lanes.  P: 4 x 256 words of LDS.
-template <bool MASS>
-__device__ SampState samp_descend(const uint64_t* hist, int G, SampState st, uint64_t thr, uint64_t* P,
-                                  SampState* out) {
-  const int t = threadIdx.x, bin = t & 255, part = t >> 8;  // blockDim.x == 1024: parts 0..3
-  uint64_t s = 0;
-  for (int g = part; g < G; g += 4) s += hist[g * 256 + bin];
-  P[part * 256 + bin] = s;
-  if (t == 0) {  // the result if no bin qualifies (an empty or invalid row): the top bin
-    SampState r = st;
-    r.prefix = (st.prefix << 8) | 255u;
-    *out = r;
-  }
-  __syncthreads();
-  if (t < 64) {
-    const int lane = t;
-    uint64_t h[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int b = 4 * lane + j;
-      h[j] = P[b] + P[256 + b] + P[512 + b] + P[768 + b];
-    }
-    const uint64_t local = h[0] + h[1] + h[2] + h[3];
-    uint64_t suf = local;  // sum over lanes >= lane
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const uint64_t v = __shfl_down(suf, o);
-      if (lane + o < 64) suf += v;
-    }
-    const uint64_t above_lane = suf - local;  // bins of higher lanes
-    // cum[j]: mass or count of the bins above bin 4 * lane + j
-    const uint64_t cum3 = above_lane, cum2 = cum3 + h[3], cum1 = cum2 + h[2], cum0 = cum1 + h[1];
-    const uint64_t cum[4] = {cum0, cum1, cum2, cum3};
-    if constexpr (!MASS) {
-      // the crossing bin: cum < rest <= cum + h (exactly one bin of the wave)
-#pragma unroll
-      for (int j = 3; j >= 0; --j)
-        if (cum[j] < st.rest && st.rest <= cum[j] + h[j]) {
-          SampState r = st;
-          r.rest -= cum[j];
-          r.prefix = (st.prefix << 8) | (uint32_t)(4 * lane + j);
-          *out = r;
-        }
-    } else {
-      // qualifying bins (rest + cum < thr) are those from some b0 up; the
-      // lowest lane holding one holds b0
-      int lowj = -1;
-#pragma unroll
-      for (int j = 3; j >= 0; --j)
-        if (st.rest + cum[j] < thr) lowj = j;
-      const uint64_t any = __ballot(lowj >= 0);
-      const int lead = any ? __ffsll((long long)any) - 1 : -1;
-      if (lane == lead) {
-        SampState r = st;
-        r.rest += cum[lowj];
-        r.prefix = (st.prefix << 8) | (uint32_t)(4 * lane + lowj);
-        *out = r;
-      }
-    }
-  }
-  __syncthreads();
-  const SampState r = *out;
-  __syncthreads();
-  return r;
-}
-
-// First launch: max of z and NaN count per workgroup; with top-k, pass 0 of
-// its selection (counts by the key's top byte).
-__global__ __launch_bounds__(kSampThreads) void samp_first_kernel(SampArgs a) {
-  __shared__ uint64_t H[256 * kSampCopies];
-  __shared__ float mred[16];
-  __shared__ int nred[16];
-  const float* row = a.x + (int64_t)blockIdx.y * a.ld;
+// First launch: max and min of z and the NaN count per slice; workgroup 0
+// clears the row's bins.
+__global__ __launch_bounds__(kSampThreads) void samp_max_kernel(SampArgs a) {
+  __shared__ float smx[kSampWaves], smn[kSampWaves];
+  __shared__ int snan[kSampWaves];
   uint8_t* w = samp_row_ws(a);
-  const bool topk = a.k > 0;
-  if (topk) hist_clear(H);
-  if (blockIdx.x == 0)  // the row histograms of the later passes
-    for (int b = threadIdx.x; b < 7 * 256; b += blockDim.x) ((uint64_t*)(w + SampRow::kGh))[b] = 0;
-  __syncthreads();
   const int i0 = blockIdx.x * a.per, i1 = min(i0 + a.per, a.V);
-  float mx = -INFINITY;
-  int nan = 0;
-  for (int i = i0 + threadIdx.x; i < i1; i += blockDim.x) {
-    const float z = samp_z(a, row, i);
-    nan += z != z;
+  SampTokens tok(a.x + (int64_t)blockIdx.y * a.ld, i0, i1, threadIdx.x, kSampThreads);
+  if (blockIdx.x == 0 && threadIdx.x < kSampBins) {
+    ((uint64_t*)(w + SampRow::kMass))[threadIdx.x] = 0;
+    ((uint32_t*)(w + SampRow::kCount))[threadIdx.x] = 0;
+  }
+  float mx = -INFINITY, mn = INFINITY;
+  bool nan = false;
+  tok.each(a.T, [&](int, float z) {
+    nan |= z != z;
     mx = fmaxf(mx, z);
-    if (topk) hist_add(H, samp_key(z) >> 24, 1);
-  }
+    mn = fminf(mn, z);
+  });
   mx = wave_max(mx);
-  nan = wave_sum_i(nan);
-  const int wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  if ((threadIdx.x & 63) == 0) {
-    mred[wv] = mx;
-    nred[wv] = nan;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    float m = mred[0];
-    int n = nred[0];
-    for (int i = 1; i < nw; ++i) {
-      m = fmaxf(m, mred[i]);
-      n += nred[i];
-    }
-    ((float*)(w + SampRow::kMax))[blockIdx.x] = m;
-    ((int*)(w + SampRow::kNan))[blockIdx.x] = n;
-    if (topk && blockIdx.x == 0) ((SampState*)(w + SampRow::kState))[0] = SampState{0u, 0u, (uint64_t)a.k};
-  }
-  if (topk) hist_store(H, (uint64_t*)(w + SampRow::kHist) + blockIdx.x * 256);
-}
-
-// Radix pass `pass` (1..3) of the top-k selection (MASS false: token counts)
-// or of the top-p boundary (MASS true: fixed-point mass of the tokens top-k
-// keeps).  Row histograms: top-k pass p in gh[p - 1] (its pass 0: the
-// per-workgroup histograms), top-p pass p in gh[3 + p]; the descent state
-// alternates between st[0] and st[1].
-template <bool MASS>
-__global__ __launch_bounds__(kSampThreads) void samp_select_kernel(SampArgs a, int pass) {
-  __shared__ uint64_t H[256 * kSampCopies];
-  __shared__ SampState bcast;
-  const float* row = a.x + (int64_t)blockIdx.y * a.ld;
-  uint8_t* w = samp_row_ws(a);
-  uint64_t* gh = (uint64_t*)(w + SampRow::kGh);
-  SampState* st = (SampState*)(w + SampRow::kState);
-  uint32_t kth = 0;
-  float m = 0.0f;
-  uint64_t thr = 0;
-  if constexpr (MASS) {
-    const SampHead* h = (const SampHead*)(w + SampRow::kHead);
-    kth = h->kth;
-    m = h->m;
-    thr = samp_thr(a.top_p, samp_sum_g((const uint64_t*)(w + SampRow::kEsum), a.G));
-  }
-  const uint64_t* src = MASS ? gh + (3 + pass - 1) * 256
-                             : (pass == 1 ? (const uint64_t*)(w + SampRow::kHist) : gh + (pass - 2) * 256);
-  const int srcG = !MASS && pass == 1 ? a.G : 1;
-  const SampState cur = samp_descend<MASS>(src, srcG, st[(pass - 1) & 1], thr, H, &bcast);
-  hist_clear(H);
-  __syncthreads();
-  const int i0 = blockIdx.x * a.per, i1 = min(i0 + a.per, a.V);
-  const int hi = 32 - 8 * pass, lo = 24 - 8 * pass;
-  for (int i = i0 + threadIdx.x; i < i1; i += blockDim.x) {
-    const float z = samp_z(a, row, i);
-    const uint32_t key = samp_key(z);
-    if ((key >> hi) != cur.prefix) continue;
-    const uint32_t bin = (key >> lo) & 255u;
-    if constexpr (MASS) {
-      const uint64_t f = samp_efix(z, kth, m);
-      if (f) hist_add(H, bin, f);
-    } else {
-      hist_add(H, bin, 1);
-    }
-  }
-  __syncthreads();
-  hist_accumulate(H, gh + (MASS ? 3 + pass : pass - 1) * 256);
-  if (blockIdx.x == 0 && threadIdx.x == 0) st[pass & 1] = cur;
-}
-
-// Softmax mass over the tokens top-k keeps, per workgroup (after the top-k
-// passes: its last digit is derived here); with top-p, pass 0 of its
-// selection.  Workgroup 0 records the k-th largest key, the max and validity.
-__global__ __launch_bounds__(kSampThreads) void samp_soft_kernel(SampArgs a) {
-  __shared__ uint64_t H[256 * kSampCopies];
-  __shared__ SampState bcast;
-  __shared__ uint64_t red[16];
-  const float* row = a.x + (int64_t)blockIdx.y * a.ld;
-  uint8_t* w = samp_row_ws(a);
-  uint32_t kth = 0;
-  if (a.k > 0)
-    kth = samp_descend<false>((const uint64_t*)(w + SampRow::kGh) + 2 * 256, 1,
-                              ((const SampState*)(w + SampRow::kState))[1], 0, H, &bcast)
-              .prefix;
-  const float* maxp = (const float*)(w + SampRow::kMax);
-  const int* nanp = (const int*)(w + SampRow::kNan);
+  mn = wave_min(mn);
+  const int any = __ballot(nan) != 0;
   const int lane = threadIdx.x & 63;
-  const float m = wave_max(lane < a.G ? maxp[lane] : -INFINITY);
-  const int nan = wave_sum_i(lane < a.G ? nanp[lane] : 0);
-  const bool valid = nan == 0 && m < INFINITY && m > -INFINITY;
-  const bool topp = a.top_p > 0.0;
-  if (topp) hist_clear(H);
+  if (lane == 0) {
+    smx[threadIdx.x >> 6] = mx;
+    smn[threadIdx.x >> 6] = mn;
+    snan[threadIdx.x >> 6] = any;
+  }
   __syncthreads();
-  const int i0 = blockIdx.x * a.per, i1 = min(i0 + a.per, a.V);
-  uint64_t part = 0;
-  if (valid)
-    for (int i = i0 + threadIdx.x; i < i1; i += blockDim.x) {
-      const float z = samp_z(a, row, i);
-      const uint64_t f = samp_efix(z, kth, m);
-      part += f;
-      if (topp && f) hist_add(H, samp_key(z) >> 24, f);
-    }
-  const uint64_t s = samp_block_sum_u64(part, red);  // its barriers also end the histogram adds
-  if (threadIdx.x == 0) {
-    ((uint64_t*)(w + SampRow::kEsum))[blockIdx.x] = s;
-    if (blockIdx.x == 0) {
-      SampHead* h = (SampHead*)(w + SampRow::kHead);
-      h->kth = kth;
-      h->tkey = 0;
-      h->m = m;
-      h->valid = valid ? 1 : 0;
-      h->tie_n = 0;
-      h->tie_f = 0;
-      if (topp) ((SampState*)(w + SampRow::kState))[0] = SampState{0u, 0u, 0u};
+  if (threadIdx.x < 64) {  // wave 0: a lane per wave's values
+    const int wv = min(lane, kSampWaves - 1);
+    mx = wave_max(smx[wv]);
+    mn = wave_min(smn[wv]);
+    const int bad = __ballot(snan[wv] != 0) != 0;
+    if (lane == 0) {
+      ((float*)(w + SampRow::kMax))[blockIdx.x] = mx;
+      ((float*)(w + SampRow::kMin))[blockIdx.x] = mn;
+      ((int*)(w + SampRow::kNan))[blockIdx.x] = bad;
     }
   }
-  if (topp) hist_accumulate(H, (uint64_t*)(w + SampRow::kGh) + 3 * 256);
 }
 
-// With top-p: the mass of the tokens both cuts keep, per workgroup (the top-p
-// boundary's last digit is derived here); workgroup 0 records the boundary.
-// The tokens of the boundary key share one z, so one mass f.  The reference's
-// sort puts them together (in vocabulary order: a stable sort) and its rule
-// keeps the j-th of them while the mass above it, A + j f, stays below
-// top_p: the first n = ceil((thr - A) / f) of them (A: the mass of the keys
-// above, the descent's rest).  When n is below their count, they are counted
-// per workgroup here and left out of its mass, and the draw adds f for each
-// of the first n; otherwise all of them are kept, as every key above.
-__global__ __launch_bounds__(kSampThreads) void samp_bsum_kernel(SampArgs a) {
-  __shared__ uint64_t H[1024];
-  __shared__ SampState bcast;
-  __shared__ uint64_t red[32];
-  const float* row = a.x + (int64_t)blockIdx.y * a.ld;
+// Second launch (with a cut): token counts (K: top-k) and masses (P: top-p)
+// per bin, in LDS, then added into the row's bins.
+template <bool K, bool P>
+__global__ __launch_bounds__(kSampThreads) void samp_bins_kernel(SampArgs a) {
+  __shared__ uint64_t H[P ? kSampBins * kSampCopies : 1];
+  __shared__ uint32_t C[K ? kSampBins * kSampCopies : 1];
   uint8_t* w = samp_row_ws(a);
-  SampHead* h = (SampHead*)(w + SampRow::kHead);
-  const uint64_t S = samp_sum_g((const uint64_t*)(w + SampRow::kEsum), a.G);
-  const uint64_t thr = samp_thr(a.top_p, S);
-  const uint64_t* last = (const uint64_t*)(w + SampRow::kGh) + 6 * 256;  // pass 3: masses by the key's low byte
-  const SampState fin = samp_descend<true>(last, 1, ((const SampState*)(w + SampRow::kState))[1], thr, H, &bcast);
-  const uint32_t tkey = fin.prefix;
-  const uint32_t kth = h->kth;
-  const float m = h->m;
-  const bool valid = h->valid != 0;
-  const uint32_t lim = kth > tkey ? kth : tkey;
   const int i0 = blockIdx.x * a.per, i1 = min(i0 + a.per, a.V);
-  uint64_t part = 0, ties = 0;  // the mass of every kept key, the tokens of the boundary key
-  if (valid)
-    for (int i = i0 + threadIdx.x; i < i1; i += blockDim.x) {
-      const float z = samp_z(a, row, i);
-      const uint32_t key = samp_key(z);
-      ties += key == tkey;
-      if (key >= lim) part += samp_efix(z, kth, m);
+  SampTokens tok(a.x + (int64_t)blockIdx.y * a.ld, i0, i1, threadIdx.x, kSampThreads);
+  for (int i = threadIdx.x; i < kSampBins * kSampCopies; i += kSampThreads) {
+    if constexpr (P) H[i] = 0;
+    if constexpr (K) C[i] = 0;
+  }
+  const SampScale sc = samp_scale(a, w);
+  if (!sc.valid) return;
+  __syncthreads();
+  const int copy = threadIdx.x & (kSampCopies - 1);
+  tok.each(a.T, [&](int, float z) {
+    const int at = samp_bin(z, sc.m, sc.inv) * kSampCopies + copy;
+    if constexpr (P) {
+      const uint64_t f = samp_efix(z, sc.m);
+      if (f) atomicAdd((unsigned long long*)&H[at], (unsigned long long)f);
     }
-  samp_block_sum2_u64(part, ties, red);
+    if constexpr (K) atomicAdd(&C[at], 1u);
+  });
+  __syncthreads();
+  for (int b = threadIdx.x; b < kSampBins; b += kSampThreads) {
+    if constexpr (P) {
+      uint64_t s = 0;
+#pragma unroll
+      for (int c = 0; c < kSampCopies; ++c) s += H[b * kSampCopies + c];
+      if (s) __hip_atomic_fetch_add((unsigned long long*)(w + SampRow::kMass) + b, (unsigned long long)s,
+                                    __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if constexpr (K) {
+      uint32_t s = 0;
+#pragma unroll
+      for (int c = 0; c < kSampCopies; ++c) s += C[b * kSampCopies + c];
+      if (s) __hip_atomic_fetch_add((uint32_t*)(w + SampRow::kCount) + b, s, __ATOMIC_RELAXED,
+                                    __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+}
+
+// The undecided bins of the row from its filled bins (identical in every
+// workgroup).  Thread b < kSampBins holds bin b.
+template <bool K, bool P>
+__device__ void samp_cuts(const SampArgs& a, const SampScale& sc, uint64_t f, uint32_t c, SampHead* h, uint64_t* red) {
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  constexpr int W = kSampBins / 64;
+  uint64_t fi = P ? wave_prefix(f) : 0;
+  uint32_t ci = K ? wave_prefix(c) : 0;
+  if (lane == 63 && wv < W) {
+    red[wv] = fi;
+    red[W + wv] = ci;
+  }
+  if (t == 0) *h = SampHead{1, sc.m, sc.inv, -1, 0, 1, 0, 0, 0, 0, 0};
+  __syncthreads();
+  uint64_t total = 0;
+#pragma unroll
+  for (int i = 0; i < W; ++i) {
+    if (i < wv) {
+      fi += red[i];
+      ci += (uint32_t)red[W + i];
+    }
+    total += red[i];
+  }
+  const uint64_t fa = fi - f;  // mass of the bins above this one
+  if constexpr (K) {
+    // the bin of the k-th largest z; a last bin of tokens without mass cuts nothing
+    const uint32_t ca = ci - c, k = (uint32_t)a.k;
+    if (t < kSampBins && ca < k && k <= ci && !(sc.clamped && t == kSampBins - 1)) {
+      h->kbin = t;
+      h->krest = (int)(k - ca);
+      h->kabove = fa;
+      red[2 * W] = fi;
+    }
+    __syncthreads();
+  }
+  if constexpr (P) {
+    const int kbin = K ? h->kbin : -1, last = kbin >= 0 ? kbin : kSampBins - 1;
+    // the mass top-k keeps: known without it, else from that of the bins
+    // above the k-th token's to that with its whole bin
+    const uint64_t s0 = kbin >= 0 ? h->kabove : total, s1 = kbin >= 0 ? red[2 * W] : total;
+    const uint64_t t0 = max(samp_thr(a.top_p, s0), (uint64_t)1), t1 = max(samp_thr(a.top_p, s1), (uint64_t)1);
+    // the boundary's bin for a bound thr: the last one (down to the k-th
+    // token's) whose mass above stays below thr
+    if (t <= last) {
+      if (fa < t0 && (t == last || fi >= t0)) {
+        h->lo = t;
+        h->labove = fa;
+      }
+      if (fa < t1 && (t == last || fi >= t1)) h->hi = t;
+    }
+    if (t == 0) h->total = total;
+    __syncthreads();
+  }
+}
+
+// Third launch: per slice, the mass of the tokens above every undecided bin
+// and the list of the tokens in them.  A slice with more of them than its
+// list holds records their key when they all share one (ties), as the key in
+// the list's first place and kSampTied in the count.
+template <bool K, bool P>
+__global__ __launch_bounds__(kSampThreads) void samp_list_kernel(SampArgs a) {
+  __shared__ SampHead h;
+  __shared__ uint64_t red[2 * (kSampBins / 64) + 1], sum[kSampWaves];
+  __shared__ uint32_t num, kmin, kmax;
+  uint8_t* w = samp_row_ws(a);
+  const int i0 = blockIdx.x * a.per, i1 = min(i0 + a.per, a.V);
+  SampTokens tok(a.x + (int64_t)blockIdx.y * a.ld, i0, i1, threadIdx.x, kSampThreads);
+  uint64_t f = 0;
+  uint32_t c = 0;
+  if (threadIdx.x < kSampBins) {
+    if constexpr (P) f = ((const uint64_t*)(w + SampRow::kMass))[threadIdx.x];
+    if constexpr (K) c = ((const uint32_t*)(w + SampRow::kCount))[threadIdx.x];
+  }
+  const SampScale sc = samp_scale(a, w);
+  if (!sc.valid) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) ((SampHead*)(w + SampRow::kHead))->valid = 0;
+    return;
+  }
   if (threadIdx.x == 0) {
-    // the boundary key's tokens: mass f0 each, tmass in all (0: none kept by
-    // top-k), from the pass-3 histogram the descent left in LDS (four
-    // partial sums per bin); the same decision in every workgroup
-    const uint32_t tb = tkey & 255u;
-    const uint64_t tmass = H[tb] + H[256 + tb] + H[512 + tb] + H[768 + tb];
-    const uint64_t f0 = valid && tmass ? samp_efix(samp_unkey(tkey), kth, m) : 0;
-    uint64_t n = 0, cnt = 0;
-    // one token (tmass == f0, the usual case) is kept whole; the quotients
-    // below are for a key of several tokens (thr > rest: the key qualifies)
-    if (f0 && tmass > f0 && thr > fin.rest) {
-      // cnt = tmass / f0 (every token of the key adds the same f0; an
-      // integer <= V, so the rounded double quotient is exact) and n =
-      // min(cnt, ceil(need / f0)): below tmass the quotient is < cnt, and
-      // its double estimate is corrected by at most one either way
-      cnt = (uint64_t)((double)tmass / (double)f0 + 0.5);
-      const uint64_t need = thr - fin.rest;
-      if (need >= tmass) {
-        n = cnt;
-      } else {
-        n = (uint64_t)ceil((double)need / (double)f0);
-        if (n > 0 && (n - 1) * f0 >= need) --n;
-        if (n * f0 < need) ++n;
+    num = 0;
+    kmin = ~0u;
+    kmax = 0;
+  }
+  if constexpr (K || P) {
+    samp_cuts<K, P>(a, sc, f, c, &h, red);
+  } else {
+    if (threadIdx.x == 0) h = SampHead{1, sc.m, sc.inv, -1, 0, 1, 0, 0, 0, 0, 0};
+    __syncthreads();
+  }
+  const int lo = h.lo, hi = h.hi, kbin = h.kbin;
+  // tokens above the first undecided bin are kept, whatever the keys say
+  const int first = lo <= hi ? lo : (kbin >= 0 ? kbin : kSampBins);
+  uint32_t* list = (uint32_t*)(w + SampRow::kList) + blockIdx.x * kSampList;
+  uint64_t part = 0;
+  tok.each(a.T, [&](int, float z) {
+    const int b = samp_bin(z, sc.m, sc.inv);
+    if (b < first) {
+      part += samp_efix(z, sc.m);
+    } else if (b <= hi || b == kbin) {
+      const uint32_t at = atomicAdd(&num, 1u), k = samp_key(z);
+      if (at < (uint32_t)kSampList) list[at] = k;
+    }
+  });
+  part = samp_block_sum_u64(part, sum);
+  const bool over = num > (uint32_t)kSampList;  // uniform
+  if (over) {  // do they share one key?
+    uint32_t k0 = ~0u, k1 = 0;
+    SampTokens again(a.x + (int64_t)blockIdx.y * a.ld, i0, i1, threadIdx.x, kSampThreads);
+    again.each(a.T, [&](int, float z) {
+      const int b = samp_bin(z, sc.m, sc.inv);
+      if (b >= first && (b <= hi || b == kbin)) {
+        k0 = min(k0, samp_key(z));
+        k1 = max(k1, samp_key(z));
+      }
+    });
+    if (k0 <= k1) {
+      atomicMin(&kmin, k0);
+      atomicMax(&kmax, k1);
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    const bool tied = over && kmin == kmax;
+    if (tied) list[0] = kmin;
+    ((uint64_t*)(w + SampRow::kSum))[blockIdx.x] = part;
+    ((uint32_t*)(w + SampRow::kNum))[blockIdx.x] = num | (tied ? kSampTied : 0u);
+    if (blockIdx.x == 0) *(SampHead*)(w + SampRow::kHead) = h;
+  }
+}
+
+// The undecided tokens of the row in the draw: gathered through LDS, up to
+// kFlat per thread in registers (the usual case: a few hundred, one per
+// thread).  When there are more, wave wv goes over the slices wv, wv + 16,
+// ... on each use: their lists, their one key if all tied, or the logits
+// again.
+struct SampUndecided {
+  static constexpr int S = kSampMaxBlocks / kSampWaves;
+  static constexpr int kFlat = 4;
+  bool flat;
+  int sets;  // flat: ceil(tokens / kSampThreads)
+  uint32_t key[kFlat];
+  uint64_t mass[kFlat];
+  int slice[kFlat];  // -1: none
+  uint32_t num[S];   // tokens of this wave's slices, not flat
+
+  // lk, ls: kFlat * kSampThreads words / bytes of LDS
+  __device__ __forceinline__ void load(const SampArgs& a, const uint8_t* w, float m, uint32_t* lk, uint8_t* ls) {
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    const uint32_t* lists = (const uint32_t*)(w + SampRow::kList);
+    uint32_t nl = ((const uint32_t*)(w + SampRow::kNum))[min(lane, a.G - 1)], k[S];
+#pragma unroll
+    for (int s = 0; s < S; ++s) k[s] = lists[min(wv + s * kSampWaves, a.G - 1) * kSampList + lane];
+    if (lane >= a.G) nl = 0;
+    const bool fits = __ballot(nl > (uint32_t)kSampList) == 0;
+    const uint32_t incl = wave_prefix(fits ? nl : 0u);
+    const int total = (int)wave_last(incl);
+    flat = fits && total <= kFlat * kSampThreads;
+    sets = (total + kSampThreads - 1) / kSampThreads;
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      const int g = wv + s * kSampWaves;
+      num[s] = (uint32_t)__builtin_amdgcn_readlane((int)nl, g);
+      if (flat) {
+        const int o = __builtin_amdgcn_readlane((int)(incl - nl), g);
+        for (int j = lane; j < (int)num[s]; j += 64) {
+          lk[o + j] = j < 64 ? k[s] : lists[g * kSampList + j];
+          ls[o + j] = (uint8_t)g;
+        }
       }
     }
-    // only a boundary key that keeps part of its tokens is split off (usually
-    // it holds one token, which is kept): its tokens leave the slice's mass
-    // (each added f0 to it) and are counted instead
-    const uint64_t f = n < cnt ? f0 : 0;
-    ((uint64_t*)(w + SampRow::kBsum))[blockIdx.x] = f ? part - ties * f0 : part;
-    ((int*)(w + SampRow::kTie))[blockIdx.x] = f ? (int)ties : 0;
-    if (blockIdx.x == 0) {
-      h->tkey = tkey;
-      h->tie_f = f;
-      h->tie_n = (int)n;
+    __syncthreads();
+    if (flat) {
+#pragma unroll
+      for (int i = 0; i < kFlat; ++i) {
+        slice[i] = -1;
+        if (i < sets) {
+          const int at = t + i * kSampThreads;
+          key[i] = lk[at];
+          if (at < total) slice[i] = ls[at];
+          mass[i] = samp_efix(samp_unkey(key[i]), m);  // (past the end: unused)
+        }
+      }
     }
   }
+
+  // f(key, mass, n, slice) for the keys in [lo, hi], n tokens of that mass each
+  template <typename F>
+  __device__ __forceinline__ void each(const SampArgs& a, const uint8_t* w, const float* row, const SampHead& h,
+                                       uint32_t lo, uint32_t hi, F f) const {
+    if (flat) {
+#pragma unroll
+      for (int i = 0; i < kFlat; ++i)
+        if (i < sets && slice[i] >= 0 && key[i] >= lo && key[i] <= hi) f(key[i], mass[i], 1u, slice[i]);
+      return;
+    }
+    const int lane = threadIdx.x & 63;
+    const auto one = [&](uint32_t k, uint32_t n, int g) {
+      if (k >= lo && k <= hi) f(k, samp_efix(samp_unkey(k), h.m), n, g);
+    };
+#pragma unroll 1
+    for (int s = 0; s < S; ++s) {
+      const int g = (threadIdx.x >> 6) + s * kSampWaves;
+      const uint32_t n = s == 0 ? num[0] : (s == 1 ? num[1] : (s == 2 ? num[2] : num[3]));
+      const uint32_t* list = (const uint32_t*)(w + SampRow::kList) + g * kSampList;
+      if (n <= (uint32_t)kSampList) {
+        for (int j = lane; j < (int)n; j += 64) one(list[j], 1u, g);
+      } else if (n & kSampTied) {
+        if (lane == 0) one(list[0], n & ~kSampTied, g);
+      } else {
+        const int i0 = g * a.per, i1 = min(i0 + a.per, a.V);
+        SampTokens tok(row, i0, i1, lane, 64);
+        tok.each(a.T, [&](int, float z) {
+          const int b = samp_bin(z, h.m, h.inv);
+          if ((b >= h.lo && b <= h.hi) || b == h.kbin) one(samp_key(z), 1u, g);
+        });
+      }
+    }
+  }
+};
+static_assert(SampUndecided::S == 4, "each() names the four counts");
+
+// The cut among the undecided keys [lo, hi] (the lowest and highest present),
+// by 256 equal ranges of keys per step until one key is left.  Counts (MASS
+// false): the key of rank `rest` from the top.  Masses: the lowest key whose
+// mass above it, `rest` on entry for `hi`, stays below thr; `rest` then is
+// that mass.  H: kCutWords of LDS, range-major per copy.
+constexpr int kCutCopies = 4;
+constexpr int kCutStride = 256 + 2;  // copies of one range lie in different banks
+constexpr int kCutWords = kCutCopies * kCutStride;
+template <bool MASS>
+__device__ uint32_t samp_descend(const SampArgs& a, const uint8_t* w, const float* row, const SampHead& h,
+                                 const SampUndecided& und, uint32_t lo, uint32_t hi, uint64_t& rest, uint64_t thr,
+                                 uint64_t* H, uint64_t* bc) {
+  const int t = threadIdx.x, lane = t & 63;
+  uint64_t* const Hc = H + (lane & (kCutCopies - 1)) * kCutStride;
+  while (lo < hi) {
+    const int shift = max(0, 24 - (int)__clz((int)(hi - lo)));
+    for (int i = t; i < kCutWords; i += kSampThreads) H[i] = 0;
+    __syncthreads();
+    und.each(a, w, row, h, lo, hi, [&](uint32_t k, uint64_t f, uint32_t n, int) {
+      atomicAdd((unsigned long long*)&Hc[(k - lo) >> shift], (unsigned long long)(MASS ? f * n : n));
+    });
+    __syncthreads();
+    if (t < 64) {  // four ranges per lane; suffix sums across the lanes
+      uint64_t r[4] = {0, 0, 0, 0};
+#pragma unroll
+      for (int c = 0; c < kCutCopies; ++c)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) r[j] += H[c * kCutStride + 4 * lane + j];
+      const uint64_t pre = wave_prefix(r[0] + r[1] + r[2] + r[3]);
+      uint64_t cum = (MASS ? rest : 0) + wave_last(pre) - pre;  // above this lane's ranges
+      int at = -1;
+      uint64_t above = 0;
+#pragma unroll
+      for (int j = 3; j >= 0; --j) {
+        if (MASS ? cum < thr : (cum < rest && rest <= cum + r[j])) {
+          at = 4 * lane + j;
+          above = cum;
+        }
+        cum += r[j];
+      }
+      // masses: of the ranges that qualify the lowest, in the lowest lane with one
+      const uint64_t any = __ballot(at >= 0);
+      if (lane == (any ? __ffsll((long long)any) - 1 : 0)) {
+        bc[0] = (uint64_t)max(at, 0);
+        bc[1] = !any ? rest : (MASS ? above : rest - above);
+      }
+    }
+    __syncthreads();
+    lo += (uint32_t)bc[0] << shift;
+    hi = lo + min(hi - lo, (1u << shift) - 1u);
+    rest = bc[1];
+    // (the next write of bc is two barriers away)
+  }
+  return lo;
 }
 
-// The draw: the first index whose prefix of kept mass exceeds u * total.
-// One workgroup per row; thread t owns a contiguous run of the chosen
-// workgroup slice; wave scans, then the wave totals in order.  With top-p,
-// of the tokens of the boundary key only the first tie_n (vocabulary order)
-// count, tie_f each: a slice keeps those of them that the slices before it
-// leave, and a token's rank among them is the slice's start plus the ties
-// of the threads before it and of its own run before it.
-__global__ __launch_bounds__(kSampThreads) void samp_pick_kernel(SampArgs a, int use_bsum) {
-  __shared__ uint64_t wtot[16];
-  __shared__ int wtie[16];
+// Last launch, one workgroup per row: the exact cuts among the undecided
+// tokens, the kept mass of each slice, and the draw: the first index whose
+// prefix of kept mass exceeds u * total.
+// The tokens of the top-p boundary key share one z, so one mass f.  The
+// reference's sort puts them together (in vocabulary order: a stable sort)
+// and its rule keeps the j-th of them while the mass above it, A + j f, stays
+// below top_p: the first n = ceil((thr - A) / f) of them (A: the mass of the
+// keys above).  When n is below their count, a slice keeps those of them that
+// the slices before it leave, and a token's rank among them is the slice's
+// start plus the ties of the threads before it and of its own run before it;
+// otherwise all of them are kept, as every key above.
+template <bool K, bool P>
+__global__ __launch_bounds__(kSampThreads) void samp_draw_kernel(SampArgs a) {
+  __shared__ uint64_t H[K || P ? kCutWords : 1];
+  __shared__ uint32_t lk[K || P ? SampUndecided::kFlat * kSampThreads : 1];
+  __shared__ uint8_t ls[K || P ? SampUndecided::kFlat * kSampThreads : 1];
+  __shared__ uint64_t bck[2], bcp[2];
+  __shared__ uint64_t red[kSampWaves], wtot[kSampWaves];
+  __shared__ float zred[4][kSampWaves];
+  __shared__ uint64_t smass[kSampMaxBlocks];
+  __shared__ int stie[kSampMaxBlocks];
+  __shared__ int wtie[kSampWaves];
   __shared__ int found;
   const int row_i = blockIdx.y;
   const float* row = a.x + (int64_t)row_i * a.ld;
   const uint8_t* w = samp_row_ws(a);
-  const SampHead hd = *(const SampHead*)(w + SampRow::kHead);  // the whole head in one load
-  if (!hd.valid) {
-    if (threadIdx.x == 0) a.tokens[row_i] = -1;
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const SampHead h = *(const SampHead*)(w + SampRow::kHead);  // the whole head in one load
+  const uint64_t base_g = ((const uint64_t*)(w + SampRow::kSum))[min(lane, a.G - 1)];
+  double uf = (double)a.u[row_i];
+  uf = uf < 0.0 ? 0.0 : uf;
+  if (!h.valid) {
+    if (t == 0) a.tokens[row_i] = -1;
     return;
   }
-  const uint64_t* bsum = (const uint64_t*)(w + (use_bsum ? SampRow::kBsum : SampRow::kEsum));
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const uint64_t tf = use_bsum ? hd.tie_f : 0;
-  const int tn = use_bsum ? hd.tie_n : 0;
-  // every wave, when the boundary key is split off (tf: uniform, the row's
-  // head): the boundary ties of the slices in lanes and their prefix ...
-  int tbefore_g = 0, tkeep_g = 0;  // ties in the slices before, ties the slice keeps
-  if (tf) {
-    const int tc_g = lane < a.G ? ((const int*)(w + SampRow::kTie))[lane] : 0;
-    int tpre_g = tc_g;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int v = __shfl_up(tpre_g, o);
-      if (lane >= o) tpre_g += v;
+  if (t == 0) found = -1;
+  uint32_t kth = 0, tkey = 0;
+  uint64_t tf = 0;  // mass of a boundary token when only the first tn are kept
+  int tn = 0;
+  if constexpr (K || P) {
+    if (t < kSampMaxBlocks) {
+      smass[t] = 0;
+      stie[t] = 0;
     }
-    tbefore_g = tpre_g - tc_g;
+    SampUndecided und;
+    und.load(a, w, h.m, lk, ls);
+    // lowest and highest undecided z, of the k-th token's bin and of the boundary's bins
+    float k0 = INFINITY, k1 = -INFINITY, p0 = INFINITY, p1 = -INFINITY;
+    und.each(a, w, row, h, 0u, ~0u, [&](uint32_t k, uint64_t, uint32_t, int) {
+      const float z = samp_unkey(k);
+      const int b = samp_bin(z, h.m, h.inv);
+      if (K && b == h.kbin) {
+        k0 = fminf(k0, z);
+        k1 = fmaxf(k1, z);
+      }
+      if (P && b >= h.lo && b <= h.hi) {
+        p0 = fminf(p0, z);
+        p1 = fmaxf(p1, z);
+      }
+    });
+    if constexpr (K) {
+      k0 = wave_min(k0);
+      k1 = wave_max(k1);
+    }
+    if constexpr (P) {
+      p0 = wave_min(p0);
+      p1 = wave_max(p1);
+    }
+    if (lane == 0) {
+      zred[0][wv] = k0;
+      zred[1][wv] = k1;
+      zred[2][wv] = p0;
+      zred[3][wv] = p1;
+    }
+    __syncthreads();
+    const int wl = min(lane, kSampWaves - 1);
+    const bool topk = K && h.kbin >= 0;  // uniform; P: the boundary always lies in a bin
+    uint64_t S = h.total;
+    uint32_t ktop = 0;
+    if constexpr (K) {
+      if (topk) {
+        ktop = samp_key(wave_max(zred[1][wl]));
+        uint64_t rank = (uint64_t)h.krest;
+        kth = samp_descend<false>(a, w, row, h, und, samp_key(wave_min(zred[0][wl])), ktop, rank, 0, H, bck);
+      }
+    }
+    if constexpr (P) {
+      if (topk) {
+        uint64_t part = 0;
+        und.each(a, w, row, h, kth, ktop, [&](uint32_t, uint64_t f, uint32_t n, int) { part += f * n; });
+        S = h.kabove + samp_block_sum_u64(part, red);
+      }
+      uint64_t above = h.labove;
+      const uint64_t thr = samp_thr(a.top_p, S);
+      const uint32_t plo = samp_key(wave_min(zred[2][wl])), phi = samp_key(wave_max(zred[3][wl]));
+      tkey = samp_descend<true>(a, w, row, h, und, max(plo, kth), phi, above, thr, H, bcp);
+      // the tokens of the boundary key per slice, and how many of them the rule keeps
+      und.each(a, w, row, h, tkey, tkey, [&](uint32_t, uint64_t, uint32_t n, int g) { atomicAdd(&stie[g], (int)n); });
+      __syncthreads();
+      const uint64_t ties = wave_total((uint32_t)stie[lane]);
+      const uint64_t f0 = samp_efix(samp_unkey(tkey), h.m), need = thr - above;
+      if (ties > 1 && f0 && thr > above && need < ties * f0) {
+        // ceil(need / f0) <= ties: the double estimate is corrected by at most one either way
+        uint64_t n = (uint64_t)ceil((double)need / (double)f0);
+        if (n > 0 && (n - 1) * f0 >= need) --n;
+        if (n * f0 < need) ++n;
+        if (n < ties) {
+          tf = f0;
+          tn = (int)n;
+        }
+      }
+    }
+    // the kept mass of each slice's undecided tokens: those from the cut up
+    // (boundary ties apart while tf is set)
+    const uint32_t lim = max(kth, tkey);
+    und.each(a, w, row, h, lim, ~0u, [&](uint32_t k, uint64_t f, uint32_t n, int g) {
+      if (!(tf && k == tkey)) atomicAdd((unsigned long long*)&smass[g], (unsigned long long)(f * n));
+    });
+  }
+  __syncthreads();
+  const uint32_t lim = max(kth, tkey);
+  // every wave: the ties before each slice (lane) and those it keeps ...
+  int tbefore_g = 0, tkeep_g = 0;
+  if (P && tf) {
+    const int tc_g = stie[lane];
+    tbefore_g = (int)wave_prefix((uint32_t)tc_g) - tc_g;
     tkeep_g = min(max(tn - tbefore_g, 0), tc_g);
   }
   // ... the slice masses, their inclusive prefix, the total
-  const uint64_t mine_g = lane < a.G ? bsum[lane] + tf * (uint64_t)tkeep_g : 0;
-  uint64_t pre_g = mine_g;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const uint64_t v = __shfl_up(pre_g, o);
-    if (lane >= o) pre_g += v;
-  }
-  const uint64_t total = __shfl(pre_g, 63);
-  double uf = (double)a.u[row_i];
-  uf = uf < 0.0 ? 0.0 : uf;
+  uint64_t mine_g = lane < a.G ? base_g + tf * (uint64_t)tkeep_g : 0;
+  if constexpr (K || P) mine_g += smass[lane];
+  const uint64_t pre_g = wave_prefix(mine_g);
+  const uint64_t total = wave_last(pre_g);
   uint64_t target = (uint64_t)(uf * (double)total);
   if (target >= total) target = total - 1;  // u = 1 (outside [0, 1)) takes the last kept token
   // the slice whose prefix first exceeds the target (the last slice at the latest)
   const uint64_t over = __ballot(lane < a.G && pre_g > target);
   const int g = over ? __ffsll((long long)over) - 1 : a.G - 1;
-  target -= __shfl(pre_g - mine_g, g);  // within workgroup slice g
-  const int trank0 = __shfl(tbefore_g, g);
-  const uint32_t kth = hd.kth, tkey = hd.tkey;
-  const uint32_t lim = kth > tkey ? kth : tkey;
-  const float m = hd.m;
   const int i0 = g * a.per, i1 = min(i0 + a.per, a.V);
-  const int e = (i1 - i0 + (int)blockDim.x - 1) / (int)blockDim.x;  // elements per thread
-  const int t0 = i0 + threadIdx.x * e, t1 = min(t0 + e, i1);
-  // the kept mass of token i (rank: the boundary ties met so far)
-  auto kept = [&](int i, int& rank) -> uint64_t {
-    const float z = samp_z(a, row, i);
-    const uint32_t key = samp_key(z);
-    if (tf && key == tkey) return rank++ < tn ? tf : 0;
-    return key >= lim ? samp_efix(z, kth, m) : 0;
-  };
-  // this thread's run: the mass of its other tokens and its boundary ties
+  const int e = (i1 - i0 + kSampThreads - 1) / kSampThreads;  // consecutive tokens per thread
+  const int t0 = i0 + t * e, t1 = min(t0 + e, i1);
+  float x[kSampUnroll];
+#pragma unroll
+  for (int j = 0; j < kSampUnroll; ++j) x[j] = row[min(t0 + j, a.V - 1)];
+  target -= __shfl(pre_g - mine_g, g);  // within slice g
+  const int trank0 = __shfl(tbefore_g, g);
+  const float m = h.m;
+  // this thread's run: the mass of its kept tokens other than split ties, and its ties
   uint64_t mine = 0;
-  int myt = 0;
-  for (int i = t0; i < t1; ++i) {
-    const float z = samp_z(a, row, i);
+  uint32_t myt = 0;
+  const auto add = [&](float z) {
     const uint32_t key = samp_key(z);
-    if (tf && key == tkey)
+    if (P && tf && key == tkey)
       ++myt;
     else if (key >= lim)
-      mine += samp_efix(z, kth, m);
-  }
-  int rank0 = 0;  // rank of this run's first boundary tie
-  if (tf) {  // uniform: the row's head
-    int tincl = myt;
+      mine += samp_efix(z, m);
+  };
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int v = __shfl_up(tincl, o);
-      if (lane >= o) tincl += v;
-    }
+  for (int j = 0; j < kSampUnroll; ++j)  // its first tokens, loaded together
+    if (t0 + j < t1) add(x[j] / a.T);
+  for (int i = t0 + kSampUnroll; i < t1; ++i) add(samp_z(a, row, i));
+  int rank0 = 0;  // rank of this run's first boundary tie
+  if (P && tf) {  // uniform
+    const int tincl = (int)wave_prefix(myt);
     if (lane == 63) wtie[wv] = tincl;
     __syncthreads();
     int tbase = trank0;
     for (int i = 0; i < wv; ++i) tbase += wtie[i];
-    rank0 = tbase + tincl - myt;
-    mine += tf * (uint64_t)min(max(tn - rank0, 0), myt);  // its ties below rank tn
+    rank0 = tbase + tincl - (int)myt;
+    mine += tf * (uint64_t)min(max(tn - rank0, 0), (int)myt);  // its ties below rank tn
   }
   // inclusive scan within the wave, then the wave totals in wave order
-  uint64_t incl = mine;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const uint64_t v = __shfl_up(incl, o);
-    if (lane >= o) incl += v;
-  }
+  uint64_t incl = wave_prefix(mine);
   if (lane == 63) wtot[wv] = incl;
-  if (threadIdx.x == 0) found = -1;
   __syncthreads();
-  uint64_t base = 0;
-  for (int i = 0; i < wv; ++i) base += wtot[i];
-  incl += base;
+  const uint64_t wl = wave_prefix(lane < kSampWaves ? wtot[lane] : (uint64_t)0);
+  if (wv > 0) incl += __shfl(wl, wv - 1);
   const uint64_t excl = incl - mine;
   if (excl <= target && target < incl) {
     uint64_t c = excl;
     int rank = rank0;
     for (int i = t0; i < t1; ++i) {
-      c += kept(i, rank);
+      const float z = samp_z(a, row, i);
+      const uint32_t key = samp_key(z);
+      if (P && tf && key == tkey)
+        c += rank++ < tn ? tf : 0;
+      else if (key >= lim)
+        c += samp_efix(z, m);
       if (c > target) {
         found = i;
         break;
@@ -600,10 +787,23 @@ __global__ __launch_bounds__(kSampThreads) void samp_pick_kernel(SampArgs a, int
     }
   }
   __syncthreads();
-  if (threadIdx.x == 0) a.tokens[row_i] = found;
+  if (t == 0) a.tokens[row_i] = found;
 }
 
 int64_t sample_workspace_bytes(int64_t M) { return M * SampRow::kBytes; }
+
+namespace {
+
+template <bool K, bool P>
+void launch_sample(const SampArgs& a, int64_t M, hipStream_t st) {
+  const dim3 grid((unsigned)a.G, (unsigned)M), block(kSampThreads);
+  hipLaunchKernelGGL(samp_max_kernel, grid, block, 0, st, a);
+  if constexpr (K || P) hipLaunchKernelGGL((samp_bins_kernel<K, P>), grid, block, 0, st, a);
+  hipLaunchKernelGGL((samp_list_kernel<K, P>), grid, block, 0, st, a);
+  hipLaunchKernelGGL((samp_draw_kernel<K, P>), dim3(1, (unsigned)M), block, 0, st, a);
+}
+
+}  // namespace
 
 int launch_sample_rows(const float* x, int64_t M, int64_t V, int64_t ld, float T, int64_t top_k, float top_p,
                        const float* u, int64_t* tokens, void* ws, hipStream_t st) {
@@ -618,19 +818,16 @@ int launch_sample_rows(const float* x, int64_t M, int64_t V, int64_t ld, float T
   a.k = top_k > 0 && top_k < V ? (int)top_k : 0;
   a.top_p = top_p > 0.0f && top_p < 1.0f ? (double)top_p : 0.0;
   a.ws = (uint8_t*)ws;
-  a.ws_row = SampRow::kBytes;
   a.u = u;
   a.tokens = tokens;
-  const dim3 grid((unsigned)a.G, (unsigned)M), block(kSampThreads);
-  hipLaunchKernelGGL(samp_first_kernel, grid, block, 0, st, a);
-  if (a.k)
-    for (int p = 1; p < 4; ++p) hipLaunchKernelGGL(samp_select_kernel<false>, grid, block, 0, st, a, p);
-  hipLaunchKernelGGL(samp_soft_kernel, grid, block, 0, st, a);
-  if (a.top_p > 0.0) {
-    for (int p = 1; p < 4; ++p) hipLaunchKernelGGL(samp_select_kernel<true>, grid, block, 0, st, a, p);
-    hipLaunchKernelGGL(samp_bsum_kernel, grid, block, 0, st, a);
-  }
-  hipLaunchKernelGGL(samp_pick_kernel, dim3(1, (unsigned)M), block, 0, st, a, a.top_p > 0.0 ? 1 : 0);
+  if (a.k && a.top_p > 0.0)
+    launch_sample<true, true>(a, M, st);
+  else if (a.k)
+    launch_sample<true, false>(a, M, st);
+  else if (a.top_p > 0.0)
+    launch_sample<false, true>(a, M, st);
+  else
+    launch_sample<false, false>(a, M, st);
   return check_launch();
 }
 

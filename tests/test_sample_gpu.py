@@ -288,3 +288,33 @@ def test_sample_drop_in_and_graph_replay(dev):
         eager = quant.sample_tokens(logits, 0.8, 0.9, 40, u=u, workspace=quant.sample_workspace(M, V, dev))
         assert torch.equal(out, eager), rep
     del graph
+
+
+@pytest.mark.parametrize("V,T,k,p", [(70000, 1.0, 0, 0.5), (70000, 0.7, 9000, 0.9), (151936, 1.0, 0, 0.9),
+                                     (151936, 1.0, 3000, 0.6), (2049, 1.0, 600, 0.5)])
+@pytest.mark.parametrize("kind", ["cluster", "wide", "grid", "bimodal"])
+def test_sample_undecided_tokens(dev, kind, V, T, k, p):
+    """Rows whose cuts fall among many tokens of one bin of max - z: a cluster
+    of distinct values within 0.01 with one far token (more than a slice's
+    list holds: read again from the logits), a cluster of one token in ten
+    (lists, but more than the draw keeps in registers), values on a coarse
+    grid (a slice's undecided tokens all tied), two far groups (top-k's cut in
+    the bin of tokens without mass)."""
+    announce(f"sample undecided {kind} V={V} T={T} k={k} p={p}")
+    g = torch.Generator().manual_seed(V + k)
+    if kind == "cluster":
+        x = 5 + 0.01 * torch.rand(1, V, generator=g)
+        x[0, V // 3] = -20.0
+    elif kind == "wide":
+        x = torch.randn(1, V, generator=g) * 2
+        at = torch.rand(1, V, generator=g) < 0.1
+        x = torch.where(at, 9 + 0.01 * torch.rand(1, V, generator=g), x)
+    elif kind == "grid":
+        x = (torch.randn(1, V, generator=g) * 1.5).round()
+    else:
+        x = torch.where(torch.rand(1, V, generator=g) < 0.002, 60.0, -60.0) + torch.randn(1, V, generator=g)
+    xn = x[0].numpy()
+    for u0 in (0.0, 0.31, 0.77, 1 - 2 ** -24):
+        tok = int(_run(x.to(dev), T, k, p, torch.tensor([u0], device=dev))[0])
+        want, ok, _ = _accept(xn, T, k, p, u0, tok)
+        assert ok, (kind, u0, tok, want)
