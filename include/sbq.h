@@ -133,6 +133,22 @@ int sbq_linear_w8(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
                   void* y, int y_dtype, int64_t ldy,
                   void* workspace, size_t workspace_bytes, void* stream);
 
+/* sbq_linear_w8 with its N columns stored as parts: the columns belong to
+ * consecutive parts whose widths are multiples of 4, and part p is a dense
+ * [M, width] matrix of y_dtype starting at element M * pstart(p) of y, where
+ * start(p) is the part's first column and pstart(p) the sum of the earlier
+ * widths, each rounded up to a multiple of 64.  For projections fused into
+ * one layer whose outputs go separate ways (model.py:262-264, 363-365): the
+ * parts leave the launch contiguous, with no copies after it.
+ * y: device, 16-byte aligned, M * (sum of the widths, each rounded up to 64)
+ * elements.  parts: device int32 [N/4][2], per 4 columns the width of their
+ * part and start/4 | ((pstart - start)/4) << 20 (so N < 2^22, and padding
+ * below 2^14 columns in all).  Everything else as sbq_linear_w8. */
+int sbq_linear_w8_parts(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
+                        const uint8_t* packed, const float* scale, const float* bias, int64_t N,
+                        void* y, int y_dtype, const int32_t* parts,
+                        void* workspace, size_t workspace_bytes, void* stream);
+
 /* `count` (1..SBQ_MAX_GROUP) independent weight-only linears that share M, K,
  * x_dtype and y_dtype, in one launch where the decode path applies: linear i
  * is y_i = linear(x_i, packed_i, scale_i, bias_i) exactly as sbq_linear_w8
@@ -242,6 +258,14 @@ int sbq_linear_w8a8(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ld
                     const float* bias, int64_t N,
                     void* y, int y_dtype, int64_t ldy, int32_t* acc_out,
                     void* workspace, size_t workspace_bytes, void* stream);
+
+/* sbq_linear_w8a8 with its columns stored as parts (see
+ * sbq_linear_w8_parts for y and parts). */
+int sbq_linear_w8a8_parts(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
+                          const uint8_t* packed, const float* scale, const int32_t* colsum,
+                          const float* bias, int64_t N, void* y, int y_dtype,
+                          const int32_t* parts, void* workspace, size_t workspace_bytes,
+                          void* stream);
 
 /* `count` (1..SBQ_MAX_GROUP) independent int8-dyn linears of one M, K and
  * dtypes: y_i = sbq_linear_w8a8(x_i, packed_i, scale_i, colsum_i, bias_i,

@@ -75,16 +75,16 @@ bool w8a8_runs_mt(int64_t M, int64_t N, int64_t K, int64_t split_bytes) {
 int linear_w8a8_run(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, const uint8_t* packed,
                     const float* scale, const int32_t* colsum, const float* bias, int64_t N, void* y, int y_dtype,
                     int64_t ldy, int32_t* acc_out, float2* parts, float* qp, int8_t* xq, uint8_t* split,
-                    int64_t split_bytes, hipStream_t st) {
+                    int64_t split_bytes, hipStream_t st, const sbq::u32x2* yparts = nullptr) {
   const bool xv = x_vec_ok(x, x_dtype, ldx), yv = y_vec_ok(y, y_dtype, ldy, N);
   // 16 < M <= 64 where the row-tile GEMV applies: the pre-passes, then that
   // GEMV on the s8 rows (inside launch_gemm_w8a8) instead of the general GEMV
   const bool mt = w8a8_runs_mt(M, N, K, split ? split_bytes : 0);
   if (!mt && sbq::gemv_supports(M, K, true, x_dtype))
     return sbq::launch_gemv_w8a8(x, x_dtype, M, K, ldx, xv, packed, scale, colsum, bias, N, y, y_dtype, ldy, acc_out,
-                                 parts, st, yv);
+                                 parts, st, yv, nullptr, yparts);
   return sbq::launch_gemm_w8a8(x, x_dtype, M, K, ldx, xv, packed, scale, colsum, bias, N, y, y_dtype, ldy, acc_out,
-                               parts, xq, qp, st, yv, split, split_bytes);
+                               parts, xq, qp, st, yv, split, split_bytes, yparts);
 }
 
 // The split-K area after a W8A8 workspace's layout, and its bytes.
@@ -196,21 +196,26 @@ int64_t sbq_w8_workspace_bytes(int64_t M, int64_t K, int x_dtype) {
   return 256 + sbq::w8_ws_layout(M, ((K + 63) / 64) * 64, x_dtype).bytes;
 }
 
-int sbq_linear_w8(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, const uint8_t* packed,
+}  // extern "C"
+
+namespace {
+
+// sbq_linear_w8 on checked operands; yparts: y stored as parts.
+int linear_w8_run(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, const uint8_t* packed,
                   const float* scale, const float* bias, int64_t N, void* y, int y_dtype, int64_t ldy,
-                  void* workspace, size_t workspace_bytes, void* stream) {
-  int rc = check_linear(x, x_dtype, M, K, ldx, packed, scale, N, y, y_dtype, ldy);
-  if (rc || M == 0) return rc;
+                  void* workspace, size_t workspace_bytes, hipStream_t st, const sbq::u32x2* yparts = nullptr) {
   const bool xv = x_vec_ok(x, x_dtype, ldx), yv = y_vec_ok(y, y_dtype, ldy, N);
-  hipStream_t st = (hipStream_t)stream;
   if (M > 16 && M <= 64) {  // several 16-row tiles of x against streamed weights
     // the tiled GEMM's mid-sized-M plan needs the full workspace (row sums, split area)
     const bool alt = workspace && (int64_t)workspace_bytes >= sbq_linear_workspace_bytes(M, N, K, x_dtype, 0);
     const int rc =
-        sbq::launch_gemv_w8_mt(x, x_dtype, M, K, ldx, xv, packed, scale, bias, N, y, y_dtype, ldy, st, yv, alt);
+        sbq::launch_gemv_w8_mt(x, x_dtype, M, K, ldx, xv, packed, scale, bias, N, y, y_dtype, ldy, st, yv,
+                                alt, yparts);
     if (rc != -1) return rc;
   }
-  if (sbq::gemv_supports(M, K, false, x_dtype)) return sbq::launch_gemv_w8(x, x_dtype, M, K, ldx, xv, packed, scale, bias, N, y, y_dtype, ldy, st, yv);
+  if (sbq::gemv_supports(M, K, false, x_dtype))
+    return sbq::launch_gemv_w8(x, x_dtype, M, K, ldx, xv, packed, scale, bias, N, y, y_dtype, ldy, st, yv, nullptr,
+                               yparts);
   // optional scratch of the prefill GEMM (row sums, staged activations), 256-byte aligned
   void* ws = nullptr;
   int64_t ws_bytes = 0;
@@ -219,7 +224,31 @@ int sbq_linear_w8(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
     ws_bytes = (int64_t)workspace_bytes - (int64_t)((uintptr_t)ws - (uintptr_t)workspace);
   }
   return sbq::launch_gemm_w8(x, x_dtype, M, K, ldx, xv, packed, scale, bias, N, y, y_dtype, ldy, ws, ws_bytes, st,
-                             yv);
+                             yv, yparts);
+}
+
+}  // namespace
+
+extern "C" {
+
+int sbq_linear_w8(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, const uint8_t* packed,
+                  const float* scale, const float* bias, int64_t N, void* y, int y_dtype, int64_t ldy,
+                  void* workspace, size_t workspace_bytes, void* stream) {
+  int rc = check_linear(x, x_dtype, M, K, ldx, packed, scale, N, y, y_dtype, ldy);
+  if (rc || M == 0) return rc;
+  return linear_w8_run(x, x_dtype, M, K, ldx, packed, scale, bias, N, y, y_dtype, ldy, workspace, workspace_bytes,
+                       (hipStream_t)stream);
+}
+
+int sbq_linear_w8_parts(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, const uint8_t* packed,
+                        const float* scale, const float* bias, int64_t N, void* y, int y_dtype, const int32_t* parts,
+                        void* workspace, size_t workspace_bytes, void* stream) {
+  int rc = check_linear(x, x_dtype, M, K, ldx, packed, scale, N, y, y_dtype, N);
+  if (rc || M == 0) return rc;
+  if (N % 4 || !parts) return SBQ_ERR_ARG;
+  if (!aligned(y, 16) || !aligned(parts, 8)) return SBQ_ERR_ALIGN;
+  return linear_w8_run(x, x_dtype, M, K, ldx, packed, scale, bias, N, y, y_dtype, N, workspace, workspace_bytes,
+                       (hipStream_t)stream, (const sbq::u32x2*)parts);
 }
 
 int sbq_linear_w8_grouped(int count, const void* const* x, const int64_t* ldx, int x_dtype, int64_t M, int64_t K,
@@ -364,6 +393,20 @@ int sbq_linear_w8a8(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ld
   return linear_w8a8_run(x, x_dtype, M, K, ldx, packed, scale, colsum, bias, N, y, y_dtype, ldy, acc_out,
                          ws_partials(workspace), ws_qp(workspace), ws_xq(workspace), ws_split(workspace, M, K),
                          ws_split_bytes(workspace, workspace_bytes, M, K), (hipStream_t)stream);
+}
+
+int sbq_linear_w8a8_parts(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, const uint8_t* packed,
+                          const float* scale, const int32_t* colsum, const float* bias, int64_t N, void* y,
+                          int y_dtype, const int32_t* parts, void* workspace, size_t workspace_bytes, void* stream) {
+  int rc = check_linear(x, x_dtype, M, K, ldx, packed, scale, N, y, y_dtype, N);
+  if (rc || M == 0) return rc;
+  if (!colsum || N % 4 || !parts) return SBQ_ERR_ARG;
+  if (!aligned(y, 16) || !aligned(parts, 8)) return SBQ_ERR_ALIGN;
+  if (!workspace || (int64_t)workspace_bytes < sbq_w8a8_workspace_bytes(M, K)) return SBQ_ERR_WORKSPACE;
+  return linear_w8a8_run(x, x_dtype, M, K, ldx, packed, scale, colsum, bias, N, y, y_dtype, N, nullptr,
+                         ws_partials(workspace), ws_qp(workspace), ws_xq(workspace), ws_split(workspace, M, K),
+                         ws_split_bytes(workspace, workspace_bytes, M, K), (hipStream_t)stream,
+                         (const sbq::u32x2*)parts);
 }
 
 int sbq_linear_w8a8_grouped(int count, const void* const* x, const int64_t* ldx, int x_dtype, int64_t M, int64_t K,

@@ -19,6 +19,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "sbq_index.h"
+
 namespace sbq {
 
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
@@ -214,6 +216,12 @@ __device__ __forceinline__ uint32_t pack_h2(_Float16 a, _Float16 b) {
 }
 __device__ __forceinline__ uint32_t pack_b2(__bf16 a, __bf16 b) {
   return (uint32_t)__builtin_bit_cast(uint16_t, a) | ((uint32_t)__builtin_bit_cast(uint16_t, b) << 16);
+}
+
+// Element offset of y[m][n], n a multiple of 4, for a y stored as parts (`e`:
+// the table entry of columns n .. n + 3) or, `parts` null, in rows of ldy.
+__device__ __forceinline__ int64_t y_offset(const u32x2* parts, u32x2 e, int M, int64_t ldy, int m, int n) {
+  return parts ? part_base(e.y, M) + (int64_t)m * e.x + n : (int64_t)m * ldy + n;
 }
 
 // Four consecutive outputs; `vec` says the 4-element group is in range and

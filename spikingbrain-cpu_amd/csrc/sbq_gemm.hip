@@ -116,7 +116,7 @@ __global__ __launch_bounds__(WN* WM * 64) void gemm_w8_kernel(const void* __rest
                                                               const float* __restrict__ scale,
                                                               const float* __restrict__ bias, int N, int Nt,
                                                               void* __restrict__ y, int yt, int64_t ldy,
-                                                              int flags) {
+                                                              const u32x2* __restrict__ parts, int flags) {
   typedef GemmOp<XT> Op;
   typedef typename Op::V V;
   constexpr int NS = Op::NS;
@@ -215,6 +215,7 @@ __global__ __launch_bounds__(WN* WM * 64) void gemm_w8_kernel(const void* __rest
     const int n = (nt0 + wn * FN + a) * 16 + 4 * g;
     if (n >= N) continue;
     const int nvalid = min(4, N - n);
+    const u32x2 pe = parts ? parts[n >> 2] : u32x2{0u, 0u};
     f32x4 sc, bi;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
@@ -233,7 +234,7 @@ __global__ __launch_bounds__(WN* WM * 64) void gemm_w8_kernel(const void* __rest
         if (bias) out = out + bi[v];
         o[v] = out;
       }
-      store_y4(y, yt, (int64_t)m * ldy + n, o, yvec && nvalid == 4, nvalid);
+      store_y4(y, yt, y_offset(parts, pe, M, ldy, m, n), o, yvec && nvalid == 4, nvalid);
     }
   }
 }
@@ -291,6 +292,7 @@ struct GemmArgs {
   void* y;
   int yt;
   int64_t ldy;
+  const u32x2* parts;   // y stored as parts (part_base), one entry per 4 columns; null: rows of stride ldy
   int32_t* acc_out;     // I8 only, may be null
   const float* qpbuf;   // I8 only: (s_x, zp as int bits)
   const float* rsum;    // fp16 W-only with RSP: per-row sums of x [M]
@@ -703,6 +705,19 @@ __global__ __launch_bounds__(KG* WN* WM * 64, (SK ? (dl_min_waves<I8, XT, BN, BM
   }
 
   const bool yvec = a.flags & 2;
+  // stores of the block: element yb + m * yld + n.  y as parts: a block within
+  // one part (nearly every block) stores rows of that part's width, others
+  // read the entry of each 4 columns.  Read only now: held through the K loop
+  // the entries cost the M = 8192 prefill 1.2%.
+  int64_t yld = a.ldy, yb = 0;
+  bool across = false, wide = (a.flags & 8) != 0;  // wide: 16-byte aligned rows
+  if (a.parts) {
+    const u32x2 p0 = a.parts[nt0 * 4], p1 = a.parts[(min(nt0 * 16 + BN, a.N) >> 2) - 1];
+    yld = __builtin_amdgcn_readfirstlane(p0.x);
+    yb = part_base(__builtin_amdgcn_readfirstlane(p0.y), M);
+    across = __builtin_amdgcn_readfirstlane(p0.y) != __builtin_amdgcn_readfirstlane(p1.y);
+    wide = !across && yld % 8 == 0 && __builtin_amdgcn_readfirstlane(p0.y) % 2 == 0;
+  }
   // I8 per-token symmetric (ptok): no zero point, y = fp32(acc) * fp32(s_t[m] * scale[n])
   // every wave is past the K loop and no stage DMA is in flight (the last wait
   // was vmcnt(0)): the stage buffers become the output tile
@@ -795,6 +810,12 @@ __global__ __launch_bounds__(KG* WN* WM * 64, (SK ? (dl_min_waves<I8, XT, BN, BM
     for (int t = 0; t < FN; ++t) {
       const int n = (nt0 + wn * FN + t) * 16 + 4 * g;
       const int nvalid = min(4, a.N - n);
+      int64_t ld = yld, base = yb;
+      if (across) {
+        const u32x2 pe = a.parts[min(n, a.N - 4) >> 2];
+        ld = pe.x;
+        base = part_base(pe.y, M);
+      }
       f32x4 sc, bi;
       i32x4 cs;
       col_ops(t, sc, bi, cs);
@@ -802,7 +823,7 @@ __global__ __launch_bounds__(KG* WN* WM * 64, (SK ? (dl_min_waves<I8, XT, BN, BM
       for (int b = 0; b < FM; ++b) {
         const int m = m0 + wm * TM + b * 16 + r;
         const f32x4 o = out4(t, b, sc, bi, cs);
-        if (m < M && n < a.N) store_y4(a.y, a.yt, (int64_t)m * a.ldy + n, o, yvec && nvalid == 4, nvalid);
+        if (m < M && n < a.N) store_y4(a.y, a.yt, base + (int64_t)m * ld + n, o, yvec && nvalid == 4, nvalid);
       }
     }
   }
@@ -829,7 +850,6 @@ __global__ __launch_bounds__(KG* WN* WM * 64, (SK ? (dl_min_waves<I8, XT, BN, BM
     constexpr int CPR = BN * 2 / 16;  // 16-byte chunks per output row of the block
     constexpr int NT = WN * WM * 64;
     static_assert((BM * CPR) % NT == 0, "output chunks split evenly over the threads");
-    const bool y16 = a.flags & 8;  // y and its row stride 16-byte aligned
     uint16_t* const y2 = (uint16_t*)a.y;
 #pragma unroll
     for (int p = 0; p < BM * CPR / NT; ++p) {
@@ -838,9 +858,17 @@ __global__ __launch_bounds__(KG* WN* WM * 64, (SK ? (dl_min_waves<I8, XT, BN, BM
       const int m = m0 + ml, n = nt0 * 16 + ch * 8;
       if (m >= M || n >= a.N) continue;
       const u32x4 v = *(const u32x4*)(lds + ml * ERS + ch * 16);
-      uint16_t* const yp = y2 + (int64_t)m * a.ldy + n;
-      if (y16 && n + 8 <= a.N) {
+      uint16_t* const yp = y2 + yb + (int64_t)m * yld + n;
+      if (wide && n + 8 <= a.N) {
         *(u32x4*)yp = v;
+      } else if (a.parts) {  // 4 columns at a time (widths and first columns are multiples of 4)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          if (n + 4 * e >= a.N) continue;
+          const u32x2 pe = a.parts[(n >> 2) + e];
+          *(u32x2*)(y2 + part_base(pe.y, M) + (int64_t)m * pe.x + n + 4 * e) =
+              e ? (u32x2){v.z, v.w} : (u32x2){v.x, v.y};
+        }
       } else {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -1325,7 +1353,7 @@ inline int y16_flag(const void* y, int yt, int64_t ldy) {
 
 int launch_gemm_w8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, bool xvec, const uint8_t* packed,
                    const float* scale, const float* bias, int64_t N, void* y, int yt, int64_t ldy, void* ws,
-                   int64_t ws_bytes, hipStream_t st, bool yvec) {
+                   int64_t ws_bytes, hipStream_t st, bool yvec, const u32x2* parts) {
   const int64_t Nt = (N + 15) / 16, Kc = (K + 63) / 64;
   const int flags = (xvec ? 1 : 0) | (yvec ? 2 : 0) | y16_flag(y, yt, ldy);
   // the direct-to-LDS path addresses a block's rows and tiles with 32-bit offsets
@@ -1336,7 +1364,7 @@ int launch_gemm_w8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, boo
     GemmArgs a{};
     a.x = x; a.ldx = ldx; a.M = (int)M; a.Kc = (int)Kc;
     a.packed = packed; a.scale = scale; a.bias = bias;
-    a.N = (int)N; a.Nt = (int)Nt; a.y = y; a.yt = yt; a.ldy = ldy; a.flags = flags;
+    a.N = (int)N; a.Nt = (int)Nt; a.y = y; a.yt = yt; a.ldy = ldy; a.parts = parts; a.flags = flags;
     const int gxt = staged ? XT_F16 : xt;  // fp32 / bf16 activations are staged as an fp16 plane
     // split K when the grid is small and the scratch after the layout holds the partials
     const DlPlan plan = plan_gemm_dl(false, gxt, M, Nt, Kc, staged);
@@ -1372,9 +1400,9 @@ int launch_gemm_w8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, boo
   }
   dim3 grid((unsigned)((Nt + kBN / 16 - 1) / (kBN / 16)), (unsigned)((M + kBM - 1) / kBM)), block(kWN * kWM * 64);
   switch (xt) {
-    case XT_F16: hipLaunchKernelGGL((gemm_w8_kernel<XT_F16, kBN, kBM, kWN, kWM>), grid, block, 0, st, x, ldx, (int)M, (int)K, (int)Kc, packed, scale, bias, (int)N, (int)Nt, y, yt, ldy, flags); break;
-    case XT_BF16: hipLaunchKernelGGL((gemm_w8_kernel<XT_BF16, kBN, kBM, kWN, kWM>), grid, block, 0, st, x, ldx, (int)M, (int)K, (int)Kc, packed, scale, bias, (int)N, (int)Nt, y, yt, ldy, flags); break;
-    case XT_F32: hipLaunchKernelGGL((gemm_w8_kernel<XT_F32, kBN, kBM, kWN, kWM>), grid, block, 0, st, x, ldx, (int)M, (int)K, (int)Kc, packed, scale, bias, (int)N, (int)Nt, y, yt, ldy, flags); break;
+    case XT_F16: hipLaunchKernelGGL((gemm_w8_kernel<XT_F16, kBN, kBM, kWN, kWM>), grid, block, 0, st, x, ldx, (int)M, (int)K, (int)Kc, packed, scale, bias, (int)N, (int)Nt, y, yt, ldy, parts, flags); break;
+    case XT_BF16: hipLaunchKernelGGL((gemm_w8_kernel<XT_BF16, kBN, kBM, kWN, kWM>), grid, block, 0, st, x, ldx, (int)M, (int)K, (int)Kc, packed, scale, bias, (int)N, (int)Nt, y, yt, ldy, parts, flags); break;
+    case XT_F32: hipLaunchKernelGGL((gemm_w8_kernel<XT_F32, kBN, kBM, kWN, kWM>), grid, block, 0, st, x, ldx, (int)M, (int)K, (int)Kc, packed, scale, bias, (int)N, (int)Nt, y, yt, ldy, parts, flags); break;
     default: return -2;
   }
   return check_launch();
@@ -1383,7 +1411,7 @@ int launch_gemm_w8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, boo
 int launch_gemm_w8a8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, bool xvec, const uint8_t* packed,
                      const float* scale, const int32_t* colsum, const float* bias, int64_t N, void* y, int yt,
                      int64_t ldy, int32_t* acc_out, float2* partials, int8_t* xq, float* qpbuf, hipStream_t st,
-                     bool yvec, uint8_t* split, int64_t split_bytes) {
+                     bool yvec, uint8_t* split, int64_t split_bytes, const u32x2* parts) {
   const int64_t Nt = (N + 15) / 16, Kc = (K + 63) / 64, Kp = Kc * 64;
   if (Kp > ((int64_t)1 << 21)) return -1;  // 32-bit block offsets of the direct-to-LDS GEMM
   GemmArgs a{};
@@ -1450,14 +1478,14 @@ int launch_gemm_w8a8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, b
     GemvArgs g{};
     g.x = xq; g.ldx = Kp; g.M = (int)M; g.K = (int)Kp; g.Kc = (int)Kc;
     g.packed = packed; g.scale = scale; g.bias = bias; g.colsum = colsum;
-    g.N = (int)N; g.Nt = (int)Nt; g.y = y; g.yt = yt; g.ldy = ldy; g.acc_out = acc_out; g.qpbuf = qpbuf;
+    g.N = (int)N; g.Nt = (int)Nt; g.y = y; g.yt = yt; g.ldy = ldy; g.parts = parts; g.acc_out = acc_out; g.qpbuf = qpbuf;
     g.flags = kGemvXVec | (yvec ? kGemvYVec : 0);
     rc = launch_gemv_mt(g, XT_S8, st, alt);
     if (rc != -1) return rc;
   }
   a.x = xq; a.ldx = Kp; a.M = (int)M; a.Kc = (int)Kc;
   a.packed = packed; a.scale = scale; a.bias = bias; a.colsum = colsum;
-  a.N = (int)N; a.Nt = (int)Nt; a.y = y; a.yt = yt; a.ldy = ldy; a.acc_out = acc_out; a.qpbuf = qpbuf;
+  a.N = (int)N; a.Nt = (int)Nt; a.y = y; a.yt = yt; a.ldy = ldy; a.parts = parts; a.acc_out = acc_out; a.qpbuf = qpbuf;
   a.flags = flags;
   return launch_gemm_dl_cfg(id, true, XT_F16, a, st);
 }

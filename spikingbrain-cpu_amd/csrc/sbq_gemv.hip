@@ -157,7 +157,8 @@ __device__ __forceinline__ void reduce_store(const GemvArgs& a, int grp, int lan
           o[v] = out;
         }
       }
-      store_y4(a.y, a.yt, (int64_t)m * a.ldy + n, o, (a.flags & 2) && nvalid == 4, nvalid);
+      const u32x2 pe = a.parts ? a.parts[n >> 2] : u32x2{0u, 0u};
+      store_y4(a.y, a.yt, y_offset(a.parts, pe, a.M, a.ldy, m, n), o, (a.flags & 2) && nvalid == 4, nvalid);
     }
   }
   __syncthreads();  // the next group reuses the reduction buffer
@@ -553,14 +554,14 @@ static GemvArgs with_argmax(GemvArgs a, const GemvArgmaxOut* am) {
 
 int launch_gemv_w8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, bool xvec, const uint8_t* packed,
                    const float* scale, const float* bias, int64_t N, void* y, int yt, int64_t ldy, hipStream_t st,
-                   bool yvec, GemvArgmaxOut* am) {
+                   bool yvec, GemvArgmaxOut* am, const u32x2* parts) {
   const int64_t Nt = (N + 15) / 16, Kc = (K + 63) / 64;
   const GemvCfg c = pick_gemv(M, Nt, Kc, false, xt);
   if (!c.ok) return -1;
   GemvArgs a{};
   a.x = x; a.ldx = ldx; a.M = (int)M; a.K = (int)K; a.Kc = (int)Kc;
   a.packed = packed; a.scale = scale; a.bias = bias;
-  a.N = (int)N; a.Nt = (int)Nt; a.y = y; a.yt = yt; a.ldy = ldy;
+  a.N = (int)N; a.Nt = (int)Nt; a.y = y; a.yt = yt; a.ldy = ldy; a.parts = parts;
   a.flags = (xvec ? 1 : 0) | (yvec ? 2 : 0);
   int fid, fks;
   if (pick_gemv_fast(M, K, N, xt, false, xvec, &fid, &fks)) {
@@ -583,11 +584,11 @@ int launch_gemv_w8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, boo
 // bf16 x with aligned rows, 64 | K); -1 when that path does not apply.
 int launch_gemv_w8_mt(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, bool xvec, const uint8_t* packed,
                       const float* scale, const float* bias, int64_t N, void* y, int yt, int64_t ldy, hipStream_t st,
-                      bool yvec, bool gemm_alt) {
+                      bool yvec, bool gemm_alt, const u32x2* parts) {
   GemvArgs a{};
   a.x = x; a.ldx = ldx; a.M = (int)M; a.K = (int)K; a.Kc = (int)((K + 63) / 64);
   a.packed = packed; a.scale = scale; a.bias = bias;
-  a.N = (int)N; a.Nt = (int)((N + 15) / 16); a.y = y; a.yt = yt; a.ldy = ldy;
+  a.N = (int)N; a.Nt = (int)((N + 15) / 16); a.y = y; a.yt = yt; a.ldy = ldy; a.parts = parts;
   a.flags = (xvec ? kGemvXVec : 0) | (yvec ? kGemvYVec : 0);
   return launch_gemv_mt(a, xt, st, gemm_alt);
 }
@@ -615,14 +616,14 @@ int launch_gemv_w8_grouped(const GemvSeg* segs, int n, int xt, int64_t M, int64_
 int launch_gemv_w8a8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, bool xvec, const uint8_t* packed,
                      const float* scale, const int32_t* colsum, const float* bias, int64_t N, void* y, int yt,
                      int64_t ldy, int32_t* acc_out, float2* partials, hipStream_t st, bool yvec,
-                     GemvArgmaxOut* am) {
+                     GemvArgmaxOut* am, const u32x2* parts) {
   const int64_t Nt = (N + 15) / 16, Kc = (K + 63) / 64;
   const GemvCfg c = pick_gemv(M, Nt, Kc, true, xt);
   if (!c.ok) return -1;
   GemvArgs a{};
   a.x = x; a.ldx = ldx; a.M = (int)M; a.K = (int)K; a.Kc = (int)Kc;
   a.packed = packed; a.scale = scale; a.bias = bias; a.colsum = colsum;
-  a.N = (int)N; a.Nt = (int)Nt; a.y = y; a.yt = yt; a.ldy = ldy; a.acc_out = acc_out;
+  a.N = (int)N; a.Nt = (int)Nt; a.y = y; a.yt = yt; a.ldy = ldy; a.acc_out = acc_out; a.parts = parts;
   a.flags = (xvec ? 1 : 0) | (yvec ? 2 : 0);
   int fid, fks;
   const bool fast = pick_gemv_fast(M, K, N, xt, true, xvec, &fid, &fks);

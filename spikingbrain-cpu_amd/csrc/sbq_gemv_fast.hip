@@ -265,7 +265,9 @@ __global__ __launch_bounds__(kFastMaxWaves * 64) void gemv_fast_kernel(GemvArgs 
   const int ne = nte * 16 + 4 * g;
   f32x4 sc = {0.f, 0.f, 0.f, 0.f}, bi = {0.f, 0.f, 0.f, 0.f};
   i32x4 cs = {0, 0, 0, 0};
+  u32x2 pe = {0u, 0u};
   if (ks < G) {
+    if (a.parts) pe = a.parts[min(ne, a.N - 4) >> 2];
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int nn = min(ne + v, a.N - 1);
@@ -666,7 +668,7 @@ __global__ __launch_bounds__(kFastMaxWaves * 64) void gemv_fast_kernel(GemvArgs 
         o[v] = out;
       }
     }
-    store_y4(a.y, a.yt, (int64_t)r * a.ldy + n, o, (a.flags & kGemvYVec) && nvalid == 4, nvalid);
+    store_y4(a.y, a.yt, y_offset(a.parts, pe, M, a.ldy, r, n), o, (a.flags & kGemvYVec) && nvalid == 4, nvalid);
     if (am) {  // fp32 y: the key of each stored value
 #pragma unroll
       for (int v = 0; v < 4; ++v)
@@ -709,7 +711,9 @@ __global__ __launch_bounds__(kFastMaxWaves * 64) void gemv_mt_kernel(GemvArgs a,
   const int ne = nte * 16 + 4 * g;
   f32x4 sc = {0.f, 0.f, 0.f, 0.f}, bi = {0.f, 0.f, 0.f, 0.f};
   i32x4 cs = {0, 0, 0, 0};
+  u32x2 pe = {0u, 0u};
   if (ks < G) {
+    if (a.parts) pe = a.parts[min(ne, a.N - 4) >> 2];
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int nn = min(ne + v, a.N - 1);
@@ -832,7 +836,7 @@ __global__ __launch_bounds__(kFastMaxWaves * 64) void gemv_mt_kernel(GemvArgs a,
         o[v] = out;
       }
     }
-    store_y4(a.y, a.yt, (int64_t)m * a.ldy + n, o, yvec, nvalid);
+    store_y4(a.y, a.yt, y_offset(a.parts, pe, M, a.ldy, m, n), o, yvec, nvalid);
   }
 }
 

@@ -35,6 +35,7 @@ struct GemvArgs {
   void* y;
   int yt;
   int64_t ldy;
+  const u32x2* parts;  // y stored as parts (part_base), one entry per 4 columns; null: rows of stride ldy
   int32_t* acc_out;
   const float2* partials;
   int nparts;

@@ -48,6 +48,20 @@ SBQ_HD unsigned argmax_slot_members(unsigned nblk, unsigned slot, unsigned slots
 }
 SBQ_HD unsigned argmax_slots_used(unsigned nblk, unsigned slots) { return nblk < slots ? nblk : slots; }
 
+// Outputs stored as parts: the columns of y [M, N] belong to consecutive parts
+// (widths multiples of 4), and part p is a dense [M, width] matrix that starts
+// at element M * pstart, pstart the part's first column with every earlier
+// width rounded up to 64 columns (so parts start 64 elements apart at least,
+// aligned for vector stores).  The table holds two words per 4 columns: the
+// part's width, and start / 4 | ((pstart - start) / 4) << kPartPadShift.
+// Element offset of column n = of the part holding it: part_base + m * width + n.
+constexpr int kPartPadShift = 20;
+SBQ_HD int64_t part_base(uint32_t word, int64_t M) {
+  const int64_t start = (int64_t)(word & ((1u << kPartPadShift) - 1u)) * 4;
+  const int64_t pstart = start + (int64_t)(word >> kPartPadShift) * 4;
+  return M * pstart - start;
+}
+
 // Column index of a key from argmax_key.
 SBQ_HD int argmax_key_index(unsigned long long key) { return (int)(0xffffffffu - (uint32_t)key); }
 

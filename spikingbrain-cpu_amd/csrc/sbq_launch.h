@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "sbq_common.h"
+
 namespace sbq {
 
 inline int check_launch() {
@@ -57,7 +59,7 @@ bool gemv_mt_applies(int64_t M, int64_t K, int64_t N, int xt, bool gemm_alt);
 int launch_gemv_mt(const GemvArgs& a, int xt, hipStream_t st, bool gemm_alt);
 int launch_gemv_w8_mt(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, bool xvec, const uint8_t* packed,
                       const float* scale, const float* bias, int64_t N, void* y, int yt, int64_t ldy, hipStream_t st,
-                      bool yvec, bool gemm_alt);
+                      bool yvec, bool gemm_alt, const u32x2* parts = nullptr);
 // Grouped launch: a.seg / a.nseg hold 2..kGemvMaxSeg linears (w8a8: int8-dyn
 // with the activation min/max reduced in the kernel).
 int launch_gemv_fast_grouped(int id, int ks, GemvArgs a, int xt, bool w8a8, hipStream_t st);
@@ -77,18 +79,20 @@ struct GemvArgmaxOut {
   bool fused;
 };
 
+// parts (the linear launchers below): y stored as parts (part_base in
+// sbq_index.h), one table entry per 4 columns; null: rows of stride ldy.
 // Weight-only linear.  xvec: x and every row of x start 16-byte aligned (vector
 // loads allowed).  yvec: y rows are 16-byte aligned and N % 4 == 0.
 int launch_gemv_w8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, bool xvec, const uint8_t* packed,
                    const float* scale, const float* bias, int64_t N, void* y, int yt, int64_t ldy, hipStream_t st,
-                   bool yvec, GemvArgmaxOut* am = nullptr);
+                   bool yvec, GemvArgmaxOut* am = nullptr, const u32x2* parts = nullptr);
 // ws: device scratch (nullable, 256-byte aligned) of ws_bytes bytes, laid out
 // by w8_ws_layout.  With enough of it the fp16 GEMM takes its per-row sums of x
 // from a pre-pass, and fp32 / bf16 activations are staged as a scaled fp16
 // plane for the same GEMM.
 int launch_gemm_w8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, bool xvec, const uint8_t* packed,
                    const float* scale, const float* bias, int64_t N, void* y, int yt, int64_t ldy, void* ws,
-                   int64_t ws_bytes, hipStream_t st, bool yvec);
+                   int64_t ws_bytes, hipStream_t st, bool yvec, const u32x2* parts = nullptr);
 // split: scratch after the workspace's layout (split_area_bytes of the plan;
 // a shorter or null one runs the shape without splitting K).
 // Direct-to-LDS GEMM plan: block configuration id and K splits (1: none);
@@ -132,12 +136,13 @@ int launch_stage_act(const void* x, int xt, int64_t ldx, int64_t M, int64_t K, _
 int launch_gemv_w8a8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, bool xvec, const uint8_t* packed,
                      const float* scale, const int32_t* colsum, const float* bias, int64_t N, void* y, int yt,
                      int64_t ldy, int32_t* acc_out, float2* partials, hipStream_t st, bool yvec,
-                     GemvArgmaxOut* am = nullptr);
+                     GemvArgmaxOut* am = nullptr, const u32x2* parts = nullptr);
 // The GEMM quantizes x once into xq (s8 [M][Kc*64]) and writes (s_x, zp) to
 // qpbuf[0..1] (zp as int bits) before the tiled pipeline reads them.
 int launch_gemm_w8a8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, bool xvec, const uint8_t* packed,
                      const float* scale, const int32_t* colsum, const float* bias, int64_t N, void* y, int yt,
                      int64_t ldy, int32_t* acc_out, float2* partials, int8_t* xq, float* qpbuf, hipStream_t st,
-                     bool yvec, uint8_t* split = nullptr, int64_t split_bytes = 0);
+                     bool yvec, uint8_t* split = nullptr, int64_t split_bytes = 0,
+                     const u32x2* parts = nullptr);
 
 }  // namespace sbq

@@ -340,6 +340,56 @@ def gemm_config(M: int, N: int, K: int, dtype: torch.dtype = torch.float16, w8a8
     return rc, splits.value
 
 
+def _parts_table(sizes: list[int]) -> tuple[torch.Tensor | None, list[int]]:
+    """(the column table of sbq_linear_w8_parts on the CPU, or None when the
+    widths do not fit it; the parts' padded first columns and, last, the
+    padded width of all of them)."""
+    pstart = [0]
+    for w in sizes:
+        pstart.append(pstart[-1] + (w + 63) // 64 * 64)
+    N = sum(sizes)
+    if any(w % 4 or w < 4 for w in sizes) or N >= 1 << 22 or pstart[-2] - (N - sizes[-1]) >= 1 << 14:
+        return None, pstart
+    rows, start = [], 0
+    for w, p in zip(sizes, pstart):
+        word = start // 4 | (p - start) // 4 << 20
+        rows.append((w, word - (1 << 32) if word >= 1 << 31 else word))
+        start += w
+    return torch.tensor(rows, dtype=torch.int32).repeat_interleave(torch.tensor([w // 4 for w in sizes]), 0), pstart
+
+
+def _linear_parts(x2: torch.Tensor, packed: torch.Tensor, scale: torch.Tensor, colsum: torch.Tensor | None,
+                  bias: torch.Tensor | None, N: int, parts: torch.Tensor, width: int,
+                  out_dtype: torch.dtype) -> torch.Tensor:
+    """linear_w8 (colsum None) or linear_w8a8 with the columns stored as the
+    parts of `parts` (_parts_table): the flat [M * width] result, part p at
+    element M * pstart[p]."""
+    x2 = _as_activation(x2)
+    M, K = x2.shape
+    y = torch.empty((M * width,), dtype=out_dtype, device=x2.device)
+    if colsum is None:
+        ws = w8_workspace(M, K, x2.device, x2.dtype, N) if M > 16 else None
+        vectors = (("scale", scale, torch.float32), ("bias", bias, torch.float32))
+    else:
+        ws = w8a8_workspace(M, K, x2.device, N, x2.dtype)
+        vectors = (("scale", scale, torch.float32), ("bias", bias, torch.float32), ("colsum", colsum, torch.int32))
+    _check_operands("linear_parts", x2, packed, N, y[:M * N].view(M, N), vectors, ws)
+    if parts.dtype != torch.int32 or parts.device != x2.device or not parts.is_contiguous() or parts.numel() * 2 != N:
+        raise ValueError(f"linear_parts: parts must be a contiguous int32 [N/4, 2] table on {x2.device}")
+    L = _lib.load()
+    with torch.cuda.device(x2.device):
+        if colsum is None:
+            rc = L.sbq_linear_w8_parts(_ptr(x2), _code(x2.dtype), M, K, _ldx(x2), _ptr(packed), _ptr(scale), _ptr(bias),
+                                       N, _ptr(y), _code(y.dtype), _ptr(parts), _ptr(ws), _nbytes(ws),
+                                       _stream(x2.device))
+        else:
+            rc = L.sbq_linear_w8a8_parts(_ptr(x2), _code(x2.dtype), M, K, _ldx(x2), _ptr(packed), _ptr(scale),
+                                         _ptr(colsum), _ptr(bias), N, _ptr(y), _code(y.dtype), _ptr(parts), _ptr(ws),
+                                         _nbytes(ws), _stream(x2.device))
+        _lib.check(rc, "sbq_linear_parts")
+    return y
+
+
 def w8a8_workspace(M: int, K: int, device: torch.device, N: int | None = None,
                    dtype: torch.dtype = torch.float16) -> torch.Tensor:
     """Scratch for the int8-dyn paths; with N, also the split-K partials of
@@ -929,7 +979,8 @@ class FusedLinear(_Fp32Buffers, nn.Module):
     bit-identical to the separate layers' (one activation quantization for the
     same x, exact int32 sums), int8 outputs agree to fp32 summation order.
 
-    forward(x) returns one tensor per part (contiguous, like the parts').
+    forward(x) returns one tensor per part (contiguous, like the parts'; the
+    parts of one call are slices of one allocation).
     part(i) is a drop-in module for part i: the parts of one call sequence
     share the result of one launch.  The first part called on an input
     launches; the other parts called on the same tensor object (same address,
@@ -970,6 +1021,8 @@ class FusedLinear(_Fp32Buffers, nn.Module):
         self.register_buffer("scale", scale, persistent=False)
         self.register_buffer("colsum", colsum, persistent=False)
         self.register_buffer("bias", bias, persistent=False)
+        table, self._pstart = _parts_table(self.sizes)
+        self.register_buffer("_parts", None if table is None else table.to(device), persistent=False)
         self.out_dtype = torch.float32
         self._memo_ref = None
         self._memo_key = None
@@ -980,15 +1033,25 @@ class FusedLinear(_Fp32Buffers, nn.Module):
         _check_in_features(x, self.in_features)
         shape = x.shape
 
+        M = x.numel() // shape[-1]
+        # several rows: the launch stores each part contiguous (one row's
+        # slices are contiguous already)
+        direct = M > 1 and self._parts is not None
+
         def run(xd):
             x2 = xd.reshape(-1, shape[-1])
             scale = self.scale.float()
             bias = None if self.bias is None else self.bias.float()
+            if direct:
+                return _linear_parts(x2, self.packed, scale, self.colsum, bias, self.out_features, self._parts,
+                                     self._pstart[-1], self.out_dtype)
             if self.w8a8:
                 return linear_w8a8(x2, self.packed, scale, self.colsum, bias, self.out_features, self.out_dtype)
             return linear_w8(x2, self.packed, scale, bias, self.out_features, self.out_dtype)
 
         y = _run_on_device(x, self.packed.device, run)
+        if direct:
+            return tuple(y[M * p:M * (p + w)].view(*shape[:-1], w) for p, w in zip(self._pstart, self.sizes))
         outs = torch.split(y, self.sizes, dim=-1)
         return tuple(o.contiguous().reshape(*shape[:-1], o.shape[-1]) for o in outs)
 

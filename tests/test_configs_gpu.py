@@ -371,6 +371,43 @@ def test_fused_hybrid_group_vs_oracle(dev, fmt, M):
             np.testing.assert_array_equal(po.cpu().numpy(), o.cpu().numpy())
 
 
+# (M, K, sizes): every kernel that stores parts (the decode GEMV, the general
+# GEMV, the row-tile GEMV, the split and the unsplit GEMM, the register-staged
+# GEMM), parts narrower than a tile, across tiles and blocks, odd M (part
+# bases), and one width that no table holds (the copying path).
+PARTS_CASES = [(2, 256, (4, 20, 64, 100)), (5, 4096, (1024, 4, 512)), (8, 2560, (4096, 128, 4, 1028)),
+               (16, 512, (36, 36, 36)), (21, 1000, (60, 4, 200)), (24, 1024, (512, 4, 508)), (47, 4096, (132, 1000)),
+               (70, 1000, (60, 4, 200)), (77, 2560, (640, 4, 260, 1024)), (128, 4096, (4096, 4, 64)),
+               (131, 512, (4, 2000, 12, 3000)), (513, 2560, (4096, 128, 4, 4096)), (33, 512, (6, 58, 64))]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", ["int8", "int8-dyn"])
+@pytest.mark.parametrize("M,K,sizes", PARTS_CASES)
+def test_fused_parts_layout(dev, fmt, M, K, sizes):
+    """A fused layer's outputs, stored part by part, equal the slices of the
+    same launch storing whole rows (linear_w8 / linear_w8a8 on the fused
+    operands), bit for bit, for every activation and output dtype."""
+    announce(f"fused parts layout {fmt} M={M} K={K} sizes={sizes}")
+    bias = cpu_x(1, sizes[0], 5).reshape(-1)
+    fused = quant.fuse_linears([quant.make_linear(fmt, gpu_weight(n, K, 30 + i, dev), bias.to(dev) if i == 0 else None)
+                                for i, n in enumerate(sizes)])
+    N = sum(sizes)
+    for xdt, ydt in ((torch.float32, torch.float32), (torch.float16, torch.float16), (torch.bfloat16, torch.bfloat16),
+                     (torch.float16, torch.float32)):
+        fused.out_dtype = ydt
+        x = cpu_x(M, K, 31).to(xdt).to(dev)
+        if fmt == "int8":
+            rows = quant.linear_w8(x, fused.packed, fused.scale, fused.bias, N, ydt)
+        else:
+            rows = quant.linear_w8a8(x, fused.packed, fused.scale, fused.colsum, fused.bias, N, ydt)
+        outs = fused(x.reshape(1, M, K))
+        assert len(outs) == len(sizes)
+        for o, want in zip(outs, torch.split(rows, list(sizes), dim=-1)):
+            assert o.is_contiguous() and o.shape == (1, *want.shape) and o.dtype == ydt
+            assert torch.equal(o[0], want), (xdt, ydt, want.shape)
+
+
 @pytest.mark.gpu
 def test_fused_parts_share_one_launch_per_call_sequence(dev):
     """FusedLinear.part(i) drop-ins under torch.inference_mode() (inference
