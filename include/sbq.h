@@ -143,7 +143,10 @@ int sbq_linear_w8(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
  * y: device, 16-byte aligned, M * (sum of the widths, each rounded up to 64)
  * elements.  parts: device int32 [N/4][2], per 4 columns the width of their
  * part and start/4 | ((pstart - start)/4) << 20 (so N < 2^22, and padding
- * below 2^14 columns in all).  Everything else as sbq_linear_w8. */
+ * below 2^14 columns before any part), written by sbq_parts_table from the
+ * widths (a host array; SBQ_ERR_ARG when they do not fit the table).
+ * Everything else as sbq_linear_w8. */
+int sbq_parts_table(const int64_t* widths, int count, int32_t* parts, void* stream);
 int sbq_linear_w8_parts(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
                         const uint8_t* packed, const float* scale, const float* bias, int64_t N,
                         void* y, int y_dtype, const int32_t* parts,

@@ -82,7 +82,7 @@ int linear_w8a8_run(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ld
   const bool mt = w8a8_runs_mt(M, N, K, split ? split_bytes : 0);
   if (!mt && sbq::gemv_supports(M, K, true, x_dtype))
     return sbq::launch_gemv_w8a8(x, x_dtype, M, K, ldx, xv, packed, scale, colsum, bias, N, y, y_dtype, ldy, acc_out,
-                                 parts, st, yv, nullptr, yparts);
+                                 parts, xq, qp, st, yv, nullptr, yparts);
   return sbq::launch_gemm_w8a8(x, x_dtype, M, K, ldx, xv, packed, scale, colsum, bias, N, y, y_dtype, ldy, acc_out,
                                parts, xq, qp, st, yv, split, split_bytes, yparts);
 }
@@ -238,6 +238,35 @@ int sbq_linear_w8(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
   if (rc || M == 0) return rc;
   return linear_w8_run(x, x_dtype, M, K, ldx, packed, scale, bias, N, y, y_dtype, ldy, workspace, workspace_bytes,
                        (hipStream_t)stream);
+}
+
+int sbq_parts_table(const int64_t* widths, int count, int32_t* parts, void* stream) {
+  if (count < 1 || !widths || !parts) return SBQ_ERR_ARG;
+  if (!aligned(parts, 8)) return SBQ_ERR_ALIGN;
+  int64_t start = 0, pstart = 0;
+  for (int i = 0; i < count; ++i) {
+    if (widths[i] < 4 || widths[i] % 4 || widths[i] > kIntMax) return SBQ_ERR_ARG;
+    if (pstart - start >= (int64_t)4 << (32 - sbq::kPartPadShift)) return SBQ_ERR_ARG;
+    start += widths[i];
+    pstart += (widths[i] + 63) / 64 * 64;
+    if (start >= (int64_t)4 << sbq::kPartPadShift) return SBQ_ERR_ARG;
+  }
+  start = pstart = 0;
+  for (int g0 = 0; g0 < count; g0 += sbq::kPartsFill) {
+    sbq::PartsFill f{};
+    const uint32_t begin4 = (uint32_t)(start / 4);
+    for (int i = g0; i < count && i < g0 + sbq::kPartsFill; ++i) {
+      const int p = f.count++;
+      f.width[p] = (uint32_t)widths[i];
+      f.word[p] = (uint32_t)(start / 4) | (uint32_t)((pstart - start) / 4) << sbq::kPartPadShift;
+      start += widths[i];
+      pstart += (widths[i] + 63) / 64 * 64;
+      f.end4[p] = (uint32_t)(start / 4);
+    }
+    const int rc = sbq::launch_parts_fill(f, begin4, parts, (hipStream_t)stream);
+    if (rc) return rc;
+  }
+  return SBQ_OK;
 }
 
 int sbq_linear_w8_parts(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, const uint8_t* packed,
@@ -442,7 +471,18 @@ int sbq_linear_w8a8_grouped(int count, const void* const* x, const int64_t* ldx,
       segs[i].N = (int)N[i];
       segs[i].Nt = (int)((N[i] + 15) / 16);
     }
-    const int rc = sbq::launch_gemv_w8_grouped(segs, count, x_dtype, M, K, xv, y_dtype, yv, st, true);
+    // `count` workspaces' worth of scratch lets inputs beyond the fused
+    // capacity be quantized together, each into its own share
+    const int64_t share = sbq_w8a8_workspace_bytes(M, K);
+    int8_t* xq[SBQ_MAX_GROUP];
+    float* qp[SBQ_MAX_GROUP];
+    for (int i = 0; i < count; ++i) {
+      xq[i] = ws_xq((uint8_t*)workspace + i * share);
+      qp[i] = ws_qp((uint8_t*)workspace + i * share);
+    }
+    const bool own = (int64_t)workspace_bytes >= count * share;
+    const int rc = sbq::launch_gemv_w8_grouped(segs, count, x_dtype, M, K, xv, y_dtype, yv, st, true,
+                                               own ? xq : nullptr, own ? qp : nullptr);
     if (rc != -1) return rc;
   }
   // one by one (stream order lets the calls share the workspace)
@@ -512,7 +552,7 @@ int sbq_linear_w8a8_argmax(const void* x, int x_dtype, int64_t M, int64_t K, int
   // own routes (bit-identical logits either way), then the row argmax
   if (M <= 16 && sbq::gemv_supports(M, K, true, x_dtype))
     rc = sbq::launch_gemv_w8a8(x, x_dtype, M, K, ldx, xv, packed, scale, colsum, bias, N, y, SBQ_F32, ldy, nullptr,
-                               ws_partials(workspace), st, yv, &am);
+                               ws_partials(workspace), ws_xq(workspace), ws_qp(workspace), st, yv, &am);
   else
     rc = sbq_linear_w8a8(x, x_dtype, M, K, ldx, packed, scale, colsum, bias, N, y, SBQ_F32, ldy, nullptr, workspace,
                          workspace_bytes, stream);

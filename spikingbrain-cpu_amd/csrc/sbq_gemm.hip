@@ -1408,27 +1408,145 @@ int launch_gemm_w8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, boo
   return check_launch();
 }
 
-int launch_gemm_w8a8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, bool xvec, const uint8_t* packed,
-                     const float* scale, const int32_t* colsum, const float* bias, int64_t N, void* y, int yt,
-                     int64_t ldy, int32_t* acc_out, float2* partials, int8_t* xq, float* qpbuf, hipStream_t st,
-                     bool yvec, uint8_t* split, int64_t split_bytes, const u32x2* parts) {
-  const int64_t Nt = (N + 15) / 16, Kc = (K + 63) / 64, Kp = Kc * 64;
-  if (Kp > ((int64_t)1 << 21)) return -1;  // 32-bit block offsets of the direct-to-LDS GEMM
-  GemmArgs a{};
-  const DlPlan plan = plan_gemm_dl(true, XT_F16, M, Nt, Kc, true);
-  int ncount = 0;
-  uint32_t* zero = attach_split(a, plan, split, split_bytes, &ncount);
-  const int id = zero || plan.splits == 1 ? plan.id : pick_gemm_dl(true, XT_F16, M, Nt, Kc);
+// Per-tensor quantization of up to SBQ_MAX_GROUP small inputs in one launch,
+// one workgroup each (rows 16-byte aligned, 64 | K, at most C * 16 KiB of x):
+// the workgroup holds its whole x in registers, so the (s_x, zp) and the s8
+// rows xq - 128 take one launch instead of two (min/max partials, then
+// quantize).  Bound by one CU's load path and the chain load - reduce -
+// parameters - store.  Values and parameters are the two-launch path's, bit
+// for bit (min and max do not depend on order).  DENSE: rows of stride K.
+// Measured (K = 2560 ... 12288): 24-80 KiB of x 2.9-3.3 us, 128 KiB 3.7,
+// 256-320 KiB 5.5-5.8, against 2.6 (min/max) + 1.1 (gap) + 2.5-3 us.
+template <int XT, int C, bool DENSE>
+__global__ __launch_bounds__(1024) void quantize_small_kernel(QuantSmall a) {
+  constexpr int NE = 16 / x_bytes<XT>();  // values per 16-byte chunk
+  typedef typename XElem<XT>::T T;
+  typedef T vN __attribute__((ext_vector_type(NE)));
+  __shared__ float2 red[16];
+  __shared__ float qs[3];
+  const void* x = a.x[0];
+  int64_t ldx = a.ldx[0];
+  int8_t* xq = a.xq[0];
+  float* qpbuf = a.qpbuf[0];
+#pragma unroll
+  for (int i = 1; i < kGemvMaxSeg; ++i)  // constant indexes only: a runtime index moves the struct to scratch
+    if ((int)blockIdx.x == i) {
+      x = a.x[i];
+      ldx = a.ldx[i];
+      xq = a.xq[i];
+      qpbuf = a.qpbuf[i];
+    }
+  const int t = threadIdx.x, lane = t & 63, cpr = a.K / NE, nch = a.M * cpr;
+  vN v[C];
+#pragma unroll
+  for (int i = 0; i < C; ++i) {  // clamped: surplus chunks repeat the last one and are not stored
+    const int c = min(t + i * 1024, nch - 1);
+    if constexpr (DENSE) {
+      v[i] = *((const vN*)x + c);
+    } else {
+      const int m = c / cpr;
+      v[i] = *(const vN*)((const T*)x + (int64_t)m * ldx + (c - m * cpr) * NE);
+    }
+  }
+  for (int i = t; i < a.nzero; i += 1024) a.zero[i] = 0u;
+  float mn = 0.0f, mx = 0.0f;  // fbgemm's range always holds 0
+#pragma unroll
+  for (int i = 0; i < C; ++i)
+#pragma unroll
+    for (int j = 0; j < NE; ++j) {
+      const float f = XElem<XT>::to_f32(v[i][j]);
+      mn = fminf(mn, f);
+      mx = fmaxf(mx, f);
+    }
+  mn = wave_min(mn);
+  mx = wave_max(mx);
+  if (lane == 0) red[t >> 6] = make_float2(mn, mx);
+  __syncthreads();
+  if (t < 64) {  // one wave: the double-precision parameter choice costs 16 waves four times its latency
+    const float2 r = red[lane & 15];
+    const ActQParams qp = choose_act_qparams(wave_min(r.x), wave_max(r.y));
+    if (t == 0) {
+      qs[0] = qp.inv;
+      qs[1] = qp.zpf;
+      qpbuf[0] = qp.scale;
+      qpbuf[1] = __int_as_float(qp.zp);
+    }
+  }
+  __syncthreads();
+  const float inv = qs[0], zpf = qs[1];
+  // the chunks stay as loaded: 2-byte values kept as the floats of the min /
+  // max pass would not fit the 128 registers of a 1024-thread workgroup
+#pragma unroll
+  for (int i = 0; i < C; ++i) asm("" : "+v"(v[i]));
+#pragma unroll
+  for (int i = 0; i < C; ++i) {
+    const int c = t + i * 1024;
+    uint32_t d[NE / 4];
+#pragma unroll
+    for (int w = 0; w < NE / 4; ++w)
+      d[w] = pack_act_s8x4(__builtin_fmaf(XElem<XT>::to_f32(v[i][4 * w]), inv, zpf),
+                           __builtin_fmaf(XElem<XT>::to_f32(v[i][4 * w + 1]), inv, zpf),
+                           __builtin_fmaf(XElem<XT>::to_f32(v[i][4 * w + 2]), inv, zpf),
+                           __builtin_fmaf(XElem<XT>::to_f32(v[i][4 * w + 3]), inv, zpf));
+    if (c < nch) {  // rows of K bytes: chunk c's values start at byte c * NE
+      if constexpr (NE == 4) *((uint32_t*)xq + c) = d[0];
+      else *((u32x2*)xq + c) = (u32x2){d[0], d[1]};
+    }
+  }
+}
+
+// x up to 320 KiB of fp32 or 160 KiB of 2-byte values (whose conversion, done
+// twice, costs more than the second launch beyond that: 304 KiB 7.9 us).
+bool quantize_small_fits(int64_t M, int64_t K, bool xvec) {
+  return xvec && K % 64 == 0 && M * K <= (int64_t)kQuantSmallChunks * 1024 * 4;
+}
+
+int launch_quantize_small(const QuantSmall& a, int count, int xt, hipStream_t st) {
+  const int64_t bytes = (int64_t)a.M * a.K * (xt == XT_F32 ? 4 : 2);
+  const int need = (int)((bytes + 1024 * 16 - 1) / (1024 * 16));
+  bool dense = true;
+  for (int i = 0; i < count; ++i) dense = dense && (a.ldx[i] == a.K || a.M == 1);
+  const dim3 grid((unsigned)count), block(1024);
+#define SBQ_QS(XT_, C_)                                                                             \
+  if (dense) hipLaunchKernelGGL((quantize_small_kernel<XT_, C_, true>), grid, block, 0, st, a);     \
+  else hipLaunchKernelGGL((quantize_small_kernel<XT_, C_, false>), grid, block, 0, st, a);
+#define SBQ_QS_XT(XT_)                      \
+  if (need <= 5) { SBQ_QS(XT_, 5) }         \
+  else if (need <= 10) { SBQ_QS(XT_, 10) }  \
+  else if constexpr (XT_ == XT_F32) { SBQ_QS(XT_, kQuantSmallChunks) } \
+  else return -1;
+  switch (xt) {
+    case XT_F32: SBQ_QS_XT(XT_F32) break;
+    case XT_F16: SBQ_QS_XT(XT_F16) break;
+    case XT_BF16: SBQ_QS_XT(XT_BF16) break;
+    default: return -2;
+  }
+#undef SBQ_QS_XT
+#undef SBQ_QS
+  return check_launch();
+}
+
+// s8 rows xq - 128 [M][Kp] and (s_x, zp) of fbgemm's per-tensor quantization
+// of x [M, K]; zero (nullable): counters to clear for the split-K GEMM after
+// it on the same stream.
+int launch_quantize_acts(const void* x, int xt, int64_t M, int64_t K, int64_t Kp, int64_t ldx, bool xvec,
+                         float2* partials, int8_t* xq, float* qpbuf, hipStream_t st, uint32_t* zero, int nzero) {
+  if (quantize_small_fits(M, K, xvec)) {
+    QuantSmall a{};
+    a.x[0] = x; a.ldx[0] = ldx; a.xq[0] = xq; a.qpbuf[0] = qpbuf;
+    a.M = (int)M; a.K = (int)K; a.zero = zero; a.nzero = nzero;
+    return launch_quantize_small(a, 1, xt, st);
+  }
   const int nparts = minmax_nparts(M, K);
-  const int prc = launch_minmax_partials(x, xt, M, K, ldx, partials, nparts, st, zero, ncount);
+  const int prc = launch_minmax_partials(x, xt, M, K, ldx, partials, nparts, st, zero, nzero);
   if (prc) return prc;
-  const int flags = (xvec ? 1 : 0) | (yvec ? 2 : 0) | y16_flag(y, yt, ldy);
   const int64_t chunks = M * (Kp / 16);
   // chunks per thread: 4 once that still gives >= 512 workgroups, 2 from 256
   // workgroups, else 1 (measured at K = 4096: M = 128 4.2 -> 3.1 us, M = 512
   // 4.4 -> 3.7 us, M = 2048 unchanged)
   const int qc = chunks >= (int64_t)256 * 4 * 512 ? 4 : (chunks >= (int64_t)256 * 2 * 256 ? 2 : 1);
   const dim3 qgrid((unsigned)((chunks + 256 * qc - 1) / (256 * qc)));
+  const int flags = xvec ? 1 : 0;
   const bool qvec = xvec && K % 16 == 0;
   const bool qdense = xvec && ldx == K && K % 64 == 0;  // flat rows in and out
 #define SBQ_QUANT_DENSE1(XT_, QC_)                                                                                  \
@@ -1469,8 +1587,23 @@ int launch_gemm_w8a8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, b
 #undef SBQ_QUANT_DENSE1
 #undef SBQ_QUANT_LAUNCH
 #undef SBQ_QUANT_LAUNCH1
-  int rc = check_launch();
+  return check_launch();
+}
+
+int launch_gemm_w8a8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, bool xvec, const uint8_t* packed,
+                     const float* scale, const int32_t* colsum, const float* bias, int64_t N, void* y, int yt,
+                     int64_t ldy, int32_t* acc_out, float2* partials, int8_t* xq, float* qpbuf, hipStream_t st,
+                     bool yvec, uint8_t* split, int64_t split_bytes, const u32x2* parts) {
+  const int64_t Nt = (N + 15) / 16, Kc = (K + 63) / 64, Kp = Kc * 64;
+  if (Kp > ((int64_t)1 << 21)) return -1;  // 32-bit block offsets of the direct-to-LDS GEMM
+  GemmArgs a{};
+  const DlPlan plan = plan_gemm_dl(true, XT_F16, M, Nt, Kc, true);
+  int ncount = 0;
+  uint32_t* zero = attach_split(a, plan, split, split_bytes, &ncount);
+  const int id = zero || plan.splits == 1 ? plan.id : pick_gemm_dl(true, XT_F16, M, Nt, Kc);
+  int rc = launch_quantize_acts(x, xt, M, K, Kp, ldx, xvec, partials, xq, qpbuf, st, zero, ncount);
   if (rc) return rc;
+  const int flags = (xvec ? 1 : 0) | (yvec ? 2 : 0) | y16_flag(y, yt, ldy);
   // small M: the row-tile GEMV on the s8 rows where it beats the tiled GEMM
   // (the GEMM's plan is available when it needs no split area or has it)
   const bool alt = plan.splits == 1 || zero != nullptr;

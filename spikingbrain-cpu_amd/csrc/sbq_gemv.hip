@@ -598,7 +598,7 @@ int launch_gemv_w8_mt(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, 
 // segment's colsum set) with the activation min/max reduced in the kernel.
 // -1: the fast path does not apply; the caller runs them one by one.
 int launch_gemv_w8_grouped(const GemvSeg* segs, int n, int xt, int64_t M, int64_t K, bool xvec, int yt, bool yvec,
-                           hipStream_t st, bool w8a8) {
+                           hipStream_t st, bool w8a8, int8_t* const* xq0, float* const* qp0) {
   if (n < 2 || n > kGemvMaxSeg) return -1;
   int64_t nt = 0;
   for (int i = 0; i < n; ++i) nt += segs[i].Nt;
@@ -610,13 +610,30 @@ int launch_gemv_w8_grouped(const GemvSeg* segs, int n, int xt, int64_t M, int64_
   a.flags = (xvec ? kGemvXVec : 0) | (yvec ? kGemvYVec : 0);
   a.nseg = n;
   for (int i = 0; i < n; ++i) a.seg[i] = segs[i];
-  return launch_gemv_fast_grouped(fid, fks, a, xt, w8a8, st);
+  const int rc = launch_gemv_fast_grouped(fid, fks, a, xt, w8a8, st);
+  if (rc != -1 || !w8a8 || !xq0 || !quantize_small_fits(M, K, xvec)) return rc;
+  QuantSmall q{};
+  q.M = (int)M;
+  q.K = (int)K;
+  for (int i = 0; i < n; ++i) {
+    q.x[i] = segs[i].x;
+    q.ldx[i] = segs[i].ldx;
+    q.xq[i] = xq0[i];
+    q.qpbuf[i] = qp0[i];
+    a.seg[i].x = xq0[i];
+    a.seg[i].ldx = K;
+    a.seg[i].qpbuf = qp0[i];
+  }
+  const int qrc = launch_quantize_small(q, n, xt, st);
+  if (qrc) return qrc;
+  pick_gemv_s8(M, K, nt * 16, &fid, &fks);
+  return launch_gemv_fast_grouped(fid, fks, a, XT_S8, true, st);
 }
 
 int launch_gemv_w8a8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, bool xvec, const uint8_t* packed,
                      const float* scale, const int32_t* colsum, const float* bias, int64_t N, void* y, int yt,
-                     int64_t ldy, int32_t* acc_out, float2* partials, hipStream_t st, bool yvec,
-                     GemvArgmaxOut* am, const u32x2* parts) {
+                     int64_t ldy, int32_t* acc_out, float2* partials, int8_t* xq, float* qpbuf, hipStream_t st,
+                     bool yvec, GemvArgmaxOut* am, const u32x2* parts) {
   const int64_t Nt = (N + 15) / 16, Kc = (K + 63) / 64;
   const GemvCfg c = pick_gemv(M, Nt, Kc, true, xt);
   if (!c.ok) return -1;
@@ -628,27 +645,23 @@ int launch_gemv_w8a8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, b
   int fid, fks;
   const bool fast = pick_gemv_fast(M, K, N, xt, true, xvec, &fid, &fks);
   if (fast) {  // small x: the kernel reduces the activation min/max itself
-    a.nparts = 0;
-    const GemvArgs f = with_argmax(a, am);
-    const int rc = launch_gemv_fast_cfg(fid, fks, f, xt, true, st);
-    if (rc != -1) {
-      if (am) am->fused = rc == 0 && (f.flags & kGemvArgmax);
-      return rc;
+    GemvArgs f = with_argmax(a, am);
+    int rc = launch_gemv_fast_cfg(fid, fks, f, xt, true, st);
+    if (rc == -1) {  // beyond that: quantized once, then the GEMV on the s8 rows
+      rc = launch_quantize_acts(x, xt, M, K, K, ldx, xvec, partials, xq, qpbuf, st);
+      if (rc) return rc;
+      f.x = xq; f.ldx = K; f.qpbuf = qpbuf;
+      pick_gemv_s8(M, K, N, &fid, &fks);
+      rc = launch_gemv_fast_cfg(fid, fks, f, XT_S8, true, st);
     }
+    if (am) am->fused = rc == 0 && (f.flags & kGemvArgmax);
+    return rc;
   }
   const int np = minmax_nparts(M, K);
   int rc = launch_minmax_partials(x, xt, M, K, ldx, partials, np, st);
   if (rc) return rc;
   a.partials = partials;
   a.nparts = np;
-  if (fast) {
-    const GemvArgs f = with_argmax(a, am);
-    rc = launch_gemv_fast_cfg(fid, fks, f, xt, true, st);
-    if (rc != -1) {
-      if (am) am->fused = rc == 0 && (f.flags & kGemvArgmax);
-      return rc;
-    }
-  }
   switch (xt) {
     case XT_F16: return launch_gemv_xt<XT_F16, true>(c, a, st);
     case XT_BF16: return launch_gemv_xt<XT_BF16, true>(c, a, st);

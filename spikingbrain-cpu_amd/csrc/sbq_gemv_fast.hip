@@ -47,7 +47,7 @@ constexpr int kFastXLdsWideBytes = 81920;  // ... with 5 row tiles per workgroup
 constexpr int kFastMaxWaves = 8;
 constexpr int kFusedChunks = 8;         // QM 2: 16-byte chunks of x per thread (at most)
 constexpr int kFusedChunksWide = 10;    // ... fp32 x with five row tiles per workgroup (one 512-thread workgroup per CU)
-constexpr int kFusedMinWaves = 4;       // W8A8 picks: 256 threads (QM 1: one min/max partial each)
+constexpr int kFusedMinWaves = 4;       // W8A8 picks: at least 256 threads share the fused x
 constexpr int kFastSplitBytes = 49152;  // fp32 x split into bf16 planes in LDS up to this size
 constexpr int kSplitChunks = 12;        // fp32 x split: 16-byte chunks of x per thread (at most)
 constexpr int kSplitRegChunks = 10;     // ... held in registers by five-row-tile workgroups
@@ -84,17 +84,6 @@ __device__ __forceinline__ void load_frag(XRaw<XT>& f, const uint8_t* p) {
     f.a = *(const V*)p;
     f.b = *(const V*)(p + 16);
   }
-}
-
-// s8 fragment (xq - 128) of 16 raw activations.
-template <int XT>
-__device__ __forceinline__ i32x4 quant16(const XRaw<XT>& f, float inv, float zpf) {
-  uint32_t d[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    d[i] = pack_act_s8x4(__builtin_fmaf(f.get(4 * i), inv, zpf), __builtin_fmaf(f.get(4 * i + 1), inv, zpf),
-                         __builtin_fmaf(f.get(4 * i + 2), inv, zpf), __builtin_fmaf(f.get(4 * i + 3), inv, zpf));
-  return (i32x4){(int)d[0], (int)d[1], (int)d[2], (int)d[3]};
 }
 
 // LDS layout: [KS][G][64] partial tiles (16 bytes each), then per-wave
@@ -180,18 +169,20 @@ __device__ __forceinline__ void argmax_epilogue(uint8_t* state, int64_t* idx, un
 
 }  // namespace
 
-// QM: 0 weight-only; 1 W8A8 with the activation min/max partials of the
-// pre-pass; 2 W8A8 that reduces min/max over the whole (small) x itself;
+// QM: 0 weight-only; 1 W8A8 on pre-quantized s8 activations (XT_S8) with the
+// (s_x, zp) a.qpbuf of the quantizing launch before it (x too large for 2);
+// 2 W8A8 that reduces min/max over the whole (small) x itself;
 // 3 per-token symmetric W8A8 on pre-quantized s8 activations (XT_S8) with
 // per-row scales a.rscale; 4 per-token symmetric W8A8 that reduces each row's
-// max |x| and quantizes the rows itself.  QM 2 and 4 (and QM 1 with five row
-// tiles) quantize x once per workgroup into s8 rows in LDS.
-// GRP: grouped launch (a.nseg linears, see GemvArgs), weight-only or QM 2
-// (each workgroup reduces the min/max of its own linear's x); a separate
-// instance, so that the single-linear kernels carry no segment lookup.
+// max |x| and quantizes the rows itself.  QM 2 and 4 quantize x once per
+// workgroup into s8 rows in LDS.
+// GRP: grouped launch (a.nseg linears, see GemvArgs), weight-only, QM 1 (each
+// linear its own rows and (s_x, zp)) or QM 2 (each workgroup reduces the
+// min/max of its own linear's x); a separate instance, so that the
+// single-linear kernels carry no segment lookup.
 template <int XT, int D, int G, bool XL, int QM, bool GRP = false>
 __global__ __launch_bounds__(kFastMaxWaves * 64) void gemv_fast_kernel(GemvArgs a, int KW, int xch) {
-  static_assert(!GRP || QM == 0 || QM == 2, "grouped launches: weight-only or fused int8-dyn");
+  static_assert(!GRP || QM == 0 || QM == 1 || QM == 2, "grouped launches: weight-only or int8-dyn");
   int bid = blockIdx.x;
   if constexpr (GRP) {
     {  // this workgroup's linear (uniform); fields read at constant indexes
@@ -204,7 +195,8 @@ __global__ __launch_bounds__(kFastMaxWaves * 64) void gemv_fast_kernel(GemvArgs 
           a.packed = a.seg[i].packed;
           a.scale = a.seg[i].scale;
           a.bias = a.seg[i].bias;
-          if constexpr (QM == 2) a.colsum = a.seg[i].colsum;
+          if constexpr (QM != 0) a.colsum = a.seg[i].colsum;
+          if constexpr (QM == 1) a.qpbuf = a.seg[i].qpbuf;
           a.y = a.seg[i].y;
           a.ldx = a.seg[i].ldx;
           a.ldy = a.seg[i].ldy;
@@ -218,7 +210,8 @@ __global__ __launch_bounds__(kFastMaxWaves * 64) void gemv_fast_kernel(GemvArgs 
   constexpr bool W8A8 = QM != 0;
   constexpr bool PT = QM == 3;
   constexpr bool PTF = QM == 4;  // per-token, x quantized in the kernel
-  static_assert(!PT || (XT == XT_S8 && !XL), "per-token: s8 fragments loaded directly");
+  constexpr bool S8 = QM == 1 || QM == 3;  // x comes quantized
+  static_assert(!S8 || (XT == XT_S8 && !XL), "pre-quantized: s8 fragments loaded directly");
   typedef typename std::conditional<W8A8, i32x4, f32x4>::type Acc;
   constexpr int EB = x_bytes<XT>();
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -252,10 +245,7 @@ __global__ __launch_bounds__(kFastMaxWaves * 64) void gemv_fast_kernel(GemvArgs 
   // QM 2: x is quantized once, from the chunks each thread holds for the
   // min/max, into s8 rows [M][K] at xs (no x copy, no per-tile quantization)
   constexpr bool kQX = QM == 2;
-  // QM 1 with five row tiles per workgroup: the (s_x, zp) of the pre-pass
-  // partials quantize the thread's chunks of x, held in registers, the same way
-  constexpr bool kQX1 = QM == 1 && G == 5;
-  constexpr bool kQXL = kQX || kQX1 || PTF;  // s8 rows in LDS
+  constexpr bool kQXL = kQX || PTF;  // s8 rows in LDS
   const int xend = kQXL ? M * K
                         : (kSplitX ? (kSplitReg ? 0 : KS * sw_cap * 16) + M * K * 4
                                    : (XL ? xch * (int)blockDim.x * 16 : 0));
@@ -276,15 +266,13 @@ __global__ __launch_bounds__(kFastMaxWaves * 64) void gemv_fast_kernel(GemvArgs 
       if constexpr (W8A8 && !PT && !PTF) cs[v] = a.colsum[nn];
     }
   }
-  // W8A8: min/max partials of the activation pre-pass, or (QM 2) up to
-  // FC 16-byte chunks of x per thread: chunk rounds past the end of x are
+  // W8A8 (QM 2, 4): up to FC 16-byte chunks of x per thread: chunk rounds past the end of x are
   // skipped (the condition is uniform over the workgroup), and the clamped
   // duplicates of a partial round are harmless
   constexpr int FC = G == 5 && XT == XT_F32 ? kFusedChunksWide : kFusedChunks;
   float2 part = {0.f, 0.f};
   u32x4 xmm[QM == 2 || PTF ? FC : 1];
   const int xm_nch = M * (K * EB / 16);  // QM 2: 16-byte chunks of x
-  if constexpr (QM == 1) part = a.partials[min(tid, a.nparts - 1)];
   if constexpr (QM == 2 || PTF) {
     const int cpr = K * EB / 16;
 #pragma unroll
@@ -301,18 +289,6 @@ __global__ __launch_bounds__(kFastMaxWaves * 64) void gemv_fast_kernel(GemvArgs 
 
   // x copy into LDS: xch 16-byte chunks per thread, sources clamped
   const uint8_t* xg = (const uint8_t*)a.x;
-  u32x4 xq1[kQX1 ? kSplitRegChunks : 1];
-  if constexpr (kQX1) {  // chunks c = tid + i * T of x, sources clamped
-    const int cpr = K * EB / 16;
-#pragma unroll
-    for (int i = 0; i < kSplitRegChunks; ++i) {
-      if (i * (int)blockDim.x < xm_nch) {
-        const int c = min(tid + i * (int)blockDim.x, xm_nch - 1);
-        const int m = c / cpr;
-        xq1[i] = *(const u32x4*)(xg + (int64_t)m * a.ldx * EB + (c - m * cpr) * 16);
-      }
-    }
-  }
   f32x4 xr[kSplitReg ? kSplitRegChunks : 1];
   if constexpr (kSplitReg) {  // chunks c = tid + i * T of x (row c / (K / 4)), sources clamped
     const int K4 = K / 4, xnch = M * K4;
@@ -373,8 +349,12 @@ __global__ __launch_bounds__(kFastMaxWaves * 64) void gemv_fast_kernel(GemvArgs 
     }
   };
   ActQParams qp = {};
+  if constexpr (QM == 1) {
+    qp.scale = a.qpbuf[0];
+    qp.zp = __float_as_int(a.qpbuf[1]);
+  }
   float tok_s = 0.0f;  // PTF: the scale of row min(r, M - 1)
-  if constexpr (XL || (W8A8 && !PT)) {
+  if constexpr (XL || (W8A8 && !S8)) {
     if constexpr (QM == 2) {
       float mn = 0.0f, mx = 0.0f;
 #pragma unroll
@@ -499,8 +479,7 @@ __global__ __launch_bounds__(kFastMaxWaves * 64) void gemv_fast_kernel(GemvArgs 
       tok_s = fmaxf(mx, 1e-8f) / 127.0f;
     }
     if constexpr (kQXL) {
-      // the s8 values xq - 128 of this thread's chunks (quant16's arithmetic:
-      // one fma and one pack per value), 16 / EB values per chunk; per-token:
+      // the s8 values xq - 128 of this thread's chunks (      // one fma and one pack per value), 16 / EB values per chunk; per-token:
       // clamp(rne(x / s), -127, 127), the row quantizer's values
       const int cpr = K * EB / 16;
       const auto quant_store = [&](const u32x4& raw, int c) {
@@ -531,19 +510,13 @@ __global__ __launch_bounds__(kFastMaxWaves * 64) void gemv_fast_kernel(GemvArgs 
         if constexpr (NE == 4) *(uint32_t*)dst = d[0];
         else *(u32x2*)dst = (u32x2){d[0], d[1]};
       };
-      if constexpr (kQX || PTF) {
 #pragma unroll
-        for (int i = 0; i < FC; ++i) {
-          if (i * (int)blockDim.x >= xm_nch) {
-        if constexpr (FC > kFusedChunks) continue;  // a break moves xmm to scratch
-        else break;
-      }
-          quant_store(xmm[i], min(tid + i * (int)blockDim.x, xm_nch - 1));
+      for (int i = 0; i < FC; ++i) {
+        if (i * (int)blockDim.x >= xm_nch) {
+          if constexpr (FC > kFusedChunks) continue;  // a break moves xmm to scratch
+          else break;
         }
-      } else {
-#pragma unroll
-        for (int i = 0; i < kSplitRegChunks; ++i)
-          if (i * (int)blockDim.x < xm_nch) quant_store(xq1[i], min(tid + i * (int)blockDim.x, xm_nch - 1));
+        quant_store(xmm[i], min(tid + i * (int)blockDim.x, xm_nch - 1));
       }
       lds_barrier();
     }
@@ -575,15 +548,11 @@ __global__ __launch_bounds__(kFastMaxWaves * 64) void gemv_fast_kernel(GemvArgs 
     XRaw<XT> f;
     if constexpr (XL) load_frag<XT>(f, xl + (kbeg + kt) * 64 * EB);
     else f = xd[p];
-    if constexpr (PT) {
+    if constexpr (S8) {
       const i32x4 q = __builtin_bit_cast(i32x4, f.v);
 #pragma unroll
       for (int j = 0; j < G; ++j) acc[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(tile_to_s8(w[p][j]), q, acc[j], 0, 0, 0);
-    } else if constexpr (W8A8) {
-      const i32x4 q = quant16<XT>(f, qp.inv, qp.zpf);
-#pragma unroll
-      for (int j = 0; j < G; ++j) acc[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(tile_to_s8(w[p][j]), q, acc[j], 0, 0, 0);
-    } else {
+    } else if constexpr (!W8A8) {
 #pragma unroll
       for (int j = 0; j < G; ++j) tile_mma<XT>(w[p][j], f, acc[j]);
     }
@@ -872,7 +841,7 @@ int launch_fast_typed(int id, const GemvArgs& a, int ks, int KW, int xch, size_t
   switch (id) {
 #define SBQ_FAST_CASE(ID, D, G, XL)                                                                     \
   case ID:                                                                                              \
-    if constexpr (QM != 3 || !XL) {                                                                     \
+    if constexpr ((QM != 1 && QM != 3) || !XL) {                                                        \
       hipLaunchKernelGGL((gemv_fast_kernel<XT, D, G, XL, QM, GRP>), dim3((a.Nt + G - 1) / G), block, lds, \
                          st, a, KW, xch);                                                               \
       return check_launch();                                                                            \
@@ -887,10 +856,10 @@ int launch_fast_typed(int id, const GemvArgs& a, int ks, int KW, int xch, size_t
 }  // namespace
 
 // Launch of fast-path configuration `id` with `ks` waves per workgroup
-// (returns -1 when the configuration cannot run this shape).  W8A8 with
-// a.nparts == 0 reduces the activation min/max in the kernel (x must fit
-// kFusedChunks 16-byte chunks per thread of the workgroup, kFusedChunksWide for
-// fp32 x with five row tiles).
+// (returns -1 when the configuration cannot run this shape).  W8A8 reduces
+// the activation min/max in the kernel (x must fit kFusedChunks 16-byte chunks
+// per thread of the workgroup, kFusedChunksWide for fp32 x with five row
+// tiles), or takes s8 rows quantized before it (xt XT_S8).
 int launch_gemv_fast_cfg(int id, int ks, const GemvArgs& a, int xt, bool w8a8, hipStream_t st) {
   if (id < 0 || id >= kNumFastCfgs || ks < 1 || ks > kFastMaxWaves) return -1;
   const FastCfg c = kFastCfgs[id];
@@ -898,32 +867,33 @@ int launch_gemv_fast_cfg(int id, int ks, const GemvArgs& a, int xt, bool w8a8, h
   const int KW = (a.Kc + ks - 1) / ks;
   ks = (a.Kc + KW - 1) / KW;  // every wave gets at least one K tile
   if (ks < c.G) return -1;                  // each row tile's epilogue belongs to one wave
-  if (xt == XT_S8) {  // per-token W8A8 on pre-quantized activations: direct fragments only
-    if (c.XL || !a.rscale) return -1;
-    return launch_fast_typed<XT_S8, 3>(id, a, ks, KW, 0, (size_t)ks * c.G * 64 * 16 + mm_bytes(), st);
+  if (xt == XT_S8) {  // pre-quantized activations (per-token a.rscale, else per-tensor): direct fragments only
+    if (c.XL) return -1;
+    size_t lds = (size_t)ks * c.G * 64 * 16 + mm_bytes();
+    if (a.flags & kGemvArgmax) lds += (size_t)c.G * 16 * 8;
+    if (a.rscale) return launch_fast_typed<XT_S8, 3>(id, a, ks, KW, 0, lds, st);
+    return a.nseg > 1 ? launch_fast_typed<XT_S8, 1, true>(id, a, ks, KW, 0, lds, st)
+                      : launch_fast_typed<XT_S8, 1>(id, a, ks, KW, 0, lds, st);
   }
-  if (w8a8 && ks * 64 < a.nparts) return -1;  // one min/max partial per thread
   const int eb = xt == XT_F32 ? 4 : 2;
   const int64_t xbytes = (int64_t)a.M * a.K * eb;
   const bool split = c.XL && xt == XT_F32 && !w8a8;  // fp32 x: raw copy + fp16 planes
   const bool split_reg = split && c.G == 5;  // fp32 x in registers, planes only in LDS
-  const bool qx1 = w8a8 && a.nparts > 0 && c.G == 5;  // pre-pass (s_x, zp), x quantized from registers
-  if (c.XL && xbytes > (split_reg || qx1 ? kSplitWideBytes
-                                         : (split ? kFastSplitBytes : (c.G == 5 ? kFastXLdsWideBytes : kFastXLdsBytes))))
+  if (c.XL && xbytes > (split_reg ? kSplitWideBytes
+                                  : (split ? kFastSplitBytes : (c.G == 5 ? kFastXLdsWideBytes : kFastXLdsBytes))))
     return -1;
   if (split && a.M > 8) return -1;  // the two planes of a row share the 16 MFMA columns
   if (c.D * c.G > 32) return -1;
   const int T = ks * 64;
   // per-token W8A8 with x quantized in the kernel: QM 4
-  const int qm = !w8a8 ? 0 : ((a.flags & kGemvPerToken) ? 4 : (a.nparts > 0 ? 1 : 2));
-  if (qm == 4 && (a.M > 16 || a.nparts > 0)) return -1;
-  const int xch = c.XL && qm != 2 && qm != 4 && !split_reg && !qx1 ? (int)((xbytes / 16 + T - 1) / T) : 0;
-  if ((split_reg || qx1) && (xbytes / 16 + T - 1) / T > kSplitRegChunks) return -1;  // the chunks each thread holds
+  const int qm = !w8a8 ? 0 : ((a.flags & kGemvPerToken) ? 4 : 2);
+  const int xch = c.XL && qm == 0 && !split_reg ? (int)((xbytes / 16 + T - 1) / T) : 0;
+  if (split_reg && (xbytes / 16 + T - 1) / T > kSplitRegChunks) return -1;  // the chunks each thread holds
   if (split && xch > kSplitChunks) return -1;  // the chunks of x each thread splits
   size_t lds = (size_t)ks * c.G * 64 * 16 + mm_bytes() + (c.XL && !split ? (size_t)xch * T * 16 : 0);
   if (split && !split_reg) lds += (size_t)ks * ((a.M * KW * 16 + 63) / 64 * 64) * 16;  // each wave's x copy
   if (split) lds += (size_t)xbytes;               // bf16 high / remainder planes
-  if (qm == 2 || qm == 4 || qx1) lds += (size_t)a.M * a.K;  // the quantized s8 rows
+  if (qm == 2 || qm == 4) lds += (size_t)a.M * a.K;  // the quantized s8 rows
   if (a.flags & kGemvArgmax) lds += (size_t)c.G * 16 * 8;  // the fused argmax's keys per row tile
   if ((qm == 2 || qm == 4) && xbytes > (int64_t)(c.G == 5 && xt == XT_F32 ? kFusedChunksWide : kFusedChunks) * 16 * T)
     return -1;  // every thread holds its chunks of x
@@ -932,7 +902,6 @@ int launch_gemv_fast_cfg(int id, int ks, const GemvArgs& a, int xt, bool w8a8, h
     case 0:                                                               \
       return a.nseg > 1 ? launch_fast_typed<XT_, 0, true>(id, a, ks, KW, xch, lds, st) \
                         : launch_fast_typed<XT_, 0>(id, a, ks, KW, xch, lds, st);      \
-    case 1: return launch_fast_typed<XT_, 1>(id, a, ks, KW, xch, lds, st); \
     case 2:                                                               \
       return a.nseg > 1 ? launch_fast_typed<XT_, 2, true>(id, a, ks, KW, xch, lds, st) \
                         : launch_fast_typed<XT_, 2>(id, a, ks, KW, xch, lds, st);      \
@@ -968,7 +937,7 @@ int launch_gemv_fast_grouped(int id, int ks, GemvArgs a, int xt, bool w8a8, hipS
   a.N = a.Nt * 16;
   a.x = a.seg[0].x;
   a.ldx = a.seg[0].ldx;
-  a.nparts = 0;
+  a.rscale = nullptr;
   a.flags &= ~(kGemvArgmax | kGemvPerToken);
   return launch_gemv_fast_cfg(id, ks, a, xt, w8a8, st);
 }
@@ -1136,19 +1105,34 @@ bool pick_gemv_fast(int64_t M, int64_t K, int64_t N, int xt, bool w8a8, bool xve
       *id = 2;
       *ks = 1;
     } else if (*ks < kFusedMinWaves) {
-      *ks = kFusedMinWaves;  // 256 threads cover the min/max partials / fused x
+      *ks = kFusedMinWaves;  // 256 threads share the fused x
     }
     // M = 4 .. 8 on a wide short-K layer: five row tiles per workgroup, as
     // for weight-only: x up to 64 KiB with the fused min/max (8 chunks per
     // thread; fp32 x up to 80 KiB, 10 chunks, so that M = 8 at K = 2560
-    // takes no pre-pass launch: checkpoint int8-dyn step 3036 -> 3240 tok/s),
-    // up to 80 KiB after the min/max pre-pass
+    // takes no quantizing launch: checkpoint int8-dyn step 3036 -> 3240 tok/s)
     if (M >= 4 && Kc < 128 && Nt > 1024 && (Nt + 4) / 5 <= 256 && xb <= kSplitWideBytes) {
       *id = 7;
       *ks = 8;
     }
   }
   return true;
+}
+
+// Choice for s8 rows quantized before the launch (QM 1, M <= 16).  Measured on
+// MI355X over every direct configuration with 2, 4 and 8 waves: short K from
+// 257 row tiles two row tiles per wave, 8-tile steps, two waves (M = 8, N =
+// 5120, K = 4096: 6.4 us against 7.2 with one row tile and four waves; M = 8 /
+// 16, N = 24576: 17.3 / 17.8, within 1% of the best), 4-tile steps on the
+// widest (M = 8, N = 151936, K = 2560: 61.2 against 64.6); else one row tile,
+// 8-tile steps, four waves (M = 8, N = 2560, K = 9728: 8.2 us, two 8.6, eight
+// 9.2; quantizing per tile in the kernel took 16.3), two at M > 8 (M = 16:
+// 9.6 against 10.3).
+void pick_gemv_s8(int64_t M, int64_t K, int64_t N, int* id, int* ks) {
+  const int64_t Kc = K / 64, Nt = (N + 15) / 16;
+  const bool wide = Kc < 128 && Nt > 256;
+  *id = wide ? (Nt > 4096 ? 4 : 5) : 3;
+  *ks = wide || M > 8 ? 2 : 4;
 }
 
 }  // namespace sbq

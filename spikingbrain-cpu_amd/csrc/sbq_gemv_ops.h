@@ -17,6 +17,7 @@ struct GemvSeg {
   const float* scale;
   const float* bias;
   const int32_t* colsum;  // int8-dyn: the weight column sums
+  const float* qpbuf;     // int8-dyn on pre-quantized rows: (s_x, zp bits)
   void* y;
   int64_t ldx, ldy;
   int N, Nt, wg0, pad;

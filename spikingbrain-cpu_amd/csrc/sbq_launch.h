@@ -16,6 +16,14 @@ inline int check_launch() {
 
 int launch_quantize_per_channel(const void* w, int wt, int64_t N, int64_t K, int64_t ldw, int8_t* q,
                                 int64_t ldq, float* scale, hipStream_t st);
+// Table entries (see sbq_linear_w8_parts) of up to kPartsFill consecutive parts.
+constexpr int kPartsFill = 16;
+struct PartsFill {
+  int count;
+  uint32_t end4[kPartsFill];   // first 4-column group past each part
+  uint32_t width[kPartsFill], word[kPartsFill];
+};
+int launch_parts_fill(const PartsFill& f, uint32_t begin4, int32_t* table, hipStream_t st);
 int launch_repack(const int8_t* q, int64_t N, int64_t K, int64_t ldq, uint8_t* packed, int32_t* colsum,
                   hipStream_t st);
 int launch_unpack(const uint8_t* packed, int64_t N, int64_t K, int8_t* q, int64_t ldq, hipStream_t st);
@@ -49,6 +57,7 @@ int gemv_config_info(int64_t M, int64_t K, bool w8a8, int xt, int32_t* info);
 // launch_gemv_fast_cfg returns -1 when that configuration cannot run the shape.
 struct GemvArgs;
 struct GemvSeg;
+void pick_gemv_s8(int64_t M, int64_t K, int64_t N, int* id, int* ks);
 bool pick_gemv_fast(int64_t M, int64_t K, int64_t N, int xt, bool w8a8, bool xvec, int* id, int* ks);
 int launch_gemv_fast_cfg(int id, int ks, const GemvArgs& a, int xt, bool w8a8, hipStream_t st);
 // Decode over several 16-row tiles of x (16 < M <= 64): weight-only on fp16 /
@@ -66,8 +75,11 @@ int launch_gemv_fast_grouped(int id, int ks, GemvArgs a, int xt, bool w8a8, hipS
 // n independent linears sharing M, K and dtypes in one launch (x / weight /
 // scale / bias / colsum / y / strides / N / Nt per segment), weight-only or
 // int8-dyn (w8a8); -1 when the fast path does not apply.
+// With xq0 / qp0 (w8a8), inputs beyond the fused capacity are quantized first, in one launch, into
+// xq0[i] and qp0[i].
 int launch_gemv_w8_grouped(const GemvSeg* segs, int n, int xt, int64_t M, int64_t K, bool xvec, int yt, bool yvec,
-                           hipStream_t st, bool w8a8 = false);
+                           hipStream_t st, bool w8a8 = false, int8_t* const* xq0 = nullptr,
+                           float* const* qp0 = nullptr);
 
 // Fused greedy token of the decode GEMV (fp32 y, M <= 16): the argmax state
 // (kArgmaxStateBytes, zero before a launch, zero again after it) and the
@@ -130,13 +142,32 @@ int launch_rowsum_f16(const void* x, int64_t ldx, int64_t M, int64_t K, float* o
 int launch_stage_act(const void* x, int xt, int64_t ldx, int64_t M, int64_t K, _Float16* xs, float* rowsum,
                      float* rscale, hipStream_t st, uint32_t* zero = nullptr, int nzero = 0);
 
-// W8A8 (fbgemm dynamic semantics).  Both launch the activation min/max
-// pre-pass into `partials` (>= kMinMaxPartials float2) when they need it (the
-// decode fast path reduces a small x in the kernel instead).
+// W8A8 (fbgemm dynamic semantics).  The decode fast path quantizes a small x
+// in the kernel; a larger one is quantized before it into xq (s8 [M][Kc*64])
+// and (s_x, zp) in qpbuf, or (ragged or misaligned rows) its min/max goes
+// into `partials` (>= kMinMaxPartials float2).
 int launch_gemv_w8a8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, bool xvec, const uint8_t* packed,
                      const float* scale, const int32_t* colsum, const float* bias, int64_t N, void* y, int yt,
-                     int64_t ldy, int32_t* acc_out, float2* partials, hipStream_t st, bool yvec,
-                     GemvArgmaxOut* am = nullptr, const u32x2* parts = nullptr);
+                     int64_t ldy, int32_t* acc_out, float2* partials, int8_t* xq, float* qpbuf, hipStream_t st,
+                     bool yvec, GemvArgmaxOut* am = nullptr, const u32x2* parts = nullptr);
+// Small activations quantized per tensor in one launch, one workgroup per
+// input (quantize_small_fits): up to 4 inputs [M, K] of one dtype.
+constexpr int kQuantSmallChunks = 20;  // 16-byte chunks of fp32 x per thread (1024 threads)
+struct QuantSmall {
+  const void* x[4];
+  int64_t ldx[4];
+  int8_t* xq[4];    // s8 rows xq - 128 [M][K]
+  float* qpbuf[4];  // (s_x, zp bits)
+  int M, K;
+  uint32_t* zero;   // counters to clear (nullable)
+  int nzero;
+};
+bool quantize_small_fits(int64_t M, int64_t K, bool xvec);
+int launch_quantize_small(const QuantSmall& a, int count, int xt, hipStream_t st);
+// ... or in two (min/max partials, then the rows) when x is larger.
+int launch_quantize_acts(const void* x, int xt, int64_t M, int64_t K, int64_t Kp, int64_t ldx, bool xvec,
+                         float2* partials, int8_t* xq, float* qpbuf, hipStream_t st, uint32_t* zero = nullptr,
+                         int nzero = 0);
 // The GEMM quantizes x once into xq (s8 [M][Kc*64]) and writes (s_x, zp) to
 // qpbuf[0..1] (zp as int bits) before the tiled pipeline reads them.
 int launch_gemm_w8a8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, bool xvec, const uint8_t* packed,

@@ -84,6 +84,23 @@ __global__ __launch_bounds__(256) void colsum_kernel(const int8_t* __restrict__ 
   if (lane == 0) colsum[n] = s;
 }
 
+// The column table of outputs stored as parts, from the parts in the kernel
+// arguments (a host copy would wait for everything launched before it).
+__global__ __launch_bounds__(256) void parts_fill_kernel(PartsFill f, uint32_t begin4, int32_t* __restrict__ table) {
+  const uint32_t i = begin4 + blockIdx.x * 256 + threadIdx.x;
+  uint32_t width = 0, word = 0, end = 0;
+#pragma unroll
+  for (int p = kPartsFill - 1; p >= 0; --p)
+    if (p < f.count && i < f.end4[p]) {
+      width = f.width[p];
+      word = f.word[p];
+      end = f.end4[p];
+    }
+  if (i >= end) return;
+  table[2 * i] = (int32_t)width;
+  table[2 * i + 1] = (int32_t)word;
+}
+
 // Zero the split-K tile counters of the GEMM that follows a pre-pass (the
 // pre-pass runs first on the same stream, so the GEMM sees them zeroed).
 __device__ __forceinline__ void zero_counters(uint32_t* c, int n) {
@@ -510,6 +527,12 @@ int launch_repack(const int8_t* q, int64_t N, int64_t K, int64_t ldq, uint8_t* p
   int rc = check_launch();
   if (rc || !colsum) return rc;
   hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)((N + 3) / 4)), dim3(256), 0, st, q, N, K, ldq, colsum);
+  return check_launch();
+}
+
+int launch_parts_fill(const PartsFill& f, uint32_t begin4, int32_t* table, hipStream_t st) {
+  const uint32_t n = f.end4[f.count - 1] - begin4;
+  hipLaunchKernelGGL(parts_fill_kernel, dim3((n + 255) / 256), dim3(256), 0, st, f, begin4, table);
   return check_launch();
 }
 

@@ -30,6 +30,7 @@ SIGNATURES = {
     "sbq_repack_w8": (_I, [_P, _L, _L, _L, _P, _P, _P]),
     "sbq_unpack_w8": (_I, [_P, _L, _L, _P, _L, _P]),
     "sbq_linear_w8": (_I, [_P, _I, _L, _L, _L, _P, _P, _P, _L, _P, _I, _L, _P, _S, _P]),
+    "sbq_parts_table": (_I, [_P, _I, _P, _P]),
     "sbq_linear_w8_parts": (_I, [_P, _I, _L, _L, _L, _P, _P, _P, _L, _P, _I, _P, _P, _S, _P]),
     "sbq_linear_w8a8_parts": (_I, [_P, _I, _L, _L, _L, _P, _P, _P, _P, _L, _P, _I, _P, _P, _S, _P]),
     "sbq_linear_w8_grouped": (_I, [_I, _P, _P, _I, _L, _L, _P, _P, _P, _P, _P, _P, _I, _P]),

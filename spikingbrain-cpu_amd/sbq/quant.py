@@ -260,7 +260,10 @@ def _run_grouped(name, xs, packeds, scales, colsums, biases, Ns, out_dtype, outs
         return [linear_w8(xs[i], packeds[i], scales[i], biases[i], Ns[i], out=ys[i]) for i in range(n)]
     ws = None
     if w8a8:
-        ws = workspace if workspace is not None else w8a8_workspace(M, K, dev)
+        ws = workspace
+        if ws is None:  # decode sizes: a share per linear of a launch, so that larger inputs are quantized together
+            ws = torch.empty((_lib.load().sbq_w8a8_workspace_bytes(M, K) * (min(n, MAX_GROUP) if M <= 16 else 1),),
+                             dtype=torch.uint8, device=dev)
     for i in range(n):
         if ys[i].dtype != ydt:
             raise ValueError(f"{name}: every output must have one dtype")
@@ -340,22 +343,21 @@ def gemm_config(M: int, N: int, K: int, dtype: torch.dtype = torch.float16, w8a8
     return rc, splits.value
 
 
-def _parts_table(sizes: list[int]) -> tuple[torch.Tensor | None, list[int]]:
-    """(the column table of sbq_linear_w8_parts on the CPU, or None when the
-    widths do not fit it; the parts' padded first columns and, last, the
-    padded width of all of them)."""
+def _parts_table(sizes: list[int], device: torch.device) -> tuple[torch.Tensor | None, list[int]]:
+    """(the column table of sbq_linear_w8_parts, or None when the widths do
+    not fit it; the parts' padded first columns and, last, the padded width of
+    all of them)."""
     pstart = [0]
     for w in sizes:
         pstart.append(pstart[-1] + (w + 63) // 64 * 64)
     N = sum(sizes)
     if any(w % 4 or w < 4 for w in sizes) or N >= 1 << 22 or pstart[-2] - (N - sizes[-1]) >= 1 << 14:
         return None, pstart
-    rows, start = [], 0
-    for w, p in zip(sizes, pstart):
-        word = start // 4 | (p - start) // 4 << 20
-        rows.append((w, word - (1 << 32) if word >= 1 << 31 else word))
-        start += w
-    return torch.tensor(rows, dtype=torch.int32).repeat_interleave(torch.tensor([w // 4 for w in sizes]), 0), pstart
+    table = torch.empty((N // 4, 2), dtype=torch.int32, device=device)
+    with torch.cuda.device(device):
+        _lib.check(_lib.load().sbq_parts_table((ctypes.c_int64 * len(sizes))(*sizes), len(sizes), _ptr(table),
+                                               _stream(device)), "sbq_parts_table")
+    return table, pstart
 
 
 def _linear_parts(x2: torch.Tensor, packed: torch.Tensor, scale: torch.Tensor, colsum: torch.Tensor | None,
@@ -1021,8 +1023,8 @@ class FusedLinear(_Fp32Buffers, nn.Module):
         self.register_buffer("scale", scale, persistent=False)
         self.register_buffer("colsum", colsum, persistent=False)
         self.register_buffer("bias", bias, persistent=False)
-        table, self._pstart = _parts_table(self.sizes)
-        self.register_buffer("_parts", None if table is None else table.to(device), persistent=False)
+        table, self._pstart = _parts_table(self.sizes, device)
+        self.register_buffer("_parts", table, persistent=False)
         self.out_dtype = torch.float32
         self._memo_ref = None
         self._memo_key = None

@@ -319,3 +319,23 @@ def test_header_compiles_standalone(tmp_path, lang, std):
     r = subprocess.run([cc, f"-std={std}", "-Wall", "-Wextra", "-pedantic", "-Werror", "-fsyntax-only",
                         f"-I{HEADER.parent}", str(src)], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr
+
+
+def test_parts_entry_points_reject_bad_arguments(lib):
+    """Widths that do not fit the column table, and N, tables or alignments the
+    parts layout does not take, are refused before any launch."""
+    P, dummy, odd = ctypes.c_void_p, ctypes.c_void_p(4096), ctypes.c_void_p(4098)
+
+    def table(widths, out=dummy):
+        return lib.sbq_parts_table((ctypes.c_int64 * len(widths))(*widths), len(widths), out, None)
+
+    assert table([6]) == -1 and table([0]) == -1 and table([4, 4], P(None)) == -1
+    assert table([1 << 22]) == -1 and table([4] * 400) == -1  # N, padding before a part
+    assert table([4, 8], odd) == -3
+    w8 = (dummy, 0, 2, 64, 64, dummy, dummy, None)
+    assert lib.sbq_linear_w8_parts(*w8, 10, dummy, 0, dummy, None, 0, None) == -1  # N % 4
+    assert lib.sbq_linear_w8_parts(*w8, 8, dummy, 0, P(None), None, 0, None) == -1
+    assert lib.sbq_linear_w8_parts(*w8, 8, odd, 0, dummy, None, 0, None) == -3
+    dyn = (dummy, 0, 2, 64, 64, dummy, dummy, dummy, None)
+    assert lib.sbq_linear_w8a8_parts(*dyn, 8, dummy, 0, dummy, None, 0, None) == -4  # no workspace
+    assert lib.sbq_linear_w8a8_parts(*dyn, 10, dummy, 0, dummy, dummy, 1 << 20, None) == -1

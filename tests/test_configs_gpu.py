@@ -371,6 +371,42 @@ def test_fused_hybrid_group_vs_oracle(dev, fmt, M):
             np.testing.assert_array_equal(po.cpu().numpy(), o.cpu().numpy())
 
 
+# x beyond what the decode GEMV quantizes itself: quantized in one launch (up
+# to 320 KiB of fp32, 160 KiB of 2-byte values) or two, then the GEMV on the s8
+# rows with one and two row tiles per wave, 2 and 4 waves.
+S8_ROUTE = [(8, 2560, 9728, "f32"), (16, 40, 4096, "f32"), (5, 5001, 4160, "f32"), (9, 4096, 9088, "f32"),
+            (10, 4000, 9728, "f32"), (8, 2560, 10240, "f16"), (16, 6150, 5120, "bf16"), (16, 100, 5184, "f16"),
+            (13, 70000, 2560, "f32"), (16, 64, 12288, "bf16"), (7, 512, 4800, "f16")]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,xd", S8_ROUTE)
+def test_w8a8_decode_quantized_before_gemv(dev, M, N, K, xd):
+    """Dense and strided rows: acc and y bit-exact against the oracle; the
+    greedy token of the same launch; two layers in one grouped call equal
+    their own calls."""
+    announce(f"w8a8 s8 route M={M} N={N} K={K} x={xd}")
+    dt = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}[xd]
+    w = gpu_weight(N, K, 3, dev)
+    lin = quant.make_linear("int8-dyn", w)
+    x = cpu_x(M, K, 4).to(dt)
+    x[:, ::97] *= 20
+    wide = torch.zeros(M, K + 64, dtype=dt, device=dev)
+    wide[:, :K] = x.to(dev)
+    cols = tile_sample(N, 7)
+    acc_ref, y_ref = ref_w8a8(x.float().numpy(), np.arange(M), *ref_rows(w, cols))
+    for xg in (x.to(dev), wide[:, :K]):
+        acc = torch.empty((M, N), dtype=torch.int32, device=dev)
+        y = quant.linear_w8a8(xg, lin.packed, lin.scale, lin.colsum, None, N, acc_out=acc)
+        np.testing.assert_array_equal(acc.cpu().numpy()[:, cols], acc_ref)
+        np.testing.assert_array_equal(y.cpu().numpy()[:, cols], y_ref)
+        yg, tok = lin.forward_greedy(xg)
+        assert torch.equal(yg, y) and torch.equal(tok, y.argmax(-1))
+        x2 = torch.roll(xg, 1, 0).contiguous() * 0.5
+        a, b = quant.grouped_forward([(lin, xg), (lin, x2)])
+        assert torch.equal(a, y) and torch.equal(b, lin(x2))
+
+
 # (M, K, sizes): every kernel that stores parts (the decode GEMV, the general
 # GEMV, the row-tile GEMV, the split and the unsplit GEMM, the register-staged
 # GEMM), parts narrower than a tile, across tiles and blocks, odd M (part
