@@ -100,6 +100,13 @@ int64_t sbq_packed_bytes(int64_t N, int64_t K);
 int sbq_repack_w8(const int8_t* q, int64_t N, int64_t K, int64_t ldq,
                   uint8_t* packed, int32_t* colsum, void* stream);
 
+/* sbq_quantize_per_channel and sbq_repack_w8 in one pass over the weight:
+ * scale, packed, and where asked for the int8 rows q (NULL: not written) and
+ * colsum (NULL: not written), the same values as those two calls. */
+int sbq_quantize_pack_w8(const void* w, int w_dtype, int64_t N, int64_t K, int64_t ldw,
+                         int8_t* q, int64_t ldq, float* scale, uint8_t* packed,
+                         int32_t* colsum, void* stream);
+
 /* Inverse of sbq_repack_w8: packed -> q [N, K] (row stride ldq). */
 int sbq_unpack_w8(const uint8_t* packed, int64_t N, int64_t K, int8_t* q, int64_t ldq,
                   void* stream);

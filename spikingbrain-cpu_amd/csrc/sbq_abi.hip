@@ -169,7 +169,16 @@ int sbq_quantize_per_channel(const void* w, int w_dtype, int64_t N, int64_t K, i
   if (N < 0 || K < 1 || ldw < K || ldq < K || N > kIntMax || K > kIntMax) return SBQ_ERR_ARG;
   if (N == 0) return SBQ_OK;
   if (!w || !q || !scale) return SBQ_ERR_ARG;
-  return sbq::launch_quantize_per_channel(w, w_dtype, N, K, ldw, q, ldq, scale, (hipStream_t)stream);
+  return sbq::launch_pack_weight(w, w_dtype, N, K, ldw, scale, q, ldq, nullptr, nullptr, (hipStream_t)stream);
+}
+
+int sbq_quantize_pack_w8(const void* w, int w_dtype, int64_t N, int64_t K, int64_t ldw, int8_t* q, int64_t ldq,
+                         float* scale, uint8_t* packed, int32_t* colsum, void* stream) {
+  if (!valid_dtype(w_dtype)) return SBQ_ERR_DTYPE;
+  if (N < 1 || K < 1 || ldw < K || (q && ldq < K) || N > kIntMax || K > kIntMax) return SBQ_ERR_ARG;
+  if (!w || !scale || !packed) return SBQ_ERR_ARG;
+  if (!aligned(packed, 16)) return SBQ_ERR_ALIGN;
+  return sbq::launch_pack_weight(w, w_dtype, N, K, ldw, scale, q, ldq, packed, colsum, (hipStream_t)stream);
 }
 
 int64_t sbq_packed_bytes(int64_t N, int64_t K) {
@@ -182,7 +191,7 @@ int sbq_repack_w8(const int8_t* q, int64_t N, int64_t K, int64_t ldq, uint8_t* p
   if (N < 1 || K < 1 || ldq < K || N > kIntMax || K > kIntMax) return SBQ_ERR_ARG;
   if (!q || !packed) return SBQ_ERR_ARG;
   if (!aligned(packed, 16)) return SBQ_ERR_ALIGN;
-  return sbq::launch_repack(q, N, K, ldq, packed, colsum, (hipStream_t)stream);
+  return sbq::launch_pack_weight(q, sbq::XT_S8, N, K, ldq, nullptr, nullptr, 0, packed, colsum, (hipStream_t)stream);
 }
 
 int sbq_unpack_w8(const uint8_t* packed, int64_t N, int64_t K, int8_t* q, int64_t ldq, void* stream) {

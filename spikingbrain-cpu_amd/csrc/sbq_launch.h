@@ -14,8 +14,11 @@ inline int check_launch() {
   return e == hipSuccess ? 0 : -5;
 }
 
-int launch_quantize_per_channel(const void* w, int wt, int64_t N, int64_t K, int64_t ldw, int8_t* q,
-                                int64_t ldq, float* scale, hipStream_t st);
+// One pass over weight rows (sbq_quant.hip pack_weight_kernel): wt a dtype
+// (quantize_per_channel) or XT_S8 (rows as they are); scale is for a dtype
+// only; q, packed, colsum: each may be null.
+int launch_pack_weight(const void* w, int wt, int64_t N, int64_t K, int64_t ldw, float* scale, int8_t* q, int64_t ldq,
+                       uint8_t* packed, int32_t* colsum, hipStream_t st);
 // Table entries (see sbq_linear_w8_parts) of up to kPartsFill consecutive parts.
 constexpr int kPartsFill = 16;
 struct PartsFill {
@@ -24,8 +27,6 @@ struct PartsFill {
   uint32_t width[kPartsFill], word[kPartsFill];
 };
 int launch_parts_fill(const PartsFill& f, uint32_t begin4, int32_t* table, hipStream_t st);
-int launch_repack(const int8_t* q, int64_t N, int64_t K, int64_t ldq, uint8_t* packed, int32_t* colsum,
-                  hipStream_t st);
 int launch_unpack(const uint8_t* packed, int64_t N, int64_t K, int8_t* q, int64_t ldq, hipStream_t st);
 
 int minmax_nparts(int64_t M, int64_t K);

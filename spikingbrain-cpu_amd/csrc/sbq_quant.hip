@@ -10,78 +10,231 @@
 
 namespace sbq {
 
-// One wavefront per weight row: exact max|w| reduction, then IEEE fp32
-// divisions and round-half-even, matching torch's CPU expression.
+// ---------------------------------------------------------------------------
+// Weights: quantize_per_channel, the packed tiles and the column sums
+// ---------------------------------------------------------------------------
+// 16 consecutive values of a weight row as loaded (WT: a source dtype, or
+// XT_S8 for rows that are int8 already).
 template <int WT>
-__global__ __launch_bounds__(256) void quantize_per_channel_kernel(const void* __restrict__ wv, int64_t N,
-                                                                   int64_t K, int64_t ldw,
-                                                                   int8_t* __restrict__ q, int64_t ldq,
-                                                                   float* __restrict__ scale) {
-  typedef typename XElem<WT>::T T;
-  const T* w = (const T*)wv;
-  const int lane = threadIdx.x & 63;
-  const int64_t n = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (n >= N) return;
-  const T* row = w + n * ldw;
-  float amax = 0.0f;
-  for (int64_t k = lane; k < K; k += 64) amax = fmaxf(amax, __builtin_fabsf(XElem<WT>::to_f32(row[k])));
-  amax = wave_max(amax);
-  const float s = fmaxf(amax, 1e-8f) / 127.0f;
-  if (lane == 0) scale[n] = s;
-  int8_t* qrow = q + n * ldq;
-  for (int64_t k = lane; k < K; k += 64) {
-    float t = __builtin_rintf(XElem<WT>::to_f32(row[k]) / s);
-    t = fminf(fmaxf(t, -127.0f), 127.0f);
-    qrow[k] = (int8_t)(int)t;
+struct WRaw {
+  static constexpr int ES = WT == XT_S8 ? 1 : (WT == XT_F32 ? 4 : 2);
+  u32x4 d[ES];
+
+  // columns k0 .. k0 + 15 of the row at p (nullptr: a row of padding); columns
+  // >= K are 0.  Rows may start at any address: whole chunks are 16-byte loads
+  // of whatever alignment (the GPU splits them), the row's last chunk goes by
+  // elements.
+  __device__ __forceinline__ void load(const uint8_t* p, int64_t k0, int64_t K) {
+    typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(1)));
+    if (p && k0 + 16 <= K) {
+#pragma unroll
+      for (int i = 0; i < ES; ++i) d[i] = *(const u32x4_any*)(p + k0 * ES + 16 * i);
+      return;
+    }
+    uint32_t w[4 * ES];
+#pragma unroll
+    for (int i = 0; i < 4 * ES; ++i) w[i] = 0u;
+    if (p && k0 < K) {
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        const int64_t k = k0 + j < K ? k0 + j : K - 1;
+        uint32_t b;
+        if constexpr (ES == 4) b = *(const uint32_t*)(p + k * 4);
+        else if constexpr (ES == 2) b = *(const uint16_t*)(p + k * 2);
+        else b = p[k];
+        if (k0 + j < K) w[j * ES / 4] |= b << (8 * (j * ES % 4));
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < ES; ++i) d[i] = (u32x4){w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]};
+  }
+  __device__ __forceinline__ float get(int j) const {
+    const uint32_t word = d[j * ES / 16][j * ES / 4 % 4];  // (a bit_cast of the element itself reads element 0)
+    if constexpr (WT == XT_F32) return __uint_as_float(word);
+    else if constexpr (WT == XT_F16) return (float)__builtin_bit_cast(f16x2, word)[j & 1];
+    else return __uint_as_float(j & 1 ? word & 0xffff0000u : word << 16);
+  }
+};
+
+// clamp(rint(v / s), -127, 127) of 16 values as bytes.  The division is IEEE
+// (about ten instructions); nearly always its rounded result is that of
+// t = v * inv, inv = fp32(1 / s): |v| <= 127 s, so t is within 2.3e-5 of the
+// fp32 quotient (1.5 units of 2^-24 each, times 127) and both round alike
+// unless t is that close to a half.  Rounding by adding 1.5 * 2^23: the low
+// byte of the sum is the integer.  A chunk with a value near a half, an
+// infinity or a NaN takes the division.
+template <int WT>
+__device__ __forceinline__ u32x4 quant_w16(const WRaw<WT>& raw, float s, float inv) {
+  constexpr float kMagic = 12582912.0f;
+  uint32_t m[16];
+  bool sure = true;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    const float t = raw.get(j) * inv, r = t + kMagic;
+    sure &= __builtin_fabsf(t - (r - kMagic)) < 0.49997f;
+    m[j] = __float_as_uint(r);
+  }
+  if (!sure) {
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const float t = __builtin_rintf(raw.get(j) / s);
+      m[j] = (uint32_t)(int)fminf(fmaxf(t, -127.0f), 127.0f);
+    }
+  }
+  u32x4 o;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    o[i] = __builtin_amdgcn_perm(m[4 * i + 1], m[4 * i], 0x0c0c0400u) |
+           __builtin_amdgcn_perm(m[4 * i + 3], m[4 * i + 2], 0x04000c0cu);
+  return o;
+}
+
+// One workgroup of 8 waves per 16 weight rows: lane (g, r) of wave v takes the
+// 16-value chunks of row r at columns 64 kc + 16 g, kc = v, v + 8, ..., the
+// chunk that is its 16 bytes of packed tile kc.  With a floating source each
+// row's max |w| is reduced (over the lanes of the row, then the waves through
+// LDS), scale = max(that, 1e-8) / 127, and the same chunks are quantized; an
+// int8 source (repack) is taken as it is.  Writes whatever is asked for: the
+// scales, the int8 rows q, the packed tiles (offset binary), the column sums.
+// C > 0: the wave's at most C chunks per lane stay in registers between the
+// two passes; C = 0: longer rows are read again (from the Infinity Cache).
+// HBM bound: one read of w, one write of each output.  Measured (whole call of
+// a module's load, eager, against a scalar quantizer, a byte-wise repack and a
+// column-sum launch, with the int8 rows written and read twice between them):
+// bf16 9728 x 2560 112 -> 25 us, 24576 x 4096 407 -> 70 us (4.3 TB/s),
+// 151936 x 2560 1661 -> 237 us (4.9 TB/s); with the int8 rows kept 26 / 96 /
+// 302 us; fp32 9728 x 2560 135 -> 26; ragged bf16 9721 x 2555 101 -> 39.  16
+// waves per workgroup: 20-45% slower except at K = 9728 (5% faster); holding
+// 24 chunks spilled (2560 x 9728: 74 us, re-reading 39).
+template <int WT, int C>
+__global__ __launch_bounds__(512) void pack_weight_kernel(const uint8_t* __restrict__ w, int64_t N, int64_t K,
+                                                          int64_t ldw, float* __restrict__ scale,
+                                                          int8_t* __restrict__ q, int64_t ldq,
+                                                          uint8_t* __restrict__ packed,
+                                                          int32_t* __restrict__ colsum) {
+  constexpr int NW = 8, U = 4;
+  constexpr bool FP = WT != XT_S8;
+  __shared__ float smax[NW][16];
+  __shared__ int ssum[NW][16];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+  const int64_t nt = blockIdx.x, n = nt * 16 + r, Kc = (K + 63) / 64;
+  const uint8_t* row = n < N ? w + n * ldw * WRaw<WT>::ES : nullptr;
+  WRaw<WT> v[C > 0 ? C : U];
+  float s = 0.0f, inv = 0.0f;
+  const auto row_max = [&](const WRaw<WT>& x, float m) {
+#pragma unroll
+    for (int j = 0; j < 16; ++j) m = fmaxf(m, __builtin_fabsf(x.get(j)));
+    return m;
+  };
+  if constexpr (FP) {
+    float m = 0.0f;
+    if constexpr (C > 0) {
+#pragma unroll
+      for (int i = 0; i < C; ++i)
+        if (wv + i * NW < Kc) v[i].load(row, (wv + i * NW) * 64 + g * 16, K);
+#pragma unroll
+      for (int i = 0; i < C; ++i)
+        if (wv + i * NW < Kc) m = row_max(v[i], m);
+    } else {
+      for (int64_t kc = wv; kc < Kc; kc += U * NW) {
+#pragma unroll
+        for (int i = 0; i < U; ++i)
+          if (kc + i * NW < Kc) v[i].load(row, (kc + i * NW) * 64 + g * 16, K);
+#pragma unroll
+        for (int i = 0; i < U; ++i)
+          if (kc + i * NW < Kc) m = row_max(v[i], m);
+      }
+    }
+    m = fmaxf(m, __shfl_xor(m, 16));
+    m = fmaxf(m, __shfl_xor(m, 32));
+    if (g == 0) smax[wv][r] = m;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NW; ++i) m = fmaxf(m, smax[i][r]);
+    s = fmaxf(m, 1e-8f) / 127.0f;
+    inv = 1.0f / s;
+    if (threadIdx.x < 16 && n < N) scale[n] = s;
+  }
+  int sum = 0;
+  const auto emit = [&](int64_t kc, const WRaw<WT>& x) {
+    u32x4 b;
+    if constexpr (FP) b = quant_w16<WT>(x, s, inv);
+    else b = x.d[0];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sum = __builtin_amdgcn_sdot4((int)b[i], 0x01010101, sum, false);
+    if (packed)
+      *(u32x4*)(packed + ((nt * Kc + kc) * 64 + lane) * 16) = b ^ (u32x4){0x80808080u, 0x80808080u, 0x80808080u, 0x80808080u};
+    const int64_t k0 = kc * 64 + g * 16;
+    if (q && n < N) {
+      typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(1)));
+      int8_t* dst = q + n * ldq + k0;
+      if (k0 + 16 <= K) {
+        *(u32x4_any*)dst = b;
+      } else {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          const uint32_t word = b[j / 4];
+          if (k0 + j < K) dst[j] = (int8_t)(word >> (8 * (j % 4)));
+        }
+      }
+    }
+  };
+  if constexpr (C > 0) {
+    // the chunks stay as loaded (the compiler would keep the 2-byte values as
+    // the floats of the first pass, twice the registers)
+#pragma unroll
+    for (int i = 0; i < C; ++i)
+#pragma unroll
+      for (int j = 0; j < WRaw<WT>::ES; ++j) asm("" : "+v"(v[i].d[j]));
+#pragma unroll
+    for (int i = 0; i < C; ++i)
+      if (wv + i * NW < Kc) emit(wv + i * NW, v[i]);
+  } else {
+    for (int64_t kc = wv; kc < Kc; kc += U * NW) {
+#pragma unroll
+      for (int i = 0; i < U; ++i)
+        if (kc + i * NW < Kc) v[i].load(row, (kc + i * NW) * 64 + g * 16, K);
+#pragma unroll
+      for (int i = 0; i < U; ++i)
+        if (kc + i * NW < Kc) emit(kc + i * NW, v[i]);
+    }
+  }
+  if (colsum) {  // uniform; exact int32: |sum| <= 127 * K
+    sum += __shfl_xor(sum, 16);
+    sum += __shfl_xor(sum, 32);
+    if (g == 0) ssum[wv][r] = sum;
+    __syncthreads();
+    if (threadIdx.x < 16 && n < N) {
+      int t = 0;
+#pragma unroll
+      for (int i = 0; i < NW; ++i) t += ssum[i][r];
+      colsum[n] = t;
+    }
   }
 }
 
-// One thread per 16-byte lane slot of the packed layout.
-__global__ __launch_bounds__(256) void repack_kernel(const int8_t* __restrict__ q, int64_t N, int64_t K,
-                                                     int64_t ldq, int64_t Kc, int64_t nslots,
-                                                     uint8_t* __restrict__ packed) {
-  const int64_t slot = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// Packed tiles -> int8 rows: one 16-byte lane slot per thread, stored at
+// whatever alignment the row has.
+__global__ __launch_bounds__(256) void unpack_kernel(const uint8_t* __restrict__ packed, int64_t N, int64_t K,
+                                                     int64_t Kc, int64_t nslots, int8_t* __restrict__ q, int64_t ldq) {
+  typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(1)));
+  const int64_t slot = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (slot >= nslots) return;
   const int lane = (int)(slot & 63);
-  const int64_t tile = slot >> 6;
-  const int64_t nt = tile / Kc, kc = tile % Kc;
-  const int64_t n = nt * 16 + (lane & 15);
-  const int64_t k0 = kc * 64 + (lane >> 4) * 16;
-  uint32_t d[4];
+  const int64_t tile = slot >> 6, nt = tile / Kc, kc = tile - nt * Kc;
+  const int64_t n = nt * 16 + (lane & 15), k0 = kc * 64 + (lane >> 4) * 16;
+  if (n >= N || k0 >= K) return;
+  const u32x4 b = *(const u32x4*)(packed + slot * 16) ^ (u32x4){0x80808080u, 0x80808080u, 0x80808080u, 0x80808080u};
+  int8_t* dst = q + n * ldq + k0;
+  if (k0 + 16 <= K) {
+    *(u32x4_any*)dst = b;
+  } else {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    uint32_t word = 0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int64_t k = k0 + i * 4 + j;
-      const uint32_t b = (n < N && k < K) ? (uint32_t)(uint8_t)q[n * ldq + k] : 0u;
-      word |= ((b ^ 0x80u) & 0xffu) << (8 * j);
+    for (int j = 0; j < 16; ++j) {
+      const uint32_t word = b[j / 4];
+      if (k0 + j < K) dst[j] = (int8_t)(word >> (8 * (j % 4)));
     }
-    d[i] = word;
   }
-  *(u32x4*)(packed + slot * 16) = (u32x4){d[0], d[1], d[2], d[3]};
-}
-
-__global__ __launch_bounds__(256) void unpack_kernel(const uint8_t* __restrict__ packed, int64_t N, int64_t K,
-                                                     int64_t Kc, int8_t* __restrict__ q, int64_t ldq) {
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= N * K) return;
-  const int64_t n = idx / K, k = idx % K;
-  const int64_t nt = n >> 4, r = n & 15, kc = k >> 6, g = (k & 63) >> 4, j = k & 15;
-  const uint8_t u = packed[((nt * Kc + kc) * 64 + g * 16 + r) * 16 + j];
-  q[n * ldq + k] = (int8_t)(u ^ 0x80u);
-}
-
-// colsum[n] = sum_k q[n,k]  (exact int32: |sum| <= 127 * K).
-__global__ __launch_bounds__(256) void colsum_kernel(const int8_t* __restrict__ q, int64_t N, int64_t K,
-                                                     int64_t ldq, int32_t* __restrict__ colsum) {
-  const int lane = threadIdx.x & 63;
-  const int64_t n = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (n >= N) return;
-  int s = 0;
-  for (int64_t k = lane; k < K; k += 64) s += (int)q[n * ldq + k];
-  s = wave_sum_i(s);
-  if (lane == 0) colsum[n] = s;
 }
 
 // The column table of outputs stored as parts, from the parts in the kernel
@@ -506,27 +659,33 @@ __global__ __launch_bounds__(1024) void argmax_rows_kernel(const float* __restri
 // ---------------------------------------------------------------------------
 // host launchers
 // ---------------------------------------------------------------------------
-int launch_quantize_per_channel(const void* w, int wt, int64_t N, int64_t K, int64_t ldw, int8_t* q,
-                                int64_t ldq, float* scale, hipStream_t st) {
-  dim3 grid((unsigned)((N + 3) / 4)), block(256);
+int launch_pack_weight(const void* w, int wt, int64_t N, int64_t K, int64_t ldw, float* scale, int8_t* q, int64_t ldq,
+                       uint8_t* packed, int32_t* colsum, hipStream_t st) {
+  const dim3 grid((unsigned)((N + 15) / 16)), block(512);
+  const int64_t per = ((K + 63) / 64 + 7) / 8;  // chunks per lane
+#define SBQ_PACK(WT_, C_) \
+  hipLaunchKernelGGL((pack_weight_kernel<WT_, C_>), grid, block, 0, st, (const uint8_t*)w, N, K, ldw, scale, q, ldq, packed, colsum)
+  // held in registers: up to 16 chunks of 2-byte values (199 VGPRs, K <= 8192), 8 of fp32 (175, K <= 4096)
+#define SBQ_PACK2(WT_)                          \
+  if (per <= 2) SBQ_PACK(WT_, 2);               \
+  else if (per <= 5) SBQ_PACK(WT_, 5);          \
+  else if (per <= 8) SBQ_PACK(WT_, 8);          \
+  else if (per <= 16) SBQ_PACK(WT_, 16);        \
+  else SBQ_PACK(WT_, 0)
   switch (wt) {
-    case XT_F32: hipLaunchKernelGGL(quantize_per_channel_kernel<XT_F32>, grid, block, 0, st, w, N, K, ldw, q, ldq, scale); break;
-    case XT_F16: hipLaunchKernelGGL(quantize_per_channel_kernel<XT_F16>, grid, block, 0, st, w, N, K, ldw, q, ldq, scale); break;
-    case XT_BF16: hipLaunchKernelGGL(quantize_per_channel_kernel<XT_BF16>, grid, block, 0, st, w, N, K, ldw, q, ldq, scale); break;
+    case XT_F16: SBQ_PACK2(XT_F16); break;
+    case XT_BF16: SBQ_PACK2(XT_BF16); break;
+    case XT_F32:
+      if (per <= 2) SBQ_PACK(XT_F32, 2);
+      else if (per <= 5) SBQ_PACK(XT_F32, 5);
+      else if (per <= 8) SBQ_PACK(XT_F32, 8);
+      else SBQ_PACK(XT_F32, 0);
+      break;
+    case XT_S8: SBQ_PACK(XT_S8, 0); break;
     default: return -2;
   }
-  return check_launch();
-}
-
-int launch_repack(const int8_t* q, int64_t N, int64_t K, int64_t ldq, uint8_t* packed, int32_t* colsum,
-                  hipStream_t st) {
-  const int64_t Nt = (N + 15) / 16, Kc = (K + 63) / 64;
-  const int64_t nslots = Nt * Kc * 64;
-  hipLaunchKernelGGL(repack_kernel, dim3((unsigned)((nslots + 255) / 256)), dim3(256), 0, st, q, N, K, ldq, Kc,
-                     nslots, packed);
-  int rc = check_launch();
-  if (rc || !colsum) return rc;
-  hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)((N + 3) / 4)), dim3(256), 0, st, q, N, K, ldq, colsum);
+#undef SBQ_PACK2
+#undef SBQ_PACK
   return check_launch();
 }
 
@@ -537,10 +696,9 @@ int launch_parts_fill(const PartsFill& f, uint32_t begin4, int32_t* table, hipSt
 }
 
 int launch_unpack(const uint8_t* packed, int64_t N, int64_t K, int8_t* q, int64_t ldq, hipStream_t st) {
-  const int64_t Kc = (K + 63) / 64;
-  const int64_t total = N * K;
-  hipLaunchKernelGGL(unpack_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, packed, N, K, Kc, q,
-                     ldq);
+  const int64_t Kc = (K + 63) / 64, nslots = (N + 15) / 16 * Kc * 64;
+  hipLaunchKernelGGL(unpack_kernel, dim3((unsigned)((nslots + 255) / 256)), dim3(256), 0, st, packed, N, K, Kc, nslots,
+                     q, ldq);
   return check_launch();
 }
 

@@ -28,6 +28,7 @@ SIGNATURES = {
     "sbq_quantize_per_channel": (_I, [_P, _I, _L, _L, _L, _P, _L, _P, _P]),
     "sbq_packed_bytes": (_L, [_L, _L]),
     "sbq_repack_w8": (_I, [_P, _L, _L, _L, _P, _P, _P]),
+    "sbq_quantize_pack_w8": (_I, [_P, _I, _L, _L, _L, _P, _L, _P, _P, _P, _P]),
     "sbq_unpack_w8": (_I, [_P, _L, _L, _P, _L, _P]),
     "sbq_linear_w8": (_I, [_P, _I, _L, _L, _L, _P, _P, _P, _L, _P, _I, _L, _P, _S, _P]),
     "sbq_parts_table": (_I, [_P, _I, _P, _P]),

@@ -161,6 +161,27 @@ def repack(q: torch.Tensor, with_colsum: bool = True) -> tuple[torch.Tensor, tor
     return packed, colsum
 
 
+def _quantize_pack(weight: torch.Tensor, with_q: bool, with_colsum: bool):
+    """quantize_per_channel_gpu and repack in one pass over the weight:
+    (q or None, scale, packed, colsum or None)."""
+    if weight.dim() != 2:
+        raise ValueError("quantize_per_channel expects a 2-D weight")
+    w = weight if weight.dtype in _DTYPE_CODE else weight.float()
+    if w.stride(-1) != 1:
+        w = w.contiguous()
+    N, K = w.shape
+    L = _lib.load()
+    dev = w.device
+    q = torch.empty((N, K), dtype=torch.int8, device=dev) if with_q else None
+    scale = torch.empty((N,), dtype=torch.float32, device=dev)
+    packed = torch.empty((packed_bytes(N, K),), dtype=torch.uint8, device=dev)
+    colsum = torch.empty((N,), dtype=torch.int32, device=dev) if with_colsum else None
+    with torch.cuda.device(dev):
+        _lib.check(L.sbq_quantize_pack_w8(_ptr(w), _code(w.dtype), N, K, _ldx(w), _ptr(q), K, _ptr(scale),
+                                          _ptr(packed), _ptr(colsum), _stream(dev)), "sbq_quantize_pack_w8")
+    return q, scale, packed, colsum
+
+
 def unpack(packed: torch.Tensor, N: int, K: int) -> torch.Tensor:
     """Packed tiles -> int8 [N, K] (the inverse of repack)."""
     if (packed.dtype != torch.uint8 or not packed.is_cuda or not packed.is_contiguous()
@@ -711,12 +732,11 @@ class Int8Linear(nn.Module):
     def __init__(self, weight: torch.Tensor, bias: torch.Tensor | None, block: int = 128):
         super().__init__()
         device = _gpu_for(weight)
-        q, scale = quantize_per_channel_gpu(weight.to(device))
+        q, scale, packed, _ = _quantize_pack(weight.to(device), with_q=True, with_colsum=False)
         self.register_buffer("qweight", q)
         self.register_buffer("scale", scale)
         self.bias = None if bias is None else nn.Parameter(bias.to(device).float(), requires_grad=False)
         self.block = block
-        packed, _ = repack(q, with_colsum=False)
         self.register_buffer("packed", packed, persistent=False)
         self.out_dtype = torch.float32
         # a loaded state_dict replaces qweight in place: rebuild the tiles from it
@@ -827,14 +847,13 @@ class DynamicInt8Linear(_Fp32Buffers, nn.Module):
             raise ValueError("granularity must be 'tensor' or 'token'")
         self.granularity = granularity
         device = _gpu_for(weight)
-        q, scale = quantize_per_channel_gpu(weight.to(device))
-        packed, colsum = repack(q, with_colsum=True)
+        _, scale, packed, colsum = _quantize_pack(weight.to(device), with_q=False, with_colsum=True)
         self.register_buffer("packed", packed, persistent=False)
         self.register_buffer("scale", scale, persistent=False)
         self.register_buffer("colsum", colsum, persistent=False)
         self.register_buffer("bias", None if bias is None else bias.to(device).float(), persistent=False)
-        self.in_features = q.shape[1]
-        self.out_features = q.shape[0]
+        self.in_features = weight.shape[1]
+        self.out_features = weight.shape[0]
         self.out_dtype = torch.float32
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:

@@ -91,6 +91,39 @@ def test_repack_roundtrip_and_colsum(dev, N, K):
     np.testing.assert_array_equal(quant.unpack(packed, N, K).cpu().numpy(), q.numpy())
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("N,K", [(1, 1), (17, 15), (5, 1000), (33, 1025), (16, 2560), (40, 4095), (130, 4100), (21, 9728),
+                                 (18, 12300)])
+def test_quantize_pack_one_pass(dev, dtype, N, K):
+    """Scales, int8 rows, packed tiles and column sums of one pass, for every
+    number of chunks a lane holds, K and row starts of any alignment, and
+    values on and next to every half of the scale (rows of maximum 127: scale
+    1): bit-equal to the oracle and to the separate entry points."""
+    announce(f"quantize pack {dtype} {N}x{K}")
+    w = make_weights(N, K, N + K)
+    if K > 600:  # half-way values and their neighbours, both signs
+        half = torch.arange(-126.5, 127, 1.0)
+        ties = torch.cat([half, torch.nextafter(half, half + 1), torch.nextafter(half, half - 1)])[:K - 1]
+        w[0, 0] = 127.0
+        w[0, 1:] = 0.0
+        w[0, 1:1 + len(ties[:K - 1])] = ties[:K - 1]
+    if N > 2:
+        w[2] = 0
+    wide = torch.zeros(N, K + 3, dtype=DT[dtype], device=dev)
+    wide[:, 1:K + 1] = w.to(DT[dtype]).to(dev)
+    qo, so = oracle.quantize_per_channel_c(w.to(DT[dtype]).float().numpy())
+    for wd in (wide[:, 1:K + 1], w.to(DT[dtype]).to(dev)):
+        q, s, packed, colsum = quant._quantize_pack(wd, True, True)
+        np.testing.assert_array_equal(q.cpu().numpy(), qo)
+        np.testing.assert_array_equal(s.cpu().numpy(), so)
+        np.testing.assert_array_equal(packed.cpu().numpy(), oracle.pack_w8(qo))
+        np.testing.assert_array_equal(colsum.cpu().numpy(), qo.astype(np.int64).sum(1))
+        p2, c2 = quant.repack(q)
+        assert torch.equal(p2, packed) and torch.equal(c2, colsum)
+        q1, s1 = quant.quantize_per_channel_gpu(wd)
+        assert torch.equal(q1, q) and torch.equal(s1, s) and torch.equal(quant.unpack(packed, N, K), q)
+
+
 # ---------------------------------------------------------------------------
 # int8 weight-only
 # ---------------------------------------------------------------------------
