@@ -1409,12 +1409,15 @@ int launch_gemm_w8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, boo
 }
 
 // Per-tensor quantization of up to SBQ_MAX_GROUP small inputs in one launch,
-// one workgroup each (rows 16-byte aligned, 64 | K, at most C * 16 KiB of x):
+// one workgroup each (at most C * 16 KiB of x with its rows padded to Kp):
 // the workgroup holds its whole x in registers, so the (s_x, zp) and the s8
 // rows xq - 128 take one launch instead of two (min/max partials, then
 // quantize).  Bound by one CU's load path and the chain load - reduce -
 // parameters - store.  Values and parameters are the two-launch path's, bit
-// for bit (min and max do not depend on order).  DENSE: rows of stride K.
+// for bit (min and max do not depend on order).  DENSE: 16-byte aligned
+// rows of stride K, 64 | K; else rows of any stride, alignment and K (16-byte
+// loads of whatever alignment, the last chunk of a row by elements, padding
+// columns as 0: inside the range, and they meet zero weights).
 // Measured (K = 2560 ... 12288): 24-80 KiB of x 2.9-3.3 us, 128 KiB 3.7,
 // 256-320 KiB 5.5-5.8, against 2.6 (min/max) + 1.1 (gap) + 2.5-3 us.
 template <int XT, int C, bool DENSE>
@@ -1436,7 +1439,8 @@ __global__ __launch_bounds__(1024) void quantize_small_kernel(QuantSmall a) {
       xq = a.xq[i];
       qpbuf = a.qpbuf[i];
     }
-  const int t = threadIdx.x, lane = t & 63, cpr = a.K / NE, nch = a.M * cpr;
+  typedef T vN_any __attribute__((ext_vector_type(NE), aligned(sizeof(T))));
+  const int t = threadIdx.x, lane = t & 63, cpr = a.Kp / NE, nch = a.M * cpr;
   vN v[C];
 #pragma unroll
   for (int i = 0; i < C; ++i) {  // clamped: surplus chunks repeat the last one and are not stored
@@ -1444,8 +1448,14 @@ __global__ __launch_bounds__(1024) void quantize_small_kernel(QuantSmall a) {
     if constexpr (DENSE) {
       v[i] = *((const vN*)x + c);
     } else {
-      const int m = c / cpr;
-      v[i] = *(const vN*)((const T*)x + (int64_t)m * ldx + (c - m * cpr) * NE);
+      const int m = c / cpr, k0 = (c - m * cpr) * NE;
+      const T* p = (const T*)x + (int64_t)m * ldx + k0;
+      if (k0 + NE <= a.K) {
+        v[i] = *(const vN_any*)p;
+      } else {
+#pragma unroll
+        for (int j = 0; j < NE; ++j) v[i][j] = k0 + j < a.K ? p[j] : (T)0.0f;
+      }
     }
   }
   for (int i = t; i < a.nzero; i += 1024) a.zero[i] = 0u;
@@ -1488,7 +1498,7 @@ __global__ __launch_bounds__(1024) void quantize_small_kernel(QuantSmall a) {
                            __builtin_fmaf(XElem<XT>::to_f32(v[i][4 * w + 1]), inv, zpf),
                            __builtin_fmaf(XElem<XT>::to_f32(v[i][4 * w + 2]), inv, zpf),
                            __builtin_fmaf(XElem<XT>::to_f32(v[i][4 * w + 3]), inv, zpf));
-    if (c < nch) {  // rows of K bytes: chunk c's values start at byte c * NE
+    if (c < nch) {  // rows of Kp bytes: chunk c's values start at byte c * NE
       if constexpr (NE == 4) *((uint32_t*)xq + c) = d[0];
       else *((u32x2*)xq + c) = (u32x2){d[0], d[1]};
     }
@@ -1496,16 +1506,19 @@ __global__ __launch_bounds__(1024) void quantize_small_kernel(QuantSmall a) {
 }
 
 // x up to 320 KiB of fp32 or 160 KiB of 2-byte values (whose conversion, done
-// twice, costs more than the second launch beyond that: 304 KiB 7.9 us).
-bool quantize_small_fits(int64_t M, int64_t K, bool xvec) {
-  return xvec && K % 64 == 0 && M * K <= (int64_t)kQuantSmallChunks * 1024 * 4;
+// twice, costs more than the second launch beyond that: 304 KiB 7.9 us); half
+// of that for rows that are not dense (M = 17, K = 4000 of fp32: the call took
+// 28.3 us with one launch, 23.7 with two).
+bool quantize_small_fits(int64_t M, int64_t K, int64_t Kp, int64_t ldx, bool xvec) {
+  const bool dense = xvec && K == Kp && (ldx == K || M == 1);
+  return M * Kp <= (int64_t)(dense ? kQuantSmallChunks : kQuantSmallChunks / 2) * 1024 * 4;
 }
 
 int launch_quantize_small(const QuantSmall& a, int count, int xt, hipStream_t st) {
-  const int64_t bytes = (int64_t)a.M * a.K * (xt == XT_F32 ? 4 : 2);
+  const int64_t bytes = (int64_t)a.M * a.Kp * (xt == XT_F32 ? 4 : 2);
   const int need = (int)((bytes + 1024 * 16 - 1) / (1024 * 16));
-  bool dense = true;
-  for (int i = 0; i < count; ++i) dense = dense && (a.ldx[i] == a.K || a.M == 1);
+  bool dense = a.K == a.Kp;
+  for (int i = 0; i < count; ++i) dense = dense && (a.ldx[i] == a.K || a.M == 1) && (uintptr_t)a.x[i] % 16 == 0;
   const dim3 grid((unsigned)count), block(1024);
 #define SBQ_QS(XT_, C_)                                                                             \
   if (dense) hipLaunchKernelGGL((quantize_small_kernel<XT_, C_, true>), grid, block, 0, st, a);     \
@@ -1531,10 +1544,10 @@ int launch_quantize_small(const QuantSmall& a, int count, int xt, hipStream_t st
 // it on the same stream.
 int launch_quantize_acts(const void* x, int xt, int64_t M, int64_t K, int64_t Kp, int64_t ldx, bool xvec,
                          float2* partials, int8_t* xq, float* qpbuf, hipStream_t st, uint32_t* zero, int nzero) {
-  if (quantize_small_fits(M, K, xvec)) {
+  if (quantize_small_fits(M, K, Kp, ldx, xvec)) {
     QuantSmall a{};
     a.x[0] = x; a.ldx[0] = ldx; a.xq[0] = xq; a.qpbuf[0] = qpbuf;
-    a.M = (int)M; a.K = (int)K; a.zero = zero; a.nzero = nzero;
+    a.M = (int)M; a.K = (int)K; a.Kp = (int)Kp; a.zero = zero; a.nzero = nzero;
     return launch_quantize_small(a, 1, xt, st);
   }
   const int nparts = minmax_nparts(M, K);

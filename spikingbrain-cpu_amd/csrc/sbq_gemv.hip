@@ -611,10 +611,12 @@ int launch_gemv_w8_grouped(const GemvSeg* segs, int n, int xt, int64_t M, int64_
   a.nseg = n;
   for (int i = 0; i < n; ++i) a.seg[i] = segs[i];
   const int rc = launch_gemv_fast_grouped(fid, fks, a, xt, w8a8, st);
-  if (rc != -1 || !w8a8 || !xq0 || !quantize_small_fits(M, K, xvec)) return rc;
+  if (rc != -1 || !w8a8 || !xq0) return rc;
+  for (int i = 0; i < n; ++i)
+    if (!quantize_small_fits(M, K, K, segs[i].ldx, xvec)) return rc;
   QuantSmall q{};
   q.M = (int)M;
-  q.K = (int)K;
+  q.K = q.Kp = (int)K;
   for (int i = 0; i < n; ++i) {
     q.x[i] = segs[i].x;
     q.ldx[i] = segs[i].ldx;
@@ -643,15 +645,20 @@ int launch_gemv_w8a8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, b
   a.N = (int)N; a.Nt = (int)Nt; a.y = y; a.yt = yt; a.ldy = ldy; a.acc_out = acc_out; a.parts = parts;
   a.flags = (xvec ? 1 : 0) | (yvec ? 2 : 0);
   int fid, fks;
-  const bool fast = pick_gemv_fast(M, K, N, xt, true, xvec, &fid, &fks);
-  if (fast) {  // small x: the kernel reduces the activation min/max itself
+  if (M <= 16) {
     GemvArgs f = with_argmax(a, am);
-    int rc = launch_gemv_fast_cfg(fid, fks, f, xt, true, st);
-    if (rc == -1) {  // beyond that: quantized once, then the GEMV on the s8 rows
-      rc = launch_quantize_acts(x, xt, M, K, K, ldx, xvec, partials, xq, qpbuf, st);
+    int rc = -1;  // small aligned x: the kernel reduces the activation min/max itself
+    if (pick_gemv_fast(M, K, N, xt, true, xvec, &fid, &fks)) rc = launch_gemv_fast_cfg(fid, fks, f, xt, true, st);
+    if (rc == -1) {
+      // beyond that, and rows of any K or alignment: quantized once into rows
+      // of whole tiles, then the GEMV on those (M = 1 ... 16, N = 2999, K =
+      // 2500: fp32 11.7 -> 7.9 us at one row, 17.7 -> 8.6 at 8, 14.8 -> 10.3 at 16)
+      const int64_t Kp = Kc * 64;
+      rc = launch_quantize_acts(x, xt, M, K, Kp, ldx, xvec, partials, xq, qpbuf, st);
       if (rc) return rc;
-      f.x = xq; f.ldx = K; f.qpbuf = qpbuf;
-      pick_gemv_s8(M, K, N, &fid, &fks);
+      f.x = xq; f.ldx = Kp; f.K = (int)Kp; f.qpbuf = qpbuf;
+      f.flags |= kGemvXVec;
+      pick_gemv_s8(M, Kp, N, &fid, &fks);
       rc = launch_gemv_fast_cfg(fid, fks, f, XT_S8, true, st);
     }
     if (am) am->fused = rc == 0 && (f.flags & kGemvArgmax);

@@ -1130,9 +1130,9 @@ bool pick_gemv_fast(int64_t M, int64_t K, int64_t N, int xt, bool w8a8, bool xve
 // 9.6 against 10.3).
 void pick_gemv_s8(int64_t M, int64_t K, int64_t N, int* id, int* ks) {
   const int64_t Kc = K / 64, Nt = (N + 15) / 16;
-  const bool wide = Kc < 128 && Nt > 256;
-  *id = wide ? (Nt > 4096 ? 4 : 5) : 3;
-  *ks = wide || M > 8 ? 2 : 4;
+  const bool wide = Kc > 4 && Kc < 128 && Nt > 256;  // (K <= 256: one wave, as elsewhere)
+  *id = wide ? (Nt > 4096 ? 4 : 5) : (Kc > 4 ? 3 : 2);
+  *ks = Kc <= 4 ? 1 : (wide || M > 8 ? 2 : 4);
 }
 
 }  // namespace sbq

@@ -144,9 +144,9 @@ int launch_stage_act(const void* x, int xt, int64_t ldx, int64_t M, int64_t K, _
                      float* rscale, hipStream_t st, uint32_t* zero = nullptr, int nzero = 0);
 
 // W8A8 (fbgemm dynamic semantics).  The decode fast path quantizes a small x
-// in the kernel; a larger one is quantized before it into xq (s8 [M][Kc*64])
-// and (s_x, zp) in qpbuf, or (ragged or misaligned rows) its min/max goes
-// into `partials` (>= kMinMaxPartials float2).
+// in the kernel; a larger one, or ragged or misaligned rows, is quantized
+// before it into xq (s8 [M][Kc*64]) and (s_x, zp) in qpbuf; above 16 rows its
+// min/max goes into `partials` (>= kMinMaxPartials float2).
 int launch_gemv_w8a8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, bool xvec, const uint8_t* packed,
                      const float* scale, const int32_t* colsum, const float* bias, int64_t N, void* y, int yt,
                      int64_t ldy, int32_t* acc_out, float2* partials, int8_t* xq, float* qpbuf, hipStream_t st,
@@ -157,13 +157,13 @@ constexpr int kQuantSmallChunks = 20;  // 16-byte chunks of fp32 x per thread (1
 struct QuantSmall {
   const void* x[4];
   int64_t ldx[4];
-  int8_t* xq[4];    // s8 rows xq - 128 [M][K]
+  int8_t* xq[4];    // s8 rows xq - 128 [M][Kp]
   float* qpbuf[4];  // (s_x, zp bits)
-  int M, K;
+  int M, K, Kp;     // Kp: K rounded up to 64
   uint32_t* zero;   // counters to clear (nullable)
   int nzero;
 };
-bool quantize_small_fits(int64_t M, int64_t K, bool xvec);
+bool quantize_small_fits(int64_t M, int64_t K, int64_t Kp, int64_t ldx, bool xvec);
 int launch_quantize_small(const QuantSmall& a, int count, int xt, hipStream_t st);
 // ... or in two (min/max partials, then the rows) when x is larger.
 int launch_quantize_acts(const void* x, int xt, int64_t M, int64_t K, int64_t Kp, int64_t ldx, bool xvec,

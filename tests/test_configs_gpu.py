@@ -371,12 +371,14 @@ def test_fused_hybrid_group_vs_oracle(dev, fmt, M):
             np.testing.assert_array_equal(po.cpu().numpy(), o.cpu().numpy())
 
 
-# x beyond what the decode GEMV quantizes itself: quantized in one launch (up
-# to 320 KiB of fp32, 160 KiB of 2-byte values) or two, then the GEMV on the s8
-# rows with one and two row tiles per wave, 2 and 4 waves.
+# x beyond what the decode GEMV quantizes itself, or of ragged K: quantized in
+# one launch (up to 320 KiB of dense fp32, 160 KiB of dense 2-byte values, half
+# of that otherwise) or two, then the GEMV on the s8 rows with one and two row
+# tiles per wave, 1, 2 and 4 waves.
 S8_ROUTE = [(8, 2560, 9728, "f32"), (16, 40, 4096, "f32"), (5, 5001, 4160, "f32"), (9, 4096, 9088, "f32"),
             (10, 4000, 9728, "f32"), (8, 2560, 10240, "f16"), (16, 6150, 5120, "bf16"), (16, 100, 5184, "f16"),
-            (13, 70000, 2560, "f32"), (16, 64, 12288, "bf16"), (7, 512, 4800, "f16")]
+            (1, 2999, 2500, "f32"), (8, 5000, 61, "f16"), (3, 300, 130, "bf16"), (16, 4999, 2501, "f32"),
+            (11, 4200, 4093, "f16"), (13, 70000, 2560, "f32"), (16, 64, 12288, "bf16"), (7, 512, 4800, "f16")]
 
 
 @pytest.mark.gpu
@@ -391,11 +393,11 @@ def test_w8a8_decode_quantized_before_gemv(dev, M, N, K, xd):
     lin = quant.make_linear("int8-dyn", w)
     x = cpu_x(M, K, 4).to(dt)
     x[:, ::97] *= 20
-    wide = torch.zeros(M, K + 64, dtype=dt, device=dev)
+    wide = torch.full((M, K + 65), float("nan"), dtype=dt, device=dev)
     wide[:, :K] = x.to(dev)
     cols = tile_sample(N, 7)
     acc_ref, y_ref = ref_w8a8(x.float().numpy(), np.arange(M), *ref_rows(w, cols))
-    for xg in (x.to(dev), wide[:, :K]):
+    for xg in (x.to(dev), wide[:, :K]):  # dense, and rows one element off alignment with NaN beside them
         acc = torch.empty((M, N), dtype=torch.int32, device=dev)
         y = quant.linear_w8a8(xg, lin.packed, lin.scale, lin.colsum, None, N, acc_out=acc)
         np.testing.assert_array_equal(acc.cpu().numpy()[:, cols], acc_ref)
