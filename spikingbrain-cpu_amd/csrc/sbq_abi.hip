@@ -202,7 +202,7 @@ int sbq_unpack_w8(const uint8_t* packed, int64_t N, int64_t K, int8_t* q, int64_
 
 int64_t sbq_w8_workspace_bytes(int64_t M, int64_t K, int x_dtype) {
   if (M < 0 || K < 0 || M > kIntMax || K > kIntMax || !valid_dtype(x_dtype)) return 0;
-  return 256 + sbq::w8_ws_layout(M, ((K + 63) / 64) * 64, x_dtype).bytes;
+  return 256 + sbq::w8_ws_layout(M, K, x_dtype).bytes;
 }
 
 }  // extern "C"
@@ -222,9 +222,6 @@ int linear_w8_run(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
                                 alt, yparts);
     if (rc != -1) return rc;
   }
-  if (sbq::gemv_supports(M, K, false, x_dtype))
-    return sbq::launch_gemv_w8(x, x_dtype, M, K, ldx, xv, packed, scale, bias, N, y, y_dtype, ldy, st, yv, nullptr,
-                               yparts);
   // optional scratch of the prefill GEMM (row sums, staged activations), 256-byte aligned
   void* ws = nullptr;
   int64_t ws_bytes = 0;
@@ -232,6 +229,18 @@ int linear_w8_run(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
     ws = (void*)(((uintptr_t)workspace + 255) & ~(uintptr_t)255);
     ws_bytes = (int64_t)workspace_bytes - (int64_t)((uintptr_t)ws - (uintptr_t)workspace);
   }
+  if (K % 64 != 0 && ws && M <= 16 && sbq::pad_decode_rows(M, N, K, x_dtype)) {
+    // ragged K at decode sizes: rows of whole tiles, then the fast GEMV
+    uint8_t* rows = (uint8_t*)ws + sbq::w8_ws_layout(M, K, x_dtype).planes;
+    const int64_t Kp = (K + 63) / 64 * 64;
+    const int rc = sbq::launch_pad_rows(x, x_dtype, M, K, ldx, rows, st);
+    if (rc) return rc;
+    return sbq::launch_gemv_w8(rows, x_dtype, M, Kp, Kp, true, packed, scale, bias, N, y, y_dtype, ldy, st, yv, nullptr,
+                               yparts);
+  }
+  if (!(K % 64 != 0 && ws && M > 16) && sbq::gemv_supports(M, K, false, x_dtype))
+    return sbq::launch_gemv_w8(x, x_dtype, M, K, ldx, xv, packed, scale, bias, N, y, y_dtype, ldy, st, yv, nullptr,
+                               yparts);
   return sbq::launch_gemm_w8(x, x_dtype, M, K, ldx, xv, packed, scale, bias, N, y, y_dtype, ldy, ws, ws_bytes, st,
                              yv, yparts);
 }
@@ -346,6 +355,7 @@ bool runs_tiled_gemm(int64_t M, int64_t N, int64_t K, int x_dtype, bool w8a8) {
     if (w8a8_runs_mt(M, N, K, sbq::split_area_bytes(p))) return false;
     return !sbq::gemv_supports(M, K, true, x_dtype);
   }
+  if (M > 16 && K % 64 != 0) return true;  // staged as rows of whole tiles
   if (M > 16 && M <= 64 && (x_dtype == SBQ_F16 || x_dtype == SBQ_BF16) && sbq::gemv_mt_applies(M, K, N, x_dtype, true))
     return false;
   return !sbq::gemv_supports(M, K, false, x_dtype);
@@ -357,6 +367,8 @@ int64_t sbq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int x_dtype,
   const int64_t Nt = (N + 15) / 16, Kc = (K + 63) / 64;
   const int64_t base = w8a8 ? sbq_w8a8_workspace_bytes(M, K) : sbq_w8_workspace_bytes(M, K, x_dtype);
   if (M == 0 || !runs_tiled_gemm(M, N, K, x_dtype, w8a8 != 0)) return base;
+  if (!w8a8 && K % 64 != 0)  // exact weights, fp32 x as two planes
+    return base + sbq::split_area_bytes(sbq::plan_gemm_dl(false, sbq::XT_BF16, M, Nt, Kc * (x_dtype == SBQ_F32 ? 2 : 1), true));
   // the GEMM's operands are s8 (W8A8) or fp16 (weight-only, fp32 / bf16 staged as an fp16 plane)
   return base + sbq::split_area_bytes(sbq::plan_gemm_dl(w8a8 != 0, 1, M, Nt, Kc, true));
 }
@@ -371,6 +383,12 @@ int sbq_gemm_config(int64_t M, int64_t N, int64_t K, int x_dtype, int w8a8, int*
   if (!valid_dtype(x_dtype)) return SBQ_ERR_DTYPE;
   if (M < 1 || N < 1 || K < 1 || M > kIntMax || N > kIntMax || K > kIntMax || (w8a8 != 0 && w8a8 != 1))
     return SBQ_ERR_ARG;
+  if (!w8a8 && K % 64 != 0) {  // exact weights, fp32 x as two planes
+    const sbq::DlPlan p = sbq::plan_gemm_dl(false, sbq::XT_BF16, M, (N + 15) / 16,
+                                            (K + 63) / 64 * (x_dtype == SBQ_F32 ? 2 : 1), true);
+    if (splits) *splits = runs_tiled_gemm(M, N, K, x_dtype, false) ? p.splits : 0;
+    return p.id;
+  }
   // with that workspace every activation dtype reaches the GEMM as fp16 (W-only:
   // fp32 / bf16 staged as an fp16 plane, row sums precomputed) or s8 (W8A8)
   const sbq::DlPlan p = sbq::plan_gemm_dl(w8a8 != 0, sbq::XT_F16, M, (N + 15) / 16, (K + 63) / 64, true);

@@ -67,6 +67,12 @@ struct GemmOp<XT_F32> {
   }
 };
 
+// fp16 activations against exactly converted weights (the direct-to-LDS GEMM's
+// XT_F16 multiplies weights offset by 128 instead and needs row sums).
+constexpr int XT_F16E = 4;
+template <>
+struct GemmOp<XT_F16E> : GemmOp<XT_F16> {};
+
 // Convert 8 fp32 activations into the operand plane(s) (16 bytes each).
 template <int XT>
 __device__ __forceinline__ void x8_to_planes(const float* t, u32x4* planes) {
@@ -284,6 +290,7 @@ struct GemmArgs {
   const void* x;  // W-only: fp16/bf16 activations; I8: s8 quantized activations
   int64_t ldx;    // row stride: elements (W-only) or bytes (I8)
   int M, Kc;
+  int Kw;         // bf16 / XT_F16E: weight tiles per row; x may hold several planes of Kw tiles (Kc = planes * Kw)
   const uint8_t* packed;
   const float* scale;
   const float* bias;
@@ -434,6 +441,9 @@ __global__ __launch_bounds__(KG* WN* WM * 64, (SK ? (dl_min_waves<I8, XT, BN, BM
   }
   const int nt0 = bx * WT, m0 = by * BM;
   const int M = a.M, Kc = a.Kc, Nt = a.Nt;
+  // planes of x (exact weights only): x tile kc meets weight tile kc mod Kw
+  constexpr bool PLANES = !I8 && !OFS;
+  const int Kw = PLANES ? a.Kw : Kc;
   // stage steps of KT K tiles (the host keeps Kc % KT == 0)
   const int KX = Kc / KT;
   // split K over gridDim.z workgroups: split z takes stage steps [zb, zb + zc)
@@ -455,7 +465,7 @@ __global__ __launch_bounds__(KG* WN* WM * 64, (SK ? (dl_min_waves<I8, XT, BN, BM
 #pragma unroll
   for (int i2 = 0; i2 < WT / GW; ++i2) {
     const int j = w * (WT / GW) + i2;
-    woff[i2] = (uint32_t)(min(nt0 + j, Nt - 1) - nt0) * (uint32_t)Kc * 1024u + lane * 16;
+    woff[i2] = (uint32_t)(min(nt0 + j, Nt - 1) - nt0) * (uint32_t)Kw * 1024u + lane * 16;
   }
 #pragma unroll
   for (int i2 = 0; i2 < XR / GW; ++i2) {
@@ -471,7 +481,7 @@ __global__ __launch_bounds__(KG* WN* WM * 64, (SK ? (dl_min_waves<I8, XT, BN, BM
     }
   }
   const __amdgpu_buffer_rsrc_t wrs =
-      raw_rsrc(a.packed + (int64_t)nt0 * Kc * 1024, (uint32_t)min((int64_t)(Nt - nt0) * Kc * 1024, (int64_t)0xffffffff));
+      raw_rsrc(a.packed + (int64_t)nt0 * Kw * 1024, (uint32_t)min((int64_t)(Nt - nt0) * Kw * 1024, (int64_t)0xffffffff));
   const __amdgpu_buffer_rsrc_t xrs =
       raw_rsrc(xg + (int64_t)m0 * xrow, (uint32_t)min((int64_t)(M - m0) * xrow, (int64_t)0xffffffff));
 
@@ -486,7 +496,8 @@ __global__ __launch_bounds__(KG* WN* WM * 64, (SK ? (dl_min_waves<I8, XT, BN, BM
       const int kc = ks * KT + j;
       const int sb = __builtin_amdgcn_readfirstlane((kg * NS + st) * STAGE + j * SUB);
 #pragma unroll
-      for (int i2 = 0; i2 < WT / GW; ++i2) lds_dma16_buf(wrs, woff[i2], kc * 1024, lds + sb + wslot + i2 * 1024);
+      for (int i2 = 0; i2 < WT / GW; ++i2)
+        lds_dma16_buf(wrs, woff[i2], (PLANES && kc >= Kw ? kc - Kw : kc) * 1024, lds + sb + wslot + i2 * 1024);
 #pragma unroll
       for (int i2 = 0; i2 < XR / GW; ++i2)
         lds_dma16_buf(xrs, xoff[i2], kc * (I8 ? 64 : 128), lds + sb + xslot + i2 * 1024);
@@ -1152,12 +1163,26 @@ int launch_dl_split(int id, bool i8, const GemmArgs& a, hipStream_t st) {
 // Launch of direct-to-LDS configuration `id` (tuning entry; -1: no such id).
 // Arguments with a split-K area (a.part) run the split instances.
 int launch_gemm_dl_cfg(int id, bool i8, int xt, const GemmArgs& a, hipStream_t st) {
-  if (a.part) return i8 || xt == XT_F16 ? launch_dl_split(id, i8, a, st) : -1;
+  if (a.part) {
+    if (!i8 && id == 22 && xt == XT_BF16) return launch_dl<false, XT_BF16, 64, 64, 4, 1, 3, 1, false, 1, true>(a, st);
+    if (!i8 && id == 22 && xt == XT_F16E) return launch_dl<false, XT_F16E, 64, 64, 4, 1, 3, 1, false, 1, true>(a, st);
+    return i8 || xt == XT_F16 ? launch_dl_split(id, i8, a, st) : -1;
+  }
   if (i8) return launch_dl_i8(id, a, st);
   // 192 x 64 blocks with K split over 4 wave groups leave no LDS for the
   // in-loop row sums: without precomputed sums the 128 x 64 split runs
   if (xt == XT_F16) return a.rsum ? launch_dl_rsp(id, a, st) : launch_dl_id<false, XT_F16>(id == 17 ? 5 : id, a, st);
   if (xt == XT_BF16) return launch_dl_id<false, XT_BF16>(id, a, st);
+  if (xt == XT_F16E) {  // the configurations pick_gemm_dl chooses for exact weights
+    switch (id) {
+      case 0: return launch_dl<false, XT_F16E, 256, 128, 4, 2, 2, 1>(a, st);
+      case 5: return launch_dl<false, XT_F16E, 128, 64, 2, 2, 2, 4>(a, st);
+      case 8: return launch_dl<false, XT_F16E, 64, 64, 1, 2, 2, 4>(a, st);
+      case 10: return launch_dl<false, XT_F16E, 256, 128, 4, 1, 2, 1>(a, st);
+      case 22: return launch_dl<false, XT_F16E, 64, 64, 4, 1, 3, 1>(a, st);
+    }
+    return -1;
+  }
   return -2;
 }
 
@@ -1293,9 +1318,13 @@ int pick_gemm_dl(bool i8, int xt, int64_t M, int64_t Nt, int64_t Kc) {
 // included).
 constexpr int kMidId = 22;
 
+// (Exact weights, the ragged-K route, take it as fp16 W-only does: their grids
+// with K over 4 wave groups of 64 x 32 wave tiles converted every weight tile
+// twice; N = 2999, K = 2500, M = 77, fp16: 17.7 -> 15.7 us;
+// N = 1000, K = 9001, fp32: 80.5 -> 37.6.)
 DlPlan plan_gemm_dl(bool i8, int xt, int64_t M, int64_t Nt, int64_t Kc, bool rsp) {
   DlPlan p{pick_gemm_dl(i8, xt, M, Nt, Kc), 1, 0, 0};
-  if (!i8 && !(xt == XT_F16 && rsp)) return p;
+  if (!i8 && !rsp) return p;
   if (M > 128) return p;
   const int64_t tiles = ((Nt + 3) / 4) * ((M + 63) / 64);
   if (tiles > 512) return p;
@@ -1335,7 +1364,10 @@ constexpr int kBN = 128, kBM = 128, kWN = 2, kWM = 2;
 
 W8Ws w8_ws_layout(int64_t M, int64_t K, int xt) {
   auto r256 = [](int64_t b) { return (b + 255) & ~(int64_t)255; };
-  const int np = xt == XT_F32 || xt == XT_BF16 ? 1 : 0;  // one staged fp16 plane
+  // one staged fp16 plane; ragged K: rows of whole tiles, fp32 as two bf16 planes
+  const bool rag = K % 64 != 0;
+  const int np = rag ? (xt == XT_F32 ? 2 : 1) : (xt == XT_F32 || xt == XT_BF16 ? 1 : 0);
+  K = (K + 63) / 64 * 64;
   W8Ws l;
   l.rowsum = 0;
   l.rscale = r256(M * 4);
@@ -1360,9 +1392,31 @@ int launch_gemm_w8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, boo
   const bool dl = xvec && K % 64 == 0 && ldx <= ((int64_t)1 << 21) && K <= ((int64_t)1 << 21);
   const W8Ws l = w8_ws_layout(M, K, xt);
   const bool staged = dl && ws && ws_bytes >= l.bytes;
+  // ragged K with a workspace: x into rows of whole tiles (any row alignment),
+  // then the direct-to-LDS GEMM on exactly converted weights: the products of
+  // the register-staged kernel below, 5-6 times faster at M = 33 ... 1000
+  // (N = 2999, K = 2500, fp16: M = 33 85.9 -> 12.7 us, M = 77 93.5 -> 15.7, M =
+  // 1000 132.8 -> 43.7; N = 1000, K = 9001, fp32, M = 77 351 -> 37.6)
+  const int64_t Kp = Kc * 64;
+  const int np = xt == XT_F32 ? 2 : 1;
+  if (K % 64 != 0 && ws && ws_bytes >= l.bytes && Kp * np <= ((int64_t)1 << 21)) {
+    uint8_t* planes = (uint8_t*)ws + l.planes;
+    GemmArgs a{};
+    const DlPlan plan = plan_gemm_dl(false, XT_BF16, M, Nt, Kc * np, true);
+    int ncount = 0;
+    uint32_t* zero = attach_split(a, plan, (uint8_t*)ws + l.bytes, ws_bytes - l.bytes, &ncount);
+    const int rc = xt == XT_F32 ? launch_split_rows(x, M, K, ldx, planes, st, zero, ncount)
+                                : launch_pad_rows(x, xt, M, K, ldx, planes, st, zero, ncount);
+    if (rc) return rc;
+    a.x = planes; a.ldx = Kp * np; a.M = (int)M; a.Kc = (int)Kc * np; a.Kw = (int)Kc;
+    a.packed = packed; a.scale = scale; a.bias = bias;
+    a.N = (int)N; a.Nt = (int)Nt; a.y = y; a.yt = yt; a.ldy = ldy; a.parts = parts; a.flags = flags | 1;
+    const int id = zero || plan.splits == 1 ? plan.id : pick_gemm_dl(false, XT_BF16, M, Nt, a.Kc);
+    return launch_gemm_dl_cfg(id, false, xt == XT_F16 ? XT_F16E : XT_BF16, a, st);
+  }
   if (dl && (xt != XT_F32 || staged)) {
     GemmArgs a{};
-    a.x = x; a.ldx = ldx; a.M = (int)M; a.Kc = (int)Kc;
+    a.x = x; a.ldx = ldx; a.M = (int)M; a.Kc = a.Kw = (int)Kc;
     a.packed = packed; a.scale = scale; a.bias = bias;
     a.N = (int)N; a.Nt = (int)Nt; a.y = y; a.yt = yt; a.ldy = ldy; a.parts = parts; a.flags = flags;
     const int gxt = staged ? XT_F16 : xt;  // fp32 / bf16 activations are staged as an fp16 plane

@@ -120,7 +120,8 @@ DlPlan plan_gemm_dl(bool i8, int xt, int64_t M, int64_t Nt, int64_t Kc, bool rsp
 int64_t split_area_bytes(const DlPlan& p);
 
 // W-only prefill scratch: [rowsum: M floats][rscale: M floats][fp16 plane: M x K for
-// fp32 and bf16 x, none for fp16], each part 256-byte aligned.
+// fp32 and bf16 x, none for fp16; ragged K: rows of whole tiles, two bf16
+// planes for fp32], each part 256-byte aligned.
 struct W8Ws {
   int64_t rowsum, rscale, planes, bytes;
 };
@@ -138,6 +139,24 @@ int launch_quantize_rows_sym(const void* x, int xt, int64_t ldx, bool xvec, int6
                              int8_t* xq, float* s_out, hipStream_t st);
 // Per-row sums in fp32 of fp16 x [M, K] (K % 8 == 0, 16-byte aligned rows).
 int launch_rowsum_f16(const void* x, int64_t ldx, int64_t M, int64_t K, float* out, hipStream_t st,
+                      uint32_t* zero = nullptr, int nzero = 0);
+// x [M, K] of any row stride, alignment and K as rows of Kp = ceil(K/64)*64
+// columns, padding 0: a copy in x's dtype, and (fp32) bf16 high and remainder
+// planes, [M][2][Kp].
+int launch_pad_rows(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, void* out, hipStream_t st,
+                    uint32_t* zero = nullptr, int nzero = 0);
+// Whether a ragged weight-only call at decode sizes (M <= 16) gains from padded
+// rows and the fast GEMV, a launch more than the general GEMV.  Measured in HIP
+// graphs (us, general -> padded): 2999 x 2500, fp32 13.0 -> 8.3 at 4 rows and
+// 9.7 -> 10.8 at 16, fp16 8.8 -> 6.7 and 15.8 -> 8.2, one row 7.2 -> 8.4 / 5.5 ->
+// 8; 11999 x 4000, fp32 31.5 -> 16.4 at 4 rows, 16.5 -> 12.8 at one; 1000 x
+// 9001, fp32 24.5 -> 9.8 at one row, 60.2 -> 24.6 at 16, fp16 33.6 -> 10.3 at 4,
+// 10.9 -> 10.8 at one.
+inline bool pad_decode_rows(int64_t M, int64_t N, int64_t K, int xt) {
+  if (xt == 0 && M > 8) return K >= 4096 || N * K >= (int64_t)1 << 23;
+  return M > 1 || (xt == 0 && (K >= 4096 || N * K >= (int64_t)1 << 24));
+}
+int launch_split_rows(const void* x, int64_t M, int64_t K, int64_t ldx, void* out, hipStream_t st,
                       uint32_t* zero = nullptr, int nzero = 0);
 // fp32 / bf16 x [M, K] -> a scaled fp16 plane, row sums and row scales.
 int launch_stage_act(const void* x, int xt, int64_t ldx, int64_t M, int64_t K, _Float16* xs, float* rowsum,

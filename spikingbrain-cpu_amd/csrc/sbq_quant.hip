@@ -593,6 +593,51 @@ __global__ __launch_bounds__(256) void stage_act_kernel(const void* __restrict__
   }
 }
 
+// x as rows of whole K tiles (PLANES 1: a copy in x's dtype; PLANES 2: fp32 as
+// bf16 high and remainder planes, [M][2][Kp]); one 8-value chunk per thread,
+// loads of whatever alignment, a row's last chunk by elements, padding 0.
+template <int XT, int PLANES>
+__global__ __launch_bounds__(256) void pad_rows_kernel(const void* __restrict__ xv, int64_t ldx, int64_t nch, int cpr,
+                                                       int K, uint8_t* __restrict__ out,
+                                                       uint32_t* __restrict__ zero, int nzero) {
+  zero_counters(zero, nzero);
+  typedef typename XElem<XT>::T T;
+  typedef T v4 __attribute__((ext_vector_type(4)));
+  typedef T v4_any __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+  const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (c >= nch) return;
+  const int64_t m = c / cpr;
+  const int k0 = (int)(c - m * cpr) * 8;
+  const T* p = (const T*)xv + m * ldx + k0;
+  v4 v[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    if (k0 + 4 * h + 4 <= K) {
+      v[h] = *(const v4_any*)(p + 4 * h);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[h][j] = k0 + 4 * h + j < K ? p[4 * h + j] : (T)0.0f;
+    }
+  }
+  if constexpr (PLANES == 1) {
+    v4* o = (v4*)(out + c * 8 * sizeof(T));
+    o[0] = v[0];
+    o[1] = v[1];
+  } else {
+    bf16x8 hi, lo;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      __bf16 a, b;
+      split_bf16(XElem<XT>::to_f32(v[j / 4][j % 4]), a, b);
+      hi[j] = a;
+      lo[j] = b;
+    }
+    __bf16* o = (__bf16*)out + m * cpr * 16 + k0;
+    *(bf16x8*)o = hi;
+    *(bf16x8*)(o + cpr * 8) = lo;
+  }
+}
+
 // One workgroup per row; each thread keeps four independent running bests
 // and has sixteen vector loads in flight at a time (a 151936-wide row is
 // three rounds of loads).
@@ -764,6 +809,27 @@ int launch_stage_act(const void* x, int xt, int64_t ldx, int64_t M, int64_t K, _
                        zero, nzero);
   else
     return -2;
+  return check_launch();
+}
+
+int launch_pad_rows(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, void* out, hipStream_t st, uint32_t* zero,
+                    int nzero) {
+  const int64_t cpr = (K + 63) / 64 * 8, nch = M * cpr;
+  const dim3 grid((unsigned)((nch + 255) / 256)), block(256);
+  switch (xt) {
+    case XT_F32: hipLaunchKernelGGL((pad_rows_kernel<XT_F32, 1>), grid, block, 0, st, x, ldx, nch, (int)cpr, (int)K, (uint8_t*)out, zero, nzero); break;
+    case XT_F16: hipLaunchKernelGGL((pad_rows_kernel<XT_F16, 1>), grid, block, 0, st, x, ldx, nch, (int)cpr, (int)K, (uint8_t*)out, zero, nzero); break;
+    case XT_BF16: hipLaunchKernelGGL((pad_rows_kernel<XT_BF16, 1>), grid, block, 0, st, x, ldx, nch, (int)cpr, (int)K, (uint8_t*)out, zero, nzero); break;
+    default: return -2;
+  }
+  return check_launch();
+}
+
+int launch_split_rows(const void* x, int64_t M, int64_t K, int64_t ldx, void* out, hipStream_t st, uint32_t* zero,
+                      int nzero) {
+  const int64_t cpr = (K + 63) / 64 * 8, nch = M * cpr;
+  hipLaunchKernelGGL((pad_rows_kernel<XT_F32, 2>), dim3((unsigned)((nch + 255) / 256)), dim3(256), 0, st, x, ldx, nch,
+                     (int)cpr, (int)K, (uint8_t*)out, zero, nzero);
   return check_launch();
 }
 

@@ -216,7 +216,7 @@ def linear_w8(x2: torch.Tensor, packed: torch.Tensor, scale: torch.Tensor, bias:
     M, K = x2.shape
     y = out if out is not None else torch.empty((M, N), dtype=out_dtype, device=x2.device)
     ws = workspace
-    if ws is None and M > 16:  # decode sizes run the GEMV, which needs none
+    if ws is None and (M > 16 or K % 64):  # aligned decode sizes run the GEMV, which needs none
         ws = w8_workspace(M, K, x2.device, x2.dtype, N)
     _check_operands("linear_w8", x2, packed, N, y, (("scale", scale, torch.float32), ("bias", bias, torch.float32)),
                     ws)
@@ -391,7 +391,7 @@ def _linear_parts(x2: torch.Tensor, packed: torch.Tensor, scale: torch.Tensor, c
     M, K = x2.shape
     y = torch.empty((M * width,), dtype=out_dtype, device=x2.device)
     if colsum is None:
-        ws = w8_workspace(M, K, x2.device, x2.dtype, N) if M > 16 else None
+        ws = w8_workspace(M, K, x2.device, x2.dtype, N) if M > 16 or K % 64 else None
         vectors = (("scale", scale, torch.float32), ("bias", bias, torch.float32))
     else:
         ws = w8a8_workspace(M, K, x2.device, N, x2.dtype)

@@ -371,6 +371,47 @@ def test_fused_hybrid_group_vs_oracle(dev, fmt, M):
             np.testing.assert_array_equal(po.cpu().numpy(), o.cpu().numpy())
 
 
+# Ragged K: padded rows and the fast GEMV (M <= 16), padded rows or bf16 planes
+# and the direct-to-LDS GEMM: K split over 4, 3 and 2 workgroups, the 64 x 64
+# grid unsplit, and the larger blocks (128 x 64 with K in 4 groups, 256 x 128).
+RAGGED_CASES = [(1, 4200, 4001), (2, 130, 65), (4, 2999, 2500), (16, 33, 1001), (17, 2999, 2500), (32, 40, 127),
+                (33, 5000, 300), (77, 2999, 2500), (128, 11999, 190), (100, 20, 9001), (129, 2999, 2500),
+                (300, 4100, 1111), (1000, 12000, 70)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("xd", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("M,N,K", RAGGED_CASES)
+def test_w8_ragged_k_routes(dev, M, N, K, xd):
+    """Dense and misaligned rows (NaN beside them), with a bias: within the
+    split's 16 bits of the float64 product of the quantized weights (fp32 x;
+    hi + lo: 2^-17 per value), or fp32 summation (2-byte x, exact products);
+    a graph replay equals the eager call (the split's counters come back)."""
+    announce(f"w8 ragged M={M} N={N} K={K} x={xd}")
+    dt = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}[xd]
+    w = gpu_weight(N, K, 13, dev)
+    bias = cpu_x(1, N, 14).reshape(-1)
+    lin = quant.Int8Linear(w, bias.to(dev))
+    x = cpu_x(M, K, 15).to(dt)
+    q, s = oracle.quantize_per_channel(w.float().cpu().numpy())
+    ref = x.double() @ torch.from_numpy(q).double().t() * torch.from_numpy(s).double() + bias.double()
+    bar = 8e-6 if xd == "f32" else 2e-6
+    wide = torch.full((M, K + 3), float("nan"), dtype=dt, device=dev)
+    wide[:, 1:K + 1] = x.to(dev)
+    for xg in (x.to(dev), wide[:, 1:K + 1]):
+        y = lin(xg)
+        assert oracle.rel_l2(y.cpu().numpy(), ref.numpy()) <= bar
+    static = x.to(dev)
+    lin(static)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = lin(static)
+    for k in range(3):
+        static.mul_(-1.0)
+        g.replay()
+        assert torch.equal(out, lin(static)), k
+
+
 # x beyond what the decode GEMV quantizes itself, or of ragged K: quantized in
 # one launch (up to 320 KiB of dense fp32, 160 KiB of dense 2-byte values, half
 # of that otherwise) or two, then the GEMV on the s8 rows with one and two row
