@@ -1012,12 +1012,15 @@ bool pick_gemv_fast(int64_t M, int64_t K, int64_t N, int xt, bool w8a8, bool xve
     // x in LDS (weight-only, M <= 8: split once into bf16 planes) when it
     // fits 24 KiB, or 48 KiB for one row (M = 1, K = 12288: 16% faster than
     // direct steps; the raw copy and the planes then hold 96 KiB of LDS, one
-    // workgroup per CU).  One row of a wide layer takes 4-tile steps over two
-    // row tiles per wave with 8 waves per workgroup (half the copies and
-    // splits: QKV and gate+up at K = 4096 2-6% faster) unless that grid needs
-    // fewer rounds of the 256 CUs than one row tile per workgroup
-    // (measured on MI355X at M = 1: N = 19456 and 18820 at K = 2560, 14.0 ->
-    // 12.0 us; N = 5120, K = 4096 keeps two tiles, 7.9 -> 7.2 us against one).
+    // workgroup per CU).  One or two rows of a wide layer (x up to 48 KiB)
+    // take 4-tile steps over two row tiles per wave (half the copies and
+    // splits) unless one row tile per workgroup needs fewer rounds of the 256
+    // CUs for its rows than that grid (N = 10000, K = 4096: 10.5 us against
+    // 10.7 with two tiles): 8 waves per workgroup at K > 3072 (M = 1, N =
+    // 5120, K = 4096: 6.7 us, four waves 7.1; one tile 7.7; M = 2, N = 6144:
+    // 7.5, direct steps 8.5), 4 waves below, where 8 leave each wave five
+    // tiles (K = 2560: N = 151936 58.3 us, eight waves over 70; 12288 8.2,
+    // 9.4; M = 2, 151936: 62.0, 71.9).
     // Long K over at most 256 row tiles takes 8 waves (N = 2560, K = 9728:
     // 8.9 -> 8.5 us; N = 4096, K = 12288: 11.6 -> 11.35 us).  Else direct steps: 8 tiles over one row tile for long
     // K, 4 tiles over two row tiles for wide layers, 4 tiles over one row
@@ -1026,17 +1029,21 @@ bool pick_gemv_fast(int64_t M, int64_t K, int64_t N, int xt, bool w8a8, bool xve
     const int64_t xb = M * K * 4;
     const bool xl = (w8a8 || M <= 8) && (xb <= 24576 || (!w8a8 && M == 1 && xb <= kFastSplitBytes));
     const auto rounds = [](int64_t wgs) { return (wgs + 255) / 256; };
-    const bool wide1 = xl && !w8a8 && M == 1 && Kc < 128 && Nt > 256 && rounds(Nt) >= 2 * rounds((Nt + 1) / 2);
+    const bool wide1 = !w8a8 && M <= 2 && xb <= kFastSplitBytes && Kc < 128 && Nt > 256 &&
+                       rounds(Nt) >= 2 * rounds((Nt + 1) / 2);
     *id = wide1 ? 6 : (xl ? 0 : (Kc >= 128 ? 3 : (Nt >= 384 ? 4 : 2)));
-    *ks = wide1 || (xl && !w8a8 && Kc >= 128 && Nt <= 256) ? 8 : 4;
+    *ks = (wide1 && Kc > 48) || (xl && !w8a8 && Kc >= 128 && Nt <= 256) ? 8 : 4;
     if (!w8a8 && Kc <= 4) {
       *id = 2;
       *ks = 1;
     }
-    // M = 4 .. 8 on a wide short-K layer whose grid of five row tiles per
+    // M <= 8 on a wide short-K layer whose grid of five row tiles per
     // workgroup fits one round of the CUs: x (up to 80 KiB) loaded into
     // registers and split into planes in LDS, read once per five row tiles
-    if (!w8a8 && M >= 4 && M <= 8 && Kc < 128 && Nt > 1024 && (Nt + 4) / 5 <= 256 && xb <= kSplitWideBytes) {
+    // (K = 2560, N = 19456 / 18820: M = 1 11.9 -> 10.9 / 11.7 -> 10.7 us
+    // against one tile, M = 2 13.6 -> 11.0, M = 3 14.4 -> 11.2; N = 17000,
+    // K = 4096, M = 1: 15.2 -> 13.9)
+    if (!w8a8 && M <= 8 && Kc < 128 && Nt > 1024 && (Nt + 4) / 5 <= 256 && xb <= kSplitWideBytes) {
       *id = 7;  // D=2, G=5, x in LDS
       *ks = 8;
     }
@@ -1058,7 +1065,10 @@ bool pick_gemv_fast(int64_t M, int64_t K, int64_t N, int xt, bool w8a8, bool xve
       //   fewer than 256 row tiles (N = 4 .. 3000: 0.1-0.4 us per launch), and
       //   on wide layers whose two-tile grid takes more rounds of 256 CUs
       //   than the one-tile grid (N = 18820: 15.0 -> 14.2 us, N = 10000:
-      //   10.2 -> 9.2 us; N = 6144, 8192, 24576 and 151936 keep two tiles).
+      //   10.2 -> 9.2 us; N = 6144, 8192, 24576 and 151936 keep two tiles);
+      //   two waves on the wide ones at K <= 3072 (M = 1, K = 2560: N = 18820
+      //   11.0 -> 10.1 us, 19456 11.0 -> 10.2, 12288 7.8 -> 7.4; K = 4096
+      //   keeps four).
       const auto rounds = [](int64_t wgs) { return (wgs + 255) / 256; };
       const bool xl = M * K * 2 <= kFastXLdsBytes;
       if (Kc <= 4) {
@@ -1066,6 +1076,7 @@ bool pick_gemv_fast(int64_t M, int64_t K, int64_t N, int xt, bool w8a8, bool xve
         *ks = 1;
       } else if (xl && (wide ? rounds(Nt) < 2 * rounds((Nt + 1) / 2) : Nt < 256)) {
         *id = 0;  // D=8, G=1, x in LDS
+        if (wide && Kc <= 48) *ks = 2;
       }
       // M = 4 .. 8, a wide layer at short K whose grid of five row tiles per
       // workgroup fills one round of the CUs: x (up to 64 KiB) in LDS, read
