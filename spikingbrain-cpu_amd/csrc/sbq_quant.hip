@@ -701,6 +701,47 @@ __global__ __launch_bounds__(1024) void argmax_rows_kernel(const float* __restri
   }
 }
 
+// Long rows over many workgroups, with no scratch but the output: out[row]
+// holds the row's largest argmax_key (sbq_index.h) until the last launch
+// replaces it by the key's column.  One workgroup per row reads 608 KB through
+// one CU (V = 151936, one row: 46 us in a HIP graph); these three launches,
+// slices of the rows over 64 workgroups: 7.1 us, 8 rows 46 -> 12.4; V = 32000
+// 14.9 -> 6.1.
+__global__ __launch_bounds__(256) void argmax_clear_kernel(unsigned long long* __restrict__ out, int64_t M) {
+  const int64_t m = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (m < M) out[m] = 0ull;  // below every key
+}
+
+__global__ __launch_bounds__(256) void argmax_slice_kernel(const float* __restrict__ y, int N, int64_t ldy, int per,
+                                                           unsigned long long* __restrict__ out) {
+  constexpr int U = 8;
+  const int64_t rowi = blockIdx.y;
+  const float* row = y + rowi * ldy;
+  const int i0 = blockIdx.x * per, i1 = min(i0 + per, N), t = threadIdx.x;
+  unsigned long long best = 0;
+  for (int b = i0 + t; b < i1; b += U * 256) {
+    float v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = row[min(b + u * 256, i1 - 1)];  // clamped: the slice's last value again
+#pragma unroll
+    for (int u = 0; u < U; ++u) best = max(best, argmax_key(v[u], min(b + u * 256, i1 - 1)));
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) best = max(best, (unsigned long long)__shfl_xor(best, o, 64));
+  __shared__ unsigned long long red[4];
+  if ((t & 63) == 0) red[t >> 6] = best;
+  __syncthreads();
+  if (t == 0) {
+    best = max(max(red[0], red[1]), max(red[2], red[3]));
+    __hip_atomic_fetch_max(out + rowi, best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+__global__ __launch_bounds__(256) void argmax_index_kernel(unsigned long long* __restrict__ out, int64_t M) {
+  const int64_t m = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (m < M) out[m] = (unsigned long long)argmax_key_index(out[m]);
+}
+
 // ---------------------------------------------------------------------------
 // host launchers
 // ---------------------------------------------------------------------------
@@ -861,6 +902,18 @@ int launch_quantize_rows_sym(const void* x, int xt, int64_t ldx, bool xvec, int6
 }
 
 int launch_argmax_rows(const float* y, int64_t M, int64_t N, int64_t ldy, int64_t* out, hipStream_t st) {
+  // rows that one workgroup takes several rounds of loads for (N = 8192: 8.6 us
+  // in one launch), until the rows alone fill the chip (V = 151936, 256 rows:
+  // 51.3 us in one launch, 52.1 in three; 64 rows 47.6 and 27.8)
+  if (N > 4096 && M <= 128) {
+    unsigned long long* keys = (unsigned long long*)out;
+    const int G = (int)min((N + 2047) / 2048, (int64_t)64), per = (int)((N + G - 1) / G);
+    const dim3 rows((unsigned)((M + 255) / 256)), block(256);
+    hipLaunchKernelGGL(argmax_clear_kernel, rows, block, 0, st, keys, M);
+    hipLaunchKernelGGL(argmax_slice_kernel, dim3((unsigned)G, (unsigned)M), block, 0, st, y, (int)N, ldy, per, keys);
+    hipLaunchKernelGGL(argmax_index_kernel, rows, block, 0, st, keys, M);
+    return check_launch();
+  }
   const int vec = ((uintptr_t)y % 16 == 0) && (ldy % 4 == 0);
   hipLaunchKernelGGL(argmax_rows_kernel, dim3((unsigned)M), dim3(1024), 0, st, y, (int)N, ldy, out, vec);
   return check_launch();

@@ -290,6 +290,29 @@ def test_sample_drop_in_and_graph_replay(dev):
     del graph
 
 
+@pytest.mark.parametrize("M,V", [(1, 4096), (1, 4097), (3, 6143), (128, 4100), (129, 4100), (2, 131073), (1, 300000)])
+def test_greedy_rows_over_slices(dev, M, V):
+    """Rows in one workgroup and over several: torch.argmax's index for random
+    rows, a maximum in the first / last place and across slices (the first of
+    equals), signed zeros, NaN first, all -inf; a padded row stride."""
+    announce(f"greedy rows M={M} V={V}")
+    x = torch.randn(M, V + 5, generator=torch.Generator().manual_seed(V))[:, :V]
+    rows = [x.clone() for _ in range(6)]
+    rows[1][:, [V - 1, V // 2 + 1, V // 2]] = 9.0
+    rows[2][:, 0] = rows[2][:, V - 1] = 9.0
+    rows[3][:] = -1.0
+    rows[3][:, V // 3] = -0.0
+    rows[3][:, V // 3 + 1] = 0.0
+    rows[4][:, [V // 2, V - 2]] = float("nan")
+    rows[5][:] = float("-inf")
+    for r in rows:
+        want = r.argmax(-1) if not torch.isnan(r).any() else torch.full((M,), V // 2)
+        wide = torch.zeros(M, V + 3, device=dev)
+        wide[:, :V] = r.to(dev)
+        for t in (r.contiguous().to(dev), wide[:, :V]):
+            assert torch.equal(quant.greedy_tokens(t).cpu(), want)
+
+
 @pytest.mark.parametrize("V,T,k,p", [(70000, 1.0, 0, 0.5), (70000, 0.7, 9000, 0.9), (151936, 1.0, 0, 0.9),
                                      (151936, 1.0, 3000, 0.6), (2049, 1.0, 600, 0.5)])
 @pytest.mark.parametrize("kind", ["cluster", "wide", "grid", "bimodal"])
