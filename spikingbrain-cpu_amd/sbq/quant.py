@@ -52,12 +52,32 @@ def _gpu_for(t: torch.Tensor) -> torch.device:
     return torch.device("cuda", torch.cuda.current_device())
 
 
-def _stream(device: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+# A small linear's kernels take about 5 us, so the host side of a call counts:
+# the stream and device queries below skip torch's Python wrappers (0.1 us each
+# against 1.9 and 1.4 us), and pointers go to ctypes as plain ints.
+def _stream(device: torch.device) -> int:
+    """The current stream of `device` (a tensor's, so it has an index)."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
-def _ptr(t: torch.Tensor | None) -> ctypes.c_void_p | None:
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+class _SameDevice:
+    def __enter__(self):
+        return None
+
+    def __exit__(self, *exc):
+        return False
+
+
+_SAME_DEVICE = _SameDevice()
+
+
+def _on_device(device: torch.device):
+    """torch.cuda.device(device), or nothing when it is the current device."""
+    return _SAME_DEVICE if torch._C._cuda_getDevice() == device.index else torch.cuda.device(device)
+
+
+def _ptr(t: torch.Tensor | None) -> int | None:
+    return None if t is None else t.data_ptr()
 
 
 def _code(dtype: torch.dtype) -> int:
@@ -97,26 +117,40 @@ def _check_operands(fn: str, x2: torch.Tensor, packed: torch.Tensor, N: int, y: 
     bounds on the GPU.  vectors: (name, tensor or None, dtype) of the [N]
     per-channel operands."""
     M, K = x2.shape
-    dev = x2.device
-    if not x2.is_cuda:
+    gpu = x2.get_device()  # (device objects compare in 0.1 us, their indexes in a third of it)
+    if gpu < 0 or not x2.is_cuda:
         raise ValueError(f"{fn}: x must be a GPU tensor")
     if N < 1:
         raise ValueError(f"{fn}: N must be >= 1")
-    need = packed_bytes(N, K)
-    if (packed.dtype != torch.uint8 or packed.device != dev or not packed.is_contiguous()
+    need = (N + 15) // 16 * 16 * ((K + 63) // 64 * 64)
+    if (packed.dtype != torch.uint8 or packed.get_device() != gpu or not packed.is_contiguous()
             or packed.numel() < need):
-        raise ValueError(f"{fn}: packed must be contiguous uint8 on {dev} with >= {need} bytes (N={N}, K={K})")
+        raise ValueError(f"{fn}: packed must be contiguous uint8 on {x2.device} with >= {need} bytes (N={N}, K={K})")
     for name, t, dt in vectors:
-        if t is not None and (t.dtype != dt or t.device != dev or not t.is_contiguous() or t.numel() < N):
-            raise ValueError(f"{fn}: {name} must be a contiguous {dt} tensor of N={N} elements on {dev}")
-    if y.device != dev or y.dim() != 2 or tuple(y.shape) != (M, N) or y.stride(-1) != 1:
-        raise ValueError(f"{fn}: out must be a [M={M}, N={N}] tensor with unit column stride on {dev}")
-    if ws is not None and (ws.device != dev or not ws.is_contiguous()):
-        raise ValueError(f"{fn}: workspace must be a contiguous tensor on {dev}")
+        if t is not None and (t.dtype != dt or t.get_device() != gpu or not t.is_contiguous() or t.numel() < N):
+            raise ValueError(f"{fn}: {name} must be a contiguous {dt} tensor of N={N} elements on {x2.device}")
+    if y.get_device() != gpu or y.shape != (M, N) or y.stride(-1) != 1:
+        raise ValueError(f"{fn}: out must be a [M={M}, N={N}] tensor with unit column stride on {x2.device}")
+    if ws is not None and (ws.get_device() != gpu or not ws.is_contiguous()):
+        raise ValueError(f"{fn}: workspace must be a contiguous tensor on {x2.device}")
 
 
 def _nbytes(t: torch.Tensor | None) -> int:
     return 0 if t is None else t.numel() * t.element_size()
+
+
+def _rows(x: torch.Tensor) -> torch.Tensor:
+    """x as [rows, features]."""
+    return x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
+
+
+def _like_rows(y: torch.Tensor, shape: torch.Size) -> torch.Tensor:
+    """A [rows, N] result in the leading dimensions of an input's shape."""
+    return y if len(shape) == 2 else y.reshape(*shape[:-1], y.shape[-1])
+
+
+def _f32(t: torch.Tensor | None) -> torch.Tensor | None:
+    return t if t is None or t.dtype == torch.float32 else t.float()
 
 
 def _check_in_features(x: torch.Tensor, K: int) -> None:
@@ -138,7 +172,7 @@ def quantize_per_channel_gpu(weight: torch.Tensor) -> tuple[torch.Tensor, torch.
     N, K = w.shape
     q = torch.empty((N, K), dtype=torch.int8, device=w.device)
     scale = torch.empty((N,), dtype=torch.float32, device=w.device)
-    with torch.cuda.device(w.device):
+    with _on_device(w.device):
         _lib.check(_lib.load().sbq_quantize_per_channel(_ptr(w), _code(w.dtype), N, K, _ldx(w), _ptr(q),
                                                         _ldx(q), _ptr(scale), _stream(w.device)),
                    "sbq_quantize_per_channel")
@@ -155,7 +189,7 @@ def repack(q: torch.Tensor, with_colsum: bool = True) -> tuple[torch.Tensor, tor
     L = _lib.load()
     packed = torch.empty((L.sbq_packed_bytes(N, K),), dtype=torch.uint8, device=q.device)
     colsum = torch.empty((N,), dtype=torch.int32, device=q.device) if with_colsum else None
-    with torch.cuda.device(q.device):
+    with _on_device(q.device):
         _lib.check(L.sbq_repack_w8(_ptr(q), N, K, _ldx(q), _ptr(packed), _ptr(colsum), _stream(q.device)),
                    "sbq_repack_w8")
     return packed, colsum
@@ -176,7 +210,7 @@ def _quantize_pack(weight: torch.Tensor, with_q: bool, with_colsum: bool):
     scale = torch.empty((N,), dtype=torch.float32, device=dev)
     packed = torch.empty((packed_bytes(N, K),), dtype=torch.uint8, device=dev)
     colsum = torch.empty((N,), dtype=torch.int32, device=dev) if with_colsum else None
-    with torch.cuda.device(dev):
+    with _on_device(dev):
         _lib.check(L.sbq_quantize_pack_w8(_ptr(w), _code(w.dtype), N, K, _ldx(w), _ptr(q), K, _ptr(scale),
                                           _ptr(packed), _ptr(colsum), _stream(dev)), "sbq_quantize_pack_w8")
     return q, scale, packed, colsum
@@ -188,7 +222,7 @@ def unpack(packed: torch.Tensor, N: int, K: int) -> torch.Tensor:
             or packed.numel() < packed_bytes(N, K)):
         raise ValueError(f"unpack expects contiguous uint8 GPU tiles of >= {packed_bytes(N, K)} bytes")
     q = torch.empty((N, K), dtype=torch.int8, device=packed.device)
-    with torch.cuda.device(packed.device):
+    with _on_device(packed.device):
         _lib.check(_lib.load().sbq_unpack_w8(_ptr(packed), N, K, _ptr(q), K, _stream(packed.device)),
                    "sbq_unpack_w8")
     return q
@@ -220,7 +254,7 @@ def linear_w8(x2: torch.Tensor, packed: torch.Tensor, scale: torch.Tensor, bias:
         ws = w8_workspace(M, K, x2.device, x2.dtype, N)
     _check_operands("linear_w8", x2, packed, N, y, (("scale", scale, torch.float32), ("bias", bias, torch.float32)),
                     ws)
-    with torch.cuda.device(x2.device):
+    with _on_device(x2.device):
         _lib.check(_lib.load().sbq_linear_w8(_ptr(x2), _code(x2.dtype), M, K, _ldx(x2), _ptr(packed),
                                              _ptr(scale), _ptr(bias), N, _ptr(y), _code(y.dtype), _ldx(y),
                                              _ptr(ws), _nbytes(ws), _stream(x2.device)),
@@ -303,7 +337,7 @@ def _run_grouped(name, xs, packeds, scales, colsums, biases, Ns, out_dtype, outs
         tail = (arr(ctypes.c_void_p, [0 if biases[i] is None else biases[i].data_ptr() for i in idx]),
                 arr(ctypes.c_int64, [Ns[i] for i in idx]), arr(ctypes.c_void_p, [ys[i].data_ptr() for i in idx]),
                 arr(ctypes.c_int64, [_ldx(ys[i]) for i in idx]), _code(ydt))
-        with torch.cuda.device(dev):
+        with _on_device(dev):
             if w8a8:
                 rc = L.sbq_linear_w8a8_grouped(*head, arr(ctypes.c_void_p, [colsums[i].data_ptr() for i in idx]),
                                                *tail, _ptr(ws), _nbytes(ws), _stream(dev))
@@ -341,15 +375,14 @@ def grouped_forward(pairs):
         _check_in_features(x, m.in_features)
         if not dyn:
             m._refresh()
-    x2s = [x.reshape(-1, shape0[-1]) for x in xs]
-    args = ([m.packed for m in layers], [m.scale if m.scale.dtype == torch.float32 else m.scale.float() for m in layers])
-    rest = ([None if m.bias is None else m.bias.float() for m in layers], [m.out_features for m in layers],
-            layers[0].out_dtype)
+    x2s = [_rows(x) for x in xs]
+    args = ([m.packed for m in layers], [_f32(m.scale) for m in layers])
+    rest = ([_f32(m.bias) for m in layers], [m.out_features for m in layers], layers[0].out_dtype)
     if dyn:
         ys = linear_w8a8_grouped(x2s, *args, [m.colsum for m in layers], *rest)
     else:
         ys = linear_w8_grouped(x2s, *args, *rest)
-    return [y.reshape(*shape0[:-1], y.shape[-1]) for y in ys]
+    return [_like_rows(y, shape0) for y in ys]
 
 
 def gemm_config(M: int, N: int, K: int, dtype: torch.dtype = torch.float16, w8a8: bool = False) -> tuple[int, int]:
@@ -375,7 +408,7 @@ def _parts_table(sizes: list[int], device: torch.device) -> tuple[torch.Tensor |
     if any(w % 4 or w < 4 for w in sizes) or N >= 1 << 22 or pstart[-2] - (N - sizes[-1]) >= 1 << 14:
         return None, pstart
     table = torch.empty((N // 4, 2), dtype=torch.int32, device=device)
-    with torch.cuda.device(device):
+    with _on_device(device):
         _lib.check(_lib.load().sbq_parts_table((ctypes.c_int64 * len(sizes))(*sizes), len(sizes), _ptr(table),
                                                _stream(device)), "sbq_parts_table")
     return table, pstart
@@ -396,11 +429,11 @@ def _linear_parts(x2: torch.Tensor, packed: torch.Tensor, scale: torch.Tensor, c
     else:
         ws = w8a8_workspace(M, K, x2.device, N, x2.dtype)
         vectors = (("scale", scale, torch.float32), ("bias", bias, torch.float32), ("colsum", colsum, torch.int32))
-    _check_operands("linear_parts", x2, packed, N, y[:M * N].view(M, N), vectors, ws)
+    _check_operands("linear_parts", x2, packed, N, y.as_strided((M, N), (N, 1)), vectors, ws)
     if parts.dtype != torch.int32 or parts.device != x2.device or not parts.is_contiguous() or parts.numel() * 2 != N:
         raise ValueError(f"linear_parts: parts must be a contiguous int32 [N/4, 2] table on {x2.device}")
     L = _lib.load()
-    with torch.cuda.device(x2.device):
+    with _on_device(x2.device):
         if colsum is None:
             rc = L.sbq_linear_w8_parts(_ptr(x2), _code(x2.dtype), M, K, _ldx(x2), _ptr(packed), _ptr(scale), _ptr(bias),
                                        N, _ptr(y), _code(y.dtype), _ptr(parts), _ptr(ws), _nbytes(ws),
@@ -436,7 +469,7 @@ def linear_w8a8(x2: torch.Tensor, packed: torch.Tensor, scale: torch.Tensor, col
         raise ValueError("acc_out must be a contiguous int32 [M, N] tensor on the input's device")
     _check_operands("linear_w8a8", x2, packed, N, y, (("scale", scale, torch.float32), ("bias", bias, torch.float32),
                                                       ("colsum", colsum, torch.int32)), ws)
-    with torch.cuda.device(x2.device):
+    with _on_device(x2.device):
         _lib.check(_lib.load().sbq_linear_w8a8(_ptr(x2), _code(x2.dtype), M, K, _ldx(x2), _ptr(packed),
                                                _ptr(scale), _ptr(colsum), _ptr(bias), N, _ptr(y), _code(y.dtype),
                                                _ldx(y), _ptr(acc_out), _ptr(ws), _nbytes(ws),
@@ -464,7 +497,7 @@ def linear_w8a8_noalloc(x2: torch.Tensor, packed: torch.Tensor, scale: torch.Ten
     _check_operands("linear_w8a8_noalloc", x2, packed, N, out, (("scale", scale, torch.float32),
                                                                  ("bias", bias, torch.float32),
                                                                  ("colsum", colsum, torch.int32)))
-    with torch.cuda.device(x2.device):
+    with _on_device(x2.device):
         _lib.check(_lib.load().sbq_linear_w8a8_noalloc(_ptr(x2), _code(x2.dtype), M, K, _ldx(x2), _ptr(packed),
                                                        _ptr(scale), _ptr(colsum), _ptr(bias), N, _ptr(out),
                                                        _code(out.dtype), _ldx(out), _ptr(acc_out),
@@ -488,7 +521,7 @@ def linear_w8a8_token(x2: torch.Tensor, packed: torch.Tensor, scale: torch.Tenso
         raise ValueError("acc_out must be a contiguous int32 [M, N] tensor on the input's device")
     _check_operands("linear_w8a8_token", x2, packed, N, y,
                     (("scale", scale, torch.float32), ("bias", bias, torch.float32)), ws)
-    with torch.cuda.device(x2.device):
+    with _on_device(x2.device):
         _lib.check(_lib.load().sbq_linear_w8a8_token(_ptr(x2), _code(x2.dtype), M, K, _ldx(x2), _ptr(packed),
                                                      _ptr(scale), _ptr(bias), N, _ptr(y), _code(y.dtype),
                                                      _ldx(y), _ptr(acc_out), _ptr(ws), _nbytes(ws),
@@ -508,7 +541,7 @@ def greedy_tokens(logits: torch.Tensor) -> torch.Tensor:
         y = y.contiguous()
     ld = _ldx(y)
     out = torch.empty((y.shape[0],), dtype=torch.int64, device=y.device)
-    with torch.cuda.device(y.device):
+    with _on_device(y.device):
         _lib.check(_lib.load().sbq_argmax_rows(_ptr(y), y.shape[0], y.shape[1], ld, _ptr(out),
                                                _stream(y.device)), "sbq_argmax_rows")
     return out.reshape(shape[:-1])
@@ -560,7 +593,7 @@ def sample_tokens(logits: torch.Tensor, temperature: float, top_p: float = 1.0, 
     ws = workspace if workspace is not None else sample_workspace(M, V, y.device)
     if ws.dtype != torch.uint8 or ws.device != y.device or not ws.is_contiguous():
         raise ValueError("workspace must be a contiguous uint8 tensor on the logits' device")
-    with torch.cuda.device(y.device):
+    with _on_device(y.device):
         _lib.check(_lib.load().sbq_sample_rows(_ptr(y), M, V, ld, float(temperature), int(top_k),
                                                float(top_p), _ptr(u), _ptr(out), _ptr(ws), _nbytes(ws),
                                                _stream(y.device)), "sbq_sample_rows")
@@ -615,7 +648,7 @@ def linear_w8_argmax(x2: torch.Tensor, packed: torch.Tensor, scale: torch.Tensor
     _check_operands("linear_w8_argmax", x2, packed, N, y, (("scale", scale, torch.float32),
                                                            ("bias", bias, torch.float32)), ws)
     idx = _check_argmax("linear_w8_argmax", x2, state, idx)
-    with torch.cuda.device(x2.device):
+    with _on_device(x2.device):
         _lib.check(_lib.load().sbq_linear_w8_argmax(_ptr(x2), _code(x2.dtype), M, K, _ldx(x2), _ptr(packed),
                                                     _ptr(scale), _ptr(bias), N, _ptr(y), _ldx(y), _ptr(idx),
                                                     _ptr(ws), _nbytes(ws), _ptr(state), _stream(x2.device)),
@@ -638,7 +671,7 @@ def linear_w8a8_argmax(x2: torch.Tensor, packed: torch.Tensor, scale: torch.Tens
                                                              ("bias", bias, torch.float32),
                                                              ("colsum", colsum, torch.int32)), ws)
     idx = _check_argmax("linear_w8a8_argmax", x2, state, idx)
-    with torch.cuda.device(x2.device):
+    with _on_device(x2.device):
         _lib.check(_lib.load().sbq_linear_w8a8_argmax(_ptr(x2), _code(x2.dtype), M, K, _ldx(x2), _ptr(packed),
                                                       _ptr(scale), _ptr(colsum), _ptr(bias), N, _ptr(y),
                                                       _ldx(y), _ptr(idx), _ptr(ws), _nbytes(ws), _ptr(state),
@@ -652,7 +685,7 @@ def _greedy_state(module: nn.Module, device: torch.device) -> torch.Tensor:
     calls on one stream run one after another and leave the state zero, so
     they share it; calls on another stream get their own."""
     states = module.__dict__.setdefault("_argmax_states", {})
-    key = (device, torch.cuda.current_stream(device).cuda_stream)
+    key = (device, _stream(device))
     st = states.get(key)
     if st is None:
         st = states[key] = argmax_state(device)
@@ -669,7 +702,7 @@ def act_qparams(x2: torch.Tensor) -> tuple[float, int]:
     s = torch.empty((1,), dtype=torch.float32, device=x2.device)
     z = torch.empty((1,), dtype=torch.int32, device=x2.device)
     ws = w8a8_workspace(M, K, x2.device)
-    with torch.cuda.device(x2.device):
+    with _on_device(x2.device):
         _lib.check(_lib.load().sbq_act_qparams(_ptr(x2), _code(x2.dtype), M, K, _ldx(x2), _ptr(s), _ptr(z),
                                                _ptr(ws), _nbytes(ws), _stream(x2.device)),
                    "sbq_act_qparams")
@@ -694,7 +727,7 @@ def act_quant_per_tensor(x2: torch.Tensor, out: torch.Tensor | None = None
     s = torch.empty((1,), dtype=torch.float32, device=x2.device)
     z = torch.empty((1,), dtype=torch.int32, device=x2.device)
     ws = w8a8_workspace(M, K, x2.device)
-    with torch.cuda.device(x2.device):
+    with _on_device(x2.device):
         _lib.check(_lib.load().sbq_act_quant_per_tensor(_ptr(x2), _code(x2.dtype), M, K, _ldx(x2), _ptr(out),
                                                         _ldx(out), _ptr(s), _ptr(z), _ptr(ws), _nbytes(ws),
                                                         _stream(x2.device)),
@@ -774,39 +807,36 @@ class Int8Linear(nn.Module):
 
     def _refresh(self):
         # packed follows qweight across .to()/.cuda(); rebuild if it was lost
-        if self.packed.device != self.qweight.device or self.packed.numel() == 0:
+        packed = self.packed
+        if packed.device != self.qweight.device or packed.numel() == 0:
             self._repack()
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        if not self.qweight.is_cuda:
+        q = self.qweight
+        if not q.is_cuda:
             raise RuntimeError("sbq Int8Linear: weights are on the CPU; move the module to a ROCm GPU")
-        _check_in_features(x, self.in_features)
+        N, K = q.shape
+        _check_in_features(x, K)
         self._refresh()
-        shape = x.shape
-        N = self.out_features
 
         def run(xd):
-            x2 = xd.reshape(-1, shape[-1])
-            scale = self.scale if self.scale.dtype == torch.float32 else self.scale.float()
-            bias = None if self.bias is None else self.bias.float()
-            return linear_w8(x2, self.packed, scale, bias, N, self.out_dtype)
+            return linear_w8(_rows(xd), self.packed, _f32(self.scale), _f32(self.bias), N, self.out_dtype)
 
-        out = _run_on_device(x, self.qweight.device, run)
-        return out.reshape(*shape[:-1], out.shape[-1])
+        return _like_rows(run(x) if x.device == q.device else _run_on_device(x, q.device, run), x.shape)
 
     def forward_greedy(self, x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
         """forward(x) and the greedy token of each row in one pass, for the
         lm_head (model.py:445-447, engine.py:30-31): (fp32 logits [..., N],
         int64 tokens [...]).  x must be on the module's GPU."""
-        _check_in_features(x, self.in_features)
+        q = self.qweight
+        N, K = q.shape
+        _check_in_features(x, K)
         self._refresh()
-        if x.device != self.qweight.device:
-            raise ValueError(f"sbq: input on {x.device} but the layer lives on {self.qweight.device}")
-        shape = x.shape
-        bias = None if self.bias is None else self.bias.float()
-        y, idx = linear_w8_argmax(x.reshape(-1, shape[-1]), self.packed, self.scale.float(), bias, self.out_features,
+        if x.device != q.device:
+            raise ValueError(f"sbq: input on {x.device} but the layer lives on {q.device}")
+        y, idx = linear_w8_argmax(_rows(x), self.packed, _f32(self.scale), _f32(self.bias), N,
                                   _greedy_state(self, x.device))
-        return y.reshape(*shape[:-1], y.shape[-1]), idx.reshape(shape[:-1])
+        return _like_rows(y, x.shape), idx.reshape(x.shape[:-1])
 
 
 class _Fp32Buffers:
@@ -857,21 +887,18 @@ class DynamicInt8Linear(_Fp32Buffers, nn.Module):
         self.out_dtype = torch.float32
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        if not self.packed.is_cuda:
+        packed = self.packed
+        if not packed.is_cuda:
             raise RuntimeError("sbq DynamicInt8Linear: weights are on the CPU; move the module to a ROCm GPU")
         _check_in_features(x, self.in_features)
-        shape = x.shape
 
         def run(xd):
-            x2 = xd.reshape(-1, shape[-1])
-            scale = self.scale.float()
-            bias = None if self.bias is None else self.bias.float()
+            x2, scale, bias = _rows(xd), _f32(self.scale), _f32(self.bias)
             if getattr(self, "granularity", "tensor") == "token":
-                return linear_w8a8_token(x2, self.packed, scale, bias, self.out_features, self.out_dtype)
-            return linear_w8a8(x2, self.packed, scale, self.colsum, bias, self.out_features, self.out_dtype)
+                return linear_w8a8_token(x2, packed, scale, bias, self.out_features, self.out_dtype)
+            return linear_w8a8(x2, packed, scale, self.colsum, bias, self.out_features, self.out_dtype)
 
-        out = _run_on_device(x, self.packed.device, run)
-        return out.reshape(*shape[:-1], out.shape[-1])
+        return _like_rows(run(x) if x.device == packed.device else _run_on_device(x, packed.device, run), x.shape)
 
     def forward_greedy(self, x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
         """forward(x) and the greedy token of each row in one pass (see
@@ -879,13 +906,12 @@ class DynamicInt8Linear(_Fp32Buffers, nn.Module):
         if getattr(self, "granularity", "tensor") != "tensor":
             raise ValueError("forward_greedy: per-tensor int8-dyn only")
         _check_in_features(x, self.in_features)
-        if x.device != self.packed.device:
-            raise ValueError(f"sbq: input on {x.device} but the layer lives on {self.packed.device}")
-        shape = x.shape
-        bias = None if self.bias is None else self.bias.float()
-        y, idx = linear_w8a8_argmax(x.reshape(-1, shape[-1]), self.packed, self.scale.float(), self.colsum, bias,
+        packed = self.packed
+        if x.device != packed.device:
+            raise ValueError(f"sbq: input on {x.device} but the layer lives on {packed.device}")
+        y, idx = linear_w8a8_argmax(_rows(x), packed, _f32(self.scale), self.colsum, _f32(self.bias),
                                     self.out_features, _greedy_state(self, x.device))
-        return y.reshape(*shape[:-1], y.shape[-1]), idx.reshape(shape[:-1])
+        return _like_rows(y, x.shape), idx.reshape(x.shape[:-1])
 
 
 def _dyn_from_quantized(qweight: torch.Tensor, scale: torch.Tensor, bias: torch.Tensor | None) -> "DynamicInt8Linear":
@@ -1060,9 +1086,7 @@ class FusedLinear(_Fp32Buffers, nn.Module):
         direct = M > 1 and self._parts is not None
 
         def run(xd):
-            x2 = xd.reshape(-1, shape[-1])
-            scale = self.scale.float()
-            bias = None if self.bias is None else self.bias.float()
+            x2, scale, bias = _rows(xd), _f32(self.scale), _f32(self.bias)
             if direct:
                 return _linear_parts(x2, self.packed, scale, self.colsum, bias, self.out_features, self._parts,
                                      self._pstart[-1], self.out_dtype)
