@@ -1118,13 +1118,56 @@ bool pick_gemv_fast(int64_t M, int64_t K, int64_t N, int xt, bool w8a8, bool xve
     } else if (*ks < kFusedMinWaves) {
       *ks = kFusedMinWaves;  // 256 threads share the fused x
     }
-    // M = 4 .. 8 on a wide short-K layer: five row tiles per workgroup, as
-    // for weight-only: x up to 64 KiB with the fused min/max (8 chunks per
-    // thread; fp32 x up to 80 KiB, 10 chunks, so that M = 8 at K = 2560
-    // takes no quantizing launch: checkpoint int8-dyn step 3036 -> 3240 tok/s)
-    if (M >= 4 && Kc < 128 && Nt > 1024 && (Nt + 4) / 5 <= 256 && xb <= kSplitWideBytes) {
+    // Short K on wide layers: every workgroup reads all of x, quantizes it
+    // and only then multiplies, so the more x, the fewer and larger workgroups
+    // pay (measured on MI355X over every configuration, M = 1 ... 8, fp32 and
+    // fp16 x):
+    // * five row tiles per workgroup where that grid fits one round of the CUs
+    //   (x up to 64 KiB, 8 chunks per thread; fp32 up to 80 KiB, 10 chunks, so
+    //   that M = 8 at K = 2560 takes no quantizing launch: checkpoint int8-dyn
+    //   step 3036 -> 3240 tok/s; M = 2, N = 19456 12.7 -> 11.7 us), else six
+    //   (M = 8, N = 24576, K = 4096, fp16: 21.4 -> 19.8);
+    // * up to 16 KiB, M <= 3: two waves, one row tile on the widest (M = 1, K =
+    //   2560: N = 19456 11.4 -> 10.3 us, 151936 57.3); at K <= 3072 four waves
+    //   of 4-tile steps (N = 12288 8.1 -> 7.6) or, up to 512 row tiles, 8-tile
+    //   steps over two (N = 5120 6.1 -> 5.7);
+    // * up to 32 KiB beyond the five- and six-tile grids, two row tiles and
+    //   four waves (M = 2, N = 151936 fp32 59.6, M = 4 fp16 60.6; eight waves
+    //   over 70);
+    // * more x on more than 4096 row tiles: quantized before the launch
+    //   instead (M = 4, N = 151936, fp32: 81 us fused, 65 so); 2-byte x on
+    //   more than 1536, five row tiles (M = 8, N = 40000, K = 4096: 31.0 ->
+    //   29.1).
+    const bool shortk = Kc > 4 && Kc < 128;
+    const bool large = M >= 4 || xb > 16384;
+    if (shortk && large && Nt > 1024 && (Nt + 4) / 5 <= 256 && xb <= kSplitWideBytes) {
       *id = 7;
       *ks = 8;
+    } else if (shortk && M <= 8 && Nt > 256) {
+      if (!large) {
+        if (Nt > 1024) {
+          *id = 3;
+          *ks = 2;
+        } else if (Kc <= 48) {
+          *id = Nt <= 512 ? 5 : 2;
+          *ks = 4;
+        }
+      } else if (xb <= 16384) {
+        // small rows at M = 4 .. 8: as picked above
+      } else if (Nt > 1024 && (Nt + 5) / 6 <= 256 && xb <= 65536) {
+        *id = 8;
+        *ks = 8;
+      } else if (xb <= 32768) {
+        if (Nt >= 384) {
+          *id = 4;
+          *ks = 4;
+        }
+      } else if (Nt > 4096) {
+        return false;
+      } else if (xt != XT_F32 && Nt > 1536) {
+        *id = 7;
+        *ks = 8;
+      }
     }
   }
   return true;
