@@ -436,7 +436,8 @@ int sbq_linear_w8a8_token(const void* x, int x_dtype, int64_t M, int64_t K, int6
   if (!workspace || (int64_t)workspace_bytes < sbq_w8a8_workspace_bytes(M, K)) return SBQ_ERR_WORKSPACE;
   const bool xv = x_vec_ok(x, x_dtype, ldx), yv = y_vec_ok(y, y_dtype, ldy, N);
   return sbq::launch_gemm_w8a8_token(x, x_dtype, M, K, ldx, xv, packed, scale, bias, N, y, y_dtype, ldy, acc_out,
-                                     ws_xq(workspace), ws_stok(workspace, M, K), (hipStream_t)stream, yv);
+                                     ws_xq(workspace), ws_stok(workspace, M, K), (hipStream_t)stream, yv,
+                                     ws_split(workspace, M, K), ws_split_bytes(workspace, workspace_bytes, M, K));
 }
 
 int sbq_linear_w8a8(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, const uint8_t* packed,

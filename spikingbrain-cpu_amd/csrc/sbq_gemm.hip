@@ -1694,7 +1694,8 @@ int launch_gemm_w8a8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, b
 // then the fast GEMV (M <= 16) or the i8 GEMM with the per-token epilogue.
 int launch_gemm_w8a8_token(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, bool xvec,
                            const uint8_t* packed, const float* scale, const float* bias, int64_t N, void* y, int yt,
-                           int64_t ldy, int32_t* acc_out, int8_t* xq, float* s_t, hipStream_t st, bool yvec) {
+                           int64_t ldy, int32_t* acc_out, int8_t* xq, float* s_t, hipStream_t st, bool yvec,
+                           uint8_t* split, int64_t split_bytes) {
   const int64_t Nt = (N + 15) / 16, Kc = (K + 63) / 64, Kp = Kc * 64;
   if (Kp > ((int64_t)1 << 21)) return -1;  // 32-bit block offsets of the direct-to-LDS GEMM
   if (M <= 16 && xvec && K % 64 == 0) {
@@ -1712,7 +1713,15 @@ int launch_gemm_w8a8_token(const void* x, int xt, int64_t M, int64_t K, int64_t 
       if (frc != -1) return frc;
     }
   }
-  int rc = launch_quantize_rows_sym(x, xt, ldx, xvec, M, K, Kp, xq, s_t, st);
+  // the per-tensor GEMM's plan: without the K split a 4096 x 4096 layer fills 32 of the
+  // 256 CUs, so its time is one workgroup's walk over K (graph replays, fp16 x, us, before -> now:
+  // 4096 x 4096 M = 32 / 64 / 128 24.5 -> 15.4 / 25.5 -> 17.4 / 25.8 -> 19.8, 12288 x 4096 M = 17 / 64 /
+  // 128 28.2 -> 24.4 / 30.1 -> 25.9 / 32.2 -> 30.0, 2560 x 9728 53.7 -> 30.0 / 56.2 -> 31.1 / 56.3 -> 33.8)
+  GemmArgs a{};
+  const DlPlan plan = plan_gemm_dl(true, XT_F16, M, Nt, Kc, true);
+  int ncount = 0;
+  uint32_t* zero = M > 16 ? attach_split(a, plan, split, split_bytes, &ncount) : nullptr;
+  int rc = launch_quantize_rows_sym(x, xt, ldx, xvec, M, K, Kp, xq, s_t, st, zero, ncount);
   if (rc) return rc;
   if (M <= 16) {  // decode sizes: the HBM-streaming GEMV on the s8 rows
     GemvArgs g{};
@@ -1729,12 +1738,22 @@ int launch_gemm_w8a8_token(const void* x, int xt, int64_t M, int64_t K, int64_t 
       if (rc != -1) return rc;
     }
   }
-  GemmArgs a{};
+  const bool alt = plan.splits == 1 || zero != nullptr;
+  if (M > 16 && gemv_mt_applies(M, Kp, N, XT_S8, alt)) {  // narrow layers: the row-tile GEMV, as per-tensor
+    GemvArgs g{};
+    g.x = xq; g.ldx = Kp; g.M = (int)M; g.K = (int)Kp; g.Kc = (int)Kc;
+    g.packed = packed; g.scale = scale; g.bias = bias;
+    g.N = (int)N; g.Nt = (int)Nt; g.y = y; g.yt = yt; g.ldy = ldy; g.acc_out = acc_out; g.rscale = s_t;
+    g.flags = kGemvXVec | (yvec ? kGemvYVec : 0);
+    rc = launch_gemv_mt(g, XT_S8, st, alt);
+    if (rc != -1) return rc;
+  }
   a.x = xq; a.ldx = Kp; a.M = (int)M; a.Kc = (int)Kc;
   a.packed = packed; a.scale = scale; a.bias = bias;
   a.N = (int)N; a.Nt = (int)Nt; a.y = y; a.yt = yt; a.ldy = ldy; a.acc_out = acc_out; a.rscale = s_t;
   a.flags = (yvec ? 2 : 0) | 4 | y16_flag(y, yt, ldy);
-  return launch_gemm_dl_cfg(pick_gemm_dl(true, XT_F16, M, Nt, Kc), true, XT_F16, a, st);
+  const int id = zero || plan.splits == 1 ? plan.id : pick_gemm_dl(true, XT_F16, M, Nt, Kc);
+  return launch_gemm_dl_cfg(id, true, XT_F16, a, st);
 }
 
 }  // namespace sbq

@@ -650,7 +650,8 @@ __global__ __launch_bounds__(kFastMaxWaves * 64) void gemv_fast_kernel(GemvArgs 
 // Decode GEMV over MT 16-row tiles of x (16 < M <= 16 * MT, 64 | K, 16-byte
 // aligned rows): weight-only on fp16 / bf16 activations, or int8-dyn (XT_S8)
 // on the s8 rows xq - 128 of the quantize pre-pass with its (s_x, zp) and
-// the GEMM's per-tensor epilogue.  The fast path's
+// the GEMM's per-tensor epilogue, or on per-token rows with their scales
+// a.rscale.  The fast path's
 // streaming of D weight tiles per step per wave, with MT activation fragments
 // per tile (loaded directly from L2, D steps ahead like the weights).  Each
 // weight tile is converted once and multiplied into MT accumulators; per-wave
@@ -688,7 +689,8 @@ __global__ __launch_bounds__(kFastMaxWaves * 64) void gemv_mt_kernel(GemvArgs a,
       const int nn = min(ne + v, a.N - 1);
       sc[v] = a.scale[nn];
       if (a.bias) bi[v] = a.bias[nn];
-      if constexpr (I8) cs[v] = a.colsum[nn];
+      if constexpr (I8)
+        if (!a.rscale) cs[v] = a.colsum[nn];
     }
   }
 
@@ -777,8 +779,10 @@ __global__ __launch_bounds__(kFastMaxWaves * 64) void gemv_mt_kernel(GemvArgs a,
   float sx = 0.0f;
   int corr = 0;
   if constexpr (I8) {
-    sx = a.qpbuf[0];
-    corr = 128 - __float_as_int(a.qpbuf[1]);
+    if (!a.rscale) {  // per-tensor
+      sx = a.qpbuf[0];
+      corr = 128 - __float_as_int(a.qpbuf[1]);
+    }
   }
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
@@ -792,9 +796,11 @@ __global__ __launch_bounds__(kFastMaxWaves * 64) void gemv_mt_kernel(GemvArgs a,
     const int m = mt * 16 + r;
     if (m >= M) continue;
     f32x4 o;
+    if constexpr (I8)
+      if (a.rscale) sx = a.rscale[m];  // per-token
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      if constexpr (I8) {  // the per-tensor epilogue of the i8 GEMM
+      if constexpr (I8) {  // the epilogue of the i8 GEMM
         const int av = s[v] + corr * cs[v];
         if (a.acc_out && v < nvalid) a.acc_out[(int64_t)m * a.N + n + v] = av;
         const float mult = sx * sc[v];
@@ -969,7 +975,7 @@ bool gemv_mt_applies(int64_t M, int64_t K, int64_t N, int xt, bool gemm_alt) {
 
 int launch_gemv_mt(const GemvArgs& a, int xt, hipStream_t st, bool gemm_alt) {
   if (a.K != a.Kc * 64 || !(a.flags & kGemvXVec) || !gemv_mt_applies(a.M, a.K, a.N, xt, gemm_alt)) return -1;
-  if (xt == XT_S8 && (!a.qpbuf || !a.colsum)) return -1;
+  if (xt == XT_S8 && !a.rscale && (!a.qpbuf || !a.colsum)) return -1;
   const int mt = (a.M + 15) / 16;
   const bool wide = a.Kc < 128 && a.Nt >= 384;
   const int G = wide ? 2 : 1;

@@ -489,7 +489,9 @@ __global__ __launch_bounds__(256) void act_quant_u8_kernel(const void* __restric
 template <int XT>
 __global__ __launch_bounds__(256) void quantize_rows_sym_kernel(const void* __restrict__ xv, int64_t ldx, int M, int K,
                                                                 int Kp, int vec, int8_t* __restrict__ xq,
-                                                                float* __restrict__ s_out) {
+                                                                float* __restrict__ s_out,
+                                                                uint32_t* __restrict__ zero, int nzero) {
+  zero_counters(zero, nzero);
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (row >= M) return;
   float amax = 0.0f;
@@ -889,13 +891,13 @@ int launch_act_quant_u8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx
 }
 
 int launch_quantize_rows_sym(const void* x, int xt, int64_t ldx, bool xvec, int64_t M, int64_t K, int64_t Kp,
-                             int8_t* xq, float* s_out, hipStream_t st) {
+                             int8_t* xq, float* s_out, hipStream_t st, uint32_t* zero, int nzero) {
   const dim3 grid((unsigned)((M + 3) / 4)), block(256);
   const int vec = xvec ? 1 : 0;
   switch (xt) {
-    case XT_F32: hipLaunchKernelGGL(quantize_rows_sym_kernel<XT_F32>, grid, block, 0, st, x, ldx, (int)M, (int)K, (int)Kp, vec, xq, s_out); break;
-    case XT_F16: hipLaunchKernelGGL(quantize_rows_sym_kernel<XT_F16>, grid, block, 0, st, x, ldx, (int)M, (int)K, (int)Kp, vec, xq, s_out); break;
-    case XT_BF16: hipLaunchKernelGGL(quantize_rows_sym_kernel<XT_BF16>, grid, block, 0, st, x, ldx, (int)M, (int)K, (int)Kp, vec, xq, s_out); break;
+    case XT_F32: hipLaunchKernelGGL(quantize_rows_sym_kernel<XT_F32>, grid, block, 0, st, x, ldx, (int)M, (int)K, (int)Kp, vec, xq, s_out, zero, nzero); break;
+    case XT_F16: hipLaunchKernelGGL(quantize_rows_sym_kernel<XT_F16>, grid, block, 0, st, x, ldx, (int)M, (int)K, (int)Kp, vec, xq, s_out, zero, nzero); break;
+    case XT_BF16: hipLaunchKernelGGL(quantize_rows_sym_kernel<XT_BF16>, grid, block, 0, st, x, ldx, (int)M, (int)K, (int)Kp, vec, xq, s_out, zero, nzero); break;
     default: return -2;
   }
   return check_launch();

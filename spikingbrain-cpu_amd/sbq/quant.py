@@ -515,7 +515,8 @@ def linear_w8a8_token(x2: torch.Tensor, packed: torch.Tensor, scale: torch.Tenso
     x2 = _as_activation(x2)
     M, K = x2.shape
     y = out if out is not None else torch.empty((M, N), dtype=out_dtype, device=x2.device)
-    ws = workspace if workspace is not None else w8a8_workspace(M, K, x2.device)
+    # (past decode sizes, the split-K partials of small grids too: the per-tensor plan)
+    ws = workspace if workspace is not None else w8a8_workspace(M, K, x2.device, N if M > 16 else None, x2.dtype)
     if acc_out is not None and (acc_out.dtype != torch.int32 or tuple(acc_out.shape) != (M, N)
                                 or not acc_out.is_contiguous() or acc_out.device != x2.device):
         raise ValueError("acc_out must be a contiguous int32 [M, N] tensor on the input's device")

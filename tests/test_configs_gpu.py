@@ -371,6 +371,36 @@ def test_fused_hybrid_group_vs_oracle(dev, fmt, M):
             np.testing.assert_array_equal(po.cpu().numpy(), o.cpu().numpy())
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(17, 1000, 4096), (20, 4096, 130), (33, 4096, 2560), (64, 2050, 4032), (48, 4100, 9728), (100, 4096, 4100), (128, 12288, 1024),
+                                   (129, 4096, 512)])
+def test_w8a8_token_split_k(dev, M, N, K):
+    """Per-token W8A8 past decode sizes: the row-tile GEMV, K split over 4, 3 and 2
+    workgroups and not at all, even and odd K tiles: acc and y bit-exact against the oracle,
+    equal without the split area, and a graph replay equals the eager call."""
+    announce(f"w8a8 token split M={M} N={N} K={K}")
+    w = gpu_weight(N, K, 21, dev)
+    lin = quant.DynamicInt8Linear(w, None, granularity="token")
+    x = cpu_x(M, K, 22)
+    cols = tile_sample(N, 7)
+    q, s = ref_rows(w, cols)
+    y_ref, info = oracle.dyn_linear_token(x.numpy(), q, s, return_intermediates=True)
+    acc = torch.empty((M, N), dtype=torch.int32, device=dev)
+    y = quant.linear_w8a8_token(x.to(dev), lin.packed, lin.scale, None, N, acc_out=acc)
+    np.testing.assert_array_equal(acc.cpu().numpy()[:, cols], info["acc"])
+    np.testing.assert_array_equal(y.cpu().numpy()[:, cols], y_ref)
+    plain = quant.linear_w8a8_token(x.to(dev), lin.packed, lin.scale, None, N, workspace=quant.w8a8_workspace(M, K, dev))
+    assert torch.equal(plain, y)
+    static = x.to(dev)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = lin(static)
+    for k in range(3):
+        static.mul_(-1.5)
+        g.replay()
+        assert torch.equal(out, lin(static)), k
+
+
 # Ragged K: padded rows and the fast GEMV (M <= 16), padded rows or bf16 planes
 # and the direct-to-LDS GEMM: K split over 4, 3 and 2 workgroups, the 64 x 64
 # grid unsplit, and the larger blocks (128 x 64 with K in 4 groups, 256 x 128).
