@@ -229,8 +229,10 @@ int linear_w8_run(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
     ws = (void*)(((uintptr_t)workspace + 255) & ~(uintptr_t)255);
     ws_bytes = (int64_t)workspace_bytes - (int64_t)((uintptr_t)ws - (uintptr_t)workspace);
   }
-  if (K % 64 != 0 && ws && M <= 16 && sbq::pad_decode_rows(M, N, K, x_dtype)) {
-    // ragged K at decode sizes: rows of whole tiles, then the fast GEMV
+  if (K % 64 != 0 && ws && M <= 16 && sbq::gemv_supports(M, K, false, x_dtype) &&
+      sbq::pad_decode_rows(M, N, K, x_dtype)) {
+    // ragged K at decode sizes: rows of whole tiles, then the fast GEMV (longer
+    // K than the GEMVs take: the GEMM below stages the rows itself)
     uint8_t* rows = (uint8_t*)ws + sbq::w8_ws_layout(M, K, x_dtype).planes;
     const int64_t Kp = (K + 63) / 64 * 64;
     const int rc = sbq::launch_pad_rows(x, x_dtype, M, K, ldx, rows, st);

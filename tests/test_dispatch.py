@@ -1,0 +1,44 @@
+"""Which kernels the C ABI launches, without a GPU (tests/host/dispatch.py):
+the library's host code runs over a recorder in place of the HIP runtime, on
+made-up addresses that nothing reads."""
+import json
+import subprocess
+import sys
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parents[1]
+HOST = ROOT / "tests" / "host"
+PKG = ROOT / "spikingbrain-cpu_amd" / "sbq"
+
+
+@pytest.fixture(scope="module")
+def dispatch(tmp_path_factory):
+    so = tmp_path_factory.mktemp("trace") / "launch_trace.so"
+    subprocess.run(["g++", "-O1", "-shared", "-fPIC", "-std=c++17", "-Wall", str(HOST / "launch_trace.cpp"),
+                    "-o", str(so)], check=True)
+
+    def run(calls):
+        """[(status, [kernel name with template arguments, ...], [grid x, ...])] of the calls."""
+        r = subprocess.run([sys.executable, str(HOST / "dispatch.py"), str(so), str(PKG / "libsbq.so"), str(PKG)],
+                           input=json.dumps(calls), capture_output=True, text=True)
+        assert r.returncode == 0, r.stderr
+        return [(t["rc"], [ln[0] for ln in t["launches"]], [ln[1][0] for ln in t["launches"]])
+                for t in json.loads(r.stdout)]
+
+    return run
+
+
+def kernels(names):
+    return [n.split("<")[0] for n in names]
+
+
+def test_ragged_k_beyond_the_decode_gemv_is_staged(dispatch):
+    """K % 64 != 0 beyond the decode GEMVs' 12288: every weight-only entry point
+    takes decode sizes (they run the tiled GEMM on rows of whole tiles)."""
+    calls = [{"op": op, "M": M, "N": 1000, "K": K, "x": x, "ws": ws}
+             for op in ("linear_w8", "linear_w8_parts", "linear_w8_argmax") for M in (1, 2, 4, 16)
+             for K in (12289, 13000, 20001) for x in ("f32", "f16", "bf16") for ws in ("base", "full")]
+    for c, (rc, names, _) in zip(calls, dispatch(calls)):
+        assert rc == 0 and kernels(names)[:2] == ["pad_rows_kernel", "gemm_dl_kernel"], (c, rc, names)

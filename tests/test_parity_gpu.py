@@ -780,6 +780,22 @@ def test_long_k_beyond_the_gemv(dev, M, K, xd):
     np.testing.assert_array_equal(yd.cpu().numpy(), oracle.dyn_linear(xv, q, s))
 
 
+@pytest.mark.parametrize("M,K,xd", [(1, 12289, "f32"), (4, 13000, "f16"), (16, 20001, "bf16"), (2, 20000, "f32")])
+def test_long_ragged_k_at_decode_sizes(dev, M, K, xd):
+    """The same with K % 64 != 0, weight-only: the layer, and two layers fused
+    (outputs stored as parts)."""
+    announce(f"long ragged K M={M} K={K} x={xd}")
+    N = 200
+    w = make_weights(N, K, 84)
+    q, s = oracle.quantize_per_channel(w.numpy())
+    x = make_x(M, K, 85, outliers=True).to(DT[xd])
+    want = oracle.int8_linear(x.float().numpy(), q, s)
+    lin = quant.Int8Linear(w, None)
+    assert oracle.rel_l2(lin(x.to(dev)).cpu().numpy(), want) <= W8_TOL
+    fused = quant.fuse_linears([quant.Int8Linear(w[:132], None), quant.Int8Linear(w[132:], None)])
+    assert oracle.rel_l2(torch.cat(fused(x.to(dev)), -1).cpu().numpy(), want) <= W8_TOL
+
+
 @pytest.mark.parametrize("M,N,K,xd", [(65536, 16, 4096, "f16"), (100003, 8, 512, "f32"), (40000, 3, 1000, "bf16")])
 def test_many_tokens_few_outputs(dev, M, N, K, xd):
     """Very tall, narrow calls (a router over a long prompt): grids of many
