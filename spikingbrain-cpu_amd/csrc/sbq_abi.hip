@@ -209,10 +209,12 @@ int64_t sbq_w8_workspace_bytes(int64_t M, int64_t K, int x_dtype) {
 
 namespace {
 
-// sbq_linear_w8 on checked operands; yparts: y stored as parts.
+// sbq_linear_w8 on checked operands; yparts: y stored as parts; am: the greedy
+// token wanted as well (fused where the decode GEMV takes it).
 int linear_w8_run(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, const uint8_t* packed,
                   const float* scale, const float* bias, int64_t N, void* y, int y_dtype, int64_t ldy,
-                  void* workspace, size_t workspace_bytes, hipStream_t st, const sbq::u32x2* yparts = nullptr) {
+                  void* workspace, size_t workspace_bytes, hipStream_t st, const sbq::u32x2* yparts = nullptr,
+                  sbq::GemvArgmaxOut* am = nullptr) {
   const bool xv = x_vec_ok(x, x_dtype, ldx), yv = y_vec_ok(y, y_dtype, ldy, N);
   if (M > 16 && M <= 64) {  // several 16-row tiles of x against streamed weights
     // the tiled GEMM's mid-sized-M plan needs the full workspace (row sums, split area)
@@ -237,11 +239,11 @@ int linear_w8_run(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
     const int64_t Kp = (K + 63) / 64 * 64;
     const int rc = sbq::launch_pad_rows(x, x_dtype, M, K, ldx, rows, st);
     if (rc) return rc;
-    return sbq::launch_gemv_w8(rows, x_dtype, M, Kp, Kp, true, packed, scale, bias, N, y, y_dtype, ldy, st, yv, nullptr,
+    return sbq::launch_gemv_w8(rows, x_dtype, M, Kp, Kp, true, packed, scale, bias, N, y, y_dtype, ldy, st, yv, am,
                                yparts);
   }
   if (!(K % 64 != 0 && ws && M > 16) && sbq::gemv_supports(M, K, false, x_dtype))
-    return sbq::launch_gemv_w8(x, x_dtype, M, K, ldx, xv, packed, scale, bias, N, y, y_dtype, ldy, st, yv, nullptr,
+    return sbq::launch_gemv_w8(x, x_dtype, M, K, ldx, xv, packed, scale, bias, N, y, y_dtype, ldy, st, yv, am,
                                yparts);
   return sbq::launch_gemm_w8(x, x_dtype, M, K, ldx, xv, packed, scale, bias, N, y, y_dtype, ldy, ws, ws_bytes, st,
                              yv, yparts);
@@ -552,16 +554,10 @@ int sbq_linear_w8_argmax(const void* x, int x_dtype, int64_t M, int64_t K, int64
   if (!aligned(argmax_ws, 8)) return SBQ_ERR_ALIGN;
   hipStream_t st = (hipStream_t)stream;
   sbq::GemvArgmaxOut am{(uint8_t*)argmax_ws, idx, false};
-  // decode sizes: the GEMV with the token fused; larger M: the logits exactly
-  // as sbq_linear_w8 computes them (its row-tile and split-K routes), then
-  // the row argmax
-  if (M <= 16 && sbq::gemv_supports(M, K, false, x_dtype)) {
-    const bool xv = x_vec_ok(x, x_dtype, ldx), yv = y_vec_ok(y, SBQ_F32, ldy, N);
-    rc = sbq::launch_gemv_w8(x, x_dtype, M, K, ldx, xv, packed, scale, bias, N, y, SBQ_F32, ldy, st, yv, &am);
-  } else {
-    rc = sbq_linear_w8(x, x_dtype, M, K, ldx, packed, scale, bias, N, y, SBQ_F32, ldy, workspace, workspace_bytes,
-                       stream);
-  }
+  // the logits exactly as sbq_linear_w8 computes them; decode GEMVs fuse the
+  // token, the row argmax follows everything else
+  rc = linear_w8_run(x, x_dtype, M, K, ldx, packed, scale, bias, N, y, SBQ_F32, ldy, workspace, workspace_bytes, st,
+                     nullptr, &am);
   if (rc || am.fused) return rc;
   return sbq::launch_argmax_rows(y, M, N, ldy, idx, st);
 }

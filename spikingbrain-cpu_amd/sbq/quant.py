@@ -637,14 +637,14 @@ def linear_w8_argmax(x2: torch.Tensor, packed: torch.Tensor, scale: torch.Tensor
     pass: (fp32 logits [M, N], int64 token [M]), the token being the first
     index of each row's maximum with NaN above every number.  `state` comes
     from argmax_state() (one per stream).  The logits are linear_w8's (the
-    same workspace rule for prefill sizes)."""
+    same workspace rule)."""
     x2 = _as_activation(x2)
     M, K = x2.shape
     y = out if out is not None else torch.empty((M, N), dtype=torch.float32, device=x2.device)
     if y.dtype != torch.float32:
         raise ValueError("linear_w8_argmax: the logits are fp32")
     ws = workspace
-    if ws is None and M > 16:
+    if ws is None and (M > 16 or K % 64):
         ws = w8_workspace(M, K, x2.device, x2.dtype, N)
     _check_operands("linear_w8_argmax", x2, packed, N, y, (("scale", scale, torch.float32),
                                                            ("bias", bias, torch.float32)), ws)

@@ -859,6 +859,22 @@ def test_greedy_one_pass_other_shapes(dev, M, N, K, xd):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("xd", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("M,N,K", [(1, 5000, 2500), (2, 2999, 2500), (5, 33000, 1111), (8, 1000, 9001), (16, 2999, 2500),
+                                   (12, 2050, 4033), (1, 300, 13000), (4, 999, 13000)])
+def test_greedy_one_pass_ragged_k(dev, M, N, K, xd):
+    """K % 64 != 0 over several waves and beyond the GEMVs' K: forward's logits,
+    bit for bit, and their token, twice (the fused state comes back to zero)."""
+    announce(f"greedy ragged M={M} N={N} K={K} x={xd}")
+    lm = quant.make_linear("int8", gpu_weight(N, K, 70, dev))
+    for seed in (71, 72):
+        x = cpu_x(M, K, seed).to(DT[xd]).to(dev)
+        y, tok = lm.forward_greedy(x)
+        assert torch.equal(y, lm(x))
+        _check_greedy(y, tok, lm)
+
+
+@pytest.mark.gpu
 def test_greedy_one_pass_graph_replays(dev):
     """The fused call captured in a HIP graph: every replay (new activations,
     eager work in between) gives the argmax of its own logits, and leaves the

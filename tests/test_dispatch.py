@@ -42,3 +42,21 @@ def test_ragged_k_beyond_the_decode_gemv_is_staged(dispatch):
              for K in (12289, 13000, 20001) for x in ("f32", "f16", "bf16") for ws in ("base", "full")]
     for c, (rc, names, _) in zip(calls, dispatch(calls)):
         assert rc == 0 and kernels(names)[:2] == ["pad_rows_kernel", "gemm_dl_kernel"], (c, rc, names)
+
+
+@pytest.mark.parametrize("fmt", ["w8", "w8a8"])
+def test_greedy_logits_take_the_route_of_the_linear(dispatch, fmt):
+    """The greedy entry points compute the logits with the launches of the plain
+    linear (decode, ragged K, long K, mid-sized and prefill M, with and without
+    the workspace): the bits of forward."""
+    ws = (None, "base", "full") if fmt == "w8" else ("base", "full")
+    shapes = [{"M": M, "N": N, "K": K, "x": x, "ws": w, "off": off} for M in (1, 2, 5, 8, 16, 17, 20, 40, 100)
+              for N, K in ((2999, 2500), (1000, 130), (18820, 128), (151936, 2561), (4096, 4096), (700, 13000))
+              for x in ("f32", "f16", "bf16") for w in ws for off in (0, 1)]
+    plain = dispatch([dict(s, op=f"linear_{fmt}") for s in shapes])
+    greedy = dispatch([dict(s, op=f"linear_{fmt}_argmax") for s in shapes])
+    for s, p, g in zip(shapes, plain, greedy):
+        assert p[0] == 0 and g[0] == 0, (s, p, g)
+        n = len(p[1])
+        assert g[1][:n] == p[1] and g[2][:n] == p[2], (s, p, g)
+        assert all("argmax" in k for k in g[1][n:]), (s, g)
