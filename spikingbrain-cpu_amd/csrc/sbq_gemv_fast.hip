@@ -1014,6 +1014,9 @@ int launch_gemv_mt(const GemvArgs& a, int xt, hipStream_t st, bool gemm_alt) {
 bool pick_gemv_fast(int64_t M, int64_t K, int64_t N, int xt, bool w8a8, bool xvec, int* id, int* ks) {
   if (M < 1 || M > 16 || K % 64 != 0 || !xvec) return false;
   const int64_t Kc = K / 64, Nt = (N + 15) / 16;
+  // waves of an 8-wave workgroup that get a K tile: five and six row tiles per
+  // workgroup need that many (each tile's epilogue belongs to one wave)
+  const int64_t kw8 = (Kc + 7) / 8, waves8 = (Kc + kw8 - 1) / kw8;
   if (xt == XT_F32) {
     // x in LDS (weight-only, M <= 8: split once into bf16 planes) when it
     // fits 24 KiB, or 48 KiB for one row (M = 1, K = 12288: 16% faster than
@@ -1049,7 +1052,8 @@ bool pick_gemv_fast(int64_t M, int64_t K, int64_t N, int xt, bool w8a8, bool xve
     // (K = 2560, N = 19456 / 18820: M = 1 11.9 -> 10.9 / 11.7 -> 10.7 us
     // against one tile, M = 2 13.6 -> 11.0, M = 3 14.4 -> 11.2; N = 17000,
     // K = 4096, M = 1: 15.2 -> 13.9)
-    if (!w8a8 && M <= 8 && Kc < 128 && Nt > 1024 && (Nt + 4) / 5 <= 256 && xb <= kSplitWideBytes) {
+    if (!w8a8 && M <= 8 && Kc < 128 && Nt > 1024 && (Nt + 4) / 5 <= 256 && waves8 >= 5 &&
+        xb <= kSplitWideBytes / kFastMaxWaves * waves8) {
       *id = 7;  // D=2, G=5, x in LDS
       *ks = 8;
     }
@@ -1090,12 +1094,14 @@ bool pick_gemv_fast(int64_t M, int64_t K, int64_t N, int xt, bool w8a8, bool xve
       // 19456 / 18820, K = 2560: 12.5 -> 10.9 / 12.7 -> 10.7 us; M = 4: 11.9
       // -> 10.5 / 11.8 -> 10.3 us; grids of more than 256 such workgroups, as
       // N = 24576 at K = 4096, run slower)
-      if (M >= 4 && Kc < 128 && Nt > 1024 && (Nt + 4) / 5 <= 256 && M * K * 2 <= kFastXLdsWideBytes) {
+      if (M >= 4 && Kc < 128 && Nt > 1024 && (Nt + 4) / 5 <= 256 && waves8 >= 5 && M * K * 2 <= kFastXLdsWideBytes) {
         *id = 7;  // D=2, G=5, x in LDS
         *ks = 8;
       }
     }
   } else {
+    // (up to four K tiles a pick below that they leave too few waves for runs
+    // the general GEMV, as fast or faster: one K tile 1.5 times)
     const bool wide = Kc <= 64 && Nt >= 384;
     *id = wide ? 5 : 3;  // D=8, G=2 | D=8, G=1
     *ks = 2;
@@ -1103,7 +1109,7 @@ bool pick_gemv_fast(int64_t M, int64_t K, int64_t N, int xt, bool w8a8, bool xve
     if (!w8a8 && Kc < 128 && Nt > 1024 && (Nt + 4) / 5 <= 256 && M * K * 2 <= kFastXLdsWideBytes) {
       *id = 7;  // D=2, G=5, x in LDS
       *ks = 8;
-    } else if (!w8a8 && Kc < 128 && Nt > 1024 && (Nt + 5) / 6 <= 256) {
+    } else if (!w8a8 && Kc < 128 && Nt > 1024 && (Nt + 5) / 6 <= 256 && (Kc <= 4 || waves8 >= 6)) {
       // six row tiles per workgroup, x fragments loaded directly: each wave
       // reads its K range of x once per six row tiles instead of two, and the
       // grid still fits one round of the CUs (M = 16, N = 24576, K = 4096:
@@ -1146,7 +1152,7 @@ bool pick_gemv_fast(int64_t M, int64_t K, int64_t N, int xt, bool w8a8, bool xve
     //   29.1).
     const bool shortk = Kc > 4 && Kc < 128;
     const bool large = M >= 4 || xb > 16384;
-    if (shortk && large && Nt > 1024 && (Nt + 4) / 5 <= 256 && xb <= kSplitWideBytes) {
+    if (shortk && large && Nt > 1024 && (Nt + 4) / 5 <= 256 && waves8 >= 5 && xb <= kSplitWideBytes) {
       *id = 7;
       *ks = 8;
     } else if (shortk && M <= 8 && Nt > 256) {
@@ -1160,7 +1166,7 @@ bool pick_gemv_fast(int64_t M, int64_t K, int64_t N, int xt, bool w8a8, bool xve
         }
       } else if (xb <= 16384) {
         // small rows at M = 4 .. 8: as picked above
-      } else if (Nt > 1024 && (Nt + 5) / 6 <= 256 && xb <= 65536) {
+      } else if (Nt > 1024 && (Nt + 5) / 6 <= 256 && waves8 >= 6 && xb <= 65536) {
         *id = 8;
         *ks = 8;
       } else if (xb <= 32768) {
@@ -1170,7 +1176,7 @@ bool pick_gemv_fast(int64_t M, int64_t K, int64_t N, int xt, bool w8a8, bool xve
         }
       } else if (Nt > 4096) {
         return false;
-      } else if (xt != XT_F32 && Nt > 1536) {
+      } else if (xt != XT_F32 && Nt > 1536 && waves8 >= 5) {
         *id = 7;
         *ks = 8;
       }

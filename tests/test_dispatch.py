@@ -60,3 +60,18 @@ def test_greedy_logits_take_the_route_of_the_linear(dispatch, fmt):
         n = len(p[1])
         assert g[1][:n] == p[1] and g[2][:n] == p[2], (s, p, g)
         assert all("argmax" in k for k in g[1][n:]), (s, g)
+
+
+def test_every_aligned_decode_pick_launches(dispatch):
+    """The configuration picked for an aligned decode call (whole K tiles) is
+    one its K leaves enough waves for: the fast GEMV runs, never the general
+    one behind it (which weight-only fp16 / bf16 keeps at M > 8 and up to four
+    K tiles).  Workgroups of five and six row tiles need as many waves, each
+    with a K tile."""
+    calls = [{"op": op, "M": M, "N": N, "K": 64 * Kc, "x": x, "ws": "full"}
+             for op in ("linear_w8", "linear_w8a8") for x in ("f32", "f16", "bf16") for M in (1, 2, 3, 4, 6, 8, 9, 12, 16)
+             for Kc in (1, 2, 3, 4, 5, 6, 7, 9, 10, 11, 13, 17, 25, 33, 40, 49, 64, 65, 127, 128, 192)
+             for N in (64, 3000, 4097, 6144, 12000, 16385, 17000, 18820, 20480, 20500, 24576, 24600, 30000, 151936)
+             if op == "linear_w8a8" or x == "f32" or M <= 8 or Kc > 4]
+    for c, (rc, names, _) in zip(calls, dispatch(calls)):
+        assert rc == 0 and kernels(names)[-1] == "gemv_fast_kernel", (c, rc, names)
