@@ -1166,6 +1166,19 @@ def test_grouped_linears(dev, M, K, Ns, xd):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,K,xd", [(1, 2500, "f32"), (1, 9001, "f32"), (4, 2500, "f16"), (9, 2500, "bf16"), (16, 1111, "f32"),
+                                    (2, 13000, "f16"), (20, 2500, "f32")])
+def test_grouped_linears_of_ragged_k(dev, M, K, xd):
+    """No grouped launch takes K % 64 != 0: each linear runs as on its own, bit
+    for bit."""
+    announce(f"grouped linears ragged M={M} K={K} x={xd}")
+    lins = [quant.Int8Linear(gpu_weight(N, K, 945 + i, dev), None) for i, N in enumerate((2999, 300))]
+    xs = [cpu_x(M, K, 947 + i).to(DT[xd]).to(dev) for i in range(2)]
+    for o, lin, x in zip(quant.grouped_forward(list(zip(lins, xs))), lins, xs):
+        assert torch.equal(o, lin(x))
+
+
+@pytest.mark.gpu
 def test_grouped_linears_graph_replays(dev):
     """The grouped launch under HIP graph capture: every replay equals the
     eager result."""
