@@ -1708,7 +1708,7 @@ int launch_gemm_w8a8_token(const void* x, int xt, int64_t M, int64_t K, int64_t 
     g.N = (int)N; g.Nt = (int)Nt; g.y = y; g.yt = yt; g.ldy = ldy; g.acc_out = acc_out;
     g.flags = kGemvXVec | (yvec ? kGemvYVec : 0) | kGemvPerToken;
     int id = 0, ks = 0;
-    if (pick_gemv_fast(M, K, N, xt, true, true, &id, &ks)) {
+    if (!gemv_quantize_first(M, K, N, xt) && pick_gemv_fast(M, K, N, xt, true, true, &id, &ks)) {
       const int frc = launch_gemv_fast_cfg(id, ks, g, xt, true, st);
       if (frc != -1) return frc;
     }

@@ -595,7 +595,8 @@ int launch_gemv_w8_mt(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, 
 
 // Independent linears of one M, K and dtypes in one fast-path launch (picked
 // as one linear of their summed rows): weight-only, or int8-dyn (w8a8: each
-// segment's colsum set) with the activation min/max reduced in the kernel.
+// segment's colsum set) with the activation min/max reduced in the kernel, or,
+// with xq0 / qp0, each input quantized in one launch before it.
 // -1: the fast path does not apply; the caller runs them one by one.
 int launch_gemv_w8_grouped(const GemvSeg* segs, int n, int xt, int64_t M, int64_t K, bool xvec, int yt, bool yvec,
                            hipStream_t st, bool w8a8, int8_t* const* xq0, float* const* qp0) {
@@ -610,10 +611,12 @@ int launch_gemv_w8_grouped(const GemvSeg* segs, int n, int xt, int64_t M, int64_
   a.flags = (xvec ? kGemvXVec : 0) | (yvec ? kGemvYVec : 0);
   a.nseg = n;
   for (int i = 0; i < n; ++i) a.seg[i] = segs[i];
-  const int rc = launch_gemv_fast_grouped(fid, fks, a, xt, w8a8, st);
-  if (rc != -1 || !w8a8 || !xq0) return rc;
-  for (int i = 0; i < n; ++i)
-    if (!quantize_small_fits(M, K, K, segs[i].ldx, xvec)) return rc;
+  bool quantize = w8a8 && xq0;
+  for (int i = 0; i < n; ++i) quantize = quantize && quantize_small_fits(M, K, K, segs[i].ldx, xvec);
+  if (!(quantize && gemv_quantize_first(M, K, nt * 16, xt))) {
+    const int rc = launch_gemv_fast_grouped(fid, fks, a, xt, w8a8, st);
+    if (rc != -1 || !quantize) return rc;
+  }
   QuantSmall q{};
   q.M = (int)M;
   q.K = q.Kp = (int)K;
@@ -648,7 +651,8 @@ int launch_gemv_w8a8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, b
   if (M <= 16) {
     GemvArgs f = with_argmax(a, am);
     int rc = -1;  // small aligned x: the kernel reduces the activation min/max itself
-    if (pick_gemv_fast(M, K, N, xt, true, xvec, &fid, &fks)) rc = launch_gemv_fast_cfg(fid, fks, f, xt, true, st);
+    if (!gemv_quantize_first(M, K, N, xt) && pick_gemv_fast(M, K, N, xt, true, xvec, &fid, &fks))
+      rc = launch_gemv_fast_cfg(fid, fks, f, xt, true, st);
     if (rc == -1) {
       // beyond that, and rows of any K or alignment: quantized once into rows
       // of whole tiles, then the GEMV on those (M = 1 ... 16, N = 2999, K =

@@ -1146,8 +1146,7 @@ bool pick_gemv_fast(int64_t M, int64_t K, int64_t N, int xt, bool w8a8, bool xve
     // * up to 32 KiB beyond the five- and six-tile grids, two row tiles and
     //   four waves (M = 2, N = 151936 fp32 59.6, M = 4 fp16 60.6; eight waves
     //   over 70);
-    // * more x on more than 4096 row tiles: quantized before the launch
-    //   instead (M = 4, N = 151936, fp32: 81 us fused, 65 so); 2-byte x on
+    // * more x: gemv_quantize_first on more than 4096 row tiles; 2-byte x on
     //   more than 1536, five row tiles (M = 8, N = 40000, K = 4096: 31.0 ->
     //   29.1).
     const bool shortk = Kc > 4 && Kc < 128;
@@ -1174,15 +1173,22 @@ bool pick_gemv_fast(int64_t M, int64_t K, int64_t N, int xt, bool w8a8, bool xve
           *id = 4;
           *ks = 4;
         }
-      } else if (Nt > 4096) {
-        return false;
-      } else if (xt != XT_F32 && Nt > 1536 && waves8 >= 5) {
+      } else if (xt != XT_F32 && Nt > 1536 && Nt <= 4096 && waves8 >= 5) {
         *id = 7;
         *ks = 8;
       }
     }
   }
   return true;
+}
+
+// Whether an int8-dyn call within the fused capacity still gains from a
+// quantizing launch before the GEMV: more than 32 KiB of x, which every
+// workgroup of the fused launch reads and quantizes whole, on more than 4096
+// row tiles of short K (M = 4, N = 151936, K = 2560, fp32: 81 us fused, 65 so).
+bool gemv_quantize_first(int64_t M, int64_t K, int64_t N, int xt) {
+  const int64_t Kc = K / 64;
+  return M <= 8 && Kc > 4 && Kc < 128 && N > 4096 * 16 && M * K * (xt == XT_F32 ? 4 : 2) > 32768;
 }
 
 // Choice for s8 rows quantized before the launch (QM 1, M <= 16).  Measured on

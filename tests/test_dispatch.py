@@ -75,3 +75,15 @@ def test_every_aligned_decode_pick_launches(dispatch):
              if op == "linear_w8a8" or x == "f32" or M <= 8 or Kc > 4]
     for c, (rc, names, _) in zip(calls, dispatch(calls)):
         assert rc == 0 and kernels(names)[-1] == "gemv_fast_kernel", (c, rc, names)
+
+
+def test_wide_grouped_int8_dyn_is_one_launch(dispatch):
+    """Groups of more than 4096 row tiles in all with more than 32 KiB of x: all
+    inputs quantized in one launch (a workgroup each) and one GEMV when every
+    linear has its share of the workspace; without it, the fused launch."""
+    for n, M, N, K, x in ((3, 4, 27866, 2688, "f32"), (3, 8, 71403, 1216, "f32"), (2, 8, 40000, 4096, "f16"),
+                          (4, 5, 33000, 4096, "bf16")):
+        c = {"op": "linear_w8a8_grouped", "M": M, "N": N, "K": K, "x": x, "count": n}
+        (rc, names, grids), (rc1, names1, _) = dispatch([dict(c, ws=str(n)), dict(c, ws="base")])
+        assert rc == 0 and kernels(names) == ["quantize_small_kernel", "gemv_fast_kernel"] and grids[0] == n, (c, names)
+        assert rc1 == 0 and kernels(names1) == ["gemv_fast_kernel"], (c, names1)
