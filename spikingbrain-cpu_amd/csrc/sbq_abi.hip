@@ -231,10 +231,11 @@ int linear_w8_run(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
     ws = (void*)(((uintptr_t)workspace + 255) & ~(uintptr_t)255);
     ws_bytes = (int64_t)workspace_bytes - (int64_t)((uintptr_t)ws - (uintptr_t)workspace);
   }
-  if (K % 64 != 0 && ws && M <= 16 && sbq::gemv_supports(M, K, false, x_dtype) &&
-      sbq::pad_decode_rows(M, N, K, x_dtype)) {
-    // ragged K at decode sizes: rows of whole tiles, then the fast GEMV (longer
-    // K than the GEMVs take: the GEMM below stages the rows itself)
+  const bool gemv = sbq::gemv_supports(M, K, false, x_dtype);
+  // ragged K with the workspace: x as rows of whole tiles, where that pays (the
+  // GEMM below writes them itself)
+  const bool pad = K % 64 != 0 && ws && sbq::pad_ragged_rows(M, N, K, x_dtype, xv);
+  if (gemv && pad && M <= 16) {
     uint8_t* rows = (uint8_t*)ws + sbq::w8_ws_layout(M, K, x_dtype).planes;
     const int64_t Kp = (K + 63) / 64 * 64;
     const int rc = sbq::launch_pad_rows(x, x_dtype, M, K, ldx, rows, st);
@@ -242,7 +243,7 @@ int linear_w8_run(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
     return sbq::launch_gemv_w8(rows, x_dtype, M, Kp, Kp, true, packed, scale, bias, N, y, y_dtype, ldy, st, yv, am,
                                yparts);
   }
-  if (!(K % 64 != 0 && ws && M > 16) && sbq::gemv_supports(M, K, false, x_dtype))
+  if (gemv && !pad)
     return sbq::launch_gemv_w8(x, x_dtype, M, K, ldx, xv, packed, scale, bias, N, y, y_dtype, ldy, st, yv, am,
                                yparts);
   return sbq::launch_gemm_w8(x, x_dtype, M, K, ldx, xv, packed, scale, bias, N, y, y_dtype, ldy, ws, ws_bytes, st,
@@ -359,7 +360,8 @@ bool runs_tiled_gemm(int64_t M, int64_t N, int64_t K, int x_dtype, bool w8a8) {
     if (w8a8_runs_mt(M, N, K, sbq::split_area_bytes(p))) return false;
     return !sbq::gemv_supports(M, K, true, x_dtype);
   }
-  if (M > 16 && K % 64 != 0) return true;  // staged as rows of whole tiles
+  if (M > 16 && K % 64 != 0)  // staged as rows of whole tiles (misaligned rows sooner than aligned ones)
+    return !sbq::gemv_supports(M, K, false, x_dtype) || sbq::pad_ragged_rows(M, N, K, x_dtype, false);
   if (M > 16 && M <= 64 && (x_dtype == SBQ_F16 || x_dtype == SBQ_BF16) && sbq::gemv_mt_applies(M, K, N, x_dtype, true))
     return false;
   return !sbq::gemv_supports(M, K, false, x_dtype);

@@ -147,16 +147,36 @@ int launch_rowsum_f16(const void* x, int64_t ldx, int64_t M, int64_t K, float* o
 // planes, [M][2][Kp].
 int launch_pad_rows(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, void* out, hipStream_t st,
                     uint32_t* zero = nullptr, int nzero = 0);
-// Whether a ragged weight-only call at decode sizes (M <= 16) gains from padded
-// rows and the fast GEMV, a launch more than the general GEMV.  Measured in HIP
-// graphs (us, general -> padded): 2999 x 2500, fp32 13.0 -> 8.3 at 4 rows and
-// 9.7 -> 10.8 at 16, fp16 8.8 -> 6.7 and 15.8 -> 8.2, one row 7.2 -> 8.4 / 5.5 ->
-// 8; 11999 x 4000, fp32 31.5 -> 16.4 at 4 rows, 16.5 -> 12.8 at one; 1000 x
-// 9001, fp32 24.5 -> 9.8 at one row, 60.2 -> 24.6 at 16, fp16 33.6 -> 10.3 at 4,
-// 10.9 -> 10.8 at one.
-inline bool pad_decode_rows(int64_t M, int64_t N, int64_t K, int xt) {
-  if (xt == 0 && M > 8) return K >= 4096 || N * K >= (int64_t)1 << 23;
-  return M > 1 || (xt == 0 && (K >= 4096 || N * K >= (int64_t)1 << 24));
+// Whether a ragged weight-only call (K % 64 != 0) that the general GEMV takes
+// (M <= 32) gains from rows of whole tiles, a launch more, on the fast GEMV (M <=
+// 16) or the tiled GEMM: as K grows, and on wide layers.  xvec: the rows are
+// 16-byte aligned as they are, which the general GEMV reads with vector loads.
+// The lines lie where both sides are equal over 6000 timings in HIP graphs (N =
+// 16 ... 150000, K = 65 ... 9000; us, general -> padded): 2999 x 2500, fp32 13.0
+// -> 8.3 at 4 rows, one row 7.2 -> 8.4; fp16, 8 rows 8.8 -> 6.7 at N = 2999, K =
+// 2500, but rows of 20 x 631 4.2 -> 6.7 and 36683 x 160 at 11 rows 6.6 -> 12.0;
+// 11999 x 4000, fp32 31.5 -> 16.4 at 4 rows, 16.5 -> 12.8 at one; 1000 x 9001,
+// fp32 24.5 -> 9.8 at one row, 60.2 -> 24.6 at 16; 20 rows of 2692 x 313, fp32 5.7
+// -> 9.0; aligned fp16 rows at 28 x 2431 x 2168 1.7 times slower padded, 32 x
+// 12780 x 3000 0.6 of it.
+inline bool pad_ragged_rows(int64_t M, int64_t N, int64_t K, int xt, bool xvec) {
+  const int64_t nk = (N * K) >> 20;
+  // K >= k0, or weights of n1 MiB at K >= k1, or of n2 MiB
+  const auto past = [&](int64_t k0, int64_t k1, int64_t n1, int64_t n2) {
+    return K >= k0 || (K >= k1 && nk >= n1) || nk >= n2;
+  };
+  if (xt == 0) {
+    if (M == 1) return past(4096, 512, 16, 32);
+    if (M == 2) return xvec ? past(8192, 512, 8, 64) : past(384, 384, 0, 10);
+    return past(M > 8 && M <= 16 ? 4096 : 1024, 256, 8, xvec ? 64 : 10);
+  }
+  if (M == 1) return false;
+  if (xvec) {
+    if (M <= 4) return past(M == 2 ? K + 1 : 6144, 512, 20, 64);
+    return M <= 16 ? past(4096, 512, 10, 64) : past(4096, 1024, 20, 64);
+  }
+  if (M == 2) return past(1536, 512, 8, 24);
+  return M <= 16 ? past(768, 320, 4, 12) : past(128, 128, 0, 6);
 }
 int launch_split_rows(const void* x, int64_t M, int64_t K, int64_t ldx, void* out, hipStream_t st,
                       uint32_t* zero = nullptr, int nzero = 0);

@@ -87,3 +87,33 @@ def test_wide_grouped_int8_dyn_is_one_launch(dispatch):
         (rc, names, grids), (rc1, names1, _) = dispatch([dict(c, ws=str(n)), dict(c, ws="base")])
         assert rc == 0 and kernels(names) == ["quantize_small_kernel", "gemv_fast_kernel"] and grids[0] == n, (c, names)
         assert rc1 == 0 and kernels(names1) == ["gemv_fast_kernel"], (c, names1)
+
+
+# (M, N, K, x, off, kernels): both sides of each line of pad_ragged_rows
+GENERAL, PADDED, STAGED = (["gemv_kernel"], ["pad_rows_kernel", "gemv_fast_kernel"], ["pad_rows_kernel", "gemm_dl_kernel"])
+RAGGED_LINES = [
+    (1, 300, 4095, "f32", 0, GENERAL), (1, 300, 4097, "f32", 0, PADDED), (1, 20000, 2500, "f16", 0, GENERAL),
+    (2, 300, 383, "f32", 0, GENERAL), (2, 300, 385, "f32", 0, PADDED), (2, 300, 2500, "f32", 0, GENERAL),
+    (2, 300, 2500, "f32", 1, PADDED), (2, 4000, 2500, "f32", 0, PADDED),
+    (4, 20, 631, "f32", 0, GENERAL), (8, 300, 1025, "f32", 0, PADDED), (8, 300, 1028, "f32", 0, PADDED),
+    (5, 20000, 500, "f32", 0, PADDED), (16, 300, 4095, "f32", 0, GENERAL), (16, 300, 4097, "f32", 0, PADDED),
+    (2, 300, 1535, "f16", 0, GENERAL), (2, 300, 1537, "f16", 0, PADDED), (2, 300, 2504, "bf16", 0, GENERAL),
+    (11, 36683, 72, "f16", 0, GENERAL), (11, 36683, 160, "f16", 0, GENERAL), (11, 36683, 161, "f16", 0, GENERAL),
+    (8, 300, 769, "bf16", 0, PADDED), (8, 300, 776, "bf16", 0, GENERAL), (8, 300, 776, "bf16", 1, PADDED),
+    (16, 4000, 2504, "f16", 0, GENERAL), (16, 5000, 2504, "f16", 0, PADDED), (4, 300, 6152, "f16", 0, PADDED),
+    (20, 300, 631, "f32", 0, GENERAL), (20, 300, 1025, "f32", 0, STAGED), (20, 2692, 313, "f32", 0, GENERAL),
+    (20, 300, 127, "f16", 0, GENERAL), (20, 300, 129, "f16", 0, STAGED), (28, 2431, 2168, "f16", 0, GENERAL),
+    (28, 2431, 2168, "f16", 1, STAGED), (32, 12780, 3000, "f16", 0, STAGED), (33, 300, 65, "f16", 0, STAGED),
+]
+
+
+@pytest.mark.parametrize("op", ["linear_w8", "linear_w8_argmax"])
+def test_ragged_rows_are_padded_where_it_pays(dispatch, op):
+    """Ragged weight-only calls that the general GEMV takes run it until K or
+    the layer outweighs the padding launch; misaligned rows sooner than rows
+    it reads with vector loads.  Without the workspace nothing is padded."""
+    calls = [{"op": op, "M": M, "N": N, "K": K, "x": x, "off": off, "ws": "full"} for M, N, K, x, off, _ in RAGGED_LINES]
+    for c, (*_, want), (rc, names, _) in zip(calls, RAGGED_LINES, dispatch(calls)):
+        assert rc == 0 and kernels(names)[:len(want)] == want, (c, names)
+    for c, (rc, names, _) in zip(calls, dispatch([dict(c, ws=None) for c in calls])):
+        assert rc == 0 and kernels(names)[0] in ("gemv_kernel", "gemm_w8_kernel"), (c, names)
