@@ -377,7 +377,7 @@ int sbq_argmax_rows(const float* y, int64_t M, int64_t N, int64_t ldy, int64_t* 
 
 /* ---- non-greedy sampling (engine.py:29-42, sample) ---- */
 
-/* Workspace bytes of sbq_sample_rows for M rows (about 130 KB per row, for
+/* Workspace bytes of sbq_sample_rows for M rows (about 270 KB per row, for
  * any vocabulary size up to 2^23).  0 for a bad argument. */
 int64_t sbq_sample_workspace_bytes(int64_t M, int64_t V);
 

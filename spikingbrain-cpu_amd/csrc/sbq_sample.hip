@@ -15,26 +15,30 @@
 //
 // No sort.  Both cuts (the k-th largest z, the top-p boundary) are found in
 // two levels.  The row's tokens are counted (top-k) and their masses
-// exp(z - max), in 2^-40 fixed point, added (top-p) in kSampBins equal bins
-// of max - z; a token more than 28 below the maximum has mass 0, so the bins
-// span at most that.  Every sum is an exact integer, independent of the order
-// the atomics land in; top_p is applied to the kept mass as top_p * sum,
-// which is the normalized condition.  The bins of the two cuts (or, while the
-// kept mass still depends on the k-th token, the few bins its bounds allow)
-// hold the only undecided tokens: a few hundred of 151936.  They are listed
-// per slice, and one workgroup per row finds the exact keys among them
-// (order-preserving 32-bit keys of z, 256 ranges per step), adds up the
-// slices and draws.  Four launches for any cut: maximum, bins, lists, draw
-// (three without a cut).
+// exp(z - max), in 2^-40 fixed point, added (top-p) in kSampBins bins of z,
+// laid between samples of the row (SampTable); a token more than 28 below the
+// maximum has mass 0, and all of those share the last bin.  Every sum is an
+// exact integer, independent of the order the atomics land in; top_p is applied
+// to the kept mass as top_p * sum, which is the normalized condition.  The bins
+// of the two cuts (or, while the kept mass still depends on the k-th token, the
+// few bins its bounds allow) hold the only undecided tokens: a few hundred of
+// 151936.  They are listed per slice, and one workgroup per row finds the exact
+// keys among them (order-preserving 32-bit keys of z, 256 ranges per step), adds
+// up the slices and draws.  Four launches for any cut: maximum and samples,
+// bins, lists, draw (three without a cut).
 //
 // What bounds it: the launches and the latency of each one's serial chain;
 // the logits (608 KB at V = 151936) are read from L2 three times.  Measured
-// in a HIP graph at V = 151936, against one launch per 8 key bits of each cut
-// over the whole row (7 launches with top-p, 10 with top-k as well): one row,
-// top-p 32.5 -> 18.4 us, top-k and top-p 49.5 -> 23.1, top-k 30.3 -> 16.8, no
-// cut 12.6 -> 10.7; eight rows, both cuts 63.6 -> 27.1.  Per launch at one
-// row: 3.0 (maximum), 4.5, 5.0, 6.6 us.  512 bins: 256 and 1024 ran within
-// 2% at one row; 1024 was 25% slower at 16 rows (more atomics per slice).
+// in a HIP graph at V = 151936 on one box, against one launch per 8 key bits of
+// each cut over the whole row (7 launches with top-p, 10 with top-k as well): one
+// row of a language model's logits, top-p 34.3 -> 21.5 us, top-k 50 and top-p 51.0
+// -> 25.5, no cut 14.1 -> 12.4; eight rows, both cuts 68 -> 34.8.  Per launch at one
+// row: 3.1 (maximum), 4.9, 5.2, 6.1 us.  Bins of equal width over the row's range
+// took 20.5, 23.6 and 30.6 us there, but 390 (both cuts 470) on a flat row with one
+// far or masked token; between samples such rows take 26 and 28, and no row of 19
+// kinds (masked, clustered, tied, sorted) more than the radix launches did (top-p
+// 38 at most).  512 bins: 256 and 1024 of equal width ran within 2% at one row;
+// 1024 was 25% slower at 16 rows (more atomics per slice).
 //
 // No workgroup waits for another: what a launch needs from the one before it
 // (maximum, bins) every workgroup derives for itself.  Rows are independent
@@ -56,11 +60,12 @@ namespace sbq {
 constexpr int kSampThreads = 1024;
 constexpr int kSampWaves = kSampThreads / 64;
 constexpr int kSampMaxBlocks = 64;   // workgroups (slices) per row: one wave's lanes hold a value of each
-constexpr int kSampBins = 512;       // bins of max - z
+constexpr int kSampBins = 512;       // bins of z
 constexpr int kSampCopies = 8;       // LDS copies of each bin (atomics of one wave spread over them)
 constexpr int kSampUnroll = 4;       // tokens in flight per thread
-constexpr int kSampList = 512;       // undecided tokens listed per slice (a slice with more is read again)
-constexpr uint32_t kSampTied = 1u << 31;  // a slice's undecided tokens are more than that and share one key
+constexpr int kSampList = 1024;      // undecided tokens listed per slice (a slice with more is read again)
+constexpr int kSampFew = 32;         // a slice with more undecided tokens looks whether they share one key
+constexpr uint32_t kSampTied = 1u << 31;  // ... and they do: the list's first place holds it
 constexpr float kSampRange = 28.0f;  // exp(-28) < 2^-40: a mass of 0 from here down
 
 // Per-row scratch, from the row's first byte (each part 256-byte aligned).
@@ -69,7 +74,8 @@ struct SampRow {
   static constexpr int64_t kMax = 256;                     // float [G]
   static constexpr int64_t kMin = kMax + 256;              // float [G]
   static constexpr int64_t kNan = kMin + 256;              // int [G]
-  static constexpr int64_t kSum = kNan + 256;              // uint64 [G]: mass above every undecided bin
+  static constexpr int64_t kSplit = kNan + 256;            // float [64]: samples of z, largest first
+  static constexpr int64_t kSum = kSplit + 256;            // uint64 [G]: mass above every undecided bin
   static constexpr int64_t kNum = kSum + 512;              // uint32 [G]: undecided tokens of the slice (| kSampTied)
   static constexpr int64_t kMass = kNum + 256;             // uint64 [kSampBins]
   static constexpr int64_t kCount = kMass + kSampBins * 8; // uint32 [kSampBins]
@@ -78,12 +84,13 @@ struct SampRow {
 };
 static_assert(kSampMaxBlocks * 8 <= 512 && kSampMaxBlocks * 4 <= 256 && kSampMaxBlocks <= 64,
               "per-slice arrays fit their slots and one wave");
+static_assert(kSampMaxBlocks == 64, "one lane per slice, its number in seven bits");
 static_assert(kSampMaxBlocks % kSampWaves == 0, "the draw's waves own whole sets of slices");
 
 // The undecided bins of a row, recorded by the list launch for the draw.
 struct SampHead {
   int valid;      // 0: a NaN or an infinite max (the reference raises)
-  float m, inv;   // max z; bins per unit of max - z
+  float m, low;   // max z; the lowest z that the bins resolve
   int kbin;       // the bin of the k-th largest z (-1: top-k masks nothing of mass)
   int krest;      // its rank within that bin, from the top
   int lo, hi;     // the top-p boundary lies in bins lo .. hi (lo > hi: no top-p)
@@ -127,10 +134,52 @@ __device__ __forceinline__ uint64_t samp_efix(float z, float m) {
   return sh >= 0 ? s << sh : s >> min(-sh, 63);
 }
 
-// Bin of z: equal steps of m - z, 0 at the maximum.  Rounding and truncation
-// are monotone, so a larger z never has a larger bin, and equal z share one.
-__device__ __forceinline__ int samp_bin(float z, float m, float inv) {
-  return (int)fminf((m - z) * inv, (float)(kSampBins - 1));
+// The bins of a row: 64 sampled z, sorted, give 15 splits of the values into
+// intervals of a few 64ths of the tokens each, whatever their distribution
+// (equal steps of max - z put most of a flat row beside one far token into one
+// bin, and one workgroup then read the row again per pass: 390 us at V =
+// 151936).  From the top: kSampTop equal steps of the interval above the first
+// split, where sampled decoding cuts; then per split one bin of the tokens
+// equal to it (ties) and kSampSteps steps of the interval below it; the last bin
+// the tokens without mass, and only those.  Steps end at `low`, below which no
+// token has mass.  Comparisons, rounding and truncation are monotone, so a
+// larger z never has a larger bin, and equal z share one.
+constexpr int kSampSplits = 15;
+constexpr int kSampTop = 200, kSampSteps = 19;
+static_assert(kSampTop + (kSampSteps + 1) * kSampSplits < kSampBins, "the intervals' bins and the last one");
+// Split t of the row is sample samp_split(t), finer towards the top.
+__device__ __forceinline__ int samp_split(int t) { return t < 2 ? t : (t < 10 ? 4 * t - 5 : 5 * t - 14); }
+struct SampTable {
+  float s[kSampSplits + 1];  // the splits, largest first
+  // per interval: its top (the split above it, the maximum), steps per unit of z, the split below it
+  f32x4 from[kSampSplits + 1];
+};
+struct SampLook {
+  const SampTable* tb;
+  float m;
+  __device__ __forceinline__ int bin(float z) const {
+    int i = 0;  // splits above z
+#pragma unroll
+    for (int step = 8; step > 0; step >>= 1) i += tb->s[i + step - 1] > z ? step : 0;
+    const f32x4 f = tb->from[i];
+    const int n = i == 0 ? kSampTop : kSampSteps;
+    int b = (int)fminf((f[0] - z) * f[1], (float)(n - 1));
+    if (i < kSampSplits && z == f[2]) b = n;  // after the interval's steps
+    b += i == 0 ? 0 : kSampTop + 1 + (kSampSteps + 1) * (i - 1);
+    return m - z <= kSampRange ? b : kSampBins - 1;
+  }
+};
+
+__device__ __forceinline__ void samp_table(const uint8_t* w, float m, float low, SampTable* tb) {
+  const int t = threadIdx.x;
+  if (t <= kSampSplits) {
+    const float* s = (const float*)(w + SampRow::kSplit);
+    const float top = t == 0 ? m : s[samp_split(t - 1)], end = t < kSampSplits ? s[samp_split(t)] : low;
+    const float width = top - fmaxf(end, low);
+    tb->s[t] = end;
+    const float steps = width > 0.0f ? (float)(t == 0 ? kSampTop : kSampSteps) / fmaxf(width, 1e-30f) : 0.0f;
+    tb->from[t] = (f32x4){top, steps, end, 0.0f};
+  }
 }
 
 // The top-p bound on the mass above a token: mass_above < top_p * S (S: the
@@ -209,11 +258,17 @@ __device__ __forceinline__ uint64_t samp_block_sum_u64(uint64_t v, uint64_t* red
   return wave_total(lane < kSampWaves ? red[lane] : (uint64_t)0);
 }
 
-// The row's maximum, bins and validity from the first launch's per-slice
-// values (identical in every wave and workgroup).
+// A lowest z beside its tokens' largest one `mx`, once the largest is `top`:
+// dropped when those are without mass beside it (masked slices).
+__device__ __forceinline__ float samp_near(float mx, float top, float mn) {
+  return mx >= top - kSampRange ? mn : INFINITY;
+}
+
+// The row's maximum, the lowest z the bins resolve, and validity from the
+// first launch's per-slice values (identical in every wave and workgroup).
 struct SampScale {
-  float m, inv;
-  bool valid, clamped;  // clamped: the last bin holds only tokens of mass 0
+  float m, low;
+  bool valid;
 };
 __device__ __forceinline__ SampScale samp_scale(const SampArgs& a, const uint8_t* w) {
   const int lane = threadIdx.x & 63, g = min(lane, a.G - 1);
@@ -221,37 +276,59 @@ __device__ __forceinline__ SampScale samp_scale(const SampArgs& a, const uint8_t
   const int nl = ((const int*)(w + SampRow::kNan))[g];
   SampScale s;
   s.m = wave_max(mxl);
-  const float mn = wave_min(mnl);
+  s.low = fmaxf(wave_min(samp_near(mxl, s.m, mnl)), s.m - kSampRange);
   s.valid = __ballot(nl != 0) == 0 && s.m < INFINITY && s.m > -INFINITY;
-  const float range = s.m - mn;
-  s.clamped = !(range < kSampRange);
-  s.inv = (float)(kSampBins - 1) / (s.clamped ? kSampRange : fmaxf(range, 1e-30f));
   return s;
 }
 
-// First launch: max and min of z and the NaN count per slice; workgroup 0
-// clears the row's bins.
+// The row's 64 samples, one in each 64th of the row (the place within it by the
+// golden ratio), sorted: each wave ranks the lanes' samples against its four,
+// one adds up the ranks.
+constexpr int kSampRanks = 64 / kSampWaves;
+__device__ __forceinline__ float samp_sample(const SampArgs& a) {
+  const uint32_t lane = threadIdx.x & 63;
+  const uint64_t V = (uint64_t)a.V, turn = (uint64_t)(lane * 2654435769u) * V >> 32;
+  return samp_z(a, a.x + (int64_t)blockIdx.y * a.ld, (int)((lane * V + turn) >> 6));
+}
+__device__ __forceinline__ int samp_rank(float z) {
+  const int lane = threadIdx.x & 63, j0 = (threadIdx.x >> 6) * kSampRanks;
+  int rank = 0;
+#pragma unroll
+  for (int j = j0; j < j0 + kSampRanks; ++j) {
+    const float o = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(z), j));
+    rank += o > z || (o == z && j < lane);
+  }
+  return rank;
+}
+
+// First launch: max z, min z of the tokens near it, and the NaN count per
+// slice; workgroup 0 clears the row's bins and sorts its samples.
 __global__ __launch_bounds__(kSampThreads) void samp_max_kernel(SampArgs a) {
   __shared__ float smx[kSampWaves], smn[kSampWaves];
-  __shared__ int snan[kSampWaves];
+  __shared__ int snan[kSampWaves], ranks[kSampWaves][64];
   uint8_t* w = samp_row_ws(a);
+  const bool sort = blockIdx.x == 0 && (a.k > 0 || a.top_p > 0.0);  // uniform
   const int i0 = blockIdx.x * a.per, i1 = min(i0 + a.per, a.V);
   SampTokens tok(a.x + (int64_t)blockIdx.y * a.ld, i0, i1, threadIdx.x, kSampThreads);
   if (blockIdx.x == 0 && threadIdx.x < kSampBins) {
     ((uint64_t*)(w + SampRow::kMass))[threadIdx.x] = 0;
     ((uint32_t*)(w + SampRow::kCount))[threadIdx.x] = 0;
   }
+  const int lane = threadIdx.x & 63;
+  const float sample = sort ? samp_sample(a) : 0.0f;
   float mx = -INFINITY, mn = INFINITY;
   bool nan = false;
   tok.each(a.T, [&](int, float z) {
     nan |= z != z;
-    mx = fmaxf(mx, z);
-    mn = fminf(mn, z);
+    const float top = fmaxf(mx, z);
+    mn = fminf(samp_near(mx, top, mn), samp_near(z, top, z));
+    mx = top;
   });
-  mx = wave_max(mx);
-  mn = wave_min(mn);
+  float top = wave_max(mx);
+  mn = wave_min(samp_near(mx, top, mn));
+  mx = top;
   const int any = __ballot(nan) != 0;
-  const int lane = threadIdx.x & 63;
+  if (sort) ranks[threadIdx.x >> 6][lane] = samp_rank(sample);
   if (lane == 0) {
     smx[threadIdx.x >> 6] = mx;
     smn[threadIdx.x >> 6] = mn;
@@ -260,14 +337,19 @@ __global__ __launch_bounds__(kSampThreads) void samp_max_kernel(SampArgs a) {
   __syncthreads();
   if (threadIdx.x < 64) {  // wave 0: a lane per wave's values
     const int wv = min(lane, kSampWaves - 1);
-    mx = wave_max(smx[wv]);
-    mn = wave_min(smn[wv]);
+    top = wave_max(smx[wv]);
+    mn = wave_min(samp_near(smx[wv], top, smn[wv]));
     const int bad = __ballot(snan[wv] != 0) != 0;
     if (lane == 0) {
-      ((float*)(w + SampRow::kMax))[blockIdx.x] = mx;
+      ((float*)(w + SampRow::kMax))[blockIdx.x] = top;
       ((float*)(w + SampRow::kMin))[blockIdx.x] = mn;
       ((int*)(w + SampRow::kNan))[blockIdx.x] = bad;
     }
+  } else if (sort && threadIdx.x < 128) {
+    int rank = 0;
+#pragma unroll
+    for (int i = 0; i < kSampWaves; ++i) rank += ranks[i][lane];
+    ((float*)(w + SampRow::kSplit))[min(rank, 63)] = sample;  // (a NaN: the row is invalid)
   }
 }
 
@@ -277,6 +359,7 @@ template <bool K, bool P>
 __global__ __launch_bounds__(kSampThreads) void samp_bins_kernel(SampArgs a) {
   __shared__ uint64_t H[P ? kSampBins * kSampCopies : 1];
   __shared__ uint32_t C[K ? kSampBins * kSampCopies : 1];
+  __shared__ SampTable tb;
   uint8_t* w = samp_row_ws(a);
   const int i0 = blockIdx.x * a.per, i1 = min(i0 + a.per, a.V);
   SampTokens tok(a.x + (int64_t)blockIdx.y * a.ld, i0, i1, threadIdx.x, kSampThreads);
@@ -286,10 +369,12 @@ __global__ __launch_bounds__(kSampThreads) void samp_bins_kernel(SampArgs a) {
   }
   const SampScale sc = samp_scale(a, w);
   if (!sc.valid) return;
+  samp_table(w, sc.m, sc.low, &tb);
   __syncthreads();
+  const SampLook look{&tb, sc.m};
   const int copy = threadIdx.x & (kSampCopies - 1);
   tok.each(a.T, [&](int, float z) {
-    const int at = samp_bin(z, sc.m, sc.inv) * kSampCopies + copy;
+    const int at = look.bin(z) * kSampCopies + copy;
     if constexpr (P) {
       const uint64_t f = samp_efix(z, sc.m);
       if (f) atomicAdd((unsigned long long*)&H[at], (unsigned long long)f);
@@ -327,7 +412,7 @@ __device__ void samp_cuts(const SampArgs& a, const SampScale& sc, uint64_t f, ui
     red[wv] = fi;
     red[W + wv] = ci;
   }
-  if (t == 0) *h = SampHead{1, sc.m, sc.inv, -1, 0, 1, 0, 0, 0, 0, 0};
+  if (t == 0) *h = SampHead{1, sc.m, sc.low, -1, 0, 1, 0, 0, 0, 0, 0};
   __syncthreads();
   uint64_t total = 0;
 #pragma unroll
@@ -340,9 +425,9 @@ __device__ void samp_cuts(const SampArgs& a, const SampScale& sc, uint64_t f, ui
   }
   const uint64_t fa = fi - f;  // mass of the bins above this one
   if constexpr (K) {
-    // the bin of the k-th largest z; a last bin of tokens without mass cuts nothing
+    // the bin of the k-th largest z; among the tokens without mass it cuts nothing
     const uint32_t ca = ci - c, k = (uint32_t)a.k;
-    if (t < kSampBins && ca < k && k <= ci && !(sc.clamped && t == kSampBins - 1)) {
+    if (t < kSampBins && ca < k && k <= ci && t < kSampBins - 1) {
       h->kbin = t;
       h->krest = (int)(k - ca);
       h->kabove = fa;
@@ -371,14 +456,15 @@ __device__ void samp_cuts(const SampArgs& a, const SampScale& sc, uint64_t f, ui
 }
 
 // Third launch: per slice, the mass of the tokens above every undecided bin
-// and the list of the tokens in them.  A slice with more of them than its
-// list holds records their key when they all share one (ties), as the key in
-// the list's first place and kSampTied in the count.
+// and the list of the tokens in them.  A slice of many that all share one key
+// (ties) records that key once, in the list's first place, and kSampTied in the
+// count.
 template <bool K, bool P>
 __global__ __launch_bounds__(kSampThreads) void samp_list_kernel(SampArgs a) {
   __shared__ SampHead h;
   __shared__ uint64_t red[2 * (kSampBins / 64) + 1], sum[kSampWaves];
   __shared__ uint32_t num, kmin, kmax;
+  __shared__ SampTable tb;
   uint8_t* w = samp_row_ws(a);
   const int i0 = blockIdx.x * a.per, i1 = min(i0 + a.per, a.V);
   SampTokens tok(a.x + (int64_t)blockIdx.y * a.ld, i0, i1, threadIdx.x, kSampThreads);
@@ -399,37 +485,33 @@ __global__ __launch_bounds__(kSampThreads) void samp_list_kernel(SampArgs a) {
     kmax = 0;
   }
   if constexpr (K || P) {
+    samp_table(w, sc.m, sc.low, &tb);
     samp_cuts<K, P>(a, sc, f, c, &h, red);
   } else {
-    if (threadIdx.x == 0) h = SampHead{1, sc.m, sc.inv, -1, 0, 1, 0, 0, 0, 0, 0};
+    if (threadIdx.x == 0) h = SampHead{1, sc.m, sc.low, -1, 0, 1, 0, 0, 0, 0, 0};
     __syncthreads();
   }
+  const SampLook look{&tb, sc.m};
   const int lo = h.lo, hi = h.hi, kbin = h.kbin;
   // tokens above the first undecided bin are kept, whatever the keys say
   const int first = lo <= hi ? lo : (kbin >= 0 ? kbin : kSampBins);
   uint32_t* list = (uint32_t*)(w + SampRow::kList) + blockIdx.x * kSampList;
   uint64_t part = 0;
+  uint32_t k0 = ~0u, k1 = 0;
   tok.each(a.T, [&](int, float z) {
-    const int b = samp_bin(z, sc.m, sc.inv);
+    const int b = K || P ? look.bin(z) : 0;
     if (b < first) {
       part += samp_efix(z, sc.m);
     } else if (b <= hi || b == kbin) {
       const uint32_t at = atomicAdd(&num, 1u), k = samp_key(z);
       if (at < (uint32_t)kSampList) list[at] = k;
+      k0 = min(k0, k);
+      k1 = max(k1, k);
     }
   });
   part = samp_block_sum_u64(part, sum);
-  const bool over = num > (uint32_t)kSampList;  // uniform
-  if (over) {  // do they share one key?
-    uint32_t k0 = ~0u, k1 = 0;
-    SampTokens again(a.x + (int64_t)blockIdx.y * a.ld, i0, i1, threadIdx.x, kSampThreads);
-    again.each(a.T, [&](int, float z) {
-      const int b = samp_bin(z, sc.m, sc.inv);
-      if (b >= first && (b <= hi || b == kbin)) {
-        k0 = min(k0, samp_key(z));
-        k1 = max(k1, samp_key(z));
-      }
-    });
+  const bool many = num > (uint32_t)kSampFew;  // uniform
+  if (many) {
     if (k0 <= k1) {
       atomicMin(&kmin, k0);
       atomicMax(&kmax, k1);
@@ -437,7 +519,7 @@ __global__ __launch_bounds__(kSampThreads) void samp_list_kernel(SampArgs a) {
     __syncthreads();
   }
   if (threadIdx.x == 0) {
-    const bool tied = over && kmin == kmax;
+    const bool tied = many && kmin == kmax;
     if (tied) list[0] = kmin;
     ((uint64_t*)(w + SampRow::kSum))[blockIdx.x] = part;
     ((uint32_t*)(w + SampRow::kNum))[blockIdx.x] = num | (tied ? kSampTied : 0u);
@@ -447,41 +529,49 @@ __global__ __launch_bounds__(kSampThreads) void samp_list_kernel(SampArgs a) {
 
 // The undecided tokens of the row in the draw: gathered through LDS, up to
 // kFlat per thread in registers (the usual case: a few hundred, one per
-// thread).  When there are more, wave wv goes over the slices wv, wv + 16,
-// ... on each use: their lists, their one key if all tied, or the logits
-// again.
+// thread).  When there are more, on each use wave wv goes over the lists of
+// the slices wv, wv + 16, ... (their one key if all tied), and all waves
+// together over the logits of the slices with more than a list.
 struct SampUndecided {
   static constexpr int S = kSampMaxBlocks / kSampWaves;
   static constexpr int kFlat = 4;
   bool flat;
   int sets;  // flat: ceil(tokens / kSampThreads)
-  uint32_t key[kFlat];
+  uint32_t key[kFlat], n[kFlat];  // n tokens of that key
   uint64_t mass[kFlat];
   int slice[kFlat];  // -1: none
   uint32_t num[S];   // tokens of this wave's slices, not flat
+  uint64_t longer;   // slices to read again
+  const SampTable* tb;
 
-  // lk, ls: kFlat * kSampThreads words / bytes of LDS
-  __device__ __forceinline__ void load(const SampArgs& a, const uint8_t* w, float m, uint32_t* lk, uint8_t* ls) {
+  // lk, ls, lc: kFlat * kSampThreads words / bytes and kSampMaxBlocks words of LDS
+  __device__ __forceinline__ void load(const SampArgs& a, const uint8_t* w, float m, uint32_t* lk, uint8_t* ls,
+                                       uint32_t* lc, const SampTable* table) {
+    tb = table;
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
     const uint32_t* lists = (const uint32_t*)(w + SampRow::kList);
     uint32_t nl = ((const uint32_t*)(w + SampRow::kNum))[min(lane, a.G - 1)], k[S];
 #pragma unroll
     for (int s = 0; s < S; ++s) k[s] = lists[min(wv + s * kSampWaves, a.G - 1) * kSampList + lane];
     if (lane >= a.G) nl = 0;
-    const bool fits = __ballot(nl > (uint32_t)kSampList) == 0;
-    const uint32_t incl = wave_prefix(fits ? nl : 0u);
+    longer = __ballot(nl > (uint32_t)kSampList && !(nl & kSampTied));
+    const uint32_t el = nl & kSampTied ? 1u : (longer ? 0u : nl);  // entries
+    const uint32_t incl = wave_prefix(el);
     const int total = (int)wave_last(incl);
-    flat = fits && total <= kFlat * kSampThreads;
+    flat = !longer && total <= kFlat * kSampThreads;
+    if (wv == 0) lc[lane] = nl & ~kSampTied;
     sets = (total + kSampThreads - 1) / kSampThreads;
 #pragma unroll
     for (int s = 0; s < S; ++s) {
       const int g = wv + s * kSampWaves;
       num[s] = (uint32_t)__builtin_amdgcn_readlane((int)nl, g);
       if (flat) {
-        const int o = __builtin_amdgcn_readlane((int)(incl - nl), g);
-        for (int j = lane; j < (int)num[s]; j += 64) {
+        const int o = __builtin_amdgcn_readlane((int)(incl - el), g), e = __builtin_amdgcn_readlane((int)el, g);
+        const uint8_t tied = num[s] & kSampTied ? 0x80 : 0;
+#pragma unroll 4
+        for (int j = lane; j < e; j += 64) {
           lk[o + j] = j < 64 ? k[s] : lists[g * kSampList + j];
-          ls[o + j] = (uint8_t)g;
+          ls[o + j] = (uint8_t)g | tied;
         }
       }
     }
@@ -493,7 +583,11 @@ struct SampUndecided {
         if (i < sets) {
           const int at = t + i * kSampThreads;
           key[i] = lk[at];
-          if (at < total) slice[i] = ls[at];
+          if (at < total) {
+            const int g = ls[at];
+            slice[i] = g & 0x7f;
+            n[i] = g & 0x80 ? lc[slice[i]] : 1u;
+          }
           mass[i] = samp_efix(samp_unkey(key[i]), m);  // (past the end: unused)
         }
       }
@@ -507,7 +601,7 @@ struct SampUndecided {
     if (flat) {
 #pragma unroll
       for (int i = 0; i < kFlat; ++i)
-        if (i < sets && slice[i] >= 0 && key[i] >= lo && key[i] <= hi) f(key[i], mass[i], 1u, slice[i]);
+        if (i < sets && slice[i] >= 0 && key[i] >= lo && key[i] <= hi) f(key[i], mass[i], n[i], slice[i]);
       return;
     }
     const int lane = threadIdx.x & 63;
@@ -523,13 +617,17 @@ struct SampUndecided {
         for (int j = lane; j < (int)n; j += 64) one(list[j], 1u, g);
       } else if (n & kSampTied) {
         if (lane == 0) one(list[0], n & ~kSampTied, g);
-      } else {
-        const int i0 = g * a.per, i1 = min(i0 + a.per, a.V);
-        SampTokens tok(row, i0, i1, lane, 64);
-        tok.each(a.T, [&](int, float z) {
-          const int b = samp_bin(z, h.m, h.inv);
-          if ((b >= h.lo && b <= h.hi) || b == h.kbin) one(samp_key(z), 1u, g);
-        });
+      }
+    }
+    const SampLook look{tb, h.m};
+#pragma unroll 1
+    for (uint64_t rest = longer; rest; rest &= rest - 1) {
+      const int g = __ffsll((long long)rest) - 1, i1 = min((g + 1) * a.per, a.V);
+#pragma unroll 1
+      for (int i = g * a.per + (int)threadIdx.x; i < i1; i += kSampThreads) {
+        const float z = samp_z(a, row, i);
+        const int b = look.bin(z);
+        if ((b >= h.lo && b <= h.hi) || b == h.kbin) one(samp_key(z), 1u, g);
       }
     }
   }
@@ -545,7 +643,7 @@ constexpr int kCutCopies = 4;
 constexpr int kCutStride = 256 + 2;  // copies of one range lie in different banks
 constexpr int kCutWords = kCutCopies * kCutStride;
 template <bool MASS>
-__device__ uint32_t samp_descend(const SampArgs& a, const uint8_t* w, const float* row, const SampHead& h,
+__device__ __forceinline__ uint32_t samp_descend(const SampArgs& a, const uint8_t* w, const float* row, const SampHead& h,
                                  const SampUndecided& und, uint32_t lo, uint32_t hi, uint64_t& rest, uint64_t thr,
                                  uint64_t* H, uint64_t* bc) {
   const int t = threadIdx.x, lane = t & 63;
@@ -608,7 +706,9 @@ __global__ __launch_bounds__(kSampThreads) void samp_draw_kernel(SampArgs a) {
   __shared__ uint64_t H[K || P ? kCutWords : 1];
   __shared__ uint32_t lk[K || P ? SampUndecided::kFlat * kSampThreads : 1];
   __shared__ uint8_t ls[K || P ? SampUndecided::kFlat * kSampThreads : 1];
+  __shared__ uint32_t lc[K || P ? kSampMaxBlocks : 1];
   __shared__ uint64_t bck[2], bcp[2];
+  __shared__ SampTable tb;
   __shared__ uint64_t red[kSampWaves], wtot[kSampWaves];
   __shared__ float zred[4][kSampWaves];
   __shared__ uint64_t smass[kSampMaxBlocks];
@@ -636,13 +736,15 @@ __global__ __launch_bounds__(kSampThreads) void samp_draw_kernel(SampArgs a) {
       smass[t] = 0;
       stie[t] = 0;
     }
+    samp_table(w, h.m, h.low, &tb);
     SampUndecided und;
-    und.load(a, w, h.m, lk, ls);
+    und.load(a, w, h.m, lk, ls, lc, &tb);
+    const SampLook look{&tb, h.m};
     // lowest and highest undecided z, of the k-th token's bin and of the boundary's bins
     float k0 = INFINITY, k1 = -INFINITY, p0 = INFINITY, p1 = -INFINITY;
     und.each(a, w, row, h, 0u, ~0u, [&](uint32_t k, uint64_t, uint32_t, int) {
       const float z = samp_unkey(k);
-      const int b = samp_bin(z, h.m, h.inv);
+      const int b = look.bin(z);
       if (K && b == h.kbin) {
         k0 = fminf(k0, z);
         k1 = fmaxf(k1, z);

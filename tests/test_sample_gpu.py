@@ -341,3 +341,85 @@ def test_sample_undecided_tokens(dev, kind, V, T, k, p):
         tok = int(_run(x.to(dev), T, k, p, torch.tensor([u0], device=dev))[0])
         want, ok, _ = _accept(xn, T, k, p, u0, tok)
         assert ok, (kind, u0, tok, want)
+
+
+def _degenerate_row(kind, V, g):
+    """Rows whose cuts fall among many tokens: flat beside a far or a masked
+    token, two neighbouring values, most of the row masked, an allowed block in
+    a masked row, values sorted along the vocabulary (one slice holds the cut),
+    a cluster that fills most of one 64th of the vocabulary and holds none of
+    the row's samples (more undecided tokens than a slice lists)."""
+    x = torch.randn(1, V, generator=g)
+    if kind == "flat-far":
+        x = 0.01 * x
+        x[0, V // 3] = -20.0
+    elif kind == "flat-masked":
+        x = 1e-6 * x
+        x[0, V // 3] = float("-inf")
+    elif kind == "peak-over-flat":
+        x = 0.01 * x
+        x[0, V // 3] = 5.0
+    elif kind == "two-values":
+        x = torch.where(x > 0, 1.0, 1.0 + 2 ** -20)
+        x[0, 3] = -19.0
+    elif kind == "masked":
+        x = torch.where(torch.rand(1, V, generator=g) < 0.99, -1e30, 2.5 * x)
+    elif kind == "block":
+        y = torch.full((1, V), float("-inf"))
+        n = min(4500, V // 2)
+        y[:, V // 5:V // 5 + n] = 0.01 * x[:, :n]
+        x = y
+    elif kind == "sorted":
+        x = (2.5 * x).sort(-1, descending=True).values
+    else:
+        sampled = [(i * V + ((i * 2654435769 % 2 ** 32) * V >> 32)) >> 6 for i in range(64)]
+        after = max(range(64), key=lambda i: (i + 1) * V // 64 - sampled[i])
+        i0, i1 = sampled[after] + 1, (after + 1) * V // 64 - 1
+        x[:, i0:i1] = 9 + 1e-4 * torch.rand(1, i1 - i0, generator=g)
+    return x
+
+
+DEGENERATE = ["flat-far", "flat-masked", "peak-over-flat", "two-values", "masked", "block", "sorted", "slice"]
+
+
+@pytest.mark.parametrize("V,T,k,p", [(151936, 0.7, 0, 0.9), (151936, 0.7, 3000, 0.6), (151936, 1.0, 40000, 1.0),
+                                     (300000, 1.0, 2000, 0.9), (5000, 0.7, 600, 0.5)])
+@pytest.mark.parametrize("kind", DEGENERATE)
+def test_sample_degenerate_rows(dev, kind, V, T, k, p):
+    """The oracle's tokens where a slice lists thousands of undecided tokens,
+    one key for all of them, or more than its list holds (read again)."""
+    announce(f"sample degenerate {kind} V={V} T={T} k={k} p={p}")
+    x = _degenerate_row(kind, V, torch.Generator().manual_seed(V + k))
+    xn = x[0].numpy()
+    for u0 in (0.0, 0.31, 0.77, 1 - 2 ** -24):
+        tok = int(_run(x.to(dev), T, k, p, torch.tensor([u0], device=dev))[0])
+        want, ok, _ = _accept(xn, T, k, p, u0, tok)
+        assert ok, (kind, u0, tok, want)
+
+
+def test_sample_time_hardly_depends_on_the_row(dev):
+    """Bins of equal width put a flat row beside one far token into one bin, and
+    the draw then read the whole row on every pass: 19 times the time of a
+    language model's row.  (1.0 - 1.8 times with bins between samples of the
+    row; the bound leaves room for a busy box.)"""
+    announce("sample time by row")
+    V, g = 151936, torch.Generator().manual_seed(1)
+    u = torch.tensor([0.31], device=dev)
+
+    def micros(x, k):
+        x, ws = x.to(dev), quant.sample_workspace(1, V, dev)
+        best = float("inf")
+        for _ in range(4):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(20):
+                quant.sample_tokens(x, 0.7, 0.9, k, u=u, workspace=ws)
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b) * 50)
+        return best
+
+    for k in (0, 3000):
+        usual = micros(2.5 * torch.randn(1, V, generator=g), k)
+        for kind in DEGENERATE:
+            assert micros(_degenerate_row(kind, V, g), k) <= 4 * usual, (kind, k, usual)
