@@ -1498,6 +1498,13 @@ __global__ __launch_bounds__(1024) void quantize_small_kernel(QuantSmall a) {
   vN v[C];
 #pragma unroll
   for (int i = 0; i < C; ++i) {  // clamped: surplus chunks repeat the last one and are not stored
+    if constexpr (!DENSE) {
+      // whole rounds past the input are skipped (uniform): a small ragged x
+      // loaded its last chunk by elements up to five times over (6 rows of 144
+      // fp16 values 8.5 -> 6.1 us with the GEMV; dense loads are faster clamped)
+      v[i] = (vN)(T)0.0f;
+      if (i * 1024 >= nch) continue;
+    }
     const int c = min(t + i * 1024, nch - 1);
     if constexpr (DENSE) {
       v[i] = *((const vN*)x + c);
@@ -1515,13 +1522,15 @@ __global__ __launch_bounds__(1024) void quantize_small_kernel(QuantSmall a) {
   for (int i = t; i < a.nzero; i += 1024) a.zero[i] = 0u;
   float mn = 0.0f, mx = 0.0f;  // fbgemm's range always holds 0
 #pragma unroll
-  for (int i = 0; i < C; ++i)
+  for (int i = 0; i < C; ++i) {
+    if (!DENSE && i * 1024 >= nch) continue;
 #pragma unroll
     for (int j = 0; j < NE; ++j) {
       const float f = XElem<XT>::to_f32(v[i][j]);
       mn = fminf(mn, f);
       mx = fmaxf(mx, f);
     }
+  }
   mn = wave_min(mn);
   mx = wave_max(mx);
   if (lane == 0) red[t >> 6] = make_float2(mn, mx);
@@ -1544,6 +1553,7 @@ __global__ __launch_bounds__(1024) void quantize_small_kernel(QuantSmall a) {
   for (int i = 0; i < C; ++i) asm("" : "+v"(v[i]));
 #pragma unroll
   for (int i = 0; i < C; ++i) {
+    if (!DENSE && i * 1024 >= nch) continue;
     const int c = t + i * 1024;
     uint32_t d[NE / 4];
 #pragma unroll
@@ -1560,12 +1570,13 @@ __global__ __launch_bounds__(1024) void quantize_small_kernel(QuantSmall a) {
 }
 
 // x up to 320 KiB of fp32 or 160 KiB of 2-byte values (whose conversion, done
-// twice, costs more than the second launch beyond that: 304 KiB 7.9 us); half
-// of that for rows that are not dense (M = 17, K = 4000 of fp32: the call took
-// 28.3 us with one launch, 23.7 with two).
+// twice, costs more than the second launch beyond that: 304 KiB 7.9 us); of
+// rows that are not dense 32768 values (M = 17, K = 4000 of fp32: the call took
+// 28.3 us with one launch, 23.7 with two; M = 56, K = 664 of fp16, 36 thousand:
+// 12.7 and 11.4).
 bool quantize_small_fits(int64_t M, int64_t K, int64_t Kp, int64_t ldx, bool xvec) {
   const bool dense = xvec && K == Kp && (ldx == K || M == 1);
-  return M * Kp <= (int64_t)(dense ? kQuantSmallChunks : kQuantSmallChunks / 2) * 1024 * 4;
+  return M * Kp <= (dense ? (int64_t)kQuantSmallChunks * 1024 * 4 : 32768);
 }
 
 int launch_quantize_small(const QuantSmall& a, int count, int xt, hipStream_t st) {

@@ -117,3 +117,18 @@ def test_ragged_rows_are_padded_where_it_pays(dispatch, op):
         assert rc == 0 and kernels(names)[:len(want)] == want, (c, names)
     for c, (rc, names, _) in zip(calls, dispatch([dict(c, ws=None) for c in calls])):
         assert rc == 0 and kernels(names)[0] in ("gemv_kernel", "gemm_w8_kernel"), (c, names)
+
+
+def test_small_activations_are_quantized_in_one_launch(dispatch):
+    """int8-dyn beyond the fused capacity: one quantizing launch up to 20 chunks
+    of dense x per thread (81920 values), 32768 values of rows that are not
+    dense, and two beyond."""
+    one, two = "quantize_small_kernel", ("minmax_partial_kernel", "minmax_dense_kernel")
+    for M, K, off, want in ((8, 4033, 0, one), (8, 4096, 1, one), (9, 4033, 0, two), (9, 4096, 1, two), (20, 4096, 0, one),
+                            (21, 4096, 0, two), (32, 1024, 1, one), (33, 1023, 0, two), (3, 77, 0, one)):
+        for x in ("f32", "f16", "bf16"):
+            c = {"op": "linear_w8a8", "M": M, "N": 5000, "K": K, "x": x, "off": off, "ws": "full"}
+            if x != "f32" and M <= 8 and K % 64 == 0 and not off:
+                continue  # within the fused capacity
+            rc, names, _ = dispatch([c])[0]
+            assert rc == 0 and kernels(names)[0] in want, (c, names)
