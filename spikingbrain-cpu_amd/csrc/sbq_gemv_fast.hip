@@ -1011,7 +1011,7 @@ int launch_gemv_mt(const GemvArgs& a, int xt, hipStream_t st, bool gemm_alt) {
 // split once into bf16 high / remainder planes when x fits (M <= 8), and
 // otherwise take direct steps with two row tiles per wave on wide layers (M =
 // 4, N = 6144 and 24576: 21-28% faster than one row tile).
-bool pick_gemv_fast(int64_t M, int64_t K, int64_t N, int xt, bool w8a8, bool xvec, int* id, int* ks) {
+bool pick_gemv_fast(int64_t M, int64_t K, int64_t N, int xt, bool w8a8, bool xvec, int* id, int* ks, bool token) {
   if (M < 1 || M > 16 || K % 64 != 0 || !xvec) return false;
   const int64_t Kc = K / 64, Nt = (N + 15) / 16;
   // waves of an 8-wave workgroup that get a K tile: five and six row tiles per
@@ -1029,7 +1029,9 @@ bool pick_gemv_fast(int64_t M, int64_t K, int64_t N, int xt, bool w8a8, bool xve
     // 5120, K = 4096: 6.7 us, four waves 7.1; one tile 7.7; M = 2, N = 6144:
     // 7.5, direct steps 8.5), 4 waves below, where 8 leave each wave five
     // tiles (K = 2560: N = 151936 58.3 us, eight waves over 70; 12288 8.2,
-    // 9.4; M = 2, 151936: 62.0, 71.9).
+    // 9.4; M = 2, 151936: 62.0, 71.9).  Two rows of K > 4096 on more than 512
+    // row tiles keep direct steps (their LDS leaves one workgroup per CU: N =
+    // 97455, K = 4864 115 us so, 88 with direct steps).
     // Long K over at most 256 row tiles takes 8 waves (N = 2560, K = 9728:
     // 8.9 -> 8.5 us; N = 4096, K = 12288: 11.6 -> 11.35 us).  Else direct steps: 8 tiles over one row tile for long
     // K, 4 tiles over two row tiles for wide layers, 4 tiles over one row
@@ -1039,7 +1041,7 @@ bool pick_gemv_fast(int64_t M, int64_t K, int64_t N, int xt, bool w8a8, bool xve
     const bool xl = (w8a8 || M <= 8) && (xb <= 24576 || (!w8a8 && M == 1 && xb <= kFastSplitBytes));
     const auto rounds = [](int64_t wgs) { return (wgs + 255) / 256; };
     const bool wide1 = !w8a8 && M <= 2 && xb <= kFastSplitBytes && Kc < 128 && Nt > 256 &&
-                       rounds(Nt) >= 2 * rounds((Nt + 1) / 2);
+                       (M == 1 || Kc <= 64 || Nt <= 512) && rounds(Nt) >= 2 * rounds((Nt + 1) / 2);
     *id = wide1 ? 6 : (xl ? 0 : (Kc >= 128 ? 3 : (Nt >= 384 ? 4 : 2)));
     *ks = (wide1 && Kc > 48) || (xl && !w8a8 && Kc >= 128 && Nt <= 256) ? 8 : 4;
     if (!w8a8 && Kc <= 4) {
@@ -1078,7 +1080,8 @@ bool pick_gemv_fast(int64_t M, int64_t K, int64_t N, int xt, bool w8a8, bool xve
       //   10.2 -> 9.2 us; N = 6144, 8192, 24576 and 151936 keep two tiles);
       //   two waves on the wide ones at K <= 3072 (M = 1, K = 2560: N = 18820
       //   11.0 -> 10.1 us, 19456 11.0 -> 10.2, 12288 7.8 -> 7.4; K = 4096
-      //   keeps four).
+      //   keeps four, and so do K = 1088 ... 2048, which four waves take in one
+      //   8-tile step each: 1-6% faster there).
       const auto rounds = [](int64_t wgs) { return (wgs + 255) / 256; };
       const bool xl = M * K * 2 <= kFastXLdsBytes;
       if (Kc <= 4) {
@@ -1086,7 +1089,7 @@ bool pick_gemv_fast(int64_t M, int64_t K, int64_t N, int xt, bool w8a8, bool xve
         *ks = 1;
       } else if (xl && (wide ? rounds(Nt) < 2 * rounds((Nt + 1) / 2) : Nt < 256)) {
         *id = 0;  // D=8, G=1, x in LDS
-        if (wide && Kc <= 48) *ks = 2;
+        if (wide && Kc <= 48 && (Kc <= 16 || Kc > 32)) *ks = 2;
       }
       // M = 4 .. 8, a wide layer at short K whose grid of five row tiles per
       // workgroup fills one round of the CUs: x (up to 64 KiB) in LDS, read
@@ -1139,16 +1142,23 @@ bool pick_gemv_fast(int64_t M, int64_t K, int64_t N, int xt, bool w8a8, bool xve
     //   that M = 8 at K = 2560 takes no quantizing launch: checkpoint int8-dyn
     //   step 3036 -> 3240 tok/s; M = 2, N = 19456 12.7 -> 11.7 us), else six
     //   (M = 8, N = 24576, K = 4096, fp16: 21.4 -> 19.8);
-    // * up to 16 KiB, M <= 3: two waves, one row tile on the widest (M = 1, K =
+    // * up to 16 KiB, M <= 3: one row tile and two waves on the widest (M = 1, K =
     //   2560: N = 19456 11.4 -> 10.3 us, 151936 57.3); at K <= 3072 four waves
     //   of 4-tile steps (N = 12288 8.1 -> 7.6) or, up to 512 row tiles, 8-tile
-    //   steps over two (N = 5120 6.1 -> 5.7);
+    //   steps over two (N = 5120 6.1 -> 5.7).  2-byte rows, whose two-tile
+    //   workgroups quantize little, gain from K = 2624, 2112 at two rows and 576
+    //   at one on, and from 8-tile steps below 384 row tiles only (M = 1 ... 3,
+    //   K = 320 ... 2048 elsewhere: 3-10% slower);
     // * up to 32 KiB beyond the five- and six-tile grids, two row tiles and
     //   four waves (M = 2, N = 151936 fp32 59.6, M = 4 fp16 60.6; eight waves
-    //   over 70);
+    //   over 70; one fp32 row from 768 row tiles on, N = 6731, K = 5248 16% slower);
     // * more x: gemv_quantize_first on more than 4096 row tiles; 2-byte x on
-    //   more than 1536, five row tiles (M = 8, N = 40000, K = 4096: 31.0 ->
-    //   29.1).
+    //   more than 1536, five row tiles where their last round of the CUs is more
+    //   than half full (M = 8, N = 40000, K = 4096: 31.0 -> 29.1; N = 25661, K =
+    //   5888, 1.25 rounds, 18% slower; per-token rows always: 0.7 of the time).
+    // Per-token rows (every thread reduces each row's maximum and divides each
+    // value, in each workgroup) take the one-tile rules only in fp32 or for one
+    // row: two and three rows of fp16 were 8-30% slower.
     const bool shortk = Kc > 4 && Kc < 128;
     const bool large = M >= 4 || xb > 16384;
     if (shortk && large && Nt > 1024 && (Nt + 4) / 5 <= 256 && waves8 >= 5 && xb <= kSplitWideBytes) {
@@ -1156,10 +1166,13 @@ bool pick_gemv_fast(int64_t M, int64_t K, int64_t N, int xt, bool w8a8, bool xve
       *ks = 8;
     } else if (shortk && M <= 8 && Nt > 256) {
       if (!large) {
+        const bool f32 = xt == XT_F32;
         if (Nt > 1024) {
-          *id = 3;
-          *ks = 2;
-        } else if (Kc <= 48) {
+          if (f32 || (M == 1 && Kc > 8) || (M == 2 && Kc > 32 && !token)) {
+            *id = 3;
+            *ks = 2;
+          }
+        } else if (Kc <= 48 && (f32 || Nt < 384 || (Kc > 40 && Nt > 512 && !token))) {
           *id = Nt <= 512 ? 5 : 2;
           *ks = 4;
         }
@@ -1169,11 +1182,11 @@ bool pick_gemv_fast(int64_t M, int64_t K, int64_t N, int xt, bool w8a8, bool xve
         *id = 8;
         *ks = 8;
       } else if (xb <= 32768) {
-        if (Nt >= 384) {
+        if (Nt >= (xt == XT_F32 && M == 1 ? 768 : 384)) {
           *id = 4;
           *ks = 4;
         }
-      } else if (xt != XT_F32 && Nt > 1536 && Nt <= 4096 && waves8 >= 5) {
+      } else if (xt != XT_F32 && Nt > 1536 && Nt <= 4096 && (token || Nt % 1280 > 640) && waves8 >= 5) {
         *id = 7;
         *ks = 8;
       }

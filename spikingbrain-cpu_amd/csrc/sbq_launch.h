@@ -60,7 +60,8 @@ struct GemvArgs;
 struct GemvSeg;
 void pick_gemv_s8(int64_t M, int64_t K, int64_t N, int* id, int* ks);
 bool gemv_quantize_first(int64_t M, int64_t K, int64_t N, int xt);
-bool pick_gemv_fast(int64_t M, int64_t K, int64_t N, int xt, bool w8a8, bool xvec, int* id, int* ks);
+bool pick_gemv_fast(int64_t M, int64_t K, int64_t N, int xt, bool w8a8, bool xvec, int* id, int* ks,
+                    bool token = false);
 int launch_gemv_fast_cfg(int id, int ks, const GemvArgs& a, int xt, bool w8a8, hipStream_t st);
 // Decode over several 16-row tiles of x (16 < M <= 64): weight-only on fp16 /
 // bf16 x, or int8-dyn on pre-quantized s8 rows (xt XT_S8).  gemm_alt: the

@@ -20,11 +20,11 @@ def dispatch(tmp_path_factory):
                     "-o", str(so)], check=True)
 
     def run(calls):
-        """[(status, [kernel name with template arguments, ...], [grid x, ...])] of the calls."""
+        """[(status, [kernel name with template arguments, ...], [(workgroups in x, threads of one), ...])]"""
         r = subprocess.run([sys.executable, str(HOST / "dispatch.py"), str(so), str(PKG / "libsbq.so"), str(PKG)],
                            input=json.dumps(calls), capture_output=True, text=True)
         assert r.returncode == 0, r.stderr
-        return [(t["rc"], [ln[0] for ln in t["launches"]], [ln[1][0] for ln in t["launches"]])
+        return [(t["rc"], [ln[0] for ln in t["launches"]], [(ln[1][0], ln[2][0]) for ln in t["launches"]])
                 for t in json.loads(r.stdout)]
 
     return run
@@ -85,7 +85,7 @@ def test_wide_grouped_int8_dyn_is_one_launch(dispatch):
                           (4, 5, 33000, 4096, "bf16")):
         c = {"op": "linear_w8a8_grouped", "M": M, "N": N, "K": K, "x": x, "count": n}
         (rc, names, grids), (rc1, names1, _) = dispatch([dict(c, ws=str(n)), dict(c, ws="base")])
-        assert rc == 0 and kernels(names) == ["quantize_small_kernel", "gemv_fast_kernel"] and grids[0] == n, (c, names)
+        assert rc == 0 and kernels(names) == ["quantize_small_kernel", "gemv_fast_kernel"] and grids[0][0] == n, (c, names)
         assert rc1 == 0 and kernels(names1) == ["gemv_fast_kernel"], (c, names1)
 
 
@@ -132,3 +132,40 @@ def test_small_activations_are_quantized_in_one_launch(dispatch):
                 continue  # within the fused capacity
             rc, names, _ = dispatch([c])[0]
             assert rc == 0 and kernels(names)[0] in want, (c, names)
+
+
+# (op, M, N, K, x, template of the GEMV: D, G, x in LDS, waves): both sides of
+# the lines between picks, where the other one was measured slower
+PICKS = [
+    ("linear_w8", 2, 97455, 4864, "f32", (4, 2, False, 4)), ("linear_w8", 2, 8000, 4864, "f32", (4, 2, True, 8)),
+    ("linear_w8", 2, 97455, 4096, "f32", (4, 2, True, 8)), ("linear_w8", 1, 97455, 4864, "f32", (4, 2, True, 8)),
+    ("linear_w8", 1, 10000, 1024, "f16", (8, 1, True, 2)), ("linear_w8", 1, 10000, 1536, "f16", (8, 1, True, 4)),
+    ("linear_w8", 1, 10000, 2560, "f16", (8, 1, True, 2)),
+    ("linear_w8a8", 1, 19456, 2560, "f16", (8, 1, False, 2)), ("linear_w8a8", 1, 19456, 384, "f16", (4, 2, False, 3)),
+    ("linear_w8a8", 2, 19456, 1024, "f16", (4, 2, False, 4)), ("linear_w8a8", 2, 19456, 2560, "f16", (8, 1, False, 2)),
+    ("linear_w8a8", 3, 60000, 1024, "bf16", (4, 2, False, 4)), ("linear_w8a8", 3, 60000, 1024, "f32", (8, 1, False, 2)),
+    ("linear_w8a8", 1, 12288, 1024, "f16", (4, 2, False, 4)), ("linear_w8a8", 1, 12288, 2688, "f16", (4, 1, False, 4)),
+    ("linear_w8a8", 1, 12288, 1024, "f32", (4, 1, False, 4)), ("linear_w8a8", 1, 5120, 1024, "f16", (8, 2, False, 4)),
+    ("linear_w8a8", 1, 7000, 1024, "f16", (4, 2, False, 4)), ("linear_w8a8", 1, 7000, 5248, "f32", (8, 1, True, 4)),
+    ("linear_w8a8", 1, 14000, 5248, "f32", (4, 2, False, 4)), ("linear_w8a8", 4, 25661, 5888, "f16", (4, 2, False, 8)),
+    ("linear_w8a8", 7, 36840, 3072, "f16", (2, 5, True, 8)), ("linear_w8a8_token", 7, 25661, 3072, "f16", (2, 5, True, 8)),
+    ("linear_w8a8_token", 2, 40000, 1024, "f16", (4, 2, False, 4)), ("linear_w8a8_token", 1, 12288, 2688, "f16", (4, 2, False, 4)),
+    ("linear_w8a8_token", 1, 40000, 1024, "bf16", (8, 1, False, 2)), ("linear_w8a8_token", 2, 40000, 1024, "f32", (8, 1, False, 2)),
+]
+
+
+def test_decode_picks_around_their_lines(dispatch):
+    for (op, M, N, K, x, want) in PICKS:
+        rc, names, dims = dispatch([{"op": op, "M": M, "N": N, "K": K, "x": x, "ws": "full"}])[0]
+        assert rc == 0 and kernels(names) == ["gemv_fast_kernel"], (op, M, N, K, x, names)
+        _, D, G, xl, *_ = [v.strip() for v in names[0].split("<")[1].split(">")[0].split(",")]
+        assert (int(D), int(G), xl == "true", dims[0][1] // 64) == want, (op, M, N, K, x, names, dims)
+
+
+def test_short_per_token_rows_are_quantized_first(dispatch):
+    """Up to four K tiles, beyond a dozen tiles of x: the row quantizer's launch."""
+    for M, Kc, first in ((3, 4, "gemv_fast_kernel"), (4, 4, "quantize_rows_sym_kernel"), (12, 1, "gemv_fast_kernel"),
+                         (13, 1, "quantize_rows_sym_kernel"), (16, 4, "quantize_rows_sym_kernel"), (3, 5, "gemv_fast_kernel")):
+        for x in ("f32", "f16"):
+            rc, names, _ = dispatch([{"op": "linear_w8a8_token", "M": M, "N": 4096, "K": 64 * Kc, "x": x, "ws": "full"}])[0]
+            assert rc == 0 and kernels(names)[0] == first and kernels(names)[-1] == "gemv_fast_kernel", (M, Kc, x, names)
