@@ -89,6 +89,12 @@ __device__ __forceinline__ u32x4 quant_w16(const WRaw<WT>& raw, float s, float i
   return o;
 }
 
+// Column sums that several workgroups add to start from zero.
+__global__ __launch_bounds__(256) void zero_ints_kernel(int32_t* __restrict__ out, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) out[i] = 0;
+}
+
 // One workgroup of 8 waves per 16 weight rows: lane (g, r) of wave v takes the
 // 16-value chunks of row r at columns 64 kc + 16 g, kc = v, v + 8, ..., the
 // chunk that is its 16 bytes of packed tile kc.  With a floating source each
@@ -103,7 +109,10 @@ __device__ __forceinline__ u32x4 quant_w16(const WRaw<WT>& raw, float s, float i
 // column-sum launch, with the int8 rows written and read twice between them):
 // bf16 9728 x 2560 112 -> 25 us, 24576 x 4096 407 -> 70 us (4.3 TB/s),
 // 151936 x 2560 1661 -> 237 us (4.9 TB/s); with the int8 rows kept 26 / 96 /
-// 302 us; fp32 9728 x 2560 135 -> 26; ragged bf16 9721 x 2555 101 -> 39.  16
+// 302 us; fp32 9728 x 2560 135 -> 26; ragged bf16 9721 x 2555 101 -> 39.  int8
+// rows alone, K over several workgroups where there are few row tiles (graph):
+// 16 x 65536 44 -> 3.6 us, 64 x 12288 10.3 -> 3.9, 300 x 9728 9.0 -> 4.4, with
+// their column sums 44 -> 6.4, 10.5 -> 5.5, 9.2 -> 6.1.  16
 // waves per workgroup: 20-45% slower except at K = 9728 (5% faster); holding
 // 24 chunks spilled (2560 x 9728: 74 us, re-reading 39).
 template <int WT, int C>
@@ -118,6 +127,9 @@ __global__ __launch_bounds__(512) void pack_weight_kernel(const uint8_t* __restr
   __shared__ int ssum[NW][16];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
   const int64_t nt = blockIdx.x, n = nt * 16 + r, Kc = (K + 63) / 64;
+  // int8 rows: K split over gridDim.y workgroups, their column sums added up
+  const int64_t share = FP ? Kc : (Kc + gridDim.y - 1) / gridDim.y;
+  const int64_t kb = FP ? 0 : blockIdx.y * share, ke = FP ? Kc : (kb + share < Kc ? kb + share : Kc);
   const uint8_t* row = n < N ? w + n * ldw * WRaw<WT>::ES : nullptr;
   WRaw<WT> v[C > 0 ? C : U];
   float s = 0.0f, inv = 0.0f;
@@ -190,13 +202,13 @@ __global__ __launch_bounds__(512) void pack_weight_kernel(const uint8_t* __restr
     for (int i = 0; i < C; ++i)
       if (wv + i * NW < Kc) emit(wv + i * NW, v[i]);
   } else {
-    for (int64_t kc = wv; kc < Kc; kc += U * NW) {
+    for (int64_t kc = kb + wv; kc < ke; kc += U * NW) {
 #pragma unroll
       for (int i = 0; i < U; ++i)
-        if (kc + i * NW < Kc) v[i].load(row, (kc + i * NW) * 64 + g * 16, K);
+        if (kc + i * NW < ke) v[i].load(row, (kc + i * NW) * 64 + g * 16, K);
 #pragma unroll
       for (int i = 0; i < U; ++i)
-        if (kc + i * NW < Kc) emit(kc + i * NW, v[i]);
+        if (kc + i * NW < ke) emit(kc + i * NW, v[i]);
     }
   }
   if (colsum) {  // uniform; exact int32: |sum| <= 127 * K
@@ -208,7 +220,10 @@ __global__ __launch_bounds__(512) void pack_weight_kernel(const uint8_t* __restr
       int t = 0;
 #pragma unroll
       for (int i = 0; i < NW; ++i) t += ssum[i][r];
-      colsum[n] = t;
+      if (!FP && gridDim.y > 1)
+        __hip_atomic_fetch_add(colsum + n, t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      else
+        colsum[n] = t;
     }
   }
 }
@@ -769,7 +784,17 @@ int launch_pack_weight(const void* w, int wt, int64_t N, int64_t K, int64_t ldw,
       else if (per <= 8) SBQ_PACK(XT_F32, 8);
       else SBQ_PACK(XT_F32, 0);
       break;
-    case XT_S8: SBQ_PACK(XT_S8, 0); break;
+    case XT_S8: {
+      // few row tiles of long rows: K over several workgroups, each with a round
+      // of K tiles at least; with column sums they start from zero, a launch more
+      const int64_t tiles = (N + 15) / 16, share = (512 + tiles - 1) / tiles;
+      const unsigned split = tiles >= 256 || (colsum && per <= 8) ? 1u : (unsigned)(share < per ? share : per);
+      if (colsum && split > 1)
+        hipLaunchKernelGGL(zero_ints_kernel, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, st, colsum, N);
+      hipLaunchKernelGGL((pack_weight_kernel<XT_S8, 0>), dim3((unsigned)tiles, split), block, 0, st, (const uint8_t*)w,
+                         N, K, ldw, scale, q, ldq, packed, colsum);
+      break;
+    }
     default: return -2;
   }
 #undef SBQ_PACK2

@@ -22,11 +22,14 @@ def call(L, c):
     (dtype), y (dtype, default f32); ws: "full" (sbq_linear_workspace_bytes),
     "base" (sbq_w8_workspace_bytes / sbq_w8a8_workspace_bytes), a number of
     base workspaces, or none; off: elements x starts beyond a 16-byte boundary;
-    pad: elements added to x's row stride; count: linears of a grouped call."""
+    pad: elements added to x's row stride; count: linears of a grouped call;
+    colsum: with column sums (repack_w8)."""
     P = ctypes.c_void_p
     at = lambda i: P((i + 1) << 40)  # noqa: E731
-    op, M, N, K = c["op"], c["M"], c["N"], c["K"]
+    op, M, N, K = c["op"], c.get("M", 0), c["N"], c["K"]
     x, y = c.get("x", "f32"), c.get("y", "f32")
+    if op == "repack_w8":
+        return L.sbq_repack_w8(at(0), N, K, K, at(1), at(4) if c.get("colsum") else None, None)
     dyn = "w8a8" in op
     xp = P(at(0).value + c.get("off", 0) * ESIZE[x])
     ldx = K + c.get("pad", 0)

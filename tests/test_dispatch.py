@@ -2,6 +2,7 @@
 the library's host code runs over a recorder in place of the HIP runtime, on
 made-up addresses that nothing reads."""
 import json
+import math
 import subprocess
 import sys
 from pathlib import Path
@@ -19,12 +20,13 @@ def dispatch(tmp_path_factory):
     subprocess.run(["g++", "-O1", "-shared", "-fPIC", "-std=c++17", "-Wall", str(HOST / "launch_trace.cpp"),
                     "-o", str(so)], check=True)
 
-    def run(calls):
-        """[(status, [kernel name with template arguments, ...], [(workgroups in x, threads of one), ...])]"""
+    def run(calls, axes=1):
+        """[(status, [kernel name with template arguments, ...], [(workgroups, threads of one), ...])]; the
+        workgroups counted along x, or over the given number of axes"""
         r = subprocess.run([sys.executable, str(HOST / "dispatch.py"), str(so), str(PKG / "libsbq.so"), str(PKG)],
                            input=json.dumps(calls), capture_output=True, text=True)
         assert r.returncode == 0, r.stderr
-        return [(t["rc"], [ln[0] for ln in t["launches"]], [(ln[1][0], ln[2][0]) for ln in t["launches"]])
+        return [(t["rc"], [ln[0] for ln in t["launches"]], [(math.prod(ln[1][:axes]), ln[2][0]) for ln in t["launches"]])
                 for t in json.loads(r.stdout)]
 
     return run
@@ -169,3 +171,18 @@ def test_short_per_token_rows_are_quantized_first(dispatch):
         for x in ("f32", "f16"):
             rc, names, _ = dispatch([{"op": "linear_w8a8_token", "M": M, "N": 4096, "K": 64 * Kc, "x": x, "ws": "full"}])[0]
             assert rc == 0 and kernels(names)[0] == first and kernels(names)[-1] == "gemv_fast_kernel", (M, Kc, x, names)
+
+
+def test_repack_spreads_few_long_rows(dispatch):
+    """A repack of few row tiles takes a workgroup of 8 waves for about every 8
+    tiles of K (16 rows of 65536 were one workgroup's serial walk); sums
+    along K start from a launch that clears them where K is split."""
+    calls = [{"op": "repack_w8", "N": N, "K": K, "colsum": cs} for cs in (False, True)
+             for N in (1, 16, 17, 64, 300, 1000, 4096, 9728) for K in (1, 64, 600, 4096, 4097, 12288, 65536)]
+    for c, (rc, names, grids) in zip(calls, dispatch(calls, axes=3)):
+        tiles, per = -(-c["N"] // 16), -(-(-(-c["K"] // 64)) // 8)
+        split = grids[-1][0] // tiles
+        assert rc == 0 and kernels(names)[-1] == "pack_weight_kernel" and grids[-1][0] % tiles == 0, (c, names)
+        assert kernels(names)[:-1] == (["zero_ints_kernel"] if c["colsum"] and split > 1 else []), (c, names)
+        if not c["colsum"] or per > 8:
+            assert split == 1 if tiles >= 256 else split == min(per, -(-512 // tiles)), (c, grids)

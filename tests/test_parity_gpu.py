@@ -124,6 +124,18 @@ def test_quantize_pack_one_pass(dev, dtype, N, K):
         assert torch.equal(q1, q) and torch.equal(s1, s) and torch.equal(quant.unpack(packed, N, K), q)
 
 
+@pytest.mark.parametrize("N,K", [(1, 577), (16, 4097), (17, 65536), (300, 9728), (1000, 4608), (4081, 4160)])
+def test_repack_of_few_long_rows(dev, N, K):
+    """K split over workgroups: tiles and (added up) column sums are the oracle's."""
+    announce(f"repack {N}x{K}")
+    q = torch.randint(-127, 128, (N, K), dtype=torch.int8, generator=torch.Generator().manual_seed(N + K))
+    packed, colsum = quant.repack(q.to(dev))
+    alone, _ = quant.repack(q.to(dev), with_colsum=False)
+    np.testing.assert_array_equal(packed.cpu().numpy(), oracle.pack_w8(q.numpy()))
+    assert torch.equal(alone, packed)
+    np.testing.assert_array_equal(colsum.cpu().numpy(), q.numpy().astype(np.int64).sum(1))
+
+
 # ---------------------------------------------------------------------------
 # int8 weight-only
 # ---------------------------------------------------------------------------
