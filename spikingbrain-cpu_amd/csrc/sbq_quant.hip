@@ -61,24 +61,28 @@ struct WRaw {
 // t = v * inv, inv = fp32(1 / s): |v| <= 127 s, so t is within 2.3e-5 of the
 // fp32 quotient (1.5 units of 2^-24 each, times 127) and both round alike
 // unless t is that close to a half.  Rounding by adding 1.5 * 2^23: the low
-// byte of the sum is the integer.  A chunk with a value near a half, an
-// infinity or a NaN takes the division.
+// byte of the sum is the integer.  A value near a half, an infinity or a NaN
+// takes the division, one by one: of bf16 values about one in 400 is half its
+// row's maximum (63.5), so most wavefronts hold one (dividing the whole chunk then
+// took 999 x 1001 10.7 us, one wave per row 6.4).
 template <int WT>
 __device__ __forceinline__ u32x4 quant_w16(const WRaw<WT>& raw, float s, float inv) {
   constexpr float kMagic = 12582912.0f;
   uint32_t m[16];
-  bool sure = true;
+  uint32_t unsure = 0;
 #pragma unroll
   for (int j = 0; j < 16; ++j) {
     const float t = raw.get(j) * inv, r = t + kMagic;
-    sure &= __builtin_fabsf(t - (r - kMagic)) < 0.49997f;
+    unsure |= __builtin_fabsf(t - (r - kMagic)) < 0.49997f ? 0u : 1u << j;
     m[j] = __float_as_uint(r);
   }
-  if (!sure) {
+  if (unsure) {
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
-      const float t = __builtin_rintf(raw.get(j) / s);
-      m[j] = (uint32_t)(int)fminf(fmaxf(t, -127.0f), 127.0f);
+      if (unsure & (1u << j)) {
+        const float t = __builtin_rintf(raw.get(j) / s);
+        m[j] = (uint32_t)(int)fminf(fmaxf(t, -127.0f), 127.0f);
+      }
     }
   }
   u32x4 o;
@@ -87,6 +91,33 @@ __device__ __forceinline__ u32x4 quant_w16(const WRaw<WT>& raw, float s, float i
     o[i] = __builtin_amdgcn_perm(m[4 * i + 1], m[4 * i], 0x0c0c0400u) |
            __builtin_amdgcn_perm(m[4 * i + 3], m[4 * i + 2], 0x04000c0cu);
   return o;
+}
+
+// quantize_per_channel of few short rows of 2-byte values, nothing packed: one
+// wavefront per row, a division per value.  A few rows leave the kernel below
+// few workgroups, its 16-byte loads of rows at odd 2-byte addresses take
+// several passes each, and near-half quotients are frequent in bf16.  That
+// kernel / this one (bf16, graph): 999 x 1001 8.7 / 6.4 us, 1000 x 2001 13.5 /
+// 10.0, 1000 x 1000 7.2 / 6.4; on the other side of the line 4000 x 2001 14.7 /
+// 19.3, 2560 x 2501 17.0 / 20.4, 1000 x 2000 9.2 / 9.9, 128 x 2560 10.1 / 11.3.
+template <int WT>
+__global__ __launch_bounds__(256) void quantize_few_rows_kernel(const void* __restrict__ wv, int64_t N, int64_t K,
+                                                                int64_t ldw, int8_t* __restrict__ q, int64_t ldq,
+                                                                float* __restrict__ scale) {
+  typedef typename XElem<WT>::T T;
+  const int lane = threadIdx.x & 63;
+  const int64_t n = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (n >= N) return;
+  const T* row = (const T*)wv + n * ldw;
+  float m = 0.0f;
+  for (int64_t k = lane; k < K; k += 64) m = fmaxf(m, __builtin_fabsf(XElem<WT>::to_f32(row[k])));
+  m = wave_max(m);
+  const float s = fmaxf(m, 1e-8f) / 127.0f;
+  if (lane == 0) scale[n] = s;
+  for (int64_t k = lane; k < K; k += 64) {
+    const float t = __builtin_rintf(XElem<WT>::to_f32(row[k]) / s);
+    q[n * ldq + k] = (int8_t)(int)fminf(fmaxf(t, -127.0f), 127.0f);
+  }
 }
 
 // Column sums that several workgroups add to start from zero.
@@ -764,6 +795,14 @@ __global__ __launch_bounds__(256) void argmax_index_kernel(unsigned long long* _
 // ---------------------------------------------------------------------------
 int launch_pack_weight(const void* w, int wt, int64_t N, int64_t K, int64_t ldw, float* scale, int8_t* q, int64_t ldq,
                        uint8_t* packed, int32_t* colsum, hipStream_t st) {
+  if (!packed && N <= 2048 && (wt == XT_F16 || wt == XT_BF16) && (K <= 1024 || (((uintptr_t)w | ldw * 2) & 2))) {
+    const dim3 rows((unsigned)((N + 3) / 4));
+    if (wt == XT_F16)
+      hipLaunchKernelGGL((quantize_few_rows_kernel<XT_F16>), rows, dim3(256), 0, st, w, N, K, ldw, q, ldq, scale);
+    else
+      hipLaunchKernelGGL((quantize_few_rows_kernel<XT_BF16>), rows, dim3(256), 0, st, w, N, K, ldw, q, ldq, scale);
+    return check_launch();
+  }
   const dim3 grid((unsigned)((N + 15) / 16)), block(512);
   const int64_t per = ((K + 63) / 64 + 7) / 8;  // chunks per lane
 #define SBQ_PACK(WT_, C_) \

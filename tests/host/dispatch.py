@@ -30,6 +30,8 @@ def call(L, c):
     x, y = c.get("x", "f32"), c.get("y", "f32")
     if op == "repack_w8":
         return L.sbq_repack_w8(at(0), N, K, K, at(1), at(4) if c.get("colsum") else None, None)
+    if op == "quantize_per_channel":
+        return L.sbq_quantize_per_channel(at(0), DT[x], N, K, K, at(1), K, at(2), None)
     dyn = "w8a8" in op
     xp = P(at(0).value + c.get("off", 0) * ESIZE[x])
     ldx = K + c.get("pad", 0)

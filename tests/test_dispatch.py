@@ -186,3 +186,14 @@ def test_repack_spreads_few_long_rows(dispatch):
         assert kernels(names)[:-1] == (["zero_ints_kernel"] if c["colsum"] and split > 1 else []), (c, names)
         if not c["colsum"] or per > 8:
             assert split == 1 if tiles >= 256 else split == min(per, -(-512 // tiles)), (c, grids)
+
+
+def test_quantize_few_rows_takes_a_wave_each(dispatch):
+    """Few short rows of 2-byte values, or at odd 2-byte addresses, quantized
+    alone: four rows per workgroup; else sixteen."""
+    calls = [{"op": "quantize_per_channel", "N": N, "K": K, "x": x} for x in ("f32", "f16", "bf16")
+             for N in (1, 16, 999, 2048, 2049) for K in (1, 64, 1000, 1001, 1024, 1026, 2001, 2500)]
+    for c, (rc, names, grids) in zip(calls, dispatch(calls)):
+        few = c["x"] != "f32" and c["N"] <= 2048 and (c["K"] <= 1024 or c["K"] % 2)
+        assert rc == 0 and kernels(names) == ["quantize_few_rows_kernel" if few else "pack_weight_kernel"], (c, names)
+        assert grids[0][0] == -(-c["N"] // (4 if few else 16)), (c, grids)

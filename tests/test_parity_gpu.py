@@ -136,6 +136,26 @@ def test_repack_of_few_long_rows(dev, N, K):
     np.testing.assert_array_equal(colsum.cpu().numpy(), q.numpy().astype(np.int64).sum(1))
 
 
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("N,K", [(1, 1), (5, 63), (2048, 65), (3, 1024), (7, 2001), (2048, 1027), (6, 12289)])
+def test_quantize_few_rows(dev, dtype, N, K):
+    """A wavefront per row: bit-equal to the oracle and to the one pass with the packing, an all-zero row and
+    rows of inf and NaN included."""
+    announce(f"quantize rows {dtype} {N}x{K}")
+    w = make_weights(N, K, N * K).to(DT[dtype])
+    if N > 4:
+        w[1] = 0
+    q, s = quant.quantize_per_channel_gpu(w.to(dev))
+    qo, so = oracle.quantize_per_channel_c(w.float().numpy())
+    np.testing.assert_array_equal(q.cpu().numpy(), qo)
+    np.testing.assert_array_equal(s.cpu().numpy(), so)
+    if N > 4:
+        w[2, K // 2], w[3, K // 3] = float("inf"), float("nan")
+    q, s = quant.quantize_per_channel_gpu(w.to(dev))
+    q2, s2, _, _ = quant._quantize_pack(w.to(dev), True, False)
+    assert torch.equal(q, q2) and torch.equal(s.view(torch.int32), s2.view(torch.int32))
+
+
 # ---------------------------------------------------------------------------
 # int8 weight-only
 # ---------------------------------------------------------------------------
