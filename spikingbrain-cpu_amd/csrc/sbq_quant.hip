@@ -968,10 +968,11 @@ int launch_quantize_rows_sym(const void* x, int xt, int64_t ldx, bool xvec, int6
 }
 
 int launch_argmax_rows(const float* y, int64_t M, int64_t N, int64_t ldy, int64_t* out, hipStream_t st) {
-  // rows that one workgroup takes several rounds of loads for (N = 8192: 8.6 us
-  // in one launch), until the rows alone fill the chip (V = 151936, 256 rows:
-  // 51.3 us in one launch, 52.1 in three; 64 rows 47.6 and 27.8)
-  if (N > 4096 && M <= 128) {
+  // rows that one workgroup takes several rounds of loads for (N = 8192, one
+  // launch / three: 8.7 us / 6.0 in a graph, 8.7 / 8.5 eager, where the host's
+  // launches count; N = 5000 8 / 6 and 7.6 / 8.5), until the rows alone fill the
+  // chip (V = 151936, 256 rows: 51.3 us / 52.1; 64 rows 47.6 / 27.8)
+  if (N >= 8192 && M <= 128) {
     unsigned long long* keys = (unsigned long long*)out;
     const int G = (int)min((N + 2047) / 2048, (int64_t)64), per = (int)((N + G - 1) / G);
     const dim3 rows((unsigned)((M + 255) / 256)), block(256);

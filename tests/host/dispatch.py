@@ -26,10 +26,12 @@ def call(L, c):
     colsum: with column sums (repack_w8)."""
     P = ctypes.c_void_p
     at = lambda i: P((i + 1) << 40)  # noqa: E731
-    op, M, N, K = c["op"], c.get("M", 0), c["N"], c["K"]
+    op, M, N, K = c["op"], c.get("M", 0), c["N"], c.get("K", 0)
     x, y = c.get("x", "f32"), c.get("y", "f32")
     if op == "repack_w8":
         return L.sbq_repack_w8(at(0), N, K, K, at(1), at(4) if c.get("colsum") else None, None)
+    if op == "argmax_rows":
+        return L.sbq_argmax_rows(at(0), M, N, N, at(1), None)
     if op == "quantize_per_channel":
         return L.sbq_quantize_per_channel(at(0), DT[x], N, K, K, at(1), K, at(2), None)
     dyn = "w8a8" in op

@@ -197,3 +197,11 @@ def test_quantize_few_rows_takes_a_wave_each(dispatch):
         few = c["x"] != "f32" and c["N"] <= 2048 and (c["K"] <= 1024 or c["K"] % 2)
         assert rc == 0 and kernels(names) == ["quantize_few_rows_kernel" if few else "pack_weight_kernel"], (c, names)
         assert grids[0][0] == -(-c["N"] // (4 if few else 16)), (c, grids)
+
+
+def test_row_argmax_below_8192_values_is_one_launch(dispatch):
+    """Three launches cost the host more than one row of fewer values gains."""
+    calls = [{"op": "argmax_rows", "M": M, "N": N} for M in (1, 8, 128, 129) for N in (1, 4096, 4097, 8191, 8192, 151936)]
+    for c, (rc, names, _) in zip(calls, dispatch(calls)):
+        want = 3 if c["N"] >= 8192 and c["M"] <= 128 else 1
+        assert rc == 0 and len(names) == want and all("argmax" in n for n in names), (c, names)
