@@ -212,8 +212,10 @@ int64_t sbq_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int x_dtype,
 int sbq_gemm_config(int64_t M, int64_t N, int64_t K, int x_dtype, int w8a8, int* splits);
 
 /* The general decode GEMV's configuration for an [M, K] input of x_dtype
- * (the kernel that runs ragged K, misaligned rows and 17..32 tokens on the
- * layers the row-tile GEMV leaves): info[0..8] = supported (0 / 1), row
+ * (weight-only: the kernel that runs misaligned rows and ragged K where
+ * padding the rows does not pay, and 17..32 tokens on the layers the
+ * row-tile GEMV leaves; int8-dyn: 17..32 tokens alone, since up to 16 never
+ * reach it and report unsupported): info[0..8] = supported (0 / 1), row
  * tiles of x, weight tiles per group, K tiles per wave, waves per
  * workgroup, activation mode (0 registers, 1 LDS, 2 chunks), staging
  * chunks per thread, LDS bytes, and whether a kernel instance exists for

@@ -38,6 +38,8 @@ namespace sbq {
 //   XM_LDS   the workgroup stages x[M][K] in LDS once; fragments are read on use
 //   XM_CHUNK fragments are re-read from global memory (L2) per group, XC K tiles
 //            at a time (for x too large for LDS; used with NB = 1)
+// W8A8 runs here with two row tiles of x in registers alone (17 <= M <= 32):
+// up to 16 rows go to gemv_fast_kernel, of any K and alignment.
 // In every mode the first activation loads are issued before the weight loads:
 // loads retire in order, so waiting for them never waits for the weights.
 // ---------------------------------------------------------------------------
@@ -94,18 +96,14 @@ __device__ __forceinline__ void load_x_frags(const GemvArgs& a, int kb, int p0, 
 // Multiply-accumulate one K tile of every weight tile of the group.
 template <int XT, int MT, int G, bool W8A8, typename Acc>
 __device__ __forceinline__ void mma_ktile(const u32x4 (&wk)[G], const XRaw<XT> (&xf)[MT], const i32x4* xq,
-                                          int nt0, int Nt, const GemvArgs& a, int lane, int k0, const ActQParams& qp,
-                                          Acc (&acc)[G][MT]) {
+                                          int nt0, int Nt, Acc (&acc)[G][MT]) {
 #pragma unroll
   for (int t = 0; t < G; ++t) {
     if (nt0 + t >= Nt) continue;
     if constexpr (W8A8) {
       const i32x4 ws = tile_to_s8(wk[t]);
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        const i32x4 q = xq ? xq[mt] : quant_frag<XT>(xf[mt], a.M, a.K, mt * 16 + (lane & 15), k0, qp.inv, qp.zpf);
-        acc[t][mt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ws, q, acc[t][mt], 0, 0, 0);
-      }
+      for (int mt = 0; mt < MT; ++mt) acc[t][mt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ws, xq[mt], acc[t][mt], 0, 0, 0);
     } else {
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) tile_mma<XT>(wk[t], xf[mt], acc[t][mt]);
@@ -191,12 +189,12 @@ __device__ __forceinline__ void process_group(const GemvArgs& a, int grp, int kb
 #pragma unroll
     for (int t = 0; t < G; ++t) wk[t] = w[t][p];
     if constexpr (XM == XM_REG) {
-      mma_ktile<XT, MT, G, W8A8>(wk, xr[p], W8A8 ? xq[p] : nullptr, nt0, a.Nt, a, lane, kc * 64 + g * 16, qp, acc);
+      mma_ktile<XT, MT, G, W8A8>(wk, xr[p], xq[p], nt0, a.Nt, acc);
     } else if constexpr (XM == XM_LDS) {
       XRaw<XT> xf[MT];
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) xf[mt].load_lds(xl, Kp, a.M, mt * 16 + r, kc * 64 + g * 16);
-      mma_ktile<XT, MT, G, W8A8>(wk, xf, nullptr, nt0, a.Nt, a, lane, kc * 64 + g * 16, qp, acc);
+      mma_ktile<XT, MT, G, false>(wk, xf, nullptr, nt0, a.Nt, acc);
     }
   }
   reduce_store<G, MT, W8A8>(a, grp, lane, acc, e, qp, red);
@@ -205,12 +203,10 @@ __device__ __forceinline__ void process_group(const GemvArgs& a, int grp, int kb
 // XM_CHUNK: the wave's P K tiles run as a pipeline of XC-tile sub-chunks; the
 // activations (re-read from L2 per group) and weight tiles of sub-chunk c+1
 // are loaded while sub-chunk c is multiplied.
-template <int XT, int MT, int G, int P, bool W8A8, int XC>
+template <int XT, int MT, int G, int P, int XC>
 __device__ __forceinline__ void process_group_chunked(const GemvArgs& a, int grp, int kb, int lane,
-                                                      const EpiVals& e, const ActQParams& qp, void* red) {
-  typedef typename std::conditional<W8A8, i32x4, f32x4>::type Acc;
+                                                      const EpiVals& e, void* red) {
   constexpr int NCH = (P + XC - 1) / XC;
-  const int g = lane >> 4;
   const int nt0 = grp * G;
   XRaw<XT> xc[2][XC][MT];
   u32x4 wc[2][G][XC];
@@ -225,27 +221,27 @@ __device__ __forceinline__ void process_group_chunked(const GemvArgs& a, int grp
           wc[b][t][j] = load_tile_nt(a.packed + ((int64_t)nt * a.Kc + kb + p) * 1024 + lane * 16);
       }
   };
-  Acc acc[G][MT];
+  f32x4 acc[G][MT];
 #pragma unroll
   for (int t = 0; t < G; ++t)
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) acc[t][mt] = Acc{0, 0, 0, 0};
+    for (int mt = 0; mt < MT; ++mt) acc[t][mt] = f32x4{0, 0, 0, 0};
   load_chunk(0, 0);
 #pragma unroll
   for (int c = 0; c < NCH; ++c) {
     if (c + 1 < NCH) load_chunk(c + 1, (c + 1) & 1);
 #pragma unroll
     for (int j = 0; j < XC; ++j) {
-      const int p = c * XC + j, kc = kb + p;
-      if (p >= P || kc >= a.Kc) continue;
+      const int p = c * XC + j;
+      if (p >= P || kb + p >= a.Kc) continue;
       u32x4 wk[G];
 #pragma unroll
       for (int t = 0; t < G; ++t) wk[t] = wc[c & 1][t][j];
-      mma_ktile<XT, MT, G, W8A8>(wk, xc[c & 1][j], nullptr, nt0, a.Nt, a, lane, kc * 64 + g * 16, qp, acc);
+      mma_ktile<XT, MT, G, false>(wk, xc[c & 1][j], nullptr, nt0, a.Nt, acc);
     }
     __builtin_amdgcn_sched_barrier(0);
   }
-  reduce_store<G, MT, W8A8>(a, grp, lane, acc, e, qp, red);
+  reduce_store<G, MT, false>(a, grp, lane, acc, e, ActQParams{}, red);
 }
 
 template <int XT, int MT, int G, int P, bool W8A8, int XM, int NB, int SC = kStageChunks>
@@ -256,6 +252,7 @@ __global__ __launch_bounds__(1024) void gemv_kernel(const GemvArgs a) {
   constexpr int XC = XT == XT_F32 ? 1 : 2;                           // XM_CHUNK sub-chunk (K tiles)
   constexpr int XR = XM == XM_REG ? P : 1;
   constexpr int XSZ = x_bytes<XT>();
+  static_assert(!W8A8 || XM == XM_REG, "W8A8 holds x in registers");
   static_assert(XM != XM_CHUNK || NB == 1, "chunked activations reload per group: one weight buffer");
   const int nw = blockDim.x >> 6;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -346,19 +343,17 @@ __global__ __launch_bounds__(1024) void gemv_kernel(const GemvArgs a) {
     }
     __syncthreads();
     qp = choose_act_qparams(mn, mx);
-    if constexpr (XM == XM_REG) {
-      const int r = lane & 15, g = lane >> 4;
+    const int r = lane & 15, g = lane >> 4;
 #pragma unroll
-      for (int p = 0; p < P; ++p)
+    for (int p = 0; p < P; ++p)
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-          xq[p][mt] = quant_frag<XT>(xr[p][mt], a.M, a.K, mt * 16 + r, (kb + p) * 64 + g * 16, qp.inv, qp.zpf);
-    }
+      for (int mt = 0; mt < MT; ++mt)
+        xq[p][mt] = quant_frag<XT>(xr[p][mt], a.M, a.K, mt * 16 + r, (kb + p) * 64 + g * 16, qp.inv, qp.zpf);
   }
 
   if constexpr (XM == XM_CHUNK) {
     while (true) {
-      process_group_chunked<XT, MT, G, P, W8A8, XC>(a, grp, kb, lane, ebuf[0], qp, red);
+      process_group_chunked<XT, MT, G, P, XC>(a, grp, kb, lane, ebuf[0], red);
       grp += gridDim.x;
       if (grp >= a.ngroups) break;
       load_epi<G, MT, W8A8>(a, grp, ebuf[0]);
@@ -407,7 +402,7 @@ struct GemvCfg {
 static GemvCfg pick_gemv(int64_t M, int64_t Nt, int64_t Kc, bool w8a8, int xt) {
   (void)Nt;
   GemvCfg c{};
-  if (M > 32 || Kc > 192) return c;
+  if (M > 32 || Kc > 192 || (w8a8 && M <= 16)) return c;
   c.mt = M <= 16 ? 1 : 2;
   c.p = Kc <= 8 ? (Kc <= 1 ? 1 : (Kc <= 2 ? 2 : (Kc <= 4 ? 4 : 8))) : (Kc <= 128 ? 8 : 12);
   c.waves = (int)((Kc + c.p - 1) / c.p);
@@ -443,7 +438,9 @@ static GemvCfg pick_gemv(int64_t M, int64_t Nt, int64_t Kc, bool w8a8, int xt) {
 
 bool gemv_supports(int64_t M, int64_t K, bool w8a8, int xt) {
   if (M < 1) return false;
-  return pick_gemv(M, 1, (K + 63) / 64, w8a8, xt).ok;
+  const int64_t Kc = (K + 63) / 64;
+  if (w8a8 && M <= 16) return Kc <= 192;  // gemv_fast_kernel, on quantized rows where x itself does not suit it
+  return pick_gemv(M, 1, Kc, w8a8, xt).ok;
 }
 
 // Forward declaration: the instance table below decides whether a picked
@@ -498,8 +495,9 @@ int gemv_config_info(int64_t M, int64_t K, bool w8a8, int xt, int32_t* info) {
 // Instances pick_gemv can select for an activation type / format.
 template <int XT, bool W8A8, int MT, int P, int XM>
 constexpr bool gemv_instance_used() {
-  if (XM == XM_REG) return P <= (XT == XT_F32 ? 1 : (W8A8 ? 2 : 4));
-  if (XM == XM_CHUNK) return MT == 1 && P > (XT == XT_F32 ? 1 : (W8A8 ? 2 : 4));
+  if (W8A8) return MT == 2 && XM == XM_REG && P <= (XT == XT_F32 ? 1 : 2);
+  if (XM == XM_REG) return P <= (XT == XT_F32 ? 1 : 4);
+  if (XM == XM_CHUNK) return MT == 1 && P > (XT == XT_F32 ? 1 : 4);
   return MT == 1;
 }
 
@@ -639,9 +637,8 @@ int launch_gemv_w8a8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, b
                      const float* scale, const int32_t* colsum, const float* bias, int64_t N, void* y, int yt,
                      int64_t ldy, int32_t* acc_out, float2* partials, int8_t* xq, float* qpbuf, hipStream_t st,
                      bool yvec, GemvArgmaxOut* am, const u32x2* parts) {
+  if (!gemv_supports(M, K, true, xt)) return -1;
   const int64_t Nt = (N + 15) / 16, Kc = (K + 63) / 64;
-  const GemvCfg c = pick_gemv(M, Nt, Kc, true, xt);
-  if (!c.ok) return -1;
   GemvArgs a{};
   a.x = x; a.ldx = ldx; a.M = (int)M; a.K = (int)K; a.Kc = (int)Kc;
   a.packed = packed; a.scale = scale; a.bias = bias; a.colsum = colsum;
@@ -668,6 +665,7 @@ int launch_gemv_w8a8(const void* x, int xt, int64_t M, int64_t K, int64_t ldx, b
     if (am) am->fused = rc == 0 && (f.flags & kGemvArgmax);
     return rc;
   }
+  const GemvCfg c = pick_gemv(M, Nt, Kc, true, xt);
   const int np = minmax_nparts(M, K);
   int rc = launch_minmax_partials(x, xt, M, K, ldx, partials, np, st);
   if (rc) return rc;

@@ -304,6 +304,19 @@ def test_general_gemv_configurations_are_launchable(lib):
     assert lib.sbq_gemv_config(1, 64, 1, 0, None) == -1
 
 
+def test_general_gemv_runs_int8_dyn_from_17_tokens(lib):
+    """Up to 16 tokens of int8-dyn never reach the general GEMV: no
+    configuration is reported for them, nor one without a kernel beyond."""
+    info = (ctypes.c_int32 * 9)()
+    for dt in (0, 1, 2):
+        for M in range(1, 33):
+            for K in (1, 63, 64, 130, 1000, 1024, 1025, 2048, 2049, 4096, 12288, 12289):
+                assert lib.sbq_gemv_config(M, K, dt, 1, info) == 0
+                want = M > 16 and K <= (1024 if dt == 0 else 2048)
+                assert (info[0], info[8]) == (want, want), (M, K, dt, list(info))
+                assert not want or (info[1], info[5]) == (2, 0), (M, K, dt, list(info))
+
+
 @pytest.mark.parametrize("lang,std", [("c", "c99"), ("c++", "c++17")])
 def test_header_compiles_standalone(tmp_path, lang, std):
     """include/sbq.h is a plain C interface: it compiles on its own as C99 and
