@@ -301,7 +301,7 @@ def lm_head_greedy_bench(ctx, V=151936, K=4096, M=1, steps=40, warmup=5):
 def sample_bench(ctx, V=151936, M=1, steps=40, warmup=5):
     """The engine's non-greedy sampling step (engine.py:29-42) over one row of
     lm_head logits (fp32, N(0, 2.5)), with the logits left on the GPU:
-    sbq_sample_rows (two-level cuts, no sort) for the engine's default
+    sbq_sample_rows (cuts by bins, no sort) for the engine's default
     parameters (temperature 0.7, top_p 0.9), with top-k 50 as well, and with
     neither; beside it the reference's expression run by torch's own GPU ops
     (division, topk, softmax, sort, cumsum, scatter, multinomial with a GPU

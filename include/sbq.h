@@ -117,24 +117,29 @@ int sbq_unpack_w8(const uint8_t* packed, int64_t N, int64_t K, int8_t* q, int64_
  * x: device [M, K] (row stride ldx), dtype F32, F16 or BF16.
  *    F16/BF16 inputs are used exactly (BF16 staged for the prefill GEMM: exact
  *    down to 2^28 below each row's maximum).  F32 inputs: on the decode paths
- *    (M <= 16, and the general GEMV up to 32 tokens) split into bf16 hi +
- *    remainder (relative representation error <= 2^-16); on the staged prefill
- *    path one fp16 plane of the row scaled by a power of two (11 significant
- *    bits: about 3e-4 relative L2 on the outputs).
+ *    (M <= 16, and the general GEMV up to 32 tokens) and on every path of a
+ *    ragged K split into bf16 hi + remainder (relative representation error
+ *    <= 2^-16); on the staged prefill path of 64 | K one fp16 plane of the row
+ *    scaled by a power of two (11 significant bits: about 3e-4 relative L2 on
+ *    the outputs).
  * packed: from sbq_repack_w8.  scale: device fp32 [N].  bias: device fp32 [N]
  * or NULL.  y: device [M, N] (row stride ldy), dtype F32, F16 or BF16.
  * Accumulation is fp32.  Routes (16-byte aligned rows, 64 | K): M <= 16 the
  * HBM-streaming MFMA GEMV; 16 < M <= 64 the row-tile GEMV on narrow layers
  * (N <= 4096 with little x to read, or wherever the workspace below is
- * missing), else the LDS-tiled MFMA GEMM; other shapes up to 32 tokens the
- * general GEMV.
+ * missing), else the LDS-tiled MFMA GEMM.  Ragged K (K % 64 != 0), with the
+ * workspace below: x copied to rows of whole tiles, then the GEMV (M <= 16) or
+ * the tiled GEMM on those, up to 32 tokens only where that pays (longer K and
+ * wider layers); what is left up to 32 tokens, and misaligned rows of whole
+ * tiles, the general GEMV.
  * workspace: optional (NULL, 0 is valid).  With >= sbq_w8_workspace_bytes(M,
- * K, x_dtype) bytes the prefill GEMM (K % 64 == 0, aligned rows) runs its
- * fastest path: F16 x with per-row sums from a pre-pass; BF16 / F32 x staged
- * as a power-of-two scaled fp16 plane for the same fp16 MFMA kernel; with
+ * K, x_dtype) bytes the prefill GEMM runs its fastest path: F16 x with per-row
+ * sums from a pre-pass; BF16 / F32 x staged as a power-of-two scaled fp16 plane
+ * for the same fp16 MFMA kernel (aligned rows, 64 | K); ragged K as above, in
+ * x's own dtype or (F32) bf16 high and remainder planes.  With
  * sbq_linear_workspace_bytes it also splits K over workgroups on small grids.
- * Without it, F16 / BF16 run a slower tiled GEMM and F32 the register-staged
- * bf16 hi + lo GEMM. */
+ * Without it, F16 / BF16 run a slower tiled GEMM and F32 and ragged K a
+ * register-staged one. */
 int sbq_linear_w8(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
                   const uint8_t* packed, const float* scale, const float* bias, int64_t N,
                   void* y, int y_dtype, int64_t ldy,
@@ -168,7 +173,8 @@ int sbq_linear_w8_parts(const void* x, int x_dtype, int64_t M, int64_t K, int64_
  * K % 64 == 0, 16-byte aligned x rows) the linears run as one GEMV launch:
  * the launch ramp and tail of a small projection are paid once per group
  * (two 4096 x 4096 projections of different inputs: 2 x 5.1 us -> 7.5 us).
- * Otherwise each runs as sbq_linear_w8 without a workspace.  Results may differ
+ * Otherwise each runs as sbq_linear_w8 without a workspace (a caller that has
+ * one is faster with separate calls for ragged K and M > 16).  Results may differ
  * from separate sbq_linear_w8 calls in the fp32 summation order (the group is
  * tiled as one layer of its summed rows).  No counterpart in the reference:
  * it is for callers holding several independent projections of one step
@@ -181,9 +187,11 @@ int sbq_linear_w8_grouped(int count, const void* const* x, const int64_t* ldx, i
                           void* const* y, const int64_t* ldy, int y_dtype, void* stream);
 
 /* Workspace bytes that let sbq_linear_w8 run its fastest prefill path for an
- * [M, K] input of x_dtype: 2 * M floats, plus M * K * 2 bytes of staged
- * activations for BF16 and F32 x, plus alignment slack.  0 for a
- * bad argument.  No counterpart in the reference (its CPU matmul needs no
+ * [M, K] input of x_dtype, and ragged K (K % 64 != 0) as rows of whole tiles:
+ * 2 * M floats, plus the staged activations, plus alignment slack.  Staged are
+ * BF16 and F32 x of 64 | K, M * K * 2 bytes, and every ragged x, M *
+ * ceil(K/64)*64 elements of 2 bytes (F16, BF16) or 4 (F32).  0 for a bad
+ * argument.  No counterpart in the reference (its CPU matmul needs no
  * scratch). */
 int64_t sbq_w8_workspace_bytes(int64_t M, int64_t K, int x_dtype);
 
@@ -228,8 +236,9 @@ int sbq_gemv_config(int64_t M, int64_t K, int x_dtype, int w8a8, int32_t* info);
 
 /* Workspace bytes sbq_linear_w8a8 / sbq_act_qparams need for an [M, K] input:
  * 2.5 KiB of activation statistics plus M * ceil(K/64)*64 bytes for the
- * quantized activations of the paths with a quantize pre-pass (M > 16), M floats of per-token
- * scales (sbq_linear_w8a8_token), plus alignment slack. */
+ * quantized activations of the paths with a quantize pre-pass (M > 16, ragged
+ * or misaligned x, and decode inputs beyond what the GEMV quantizes itself), M
+ * floats of per-token scales (sbq_linear_w8a8_token), plus alignment slack. */
 int64_t sbq_w8a8_workspace_bytes(int64_t M, int64_t K);
 
 /* The activation quantization parameters that fbgemm's dynamic linear chooses
@@ -285,8 +294,10 @@ int sbq_linear_w8a8_parts(const void* x, int x_dtype, int64_t M, int64_t K, int6
  * in sbq_linear_w8_grouped, plus host arrays of the column sums (required)
  * and one workspace of >= sbq_w8a8_workspace_bytes(M, K) bytes.  For decode
  * shapes whose x fits the fused GEMV (each workgroup reduces its linear's
- * min/max itself) the linears run as one launch; otherwise one by one as
- * sbq_linear_w8a8, sharing the workspace in stream order.  Bit-exact with
+ * min/max itself) the linears run as one launch; larger decode inputs, given
+ * `count` times those bytes, as two: every input quantized into its own share,
+ * then one GEMV; otherwise one by one as sbq_linear_w8a8, sharing the
+ * workspace in stream order.  Bit-exact with
  * separate calls (integer accumulation).  No counterpart in the reference:
  * it is for callers holding several independent int8-dyn projections of one
  * step (model.py: the two lora up-projections, the SSE and SWA output
@@ -330,9 +341,12 @@ int sbq_linear_w8a8_noalloc(const void* x, int x_dtype, int64_t M, int64_t K, in
  *   xq[m,k] = clamp(rne(x[m,k] / s_t[m]), -127, 127)
  *   acc[m,n] = sum_k xq[m,k] * q[n,k]            (int32, exact; acc_out nullable)
  *   y[m,n] = fp32(acc) * fp32(s_t[m] * scale[n]) (with a bias: one fma)
- * workspace: >= sbq_w8a8_workspace_bytes(M, K) bytes.  The row quantizer runs
- * first; then M <= 16 runs the HBM-streaming int8 MFMA GEMV on the s8 rows,
- * larger M the tiled int8 MFMA GEMM. */
+ * workspace: >= sbq_w8a8_workspace_bytes(M, K) bytes; with
+ * sbq_linear_workspace_bytes the GEMM splits K over workgroups on small grids.
+ * Small decode inputs are quantized in the HBM-streaming int8 MFMA GEMV itself;
+ * otherwise the row quantizer runs first, then that GEMV on the s8 rows (M <=
+ * 16), the row-tile GEMV on narrow layers (M <= 64) or the tiled int8 MFMA
+ * GEMM. */
 int sbq_linear_w8a8_token(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
                           const uint8_t* packed, const float* scale, const float* bias, int64_t N,
                           void* y, int y_dtype, int64_t ldy, int32_t* acc_out,

@@ -360,9 +360,9 @@ __global__ __launch_bounds__(kFastMaxWaves * 64) void gemv_fast_kernel(GemvArgs 
 #pragma unroll
       for (int i = 0; i < FC; ++i) {
         if (i * (int)blockDim.x >= xm_nch) {
-        if constexpr (FC > kFusedChunks) continue;  // a break moves xmm to scratch
-        else break;
-      }
+          if constexpr (FC > kFusedChunks) continue;  // a break moves xmm to scratch
+          else break;
+        }
         constexpr int NE = 16 / EB;
 #pragma unroll
         for (int j = 0; j < NE; ++j) {
@@ -393,9 +393,9 @@ __global__ __launch_bounds__(kFastMaxWaves * 64) void gemv_fast_kernel(GemvArgs 
 #pragma unroll
         for (int i = 0; i < FC; ++i) {
           if (i * (int)blockDim.x >= xm_nch) {
-        if constexpr (FC > kFusedChunks) continue;  // a break moves xmm to scratch
-        else break;
-      }
+            if constexpr (FC > kFusedChunks) continue;  // a break moves xmm to scratch
+            else break;
+          }
           const int c = min(tid + i * (int)blockDim.x, xm_nch - 1);
           if (c >= m * cpr && c < (m + 1) * cpr) {
             float v[NE];
@@ -479,8 +479,9 @@ __global__ __launch_bounds__(kFastMaxWaves * 64) void gemv_fast_kernel(GemvArgs 
       tok_s = fmaxf(mx, 1e-8f) / 127.0f;
     }
     if constexpr (kQXL) {
-      // the s8 values xq - 128 of this thread's chunks (      // one fma and one pack per value), 16 / EB values per chunk; per-token:
-      // clamp(rne(x / s), -127, 127), the row quantizer's values
+      // the s8 values xq - 128 of this thread's chunks (one fma and one pack
+      // per value), 16 / EB values per chunk; per-token: clamp(rne(x / s), -127,
+      // 127), the row quantizer's values
       const int cpr = K * EB / 16;
       const auto quant_store = [&](const u32x4& raw, int c) {
         const int m = c / cpr;

@@ -45,7 +45,8 @@ int64_t sample_workspace_bytes(int64_t M);
 int launch_sample_rows(const float* x, int64_t M, int64_t V, int64_t ld, float T, int64_t top_k, float top_p,
                        const float* u, int64_t* tokens, void* ws, hipStream_t st);
 
-// True when the streaming GEMV kernels take this M and K (otherwise the GEMM).
+// True when the streaming GEMV kernels take this M and K (otherwise the GEMM):
+// up to 32 rows, and int8-dyn up to 16 of any x.
 bool gemv_supports(int64_t M, int64_t K, bool w8a8, int xt);
 // The general GEMV's configuration for an [M, K] input (sbq_gemv_config):
 // info[0..8] = ok, row tiles of x, weight tiles per group, K tiles per wave,

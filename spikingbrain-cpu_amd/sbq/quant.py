@@ -230,8 +230,8 @@ def unpack(packed: torch.Tensor, N: int, K: int) -> torch.Tensor:
 
 def w8_workspace(M: int, K: int, device: torch.device, dtype: torch.dtype = torch.float16,
                  N: int | None = None) -> torch.Tensor:
-    """Scratch for linear_w8's prefill path with [M, K] activations of `dtype`;
-    with N, also the split-K partials of shapes that need them."""
+    """Scratch for linear_w8's prefill path with [M, K] activations of `dtype`,
+    or its padded rows of ragged K; with N, also the split-K partials of shapes that need them."""
     L = _lib.load()
     n = L.sbq_w8_workspace_bytes(M, K, _code(dtype)) if N is None else L.sbq_linear_workspace_bytes(
         M, N, K, _code(dtype), 0)
@@ -243,9 +243,10 @@ def linear_w8(x2: torch.Tensor, packed: torch.Tensor, scale: torch.Tensor, bias:
               workspace: torch.Tensor | None = None) -> torch.Tensor:
     """y = (x2 @ q^T) * scale (+ bias) for x2 [M, K] on the GPU.
 
-    Prefill-sized inputs (M > 16) get the scratch of the fastest GEMM path
-    (row sums; staged fp16 planes for fp32 / bf16 activations) unless the
-    caller passes one; the library itself never allocates."""
+    Prefill-sized inputs (M > 16) and those of ragged K get the scratch of the
+    fastest path (row sums; staged fp16 planes for fp32 / bf16 activations;
+    rows of whole K tiles) unless the caller passes one; the library itself
+    never allocates."""
     x2 = _as_activation(x2)
     M, K = x2.shape
     y = out if out is not None else torch.empty((M, N), dtype=out_dtype, device=x2.device)
@@ -270,9 +271,9 @@ def linear_w8_grouped(xs, packeds, scales, biases, Ns, out_dtype: torch.dtype = 
     ys[i] = linear_w8(xs[i], packeds[i], scales[i], biases[i], Ns[i]).
 
     All xs are [M, K] GPU tensors of one dtype and device, all outputs one
-    dtype.  Decode shapes (M <= 16) run as a single GEMV launch over the
-    summed rows (the per-launch ramp and tail paid once); other shapes run one
-    by one.  Results can differ from separate calls in the fp32 summation
+    dtype.  Decode shapes (M <= 16, K % 64 == 0) run as a single GEMV launch
+    over the summed rows (the per-launch ramp and tail paid once); other shapes
+    run one by one.  Results can differ from separate calls in the fp32 summation
     order.  More than MAX_GROUP linears are split into groups."""
     return _run_grouped("linear_w8_grouped", xs, packeds, scales, None, biases, Ns, out_dtype, outs, None)
 
@@ -284,8 +285,10 @@ def linear_w8a8_grouped(xs, packeds, scales, colsums, biases, Ns, out_dtype: tor
     Ns[i]), each x quantized with its own (s_x, zp).
 
     Shapes as in linear_w8_grouped.  Decode shapes whose x fits the fused
-    GEMV run as one launch; others run one by one, sharing `workspace`
-    (default: allocated for [M, K]).  Bit-exact with separate calls."""
+    GEMV run as one launch; larger decode inputs as two, all quantized first,
+    when `workspace` holds a share of w8a8_workspace(M, K) bytes for each (the
+    default does); others run one by one, sharing it.  Bit-exact with separate
+    calls."""
     return _run_grouped("linear_w8a8_grouped", xs, packeds, scales, colsums, biases, Ns, out_dtype, outs, workspace)
 
 
