@@ -31,13 +31,14 @@
 // the logits (608 KB at V = 151936) are read from L2 three times.  Measured
 // in a HIP graph at V = 151936 on one box, against one launch per 8 key bits of
 // each cut over the whole row (7 launches with top-p, 10 with top-k as well): one
-// row of a language model's logits, top-p 34.3 -> 21.5 us, top-k 50 and top-p 51.0
-// -> 25.5, no cut 14.1 -> 12.4; eight rows, both cuts 68 -> 34.8.  Per launch at one
-// row: 3.1 (maximum), 4.9, 5.2, 6.1 us.  Bins of equal width over the row's range
-// took 20.5, 23.6 and 30.6 us there, but 390 (both cuts 470) on a flat row with one
-// far or masked token; between samples such rows take 26 and 28, and no row of 19
+// row of a language model's logits, top-p 35.0 -> 20.7 us, top-k 50 and top-p 51.2
+// -> 24.4, no cut 14.1 -> 12.3; eight rows, both cuts 67.2 -> 31.9.  Per launch at one
+// row: 3.2 (maximum), 4.6, 4.8, 6.0 us.  Bins of equal width over the row's range
+// took 20.4, 24.0 and 30.1 us there, but 390 (both cuts 470) on a flat row with one
+// far or masked token; between samples such rows take 26 and 27, and no row of 19
 // kinds (masked, clustered, tied, sorted) more than the radix launches did (top-p
-// 38 at most).  512 bins: 256 and 1024 of equal width ran within 2% at one row;
+// 38 at most).  Over many rows the vector units bound the bins launch (eight rows:
+// 7.4 us, equal bins 5.8): the lookup is a fifth of a token's 100 instructions.  512 bins: 256 and 1024 of equal width ran within 2% at one row;
 // 1024 was 25% slower at 16 rows (more atomics per slice).
 //
 // No workgroup waits for another: what a launch needs from the one before it
@@ -125,62 +126,94 @@ __device__ __forceinline__ float samp_unkey(uint32_t k) {
 
 __device__ __forceinline__ float samp_z(const SampArgs& a, const float* row, int i) { return row[i] / a.T; }
 
-// fixed-point mass exp(z - m) * 2^40, truncated: the 24-bit significand of
-// the float exp(z - m) <= 1, shifted (its exponent field is at most 127)
+// fixed-point mass exp(z - m) * 2^40, truncated: exp(z - m) <= 1 in units of
+// 2^-16, then the rest of them in units of 2^-24 (every step but the two
+// truncations exact)
 __device__ __forceinline__ uint64_t samp_efix(float z, float m) {
-  const uint32_t b = __float_as_uint(expf(z - m));
-  const int sh = (int)(b >> 23) - (150 - 40);
-  const uint64_t s = (b & 0x7fffffu) | 0x800000u;
-  return sh >= 0 ? s << sh : s >> min(-sh, 63);
+  const float f = expf(z - m) * 65536.0f;
+  const uint32_t hi = (uint32_t)f, lo = (uint32_t)((f - (float)hi) * 16777216.0f);
+  return (uint64_t)hi << 24 | lo;
 }
 
-// The bins of a row: 64 sampled z, sorted, give 15 splits of the values into
+// The bins of a row: 64 sampled z, sorted, give 14 splits of the values into
 // intervals of a few 64ths of the tokens each, whatever their distribution
 // (equal steps of max - z put most of a flat row beside one far token into one
 // bin, and one workgroup then read the row again per pass: 390 us at V =
-// 151936).  From the top: kSampTop equal steps of the interval above the first
-// split, where sampled decoding cuts; then per split one bin of the tokens
-// equal to it (ties) and kSampSteps steps of the interval below it; the last bin
-// the tokens without mass, and only those.  Steps end at `low`, below which no
-// token has mass.  Comparisons, rounding and truncation are monotone, so a
-// larger z never has a larger bin, and equal z share one.
-constexpr int kSampSplits = 15;
-constexpr int kSampTop = 200, kSampSteps = 19;
-static_assert(kSampTop + (kSampSteps + 1) * kSampSplits < kSampBins, "the intervals' bins and the last one");
+// 151936).  Interval i lies below split i - 1 (the maximum); its first bin holds
+// the tokens equal to that (ties), the rest are equal steps down to split i
+// (in the last interval to `low`, the lowest z that can have mass): kSampTop of
+// them in the first interval, where sampled decoding cuts, kSampSteps in the
+// others.  A last split, the largest z below max - kSampRange, leaves the last
+// bin to tokens without mass, and splits below it count as it.  Comparisons,
+// rounding and ceil are monotone, so a larger z never has a larger bin, and
+// equal z share one.
+constexpr int kSampSplits = 14;
+constexpr int kSampTop = 200, kSampSteps = 21;
+static_assert(kSampSplits == 14, "the last split is the 15th, of a search in four steps");
+static_assert(kSampTop + 1 + (kSampSteps + 1) * kSampSplits < kSampBins, "the intervals' bins and the last one");
 // Split t of the row is sample samp_split(t), finer towards the top.
-__device__ __forceinline__ int samp_split(int t) { return t < 2 ? t : (t < 10 ? 4 * t - 5 : 5 * t - 14); }
+__device__ __forceinline__ int samp_split(int t) {
+  return t < 2 ? t : (t < 4 ? 4 * t - 5 : (27 * t - 46) / 5);  // 0, 1, 3, 7, 12 ... 61
+}
 struct SampTable {
-  float s[kSampSplits + 1];  // the splits, largest first
-  // per interval: its top (the split above it, the maximum), steps per unit of z, the split below it
-  f32x4 from[kSampSplits + 1];
+  float s[16];     // the splits, largest first
+  f32x4 from[16];  // per interval: its top, steps per unit of z, steps, (int bits) first bin
 };
+// (Splits compared two levels deep or all at once, from scalar registers, and four
+// tokens looked up together were slower: 0.3 to 1.5 us of the bins launch at
+// eight rows.)
 struct SampLook {
   const SampTable* tb;
-  float m;
   __device__ __forceinline__ int bin(float z) const {
-    int i = 0;  // splits above z
+    int i = 0;  // splits at or above z
 #pragma unroll
-    for (int step = 8; step > 0; step >>= 1) i += tb->s[i + step - 1] > z ? step : 0;
+    for (int step = 8; step > 0; step >>= 1) i += tb->s[i + step - 1] >= z ? step : 0;
     const f32x4 f = tb->from[i];
-    const int n = i == 0 ? kSampTop : kSampSteps;
-    int b = (int)fminf((f[0] - z) * f[1], (float)(n - 1));
-    if (i < kSampSplits && z == f[2]) b = n;  // after the interval's steps
-    b += i == 0 ? 0 : kSampTop + 1 + (kSampSteps + 1) * (i - 1);
-    return m - z <= kSampRange ? b : kSampBins - 1;
+    return (int)__float_as_uint(f[3]) + (int)__builtin_ceilf(fminf((f[0] - z) * f[1], f[2]));
   }
 };
 
-__device__ __forceinline__ void samp_table(const uint8_t* w, float m, float low, SampTable* tb) {
-  const int t = threadIdx.x;
-  if (t <= kSampSplits) {
-    const float* s = (const float*)(w + SampRow::kSplit);
-    const float top = t == 0 ? m : s[samp_split(t - 1)], end = t < kSampSplits ? s[samp_split(t)] : low;
-    const float width = top - fmaxf(end, low);
-    tb->s[t] = end;
-    const float steps = width > 0.0f ? (float)(t == 0 ? kSampTop : kSampSteps) / fmaxf(width, 1e-30f) : 0.0f;
-    tb->from[t] = (f32x4){top, steps, end, 0.0f};
+// This lane's split (lane t: split t), for samp_table: one load, to be issued
+// ahead of what the caller still has to find out.
+__device__ __forceinline__ float samp_lane_split(const uint8_t* w) {
+  return ((const float*)(w + SampRow::kSplit))[samp_split(min((int)(threadIdx.x & 63), kSampSplits - 1))];
+}
+// v of the lane before, within each 16 lanes
+__device__ __forceinline__ float samp_lane_before(float v) {
+  return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), 0x111, 0xf, 0xf, false));
+}
+
+// (one wave: a lane per interval)
+__device__ __forceinline__ void samp_table(float lane_split, float m, float low, SampTable* tb) {
+  const int t = threadIdx.x & 63;
+  const float bound = samp_unkey(samp_key(m - kSampRange) - 1u);
+  const float split = t < kSampSplits ? fmaxf(lane_split, bound) : bound, before = samp_lane_before(split);
+  if (t < 16) {
+    const float top = t == 0 ? m : before, n = t == 0 ? (float)kSampTop : (t <= kSampSplits ? (float)kSampSteps : 0.0f);
+    const float width = top - fmaxf(split, low);
+    const int base = t == 0 ? 0 : (t <= kSampSplits ? kSampTop + 1 + (kSampSteps + 1) * (t - 1) : kSampBins - 1);
+    tb->s[t] = split;
+    tb->from[t] = (f32x4){top, width > 0.0f ? n / fmaxf(width, 1e-30f) : 0.0f, n, __uint_as_float((uint32_t)base)};
   }
 }
+
+// Tokens whose bin is sure to lie after `last`, without the lookup: those of a
+// later interval, or past its step in bin()'s own arithmetic (the list launch,
+// which needs only the others: 5.4 -> 4.8 us at one row, 7.9 -> 6.2 at eight).
+struct SampAfter {
+  float top, steps, end, step;
+  __device__ __forceinline__ SampAfter(const SampTable* tb, int last)
+      : top(0.0f), steps(0.0f), end(-INFINITY), step(INFINITY) {
+    if (last < 0 || last >= kSampBins - 1) return;  // uniform: no bins, or none after it
+    const int q = last - (kSampTop + 1), i = q < 0 ? 0 : 1 + q / (kSampSteps + 1);
+    const int j = q < 0 ? last : q % (kSampSteps + 1);  // 0: the ties
+    top = tb->from[i][0];
+    steps = tb->from[i][1];
+    end = tb->s[i];
+    if (j < (i == 0 ? kSampTop : kSampSteps)) step = (float)j;
+  }
+  __device__ __forceinline__ bool operator()(float z) const { return z <= end || (top - z) * steps > step; }
+};
 
 // The top-p bound on the mass above a token: mass_above < top_p * S (S: the
 // mass top-k keeps) <=> mass_above < thr, for integer masses.
@@ -205,6 +238,18 @@ struct SampTokens {
   __device__ __forceinline__ void load(int b) {
 #pragma unroll
     for (int u = 0; u < kSampUnroll; ++u) x[u] = row[max(min(b + u * n, i1 - 1), 0)];
+  }
+  // f(z[kSampUnroll], b) for each round: the tokens b + u n, those past the
+  // range repeating its last one
+  template <typename F>
+  __device__ __forceinline__ void rounds(float T, F f) {
+    for (int b = i0 + t; b < i1; b += kSampUnroll * n) {
+      if (b != i0 + t) load(b);
+      float z[kSampUnroll];
+#pragma unroll
+      for (int u = 0; u < kSampUnroll; ++u) z[u] = x[u] / T;
+      f(z, b);
+    }
   }
   // f(i, z) for each token
   template <typename F>
@@ -281,6 +326,17 @@ __device__ __forceinline__ SampScale samp_scale(const SampArgs& a, const uint8_t
   return s;
 }
 
+// The same, and with TABLE the bins' table, by one wave for its workgroup (all 16
+// waves reading the row's three or four lines: the bins launch 0.4 us longer at
+// eight rows, 0.3 at one).
+template <bool TABLE>
+__device__ __forceinline__ void samp_scale_table(const SampArgs& a, const uint8_t* w, SampScale* out, SampTable* tb) {
+  const float split = TABLE ? samp_lane_split(w) : 0.0f;
+  const SampScale sc = samp_scale(a, w);
+  if constexpr (TABLE) samp_table(split, sc.m, sc.low, tb);
+  if ((threadIdx.x & 63) == 0) *out = sc;
+}
+
 // The row's 64 samples, one in each 64th of the row (the place within it by the
 // golden ratio), sorted: each wave ranks the lanes' samples against its four,
 // one adds up the ranks.
@@ -318,10 +374,16 @@ __global__ __launch_bounds__(kSampThreads) void samp_max_kernel(SampArgs a) {
   const float sample = sort ? samp_sample(a) : 0.0f;
   float mx = -INFINITY, mn = INFINITY;
   bool nan = false;
-  tok.each(a.T, [&](int, float z) {
-    nan |= z != z;
-    const float top = fmaxf(mx, z);
-    mn = fminf(samp_near(mx, top, mn), samp_near(z, top, z));
+  tok.rounds(a.T, [&](const float (&z)[kSampUnroll], int) {
+    float top = mx;
+#pragma unroll
+    for (int u = 0; u < kSampUnroll; ++u) {
+      nan |= z[u] != z[u];
+      top = fmaxf(top, z[u]);
+    }
+    mn = samp_near(mx, top, mn);
+#pragma unroll
+    for (int u = 0; u < kSampUnroll; ++u) mn = fminf(mn, samp_near(z[u], top, z[u]));
     mx = top;
   });
   float top = wave_max(mx);
@@ -360,23 +422,24 @@ __global__ __launch_bounds__(kSampThreads) void samp_bins_kernel(SampArgs a) {
   __shared__ uint64_t H[P ? kSampBins * kSampCopies : 1];
   __shared__ uint32_t C[K ? kSampBins * kSampCopies : 1];
   __shared__ SampTable tb;
+  __shared__ SampScale sc;
   uint8_t* w = samp_row_ws(a);
   const int i0 = blockIdx.x * a.per, i1 = min(i0 + a.per, a.V);
   SampTokens tok(a.x + (int64_t)blockIdx.y * a.ld, i0, i1, threadIdx.x, kSampThreads);
+  if (threadIdx.x < 64) samp_scale_table<true>(a, w, &sc, &tb);
   for (int i = threadIdx.x; i < kSampBins * kSampCopies; i += kSampThreads) {
     if constexpr (P) H[i] = 0;
     if constexpr (K) C[i] = 0;
   }
-  const SampScale sc = samp_scale(a, w);
-  if (!sc.valid) return;
-  samp_table(w, sc.m, sc.low, &tb);
   __syncthreads();
-  const SampLook look{&tb, sc.m};
+  if (!sc.valid) return;
+  const float m = sc.m;
+  const SampLook look{&tb};
   const int copy = threadIdx.x & (kSampCopies - 1);
   tok.each(a.T, [&](int, float z) {
     const int at = look.bin(z) * kSampCopies + copy;
     if constexpr (P) {
-      const uint64_t f = samp_efix(z, sc.m);
+      const uint64_t f = samp_efix(z, m);
       if (f) atomicAdd((unsigned long long*)&H[at], (unsigned long long)f);
     }
     if constexpr (K) atomicAdd(&C[at], 1u);
@@ -403,7 +466,7 @@ __global__ __launch_bounds__(kSampThreads) void samp_bins_kernel(SampArgs a) {
 // The undecided bins of the row from its filled bins (identical in every
 // workgroup).  Thread b < kSampBins holds bin b.
 template <bool K, bool P>
-__device__ void samp_cuts(const SampArgs& a, const SampScale& sc, uint64_t f, uint32_t c, SampHead* h, uint64_t* red) {
+__device__ void samp_cuts(const SampArgs& a, uint64_t f, uint32_t c, SampHead* h, uint64_t* red) {
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
   constexpr int W = kSampBins / 64;
   uint64_t fi = P ? wave_prefix(f) : 0;
@@ -412,8 +475,7 @@ __device__ void samp_cuts(const SampArgs& a, const SampScale& sc, uint64_t f, ui
     red[wv] = fi;
     red[W + wv] = ci;
   }
-  if (t == 0) *h = SampHead{1, sc.m, sc.low, -1, 0, 1, 0, 0, 0, 0, 0};
-  __syncthreads();
+  __syncthreads();  // (the caller's *h as well)
   uint64_t total = 0;
 #pragma unroll
   for (int i = 0; i < W; ++i) {
@@ -465,6 +527,7 @@ __global__ __launch_bounds__(kSampThreads) void samp_list_kernel(SampArgs a) {
   __shared__ uint64_t red[2 * (kSampBins / 64) + 1], sum[kSampWaves];
   __shared__ uint32_t num, kmin, kmax;
   __shared__ SampTable tb;
+  __shared__ SampScale sc;
   uint8_t* w = samp_row_ws(a);
   const int i0 = blockIdx.x * a.per, i1 = min(i0 + a.per, a.V);
   SampTokens tok(a.x + (int64_t)blockIdx.y * a.ld, i0, i1, threadIdx.x, kSampThreads);
@@ -474,34 +537,35 @@ __global__ __launch_bounds__(kSampThreads) void samp_list_kernel(SampArgs a) {
     if constexpr (P) f = ((const uint64_t*)(w + SampRow::kMass))[threadIdx.x];
     if constexpr (K) c = ((const uint32_t*)(w + SampRow::kCount))[threadIdx.x];
   }
-  const SampScale sc = samp_scale(a, w);
-  if (!sc.valid) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) ((SampHead*)(w + SampRow::kHead))->valid = 0;
-    return;
-  }
+  if (threadIdx.x < 64) samp_scale_table<K || P>(a, w, &sc, &tb);
   if (threadIdx.x == 0) {
     num = 0;
     kmin = ~0u;
     kmax = 0;
+    h = SampHead{1, sc.m, sc.low, -1, 0, 1, 0, 0, 0, 0, 0};  // (sc: this lane's own store)
   }
-  if constexpr (K || P) {
-    samp_table(w, sc.m, sc.low, &tb);
-    samp_cuts<K, P>(a, sc, f, c, &h, red);
-  } else {
-    if (threadIdx.x == 0) h = SampHead{1, sc.m, sc.low, -1, 0, 1, 0, 0, 0, 0, 0};
+  if constexpr (K || P)
+    samp_cuts<K, P>(a, f, c, &h, red);
+  else
     __syncthreads();
+  if (!sc.valid) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) ((SampHead*)(w + SampRow::kHead))->valid = 0;
+    return;
   }
-  const SampLook look{&tb, sc.m};
+  const float m = sc.m;
+  const SampLook look{&tb};
   const int lo = h.lo, hi = h.hi, kbin = h.kbin;
+  const SampAfter after(&tb, K || P ? max(lo <= hi ? hi : -1, kbin) : -1);  // most of a usual row
   // tokens above the first undecided bin are kept, whatever the keys say
   const int first = lo <= hi ? lo : (kbin >= 0 ? kbin : kSampBins);
   uint32_t* list = (uint32_t*)(w + SampRow::kList) + blockIdx.x * kSampList;
   uint64_t part = 0;
   uint32_t k0 = ~0u, k1 = 0;
   tok.each(a.T, [&](int, float z) {
+    if ((K || P) && after(z)) return;
     const int b = K || P ? look.bin(z) : 0;
     if (b < first) {
-      part += samp_efix(z, sc.m);
+      part += samp_efix(z, m);
     } else if (b <= hi || b == kbin) {
       const uint32_t at = atomicAdd(&num, 1u), k = samp_key(z);
       if (at < (uint32_t)kSampList) list[at] = k;
@@ -542,12 +606,10 @@ struct SampUndecided {
   int slice[kFlat];  // -1: none
   uint32_t num[S];   // tokens of this wave's slices, not flat
   uint64_t longer;   // slices to read again
-  const SampTable* tb;
 
   // lk, ls, lc: kFlat * kSampThreads words / bytes and kSampMaxBlocks words of LDS
   __device__ __forceinline__ void load(const SampArgs& a, const uint8_t* w, float m, uint32_t* lk, uint8_t* ls,
-                                       uint32_t* lc, const SampTable* table) {
-    tb = table;
+                                       uint32_t* lc) {
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
     const uint32_t* lists = (const uint32_t*)(w + SampRow::kList);
     uint32_t nl = ((const uint32_t*)(w + SampRow::kNum))[min(lane, a.G - 1)], k[S];
@@ -597,7 +659,7 @@ struct SampUndecided {
   // f(key, mass, n, slice) for the keys in [lo, hi], n tokens of that mass each
   template <typename F>
   __device__ __forceinline__ void each(const SampArgs& a, const uint8_t* w, const float* row, const SampHead& h,
-                                       uint32_t lo, uint32_t hi, F f) const {
+                                       const SampLook& look, uint32_t lo, uint32_t hi, F f) const {
     if (flat) {
 #pragma unroll
       for (int i = 0; i < kFlat; ++i)
@@ -619,7 +681,6 @@ struct SampUndecided {
         if (lane == 0) one(list[0], n & ~kSampTied, g);
       }
     }
-    const SampLook look{tb, h.m};
 #pragma unroll 1
     for (uint64_t rest = longer; rest; rest &= rest - 1) {
       const int g = __ffsll((long long)rest) - 1, i1 = min((g + 1) * a.per, a.V);
@@ -644,7 +705,7 @@ constexpr int kCutStride = 256 + 2;  // copies of one range lie in different ban
 constexpr int kCutWords = kCutCopies * kCutStride;
 template <bool MASS>
 __device__ __forceinline__ uint32_t samp_descend(const SampArgs& a, const uint8_t* w, const float* row, const SampHead& h,
-                                 const SampUndecided& und, uint32_t lo, uint32_t hi, uint64_t& rest, uint64_t thr,
+                                 const SampUndecided& und, const SampLook& look, uint32_t lo, uint32_t hi, uint64_t& rest, uint64_t thr,
                                  uint64_t* H, uint64_t* bc) {
   const int t = threadIdx.x, lane = t & 63;
   uint64_t* const Hc = H + (lane & (kCutCopies - 1)) * kCutStride;
@@ -652,7 +713,7 @@ __device__ __forceinline__ uint32_t samp_descend(const SampArgs& a, const uint8_
     const int shift = max(0, 24 - (int)__clz((int)(hi - lo)));
     for (int i = t; i < kCutWords; i += kSampThreads) H[i] = 0;
     __syncthreads();
-    und.each(a, w, row, h, lo, hi, [&](uint32_t k, uint64_t f, uint32_t n, int) {
+    und.each(a, w, row, h, look, lo, hi, [&](uint32_t k, uint64_t f, uint32_t n, int) {
       atomicAdd((unsigned long long*)&Hc[(k - lo) >> shift], (unsigned long long)(MASS ? f * n : n));
     });
     __syncthreads();
@@ -721,6 +782,7 @@ __global__ __launch_bounds__(kSampThreads) void samp_draw_kernel(SampArgs a) {
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
   const SampHead h = *(const SampHead*)(w + SampRow::kHead);  // the whole head in one load
   const uint64_t base_g = ((const uint64_t*)(w + SampRow::kSum))[min(lane, a.G - 1)];
+  const float split = (K || P) && t < 64 ? samp_lane_split(w) : 0.0f;
   double uf = (double)a.u[row_i];
   uf = uf < 0.0 ? 0.0 : uf;
   if (!h.valid) {
@@ -736,13 +798,13 @@ __global__ __launch_bounds__(kSampThreads) void samp_draw_kernel(SampArgs a) {
       smass[t] = 0;
       stie[t] = 0;
     }
-    samp_table(w, h.m, h.low, &tb);
+    if (t < 64) samp_table(split, h.m, h.low, &tb);
     SampUndecided und;
-    und.load(a, w, h.m, lk, ls, lc, &tb);
-    const SampLook look{&tb, h.m};
+    und.load(a, w, h.m, lk, ls, lc);
+    const SampLook look{&tb};
     // lowest and highest undecided z, of the k-th token's bin and of the boundary's bins
     float k0 = INFINITY, k1 = -INFINITY, p0 = INFINITY, p1 = -INFINITY;
-    und.each(a, w, row, h, 0u, ~0u, [&](uint32_t k, uint64_t, uint32_t, int) {
+    und.each(a, w, row, h, look, 0u, ~0u, [&](uint32_t k, uint64_t, uint32_t, int) {
       const float z = samp_unkey(k);
       const int b = look.bin(z);
       if (K && b == h.kbin) {
@@ -777,21 +839,21 @@ __global__ __launch_bounds__(kSampThreads) void samp_draw_kernel(SampArgs a) {
       if (topk) {
         ktop = samp_key(wave_max(zred[1][wl]));
         uint64_t rank = (uint64_t)h.krest;
-        kth = samp_descend<false>(a, w, row, h, und, samp_key(wave_min(zred[0][wl])), ktop, rank, 0, H, bck);
+        kth = samp_descend<false>(a, w, row, h, und, look, samp_key(wave_min(zred[0][wl])), ktop, rank, 0, H, bck);
       }
     }
     if constexpr (P) {
       if (topk) {
         uint64_t part = 0;
-        und.each(a, w, row, h, kth, ktop, [&](uint32_t, uint64_t f, uint32_t n, int) { part += f * n; });
+        und.each(a, w, row, h, look, kth, ktop, [&](uint32_t, uint64_t f, uint32_t n, int) { part += f * n; });
         S = h.kabove + samp_block_sum_u64(part, red);
       }
       uint64_t above = h.labove;
       const uint64_t thr = samp_thr(a.top_p, S);
       const uint32_t plo = samp_key(wave_min(zred[2][wl])), phi = samp_key(wave_max(zred[3][wl]));
-      tkey = samp_descend<true>(a, w, row, h, und, max(plo, kth), phi, above, thr, H, bcp);
+      tkey = samp_descend<true>(a, w, row, h, und, look, max(plo, kth), phi, above, thr, H, bcp);
       // the tokens of the boundary key per slice, and how many of them the rule keeps
-      und.each(a, w, row, h, tkey, tkey, [&](uint32_t, uint64_t, uint32_t n, int g) { atomicAdd(&stie[g], (int)n); });
+      und.each(a, w, row, h, look, tkey, tkey, [&](uint32_t, uint64_t, uint32_t n, int g) { atomicAdd(&stie[g], (int)n); });
       __syncthreads();
       const uint64_t ties = wave_total((uint32_t)stie[lane]);
       const uint64_t f0 = samp_efix(samp_unkey(tkey), h.m), need = thr - above;
@@ -809,7 +871,7 @@ __global__ __launch_bounds__(kSampThreads) void samp_draw_kernel(SampArgs a) {
     // the kept mass of each slice's undecided tokens: those from the cut up
     // (boundary ties apart while tf is set)
     const uint32_t lim = max(kth, tkey);
-    und.each(a, w, row, h, lim, ~0u, [&](uint32_t k, uint64_t f, uint32_t n, int g) {
+    und.each(a, w, row, h, look, lim, ~0u, [&](uint32_t k, uint64_t f, uint32_t n, int g) {
       if (!(tf && k == tkey)) atomicAdd((unsigned long long*)&smass[g], (unsigned long long)(f * n));
     });
   }
