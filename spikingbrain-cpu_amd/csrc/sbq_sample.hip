@@ -38,8 +38,9 @@
 // far or masked token; between samples such rows take 26 and 27, and no row of 19
 // kinds (masked, clustered, tied, sorted) more than the radix launches did (top-p
 // 38 at most).  Over many rows the vector units bound the bins launch (eight rows:
-// 7.4 us, equal bins 5.8): the lookup is a fifth of a token's 100 instructions.  512 bins: 256 and 1024 of equal width ran within 2% at one row;
-// 1024 was 25% slower at 16 rows (more atomics per slice).
+// 7.4 us, equal bins 5.8): the lookup is a fifth of a token's 100 instructions.
+// 512 bins: 256 and 1024 of equal width ran within 2% at one row; 1024 was 25%
+// slower at 16 rows (more atomics per slice).
 //
 // No workgroup waits for another: what a launch needs from the one before it
 // (maximum, bins) every workgroup derives for itself.  Rows are independent

@@ -1080,6 +1080,12 @@ class FusedLinear(_Fp32Buffers, nn.Module):
         self._memo_out = None
         self._memo_taken = set()
 
+    def __setstate__(self, state):
+        super().__setstate__(state)
+        if "_parts" not in self._buffers:  # saved whole before layers had the table: their outputs are sliced
+            self.register_buffer("_parts", None, persistent=False)
+            self._pstart = []
+
     def forward(self, x: torch.Tensor) -> tuple[torch.Tensor, ...]:
         _check_in_features(x, self.in_features)
         shape = x.shape

@@ -980,6 +980,23 @@ def test_fuse_linears_rejects_mixed_parts(dev):
 # ---------------------------------------------------------------------------
 # greedy token selection on the GPU (engine.py:30-31)
 # ---------------------------------------------------------------------------
+@pytest.mark.parametrize("cls", ["Int8Linear", "DynamicInt8Linear"])
+def test_fused_layer_saved_whole_before_the_parts_table(dev, cls):
+    """A fused layer pickled without the column table (as layers once were)
+    loads and slices its outputs: the same values."""
+    announce(f"fused saved whole {cls}")
+    fused = quant.fuse_linears([getattr(quant, cls)(make_weights(n, 256, n).to(dev), None) for n in (64, 20)])
+    state = fused.__getstate__() if hasattr(fused, "__getstate__") else fused.__dict__
+    state = {k: v for k, v in state.items() if k != "_pstart"}
+    state["_buffers"] = {k: v for k, v in state["_buffers"].items() if k != "_parts"}
+    state["_non_persistent_buffers_set"] = state["_non_persistent_buffers_set"] - {"_parts"}
+    old = quant.FusedLinear.__new__(quant.FusedLinear)
+    old.__setstate__(state)
+    x = torch.randn(3, 256, device=dev, generator=torch.Generator(dev).manual_seed(5))
+    assert all(torch.equal(a, b) for a, b in zip(old(x), fused(x)))
+    assert all(torch.equal(a, b) for a, b in zip(old(x[:1]), fused(x[:1])))
+
+
 def test_greedy_tokens_match_torch_argmax(dev):
     announce("greedy tokens")
     g = torch.Generator().manual_seed(3)
