@@ -38,7 +38,7 @@
 // far or masked token; between samples such rows take 26 and 27, and no row of 19
 // kinds (masked, clustered, tied, sorted) more than the radix launches did (top-p
 // 38 at most).  Over many rows the vector units bound the bins launch (eight rows:
-// 7.4 us, equal bins 5.8): the lookup is a fifth of a token's 100 instructions.
+// 7.4 us, equal bins 5.8): a token takes 62 instructions, 38 with equal bins.
 // 512 bins: 256 and 1024 of equal width ran within 2% at one row; 1024 was 25%
 // slower at 16 rows (more atomics per slice).
 //
@@ -339,9 +339,11 @@ __device__ __forceinline__ void samp_scale_table(const SampArgs& a, const uint8_
 }
 
 // The row's 64 samples, one in each 64th of the row (the place within it by the
-// golden ratio), sorted: each wave ranks the lanes' samples against its four,
-// one adds up the ranks.
-constexpr int kSampRanks = 64 / kSampWaves;
+// golden ratio), sorted: each of four waves ranks the lanes' samples against
+// its sixteen, one adds up the ranks.  (On cold logits the launch takes 3.7 us
+// so, 4.0 with four ranks in each of 16 waves, which all load the 64
+// scattered samples, and 4.2 with two waves.)
+constexpr int kSampRankWaves = 4, kSampRanks = 64 / kSampRankWaves;
 __device__ __forceinline__ float samp_sample(const SampArgs& a) {
   const uint32_t lane = threadIdx.x & 63;
   const uint64_t V = (uint64_t)a.V, turn = (uint64_t)(lane * 2654435769u) * V >> 32;
@@ -362,9 +364,9 @@ __device__ __forceinline__ int samp_rank(float z) {
 // slice; workgroup 0 clears the row's bins and sorts its samples.
 __global__ __launch_bounds__(kSampThreads) void samp_max_kernel(SampArgs a) {
   __shared__ float smx[kSampWaves], smn[kSampWaves];
-  __shared__ int snan[kSampWaves], ranks[kSampWaves][64];
+  __shared__ int snan[kSampWaves], ranks[kSampRankWaves][64];
   uint8_t* w = samp_row_ws(a);
-  const bool sort = blockIdx.x == 0 && (a.k > 0 || a.top_p > 0.0);  // uniform
+  const bool sort = blockIdx.x == 0 && threadIdx.x < kSampRankWaves * 64 && (a.k > 0 || a.top_p > 0.0);
   const int i0 = blockIdx.x * a.per, i1 = min(i0 + a.per, a.V);
   SampTokens tok(a.x + (int64_t)blockIdx.y * a.ld, i0, i1, threadIdx.x, kSampThreads);
   if (blockIdx.x == 0 && threadIdx.x < kSampBins) {
@@ -411,7 +413,7 @@ __global__ __launch_bounds__(kSampThreads) void samp_max_kernel(SampArgs a) {
   } else if (sort && threadIdx.x < 128) {
     int rank = 0;
 #pragma unroll
-    for (int i = 0; i < kSampWaves; ++i) rank += ranks[i][lane];
+    for (int i = 0; i < kSampRankWaves; ++i) rank += ranks[i][lane];
     ((float*)(w + SampRow::kSplit))[min(rank, 63)] = sample;  // (a NaN: the row is invalid)
   }
 }
