@@ -138,14 +138,14 @@ __global__ __launch_bounds__(256) void zero_ints_kernel(int32_t* __restrict__ ou
 // HBM bound: one read of w, one write of each output.  Measured (whole call of
 // a module's load, eager, against a scalar quantizer, a byte-wise repack and a
 // column-sum launch, with the int8 rows written and read twice between them):
-// bf16 9728 x 2560 112 -> 25 us, 24576 x 4096 407 -> 70 us (4.3 TB/s),
-// 151936 x 2560 1661 -> 237 us (4.9 TB/s); with the int8 rows kept 26 / 96 /
-// 302 us; fp32 9728 x 2560 135 -> 26; ragged bf16 9721 x 2555 101 -> 39.  int8
+// bf16 9728 x 2560 112 -> 22 us, 24576 x 4096 407 -> 65 us (4.7 TB/s),
+// 151936 x 2560 1661 -> 213 us (5.5 TB/s); with the int8 rows kept 24 / 89 /
+// 300 us; fp32 9728 x 2560 135 -> 24; ragged bf16 9721 x 2555 101 -> 37.  int8
 // rows alone, K over several workgroups where there are few row tiles (graph):
 // 16 x 65536 44 -> 3.6 us, 64 x 12288 10.3 -> 3.9, 300 x 9728 9.0 -> 4.4, with
 // their column sums 44 -> 6.4, 10.5 -> 5.5, 9.2 -> 6.1.  16
 // waves per workgroup: 20-45% slower except at K = 9728 (5% faster); holding
-// 24 chunks spilled (2560 x 9728: 74 us, re-reading 39).
+// 24 chunks spilled (2560 x 9728: 74 us, re-reading 32).
 template <int WT, int C>
 __global__ __launch_bounds__(512) void pack_weight_kernel(const uint8_t* __restrict__ w, int64_t N, int64_t K,
                                                           int64_t ldw, float* __restrict__ scale,
